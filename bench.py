@@ -86,24 +86,27 @@ def cpu_sample_case(workload, case):
 
 def launch_plan(prm, nstages):
     """Launches per time step by profiling group, as Solver::step issues them:
-    {group: (launches, kernel name)}.  FP32 inviscid M1/M2 runs every stage
-    (but a residual stage 0) as one stage_fused32 launch; other paths run
+    {group: (launches, kernel name up to the parameters that depend on the
+    mesh)}.  Inviscid M1/M2 runs every stage (but a residual stage 0) as one
+    stage_fused32 / stage_fused64 launch; other paths run
     grad_vis (when it has work), face_flux and cell_update per stage.  The
     last stage's launch also forms the CFL/dt block extrema, except on the
     FP64 3D path, where they keep a launch of their own.  Their final
     reduction is one single-block launch, or, inside a run that steps
-    again, one extra block of the next step's first FP32 launch."""
+    again, one extra block of the next step's first launch (one-launch
+    stages and FP32)."""
     D, S = prm["dim"], prm["solver"]
     fp32 = prm["precision"] == 32
     visc = prm["mu"] != 0.0 or not prm.get("laminar", 1)
     sfx = "32" if fp32 else ""
     mode = 0 if prm.get("adjust_dt") else 1
-    if fp32 and not visc and S < 2:
+    if not visc and S < 2:
         first = 1 if prm.get("have_res") else 0
-        plan = {"cell_update": (nstages - 1 - first, f"stage_fused32<{D}, {S}, -1>"),
-                "cell_update_cfl": (1, f"stage_fused32<{D}, {S}, {mode}>")}
+        name = "stage_fused32" if fp32 else "stage_fused64"
+        plan = {"cell_update": (nstages - 1 - first, f"{name}<{D}, {S}, -1"),
+                "cell_update_cfl": (1, f"{name}<{D}, {S}, {mode}")}
         if first:
-            plan["face_flux"] = (first, f"face_flux32<{D}, {S}, false, false>")
+            plan["face_flux"] = (first, f"face_flux{sfx}<{D}, {S}, false, false")
         return plan
     rg = S == 2 and prm.get("minmod")
     plan = {"face_flux": (nstages, f"face_flux{sfx}<{D}, {S}, {str(visc).lower()}, false>")}
@@ -281,7 +284,7 @@ def traffic_of(key, kernel):
             t = json.load(fh)
     except (OSError, ValueError):
         return None, None
-    k = t.get("kernels", {}).get(kernel)
+    k = next((v for n, v in t.get("kernels", {}).items() if n.startswith(kernel)), None)
     if t.get("workload") != key or not k:
         return None, None
     src = (f"profiles/{key}_traffic.json: rocprofv3 FETCH_SIZE x{t['fetch_factor']:.3f} + WRITE_SIZE "

@@ -357,20 +357,6 @@ struct UpdateUnroll32 {
     static constexpr int value = GatherUnroll<D>::value;
 };
 
-// Face slot storage: for each group of 64 consecutive cells (one wave's
-// cells), slot j's field f (NF fields per slot) at
-// [c / 64][j][f][c % 64], so that a wave reads one contiguous block of each
-// slot array instead of a separate strided stream per slot and field
-// (kSlotBlocked; otherwise [j][f][c]).  Arrays hold whole groups.
-constexpr bool kSlotBlocked = true;
-template <int D, int NF>
-__device__ __forceinline__ size_t slot_at(int nc, int j, int f, int c) {
-    if constexpr (kSlotBlocked)
-        return ((size_t)(c >> 6) * (GatherUnroll<D>::value * NF) + (size_t)(j * NF + f)) * 64 + (size_t)(c & 63);
-    return ((size_t)j * NF + f) * (size_t)nc + c;
-}
-inline size_t slot_array_len(int nc, int U, int NF) { return (size_t)(nc + 63) / 64 * 64 * U * NF; }
-
 // gather entry j of cell c (entry e of the list): its side, other cell,
 // weight and area vector.  SL: from the per-cell face slots for the first
 // GatherUnroll entries (streamed, no face index to chase); otherwise, and

@@ -29,8 +29,25 @@ struct KArgs {
     const int32_t *g_off, *g_ent;   // gather lists
     const int32_t *s_off, *s_ent;   // slot lists
     const int32_t *ghost_cell, *ghost_role;
-    const double *vinv, *sigma;
+    const double *vinv;
+    const double *sigma;            // nullptr where every cell's sponge sigma is zero
     const double *smag;             // [nc] Smagorinsky constants, nullptr when laminar
+    // per-cell face slots of the one-launch stage (nullptr until built), the
+    // first GatherUnroll gather entries of each cell, slot_at places them:
+    // either packed words (the other cell in the low pk_shift bits, above
+    // them the face's record in the geometry table pk_tab) or, where the mesh
+    // has too many distinct records, keys (~other on N entries) with the
+    // face's own area vector and weight.  A slot past the cell's last entry
+    // holds the cell itself.  s_perm: 3 bits per gather entry, its position
+    // in the cell's slot list.  more_faces: some cell has entries beyond the
+    // slots.
+    const uint32_t *pk;
+    const double *pk_tab;
+    int pk_shift;
+    const int32_t *sl_nb;
+    const double *sl_S, *sl_w;
+    const int32_t *s_perm;
+    int more_faces;
     double *q;                      // cell records (q64_index), ghosts included
     double *dq;                     // [(D+2)][nc]
     double *res_cell;               // [(D+2)][nc]
@@ -89,6 +106,20 @@ struct GatherUnroll {
     static constexpr int value = D == 2 ? 4 : 6;
 };
 
+// Face slot storage: for each group of 64 consecutive cells (one wave's
+// cells), slot j's field f (NF fields per slot) at
+// [c / 64][j][f][c % 64], so that a wave reads one contiguous block of each
+// slot array instead of a separate strided stream per slot and field
+// (kSlotBlocked; otherwise [j][f][c]).  Arrays hold whole groups.
+constexpr bool kSlotBlocked = true;
+template <int D, int NF>
+__device__ __forceinline__ size_t slot_at(int nc, int j, int f, int c) {
+    if constexpr (kSlotBlocked)
+        return ((size_t)(c >> 6) * (GatherUnroll<D>::value * NF) + (size_t)(j * NF + f)) * 64 + (size_t)(c & 63);
+    return ((size_t)j * NF + f) * (size_t)nc + c;
+}
+inline size_t slot_array_len(int nc, int U, int NF) { return (size_t)(nc + 63) / 64 * 64 * U * NF; }
+
 // FP64 loads and stores of data a kernel touches once, non-temporal where
 // kStreamNT64 allows (levels as on the FP32 path: 2 the RK register, 3 the
 // new states, the face kernel's face lists and geometry, the face fluxes,
@@ -98,23 +129,23 @@ struct GatherUnroll {
 // 4.2 M-cell O-grid 5.96 -> 5.65, 1 M-cell annulus 0.880 -> 0.848.
 template <int D>
 constexpr int kStreamNT64 = 3;
-template <int D, int LEVEL, class T>
+template <int D, int LEVEL, int NT = kStreamNT64<D>, class T>
 __device__ __forceinline__ T ld64_once(const T *p) {
-    if constexpr (kStreamNT64<D> >= LEVEL) return __builtin_nontemporal_load(p);
+    if constexpr (NT >= LEVEL) return __builtin_nontemporal_load(p);
     return *p;
 }
-template <int D, int LEVEL, class T>
+template <int D, int LEVEL, int NT = kStreamNT64<D>, class T>
 __device__ __forceinline__ void st64_once(T *p, T v) {
-    if constexpr (kStreamNT64<D> >= LEVEL)
+    if constexpr (NT >= LEVEL)
         __builtin_nontemporal_store(v, p);
     else
         *p = v;
 }
 using d2v = double __attribute__((ext_vector_type(2)));
-template <int D, int LEVEL>
+template <int D, int LEVEL, int NT = kStreamNT64<D>>
 __device__ __forceinline__ void st64x2_once(double *p, double x, double y) {
     const d2v v = {x, y};
-    st64_once<D, LEVEL>(reinterpret_cast<d2v *>(p), v);
+    st64_once<D, LEVEL, NT>(reinterpret_cast<d2v *>(p), v);
 }
 
 // face f's area vector (one 16-byte load in 2D)
@@ -148,11 +179,11 @@ __device__ __forceinline__ void load_q(const KArgs &a, int i, double *q) {
     if (D == 3) q[4] = a.q[(size_t)4 * a.ntot + i];
 }
 
-template <int D>
+template <int D, int NT = kStreamNT64<D>>
 __device__ __forceinline__ void store_q(double *qv, size_t ntot, int i, const double *q) {
-    st64x2_once<D, 3>(qv + 4 * (size_t)i, q[0], q[1]);
-    st64x2_once<D, 3>(qv + 4 * (size_t)i + 2, q[2], q[3]);
-    if (D == 3) st64_once<D, 3>(qv + 4 * ntot + i, q[4]);
+    st64x2_once<D, 3, NT>(qv + 4 * (size_t)i, q[0], q[1]);
+    st64x2_once<D, 3, NT>(qv + 4 * (size_t)i + 2, q[2], q[3]);
+    if (D == 3) st64_once<D, 3, NT>(qv + 4 * ntot + i, q[4]);
 }
 
 // One cell's gradients as one record, padded to whole 16-byte words: dudx
@@ -531,6 +562,141 @@ __global__ void __launch_bounds__(256) grad_vis(KArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// Convective flux of one face (M1 cfd_v0.cpp:2589-2675, M2 1968-2023) seen
+// from one of its cells: c that cell, o the other, S pointing out of c, wc / wo
+// the weights of INTERP_LINEAR(wc, c, o) and INTERP_LINEAR(wo, o, c) (w and
+// 1 - w for the face's P, 1 - w and w for its N).  With c = P these are the
+// reference's operations; from N every product and sum is the same one with
+// both signs reversed or the two addends exchanged, so the result is P's
+// negated, bit for bit, and a cell can form its faces' fluxes without
+// selecting which side it is on.
+// ---------------------------------------------------------------------------
+template <int D>
+struct Prim64 {
+    double R, c, e;  // p / rho, speed of sound, internal energy (M2: R and e = H)
+};
+template <int D, int SOLVER>
+__device__ __forceinline__ Prim64<D> prim64(const KArgs &a, const double (&q)[D + 2]) {
+    Prim64<D> s;
+    s.R = rpsi<D>(a, q);
+    if constexpr (SOLVER == 0) {
+        const double ri = 1.0 / q[0];
+        double e = 2 * q[D + 1] * ri;
+#pragma unroll
+        for (int k = 0; k < D; k++) {
+            const double u = q[k + 1] * ri;
+            e -= u * u;
+        }
+        s.e = e * 0.5;
+        s.c = sqrt(a.gamma * s.R);
+    } else {
+        s.e = q[D + 1] / q[0] + s.R;
+        s.c = 0.0;
+    }
+    return s;
+}
+
+template <int D>
+__device__ __forceinline__ void flux_m1(const double (&qc)[D + 2], const Prim64<D> &sc, const double (&qo)[D + 2],
+                                        const Prim64<D> &so, const double (&S)[D], const double Sm, const double wc,
+                                        const double wo, double (&rhs)[D + 2]) {
+    const double rhoPos = INTERP_LINEAR(wc, qc[0], qo[0]);
+    const double rhoNeg = INTERP_LINEAR(wo, qo[0], qc[0]);
+    const double rPi = 1.0 / rhoPos, rNi = 1.0 / rhoNeg;
+    double rUP[D], rUN[D], uP[D], uN[D];
+#pragma unroll
+    for (int k = 0; k < D; k++) {
+        rUP[k] = INTERP_LINEAR(wc, qc[k + 1], qo[k + 1]);
+        rUN[k] = INTERP_LINEAR(wo, qo[k + 1], qc[k + 1]);
+    }
+    const double eP = INTERP_LINEAR(wc, sc.e, so.e), eN = INTERP_LINEAR(wo, so.e, sc.e);
+    const double RP = INTERP_LINEAR(wc, sc.R, so.R), RN = INTERP_LINEAR(wo, so.R, sc.R);
+    const double pP = rhoPos * RP, pN = rhoNeg * RN;
+    const double cPos = INTERP_LINEAR(wc, sc.c, so.c), cNeg = INTERP_LINEAR(wo, so.c, sc.c);
+    double phP = 0.0, phN = 0.0;
+#pragma unroll
+    for (int k = 0; k < D; k++) {
+        uP[k] = rUP[k] * rPi;
+        uN[k] = rUN[k] * rNi;
+        phP += uP[k] * S[k];
+        phN += -uN[k] * S[k];
+    }
+    // std::max({x1, x2, 0}) / std::min({y1, y2, 0}): first extreme wins
+    const double x1 = phP + cPos * Sm, x2 = -phN + cNeg * Sm;
+    double psiP = (x1 < x2) ? x2 : x1;
+    if (psiP < 0.0) psiP = 0.0;
+    const double y1 = phP - cPos * Sm, y2 = -phN - cNeg * Sm;
+    double psiN = (y2 < y1) ? y2 : y1;
+    if (0.0 < psiN) psiN = 0.0;
+    const double a0 = 1.0 / (psiP - psiN);
+    const double a1 = psiP * psiN;
+    const double aP = psiP * phP, aN = psiN * phN;
+    double rEP = eP, rEN = eN;
+#pragma unroll
+    for (int k = 0; k < D; k++) {
+        rEP += 0.5 * uP[k] * uP[k];
+        rEN += 0.5 * uN[k] * uN[k];
+    }
+    rEP *= rhoPos;
+    rEN *= rhoNeg;
+    rhs[0] = -(aP * rhoPos + aN * rhoNeg + (rhoNeg - rhoPos) * a1) * a0;
+#pragma unroll
+    for (int k = 0; k < D; k++)
+        rhs[k + 1] = -((aP * rUP[k] + aN * rUN[k] + (rUN[k] - rUP[k]) * a1) * a0 +
+                       (pP * psiP - pN * psiN) * a0 * S[k]);
+    rhs[D + 1] = -(aP * rEP + aN * rEN + (rEN - rEP) * a1 + (aP * pP + aN * pN)) * a0;
+}
+
+// flux_m1 where 1 - wc == wo and 1 - wo == wc hold exactly (any w >= 1/2, and
+// half of those below): both reconstructed states are then the same sums of
+// the same products, so the second one's operations are left out and the
+// result is the same to the bit.
+template <int D>
+__device__ __forceinline__ void flux_m1_sym(const double (&qc)[D + 2], const Prim64<D> &sc, const double (&qo)[D + 2],
+                                            const Prim64<D> &so, const double (&S)[D], const double Sm,
+                                            const double wc, const double wo, double (&rhs)[D + 2]) {
+    const double rho = wc * qc[0] + wo * qo[0];
+    const double ri = 1.0 / rho;
+    double rU[D], ph = 0.0;
+    double rE = wc * sc.e + wo * so.e;
+#pragma unroll
+    for (int k = 0; k < D; k++) {
+        rU[k] = wc * qc[k + 1] + wo * qo[k + 1];
+        const double u = rU[k] * ri;
+        ph += u * S[k];
+        rE += 0.5 * u * u;
+    }
+    rE *= rho;
+    const double p = rho * (wc * sc.R + wo * so.R);
+    const double cS = (wc * sc.c + wo * so.c) * Sm;
+    double psiP = ph + cS, psiN = ph - cS;
+    if (psiP < 0.0) psiP = 0.0;
+    if (0.0 < psiN) psiN = 0.0;
+    const double a0 = 1.0 / (psiP - psiN);
+    const double aP = psiP * ph, aN = psiN * -ph;
+    rhs[0] = -(aP * rho + aN * rho) * a0;
+    const double pS = (p * psiP - p * psiN) * a0;
+#pragma unroll
+    for (int k = 0; k < D; k++) rhs[k + 1] = -((aP * rU[k] + aN * rU[k]) * a0 + pS * S[k]);
+    rhs[D + 1] = -(aP * rE + aN * rE + (aP * p + aN * p)) * a0;
+}
+
+// M2's face pressure and mass flux are formed by the face kernel too, which
+// adds the AUSM correction to the pressure in between
+template <int D>
+__device__ __forceinline__ void flux_m2(const double rhoavg, const double (&rUa)[D], const double Havg,
+                                        const double pavg, const double (&S)[D], double (&rhs)[D + 2]) {
+    const double rai = 1.0 / rhoavg;
+    double phi = 0.0;
+#pragma unroll
+    for (int k = 0; k < D; k++) phi += (rUa[k] * rai) * S[k];
+    rhs[0] = -rhoavg * phi;
+#pragma unroll
+    for (int k = 0; k < D; k++) rhs[k + 1] = -(rUa[k] * phi + pavg * S[k]);
+    rhs[D + 1] = -(rhoavg * Havg * phi);
+}
+
+// ---------------------------------------------------------------------------
 // Face fluxes: convective (M1 2589-2675, M2 1968-2023, M2AUSM 2256-2366) plus
 // the viscous terms shared by all three (2682-2790).  One thread per face.
 // VISC false (mu = 0): every viscous term is mu or k = cp mu / Pr times a
@@ -579,65 +745,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 2
     Sm = sqrt(Sm);
 
     if (SOLVER == 0) {
-        const double omw = 1.0 - w;
-        const double rhoPos = INTERP_LINEAR(w, qP[0], qN[0]);
-        const double rhoNeg = INTERP_LINEAR(omw, qN[0], qP[0]);
-        const double rPi = 1.0 / rhoPos, rNi = 1.0 / rhoNeg;
-        double rUP[D], rUN[D], uP[D], uN[D];
-#pragma unroll
-        for (int k = 0; k < D; k++) {
-            rUP[k] = INTERP_LINEAR(w, qP[k + 1], qN[k + 1]);
-            rUN[k] = INTERP_LINEAR(omw, qN[k + 1], qP[k + 1]);
-        }
-        double ce = 2 * qP[D + 1] * cri;
-        double ae = 2 * qN[D + 1] * ari;
-#pragma unroll
-        for (int k = 0; k < D; k++) {
-            ce -= cU[k] * cU[k];
-            ae -= aU[k] * aU[k];
-        }
-        ce *= 0.5;
-        ae *= 0.5;
-        const double eP = INTERP_LINEAR(w, ce, ae), eN = INTERP_LINEAR(omw, ae, ce);
-        const double RP = INTERP_LINEAR(w, cR, aR), RN = INTERP_LINEAR(omw, aR, cR);
-        const double pP = rhoPos * RP, pN = rhoNeg * RN;
-        const double cP = sqrt(a.gamma * cR), cN = sqrt(a.gamma * aR);
-        const double cPos = INTERP_LINEAR(w, cP, cN), cNeg = INTERP_LINEAR(omw, cN, cP);
-        double phP = 0.0, phN = 0.0;
-#pragma unroll
-        for (int k = 0; k < D; k++) {
-            uP[k] = rUP[k] * rPi;
-            uN[k] = rUN[k] * rNi;
-            phP += uP[k] * S[k];
-            phN += -uN[k] * S[k];
-        }
-        // std::max({x1, x2, 0}) / std::min({y1, y2, 0}): first extreme wins
-        const double x1 = phP + cPos * Sm, x2 = -phN + cNeg * Sm;
-        double psiP = (x1 < x2) ? x2 : x1;
-        if (psiP < 0.0) psiP = 0.0;
-        const double y1 = phP - cPos * Sm, y2 = -phN - cNeg * Sm;
-        double psiN = (y2 < y1) ? y2 : y1;
-        if (0.0 < psiN) psiN = 0.0;
-        const double a0 = 1.0 / (psiP - psiN);
-        const double a1 = psiP * psiN;
-        const double aP = psiP * phP, aN = psiN * phN;
-        double rEP = eP, rEN = eN;
-#pragma unroll
-        for (int k = 0; k < D; k++) {
-            rEP += 0.5 * uP[k] * uP[k];
-            rEN += 0.5 * uN[k] * uN[k];
-        }
-        rEP *= rhoPos;
-        rEN *= rhoNeg;
-        rhs[0] = -(aP * rhoPos + aN * rhoNeg + (rhoNeg - rhoPos) * a1) * a0;
-#pragma unroll
-        for (int k = 0; k < D; k++)
-            rhs[k + 1] = -((aP * rUP[k] + aN * rUN[k] + (rUN[k] - rUP[k]) * a1) * a0 +
-                           (pP * psiP - pN * psiN) * a0 * S[k]);
-        rhs[D + 1] = -(aP * rEP + aN * rEN + (rEN - rEP) * a1 + (aP * pP + aN * pN)) * a0;
+        const Prim64<D> sp = prim64<D, 0>(a, qP), sn = prim64<D, 0>(a, qN);
+        flux_m1<D>(qP, sp, qN, sn, S, Sm, w, 1.0 - w, rhs);
     } else {
         const double rhoavg = 0.5 * (qP[0] + qN[0]);
-        const double rai = 1.0 / rhoavg;
         double rUa[D];
 #pragma unroll
         for (int k = 0; k < D; k++) rUa[k] = 0.5 * (qP[k + 1] + qN[k + 1]);
@@ -717,13 +828,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 2
             const double pu = -0.75 * p5pos(MP, alpha) * p5neg(MN, alpha) * (rhoP + rhoN) * cavg * fa * (unN - unP);
             pavg += tha * (pu - 0.5 * phalf);
         }
-        double phi = 0.0;
-#pragma unroll
-        for (int k = 0; k < D; k++) phi += (rUa[k] * rai) * S[k];
-        rhs[0] = -rhoavg * phi;
-#pragma unroll
-        for (int k = 0; k < D; k++) rhs[k + 1] = -(rUa[k] * phi + pavg * S[k]);
-        rhs[D + 1] = -(rhoavg * Havg * phi);
+        flux_m2<D>(rhoavg, rUa, Havg, pavg, S, rhs);
     }
 
     // viscous terms (cfd_v0.cpp:2682-2790)
@@ -854,6 +959,23 @@ __global__ void __launch_bounds__(256) vis_tensor_field(KArgs a, double *tmc_out
     }
 }
 
+// dt_c (MODE 0) or cfl_c (MODE 1) from a cell's sum over its faces, combined
+// with the block's starting value
+template <int D, int MODE>
+__device__ __forceinline__ double cfl_value64(const double rho, const double vinv, const double sum,
+                                              const double param) {
+    double v = MODE == 0 ? 100.0 : 0.0;
+    if (MODE == 0) {
+        const double vol = 1.0 / vinv;
+        const double dtc = param * rho * 2.0 * vol / sum;
+        if (v > dtc) v = dtc;
+    } else {
+        const double cfl = sum * ((1.0 / rho) * vinv * param);
+        if (v < cfl) v = cfl;
+    }
+    return v;
+}
+
 // ---------------------------------------------------------------------------
 // compute_dt / compute_cfl (cfd_v0.cpp:2887-2942) of one cell from its state
 // q: the sum over its faces in slot order, then dt_c (MODE 0) or cfl_c
@@ -907,16 +1029,7 @@ __device__ __forceinline__ double cfl_cell(const KArgs &a, const int c, const do
         for (int k = 0; k < D; k++) S[k] = ent >= 0 ? sf[k] : -sf[k];
         add(S);
     }
-    double v = MODE == 0 ? 100.0 : 0.0;
-    if (MODE == 0) {
-        const double vol = 1.0 / a.vinv[c];
-        const double dtc = param * q[0] * 2.0 * vol / sum;
-        if (v > dtc) v = dtc;
-    } else {
-        const double cfl = sum * ((1.0 / q[0]) * a.vinv[c] * param);
-        if (v < cfl) v = cfl;
-    }
-    return v;
+    return cfl_value64<D, MODE>(q[0], a.vinv[c], sum, param);
 }
 
 // Block-wide min (MODE 0) / max (MODE 1) of v into *dst; every thread of the
@@ -937,6 +1050,17 @@ __device__ __forceinline__ void block_extremum(double v, double *dst) {
         for (int i = 1; i < (int)(blockDim.x >> 6); i++) r = pick(r, ext[i]);
         *dst = r;
     }
+}
+
+// the sponge term of one cell (cfd_v0.cpp:2808-2811)
+template <int D, int NT = kStreamNT64<D>>
+__device__ __forceinline__ void sponge64(const KArgs &a, const int c, const double dt, const double (&q)[D + 2],
+                                         double (&dq)[D + 2]) {
+    const double sg = ld64_once<D, 3, NT>(a.sigma + c);
+    dq[0] += dt * sg * (a.rho_inf - q[0]);
+#pragma unroll
+    for (int k = 0; k < D; k++) dq[k + 1] += dt * sg * (a.rho_inf * a.U_inf[k] - q[k + 1]);
+    dq[D + 1] += dt * sg * (a.rho_inf * a.E_inf - q[D + 1]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1005,11 +1129,7 @@ __global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, 
         }
         double q[D + 2];
         load_q<D>(a, c, q);
-        const double sg = ld64_once<D, 3>(a.sigma + c);
-        dq[0] += dt * sg * (a.rho_inf - q[0]);
-#pragma unroll
-        for (int k = 0; k < D; k++) dq[k + 1] += dt * sg * (a.rho_inf * a.U_inf[k] - q[k + 1]);
-        dq[D + 1] += dt * sg * (a.rho_inf * a.E_inf - q[D + 1]);
+        if (a.sigma) sponge64<D>(a, c, dt, q, dq);
 #pragma unroll
         for (int k = 0; k < D + 2; k++) {
             q[k] += B * dq[k];
@@ -1119,6 +1239,280 @@ __device__ __forceinline__ void cfl_dt_final_block(const double *partial, int nb
         for (int i = 1; i < NT / 64; i++) r = pick(r, w[i]);
         *out = r;
         if (dt_dst) *dt_dst = r;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// One RK stage of the inviscid M1 / M2 schemes in one launch: each cell forms
+// its faces' fluxes from its own and the other cells' states as it gathers
+// them (every interior face by both of its cells, to the same bits), adds
+// sponge and RK update and writes the new state and its boundary ghosts to
+// qout, another buffer.  The face fluxes' round trip through memory (write,
+// two gathered reads: 120 B of the 773 B per 3D cell and stage that the face
+// and update launches move) and the second read of the states are gone.
+// PK: the face's area vector and weights come from the geometry table, 4 B
+// per slot instead of 36: a uniform mesh has a few dozen distinct records,
+// which stay in the L1 caches.
+// ---------------------------------------------------------------------------
+// Faces whose loads are issued together: two leave 126 VGPRs and 4 waves per
+// SIMD (3D box of 1.4 M cells: one 495, two 485, three 526 us per step).
+constexpr int kFusedGroup64 = 2;
+// geometry table record: S out of the cell [D], |S|, wc, wo, padded to whole
+// 16-byte words (6 doubles in 2D and 3D)
+constexpr int kTabRec64 = 6;
+
+// the face data of gather entry j of cell c as that cell sees them; key: the
+// packed word, or the slot's key
+template <int D, bool PK, int NT>
+struct FaceOf64 {
+    int other;
+    double S[D], Sm, wc, wo;
+    __device__ __forceinline__ static int load_key(const KArgs &a, const int j, const int c) {
+        const size_t i = slot_at<D, 1>(a.nc, j, 0, c);
+        if constexpr (PK) return (int)ld64_once<D, 1, NT>(a.pk + i);
+        return ld64_once<D, 1, NT>(a.sl_nb + i);
+    }
+    __device__ __forceinline__ static int other_of(const KArgs &a, const int key) {
+        if constexpr (PK) return (int)((uint32_t)key & ((1u << a.pk_shift) - 1u));
+        return key >= 0 ? key : ~key;
+    }
+    // geometry of a face stored with P's orientation
+    __device__ __forceinline__ void from_face(const bool isP, const double (&s)[D], const double w) {
+        double m = 0.0;
+#pragma unroll
+        for (int k = 0; k < D; k++) {
+            m += s[k] * s[k];
+            S[k] = isP ? s[k] : -s[k];
+        }
+        Sm = sqrt(m);
+        const double omw = 1.0 - w;
+        wc = isP ? w : omw;
+        wo = isP ? omw : w;
+    }
+    __device__ __forceinline__ void load(const KArgs &a, const int j, const int c, const int key) {
+        other = other_of(a, key);
+        if constexpr (PK) {
+            const double2 *p =
+                reinterpret_cast<const double2 *>(a.pk_tab + (size_t)((uint32_t)key >> a.pk_shift) * kTabRec64);
+            const double2 v0 = p[0], v1 = p[1], v2 = p[2];
+            const double r[6] = {v0.x, v0.y, v1.x, v1.y, v2.x, v2.y};
+#pragma unroll
+            for (int k = 0; k < D; k++) S[k] = r[k];
+            Sm = r[D];
+            wc = r[D + 1];
+            wo = r[D + 2];
+        } else {
+            double s[D];
+#pragma unroll
+            for (int k = 0; k < D; k++) s[k] = ld64_once<D, 1, NT>(a.sl_S + slot_at<D, D>(a.nc, j, k, c));
+            from_face(key >= 0, s, ld64_once<D, 1, NT>(a.sl_w + slot_at<D, 1>(a.nc, j, 0, c)));
+        }
+    }
+    // an entry of the gather list (beyond the slots)
+    __device__ __forceinline__ void load_list(const KArgs &a, const int ent) {
+        const bool isP = ent >= 0;
+        const int f = isP ? (ent & kFaceMask) : ~ent;
+        other = isP ? a.fN[f] : a.fP[f];
+        double s[D];
+        load_S64<D>(a.S, f, s);
+        from_face(isP, s, a.w[f]);
+    }
+};
+
+template <int D, int SOLVER, bool SYM>
+__device__ __forceinline__ void own_flux64(const KArgs &a, const double (&qc)[D + 2], const Prim64<D> &sc,
+                                           const double (&qo)[D + 2], const double (&S)[D], const double Sm,
+                                           const double wc, const double wo, double (&r)[D + 2]) {
+    const Prim64<D> so = prim64<D, SOLVER>(a, qo);
+    if constexpr (SOLVER == 0) {
+        SYM ? flux_m1_sym<D>(qc, sc, qo, so, S, Sm, wc, wo, r) : flux_m1<D>(qc, sc, qo, so, S, Sm, wc, wo, r);
+    } else {
+        const double rhoavg = 0.5 * (qc[0] + qo[0]);
+        double rUa[D];
+#pragma unroll
+        for (int k = 0; k < D; k++) rUa[k] = 0.5 * (qc[k + 1] + qo[k + 1]);
+        const double Ravg = 0.5 * (sc.R + so.R);
+        const double Havg = 0.5 * (sc.e + so.e);
+        flux_m2<D>(rhoavg, rUa, Havg, rhoavg * Ravg, S, r);
+    }
+}
+
+// |m.S| (MODE 1) or |m.S| / |S| (MODE 0) of one face, as cfl_cell forms it
+template <int D, int MODE>
+__device__ __forceinline__ double cfl_term64(const double (&q)[D + 2], const double (&S)[D], const double Sm) {
+    double fl = 0.0;
+#pragma unroll
+    for (int k = 0; k < D; k++) fl += MODE == 0 ? q[k + 1] * S[k] / Sm : q[k + 1] * S[k];
+    return fabs(fl);
+}
+
+// fin_nblk > 0 (a stage without CFL/dt sums): one block more, the last,
+// reduces the fin_nblk per-block CFL maxima that the previous step's last
+// stage left in a.partial into *fin_out.
+// SYM: every face's weights allow flux_m1_sym.
+template <int D, int SOLVER, int CFL, bool PK, bool SYM, int NT>
+__global__ void __launch_bounds__(256) stage_fused64(KArgs a, double *qout, double A, double B, int zero_dq,
+                                                     double cfl_param, int fin_nblk, double *fin_out) {
+    int nb = (int)gridDim.x;
+    if constexpr (CFL < 0) {
+        if (fin_nblk > 0) {
+            nb -= 1;
+            if ((int)blockIdx.x == nb) {
+                cfl_dt_final_block<1, 256>(a.partial, fin_nblk, fin_out, nullptr);
+                return;
+            }
+        }
+    }
+    constexpr int U = GatherUnroll<D>::value;
+    using F = FaceOf64<D, PK, NT>;
+    const int blk = xcd_block((int)blockIdx.x, nb);
+    const int c = blk * (int)blockDim.x + (int)threadIdx.x;
+    double cv = CFL == 0 ? 100.0 : 0.0;
+    // the CFL/dt terms of a cell's faces in slot order (own thread only)
+    __shared__ double terms[CFL >= 0 ? kMaxFaces * 256 : 1];
+    if (c < a.nc) {
+        constexpr int G = kFusedGroup64;
+        int key[G];
+#pragma unroll
+        for (int u = 0; u < G; u++) key[u] = F::load_key(a, u, c);
+        double qc[D + 2], dq[D + 2];
+        load_q<D>(a, c, qc);
+        const double dt = *a.dt;
+        const double vinv = ld64_once<D, 3, NT>(a.vinv + c);
+#pragma unroll
+        for (int k = 0; k < D + 2; k++) dq[k] = zero_dq ? 0.0 : ld64_once<D, 2, NT>(a.dq + (size_t)k * a.nc + c) * A;
+        const Prim64<D> sc = prim64<D, SOLVER>(a, qc);
+        unsigned gmask = 0;  // bit j: slot j leads to a boundary ghost
+        // a rolled loop over groups of G faces, the next group's keys loaded a
+        // group ahead: unrolled, the compiler gathers all faces' loads at the
+        // top and spills
+#pragma unroll 1
+        for (int j0 = 0; j0 < U; j0 += G) {
+            F f[G];
+            double qo[G][D + 2];
+            int next[G];
+#pragma unroll
+            for (int u = 0; u < G; u++) {
+                f[u].load(a, j0 + u, c, key[u]);
+                load_q<D>(a, f[u].other, qo[u]);
+                next[u] = F::load_key(a, j0 + G < U ? j0 + G + u : u, c);
+            }
+#pragma unroll
+            for (int u = 0; u < G; u++) {
+                if (f[u].other != c) {
+                    double r[D + 2];
+                    own_flux64<D, SOLVER, SYM>(a, qc, sc, qo[u], f[u].S, f[u].Sm, f[u].wc, f[u].wo, r);
+                    gmask |= f[u].other >= a.nc ? 1u << (j0 + u) : 0u;
+#pragma unroll
+                    for (int k = 0; k < D + 2; k++) dq[k] += dt * r[k] * vinv;
+                }
+                key[u] = next[u];
+            }
+        }
+        int e1 = 0, e2 = 0;  // gather entries beyond the slots
+        if (U < kMaxFaces && a.more_faces) {
+            e1 = a.g_off[c] + U;
+            e2 = a.g_off[c + 1];
+            for (int e = e1; e < e2; e++) {
+                F f;
+                f.load_list(a, a.g_ent[e]);
+                double qo[D + 2], r[D + 2];
+                load_q<D>(a, f.other, qo);
+                own_flux64<D, SOLVER, false>(a, qc, sc, qo, f.S, f.Sm, f.wc, f.wo, r);
+                gmask |= f.other >= a.nc ? 1u << (U + e - e1) : 0u;
+#pragma unroll
+                for (int k = 0; k < D + 2; k++) dq[k] += dt * r[k] * vinv;
+            }
+        }
+        double q[D + 2];
+#pragma unroll
+        for (int k = 0; k < D + 2; k++) q[k] = qc[k];
+        if (a.sigma) sponge64<D, NT>(a, c, dt, q, dq);
+#pragma unroll
+        for (int k = 0; k < D + 2; k++) {
+            q[k] += B * dq[k];
+            st64_once<D, 2, NT>(a.dq + (size_t)k * a.nc + c, dq[k]);
+        }
+        store_q<D, NT>(qout, a.ntot, c, q);
+        // this cell's boundary ghosts for the next stage
+        for (unsigned m = gmask; m; m &= m - 1) {
+            const int j = __builtin_ctz(m);
+            int g;
+            if (U >= kMaxFaces || j < U) {
+                g = F::other_of(a, F::load_key(a, j, c));
+            } else {
+                g = a.fN[a.g_ent[e1 + j - U] & kFaceMask];
+            }
+            double qg[D + 2];
+            if (!ghost_state<D>(a, a.ghost_role[g - a.nc], q, qg)) load_q<D>(a, g, qg);
+            store_q<D, NT>(qout, a.ntot, g, qg);
+        }
+        if constexpr (CFL >= 0) {
+            const int perm = a.s_perm[c];
+#pragma unroll
+            for (int j = 0; j < U; j++) {
+                F f;
+                f.load(a, j, c, F::load_key(a, j, c));
+                if (f.other != c)
+                    terms[((perm >> (3 * j)) & 7) * 256 + threadIdx.x] = cfl_term64<D, CFL>(q, f.S, f.Sm);
+            }
+            for (int e = e1; U < kMaxFaces && e < e2; e++) {
+                F f;
+                f.load_list(a, a.g_ent[e]);
+                terms[((perm >> (3 * (U + e - e1))) & 7) * 256 + threadIdx.x] = cfl_term64<D, CFL>(q, f.S, f.Sm);
+            }
+            const int n = (perm >> 18) & 7;
+            double sum = 0.0;
+            for (int j = 0; j < n; j++) sum += terms[j * 256 + threadIdx.x];
+            cv = cfl_value64<D, CFL>(q[0], a.vinv[c], sum, cfl_param);
+        }
+    }
+    if constexpr (CFL >= 0) block_extremum<CFL>(cv, a.partial + blk);
+}
+
+// the one-launch stage's slots from the gather list and, with face_rec, each
+// face's record number in the geometry table (2 face_rec + 1 from the N side;
+// none: a placeholder's record)
+template <int D>
+__global__ void __launch_bounds__(256) build_slots64(KArgs a, const uint16_t *face_rec, int none, uint32_t *pk,
+                                                     int32_t *nb, double *S, double *w, int32_t *perm) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= a.nc) return;
+    const int e0 = a.g_off[c], ne = a.g_off[c + 1] - e0;
+    const int s0 = a.s_off[c], ns = a.s_off[c + 1] - s0;
+    int p = ns << 18;
+    for (int j = 0; j < ne && j < kMaxFaces; j++) {
+        const int ent = a.g_ent[e0 + j];
+        const int bare = ent >= 0 ? (ent & kFaceMask) : ent;
+        for (int i = 0; i < ns; i++)
+            if (a.s_ent[s0 + i] == bare) p |= i << (3 * j);
+    }
+    perm[c] = p;
+    constexpr int U = GatherUnroll<D>::value;
+    for (int j = 0; j < U; j++) {
+        const size_t i1 = slot_at<D, 1>(a.nc, j, 0, c);
+        if (j >= ne) {
+            // placeholder past the cell's last entry: the cell itself, unit
+            // area (read by unbranched gathers, never added)
+            if (pk) {
+                pk[i1] = (uint32_t)c | (uint32_t)none << a.pk_shift;
+            } else {
+                nb[i1] = c;
+                for (int k = 0; k < D; k++) S[slot_at<D, D>(a.nc, j, k, c)] = 1.0;
+                w[i1] = 0.5;
+            }
+            continue;
+        }
+        const int ent = a.g_ent[e0 + j];
+        const int f = ent >= 0 ? (ent & kFaceMask) : ~ent;
+        const int o = ent >= 0 ? a.fN[f] : a.fP[f];
+        if (pk) {
+            pk[i1] = (uint32_t)o | (uint32_t)(2 * face_rec[f] + (ent >= 0 ? 0 : 1)) << a.pk_shift;
+        } else {
+            nb[i1] = ent >= 0 ? o : ~o;
+            for (int k = 0; k < D; k++) S[slot_at<D, D>(a.nc, j, k, c)] = a.S[(size_t)f * D + k];
+            w[i1] = a.w[f];
+        }
     }
 }
 

@@ -574,6 +574,66 @@ std::string build_layout(const lfm_polymesh &m, const lfm_partition *part, const
     return "";
 }
 
+template <typename T>
+FaceTable<T> face_table(const SolverLayout &L, int max_n) {
+    FaceTable<T> t;
+    const size_t nf = L.nf;
+    const int D = L.D;
+    if (max_n < 1 || nf == 0) return t;
+    max_n = std::min(max_n, 65535);
+    // open addressing over at most half-full power-of-two buckets
+    size_t cap = 16;
+    while (cap < 2 * (size_t)(max_n + 1)) cap *= 2;
+    std::vector<int32_t> bucket(cap, -1);
+    struct Key {
+        T v[4];
+    };
+    std::vector<Key> keys;
+    t.rec.resize(nf);
+    // consecutive cells repeat the previous cells' records: the few last
+    // used ones are tried before the hash
+    constexpr int kLast = 4;
+    int last[kLast] = {-1, -1, -1, -1}, at = 0;
+    for (size_t f = 0; f < nf; f++) {
+        Key k{};
+        for (int i = 0; i < D; i++) k.v[i] = (T)L.S[i * nf + f];
+        k.v[3] = (T)L.w[f];
+        int r = -1;
+        for (int i = 0; i < kLast && r < 0; i++)
+            if (last[i] >= 0 && std::memcmp(&keys[last[i]], &k, sizeof k) == 0) r = last[i];
+        if (r < 0) {
+            uint64_t h = 1469598103934665603ull;
+            for (T x : k.v) {
+                uint64_t b = 0;
+                std::memcpy(&b, &x, sizeof x);
+                h = (h ^ b) * 0x9E3779B97F4A7C15ull;
+                h ^= h >> 29;
+            }
+            size_t i = (size_t)h & (cap - 1);
+            while (bucket[i] >= 0 && std::memcmp(&keys[bucket[i]], &k, sizeof k) != 0) i = (i + 1) & (cap - 1);
+            if (bucket[i] < 0) {
+                if ((int)keys.size() == max_n) return FaceTable<T>();
+                bucket[i] = (int32_t)keys.size();
+                keys.push_back(k);
+            }
+            r = bucket[i];
+            last[at] = r;
+            at = (at + 1) % kLast;
+        }
+        t.rec[f] = (uint16_t)r;
+    }
+    t.n = (int)keys.size();
+    t.S.resize((size_t)t.n * D);
+    t.w.resize(t.n);
+    for (int i = 0; i < t.n; i++) {
+        for (int k = 0; k < D; k++) t.S[(size_t)i * D + k] = keys[i].v[k];
+        t.w[i] = keys[i].v[3];
+    }
+    return t;
+}
+template FaceTable<float> face_table<float>(const SolverLayout &, int);
+template FaceTable<double> face_table<double>(const SolverLayout &, int);
+
 std::string halo_import(SolverLayout &L, int ni, int n, const int32_t *key, const int32_t *cell,
                         const double *disp) {
     if (ni < 0 || ni >= (int)L.halo.size()) return "unknown neighbour";

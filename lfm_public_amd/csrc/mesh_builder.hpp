@@ -86,6 +86,26 @@ std::string build_layout(const lfm_polymesh &m, const lfm_partition *part, const
 std::string halo_import(SolverLayout &L, int ni, int n, const int32_t *key, const int32_t *cell,
                         const double *disp);
 
+// The distinct face records (area vector and weight as T holds them) of a
+// layout, for kernels that read a small table instead of per-face data: a
+// uniform mesh has a few dozen.  n = 0 where there are more than max_n; rec:
+// each face's record.
+template <typename T>
+struct FaceTable {
+    int n = 0;
+    std::vector<T> S, w;        // [n][D], [n]
+    std::vector<uint16_t> rec;  // [nf]
+};
+template <typename T>
+FaceTable<T> face_table(const SolverLayout &L, int max_n);
+
+// bits that hold an index below n
+inline int index_bits(long n) {
+    int b = 1;
+    while ((1L << b) < n) b++;
+    return b;
+}
+
 // Gas constants derived as set_init_conditions does (cfd_v0.cpp:880-902).
 struct Gas {
     double R, R_inv, gamma, gm1, cp, mu, pr_inv;

@@ -4,6 +4,7 @@
 // HBM in SoA layout and drives the stage kernels on its own HIP stream.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -31,6 +32,9 @@ std::mutex &device_setup_mutex() {
     return m;
 }
 
+// records of the FP64 geometry table: both orientations of them are at most
+// 192 KiB, which stay in an XCD's 4 MiB L2 beside the gathered states
+static constexpr int kMaxTable64 = 2048;
 static constexpr int kBlock = 256;
 static inline int nblocks(long n) { return (int)((n + kBlock - 1) / kBlock); }
 
@@ -104,7 +108,8 @@ static int create_fp64(Solver *s) {
     rc |= dev_upload(s, (int32_t **)&a.ghost_cell, L.ghost_cell.data(), L.ng);
     rc |= dev_upload(s, (int32_t **)&a.ghost_role, L.ghost_role.data(), L.ng);
     rc |= dev_upload(s, (double **)&a.vinv, L.vinv.data(), nc);
-    rc |= dev_upload(s, (double **)&a.sigma, L.sigma.data(), nc);
+    if (std::any_of(L.sigma.begin(), L.sigma.end(), [](double v) { return v != 0.0; }))
+        rc |= dev_upload(s, (double **)&a.sigma, L.sigma.data(), nc);
     if (!L.smag.empty()) rc |= dev_upload(s, (double **)&a.smag, L.smag.data(), nc);
     rc |= dev_zeros(s, &a.q, (size_t)(D + 2) * ntot);
     rc |= dev_zeros(s, &a.dq, (size_t)(D + 2) * nc);
@@ -157,6 +162,19 @@ static int create_fp64(Solver *s) {
         HIP_TRY(hipMemcpy(a.q, q0.data(), q0.size() * sizeof(double), hipMemcpyHostToDevice));
     }
     HIP_TRY(hipMemcpy(s->d_scalar, &s->dt, sizeof(double), hipMemcpyHostToDevice));
+    // one-launch stages; a cell that is its own neighbour (a cyclic pair one
+    // cell apart) has more gather entries than slots and keeps the launches
+    // that walk the list
+    s->fused_ok = !s->visc && s->prm.solver < 2 && L.halo.empty();
+    for (size_t f = 0; f < nf && s->fused_ok; f++) s->fused_ok = L.fP[f] != L.fN[f];
+    a.more_faces = L.max_faces > (D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value);
+    if (s->fused_ok) {
+        // records in both orientations and a placeholder's fit above the
+        // cell index; kMaxTable64 keeps the table in an XCD's L2
+        a.pk_shift = index_bits((long)ntot);
+        const long fit = ((1L << (32 - a.pk_shift)) - 1) / 2;
+        s->table64 = face_table<double>(L, (int)std::min<long>(fit, kMaxTable64));
+    }
     return 0;
 }
 
@@ -248,6 +266,45 @@ int integrals64(Solver *s, double *out_dev) {
         hipLaunchKernelGGL(integrals64<3>, dim3(nb), dim3(kBlock), 0, s->stream, s->k64);
     hipLaunchKernelGGL(reduce_sum, dim3(1), dim3(kBlock), 0, s->stream, s->k64.partial, nb, s->L.D + 2, out_dev, 0);
     return 0;
+}
+
+template <int D, int SOLVER, bool PK, bool SYM, int NT>
+static void launch_fused64_nt(Solver *s, double A, double B, int zero_dq, const KArgs &a, double *qout,
+                             const Solver::CflJob *cfl, bool fin) {
+    const int nb = nblocks(s->L.nc);
+    if (!cfl)
+        hipLaunchKernelGGL((stage_fused64<D, SOLVER, -1, PK, SYM, NT>), dim3(nb + (fin ? 1 : 0)), dim3(kBlock), 0, s->stream, a,
+                           qout, A, B, zero_dq, 0.0, fin ? nb : 0, s->d_cfl);
+    else if (cfl->mode == 0)
+        hipLaunchKernelGGL((stage_fused64<D, SOLVER, 0, PK, SYM, NT>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
+                           zero_dq, cfl->param, 0, s->d_cfl);
+    else
+        hipLaunchKernelGGL((stage_fused64<D, SOLVER, 1, PK, SYM, NT>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
+                           zero_dq, cfl->param, 0, s->d_cfl);
+}
+
+template <int D, int SOLVER, bool PK, bool SYM>
+static void launch_fused64_v(Solver *s, double A, double B, int zero_dq, const KArgs &a, double *qout,
+                             const Solver::CflJob *cfl, bool fin) {
+    s->stream_nt ? launch_fused64_nt<D, SOLVER, PK, SYM, 3>(s, A, B, zero_dq, a, qout, cfl, fin)
+                 : launch_fused64_nt<D, SOLVER, PK, SYM, 0>(s, A, B, zero_dq, a, qout, cfl, fin);
+}
+
+// fin: the launch also reduces the previous step's CFL maxima (left in
+// a.partial) into d_cfl, in one extra block
+template <int D>
+static void launch_stage_fused64(Solver *s, double A, double B, bool zero_dq, const double *qin, double *qout,
+                                 const Solver::CflJob *cfl, bool fin) {
+    KArgs a = s->k64;
+    a.q = const_cast<double *>(qin);
+    if (s->prm.solver == 1)
+        a.pk ? launch_fused64_v<D, 1, true, false>(s, A, B, zero_dq, a, qout, cfl, fin)
+             : launch_fused64_v<D, 1, false, false>(s, A, B, zero_dq, a, qout, cfl, fin);
+    else if (a.pk)
+        s->sym64 ? launch_fused64_v<D, 0, true, true>(s, A, B, zero_dq, a, qout, cfl, fin)
+                 : launch_fused64_v<D, 0, true, false>(s, A, B, zero_dq, a, qout, cfl, fin);
+    else
+        launch_fused64_v<D, 0, false, false>(s, A, B, zero_dq, a, qout, cfl, fin);
 }
 
 // dispatch helpers over dimension
@@ -422,9 +479,121 @@ bool Solver::ensure_slots32() {
     return true;
 }
 
+// Whether a stage that touches this many bytes marks what a kernel reads or
+// writes once as non-temporal.  Up to about a third more than the 256 MB
+// Infinity Cache the next launch finds part of it there if it is not marked;
+// beyond, marking keeps the gathered neighbour states in L2.  FP64 3D box,
+// one launch per stage, us per step marked / not: 134 MB 313 / 255, 214 MB
+// 460 / 386, 261 MB 553 / 487, 319 MB 654 / 645, 454 MB 903 / 915, 829 MB
+// 1560 / 1607.
+static bool stream_once(size_t bytes) { return bytes > (size_t)340 << 20; }
+
+bool Solver::alloc_all(void **p, const size_t *bytes, int n) {
+    for (int i = 0; i < n; i++)
+        if (hipMalloc(&p[i], bytes[i]) != hipSuccess) {
+            (void)hipGetLastError();
+            for (int k = 0; k < i; k++) (void)hipFree(p[k]);
+            return false;
+        }
+    for (int i = 0; i < n; i++) {
+        allocs.push_back(p[i]);
+        device_bytes += (int64_t)bytes[i];
+    }
+    return true;
+}
+
+// the FP64 one-launch stage's slots: packed words over the geometry table
+// where the mesh has few distinct face records, else each slot's key, area
+// vector and weight
+bool Solver::ensure_slots64() {
+    if (k64.s_perm) return true;
+    const int D = L.D, U = D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value;
+    const size_t words = slot_array_len(L.nc, U, 1) * sizeof(int32_t), perm = (size_t)L.nc * sizeof(int32_t);
+    std::lock_guard<std::mutex> lock(device_setup_mutex());
+    void *p[4] = {nullptr, nullptr, nullptr, nullptr}, *rec = nullptr;
+    const int nt = table64.n;
+    std::vector<double> tab;
+    if (nt) {
+        // each record as P sees it, then as N does (flux_m1), and a
+        // placeholder's; |S| summed and rooted as the kernels would
+        tab.assign((size_t)(2 * nt + 1) * kTabRec64, 0.0);
+        sym64 = true;
+        for (int i = 0; i < 2 * nt; i++) {
+            double *r = &tab[(size_t)i * kTabRec64], m = 0.0;
+            const double w = table64.w[i / 2], omw = 1.0 - w;
+            for (int k = 0; k < D; k++) {
+                const double x = table64.S[(size_t)(i / 2) * D + k];
+                m += x * x;
+                r[k] = i % 2 ? -x : x;
+            }
+            r[D] = std::sqrt(m);
+            r[D + 1] = i % 2 ? omw : w;
+            r[D + 2] = i % 2 ? w : omw;
+            sym64 = sym64 && 1.0 - omw == w;
+        }
+        double *r = &tab[(size_t)2 * nt * kTabRec64];
+        r[0] = r[D] = 1.0;
+        r[D + 1] = r[D + 2] = 0.5;
+        const size_t bytes[3] = {words, tab.size() * sizeof(double), perm};
+        if (!alloc_all(p, bytes, 3)) return false;
+        if (hipMalloc(&rec, table64.rec.size() * sizeof(uint16_t)) != hipSuccess ||
+            hipMemcpy(rec, table64.rec.data(), table64.rec.size() * sizeof(uint16_t), hipMemcpyHostToDevice) !=
+                hipSuccess ||
+            hipMemcpy(p[1], tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
+            (void)hipGetLastError();
+            if (rec) (void)hipFree(rec);
+            return false;
+        }
+    } else {
+        const size_t bytes[4] = {words, slot_array_len(L.nc, U, D) * sizeof(double),
+                                 slot_array_len(L.nc, U, 1) * sizeof(double), perm};
+        if (!alloc_all(p, bytes, 4)) return false;
+    }
+    const int nb = nblocks(L.nc);
+    uint32_t *pk = nt ? (uint32_t *)p[0] : nullptr;
+    int32_t *key = nt ? nullptr : (int32_t *)p[0], *pm = (int32_t *)(nt ? p[2] : p[3]);
+    double *sS = nt ? nullptr : (double *)p[1], *sw = nt ? nullptr : (double *)p[2];
+    if (D == 2)
+        hipLaunchKernelGGL(build_slots64<2>, dim3(nb), dim3(kBlock), 0, stream, k64, (const uint16_t *)rec, 2 * nt, pk,
+                           key, sS, sw, pm);
+    else
+        hipLaunchKernelGGL(build_slots64<3>, dim3(nb), dim3(kBlock), 0, stream, k64, (const uint16_t *)rec, 2 * nt, pk,
+                           key, sS, sw, pm);
+    if (rec) {
+        (void)hipStreamSynchronize(stream);
+        (void)hipFree(rec);
+    }
+    table64 = FaceTable<double>();
+    k64.pk = pk;
+    k64.pk_tab = nt ? (const double *)p[1] : nullptr;
+    k64.sl_nb = key;
+    k64.sl_S = sS;
+    k64.sl_w = sw;
+    k64.s_perm = pm;
+    // what one stage touches: two states, the RK register, the slots, 1/V
+    // and sponge
+    stream_nt = stream_once((size_t)(3 * (D + 2) + 1 + (k64.sigma ? 1 : 0)) * L.nc * sizeof(double) + words +
+                            (nt ? 0 : words / sizeof(int32_t) * (D + 1) * sizeof(double)));
+    return true;
+}
+
 // the second state buffer of the one-launch stages (and the slots they
 // read), allocated on first use; without them the step runs the separate
 // launches, which compute the same bits
+bool Solver::ensure_alt64() {
+    if (!fused_ok) return false;
+    if (q_alt64) return true;
+    void *p = nullptr;
+    const size_t bytes = (size_t)(L.D + 2) * ((size_t)L.nc + L.ng) * sizeof(double);
+    fused_ok = ensure_slots64();
+    if (fused_ok) {
+        std::lock_guard<std::mutex> lock(device_setup_mutex());
+        fused_ok = alloc_all(&p, &bytes, 1);
+    }
+    q_alt64 = (double *)p;
+    return fused_ok;
+}
+
 bool Solver::ensure_alt32() {
     if (!fused_ok) return false;
     if (q_alt32) return true;
@@ -457,12 +626,21 @@ int Solver::fused_from() const {
 
 void Solver::stage_fused(int rk, bool from_alt) {
     stage_a(rk);  // the ghost fill after an outside write (no gradients here)
-    float *qin = from_alt ? q_alt32 : k32->q, *qout = from_alt ? k32->q : q_alt32;
+    auto launch = [&](const CflJob *job, bool fin) {
+        if (!fp32) {
+            double *qin = from_alt ? q_alt64 : k64.q, *qout = from_alt ? k64.q : q_alt64;
+            LFM_DISPATCH_D(this, launch_stage_fused64<2>(this, A[rk], B[rk], rk == 0, qin, qout, job, fin),
+                           launch_stage_fused64<3>(this, A[rk], B[rk], rk == 0, qin, qout, job, fin));
+            return;
+        }
+        float *qin = from_alt ? q_alt32 : k32->q, *qout = from_alt ? k32->q : q_alt32;
+        LFM_DISPATCH_D(this, launch_stage_fused32<2>(this, A[rk], B[rk], rk == 0, qin, qout, job, fin),
+                       launch_stage_fused32<3>(this, A[rk], B[rk], rk == 0, qin, qout, job, fin));
+    };
     if (rk == nstages - 1) {
         const CflJob job = cfl_job(true);
         prof_mark(5, true);
-        LFM_DISPATCH_D(this, launch_stage_fused32<2>(this, A[rk], B[rk], rk == 0, qin, qout, &job, false),
-                       launch_stage_fused32<3>(this, A[rk], B[rk], rk == 0, qin, qout, &job, false));
+        launch(&job, false);
         prof_mark(5, false);
         final_or_carry(job);
         cfl_fused = true;
@@ -471,8 +649,7 @@ void Solver::stage_fused(int rk, bool from_alt) {
         const bool fin = cfl_pending && carry_target() == 1;
         if (fin) cfl_pending = false;
         prof_mark(3, true);
-        LFM_DISPATCH_D(this, launch_stage_fused32<2>(this, A[rk], B[rk], rk == 0, qin, qout, nullptr, fin),
-                       launch_stage_fused32<3>(this, A[rk], B[rk], rk == 0, qin, qout, nullptr, fin));
+        launch(nullptr, fin);
         prof_mark(3, false);
     }
 }
@@ -484,7 +661,7 @@ void Solver::stage_fused(int rk, bool from_alt) {
 // viscous or M2AUSM solver has one, before its update); 0, none
 int Solver::carry_target() const {
     if (!L.halo.empty()) return 0;
-    if (fused_ok) return q_alt32 && fused_from() == 0 && nstages > 1 ? 1 : 0;
+    if (fused_ok) return have_alt() && fused_from() == 0 && nstages > 1 ? 1 : 0;
     return fp32 && (visc || prm.solver == 2) ? 2 : 0;
 }
 
@@ -510,7 +687,7 @@ void Solver::flush_cfl() {
 
 // one full time step (Mesh::solve loop body), no host synchronisation
 void Solver::step() {
-    const int first = fused_ok && ensure_alt32() ? fused_from() : nstages;
+    const int first = fused_ok && ensure_alt() ? fused_from() : nstages;
     if (carry_target() == 0) flush_cfl();
     for (int rk = 0; rk < first; rk++) {
         stage_a(rk);
@@ -524,7 +701,7 @@ void Solver::step() {
     // an odd number of one-launch stages left the state in the second
     // buffer: it becomes the state buffer (kernels take k32 by value at
     // launch, so later launches see the swap)
-    if (in_alt) std::swap(k32->q, q_alt32);
+    if (in_alt) fp32 ? std::swap(k32->q, q_alt32) : std::swap(k64.q, q_alt64);
     end_step(true);
 }
 

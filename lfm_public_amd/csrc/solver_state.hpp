@@ -146,15 +146,28 @@ struct Solver {
     // then launches nothing.
     void stage_a(int rk);
     void stage_b(int rk, bool fuse_cfl = false, bool own_dt = true);
-    // FP32 inviscid M1 / M2 without halos or wall forces (fused_ok): stages
-    // from fused_from() on are one launch each, reading one state buffer and
+    // Inviscid M1 / M2 without halos or wall forces (fused_ok): stages from
+    // fused_from() on are one launch each, reading one state buffer and
     // writing the other; after an odd count the two buffers swap roles, so
-    // k32->q always holds the state between steps.  The second buffer is
-    // allocated by the first step that uses it (ensure_alt32), so solvers
-    // that only step through a batch never hold it.
+    // k32->q / k64.q always holds the state between steps.  The second buffer
+    // is allocated by the first step that uses it (ensure_alt), so solvers
+    // driven through the per-stage calls never hold it.
     bool fused_ok = false;
     float *q_alt32 = nullptr;
+    double *q_alt64 = nullptr;
+    bool ensure_alt() { return fp32 ? ensure_alt32() : ensure_alt64(); }
+    bool have_alt() const { return fp32 ? q_alt32 != nullptr : q_alt64 != nullptr; }
     bool ensure_alt32();
+    bool ensure_alt64();
+    // the FP64 one-launch stage's slots (k64.pk or k64.sl_*, k64.s_perm), on
+    // first use; the distinct face records found when the handle was created
+    FaceTable<double> table64;
+    bool ensure_slots64();
+    bool stream_nt = true;  // the stage outgrows the Infinity Cache (stream_once)
+    bool sym64 = false;  // every record's weights allow flux_m1_sym
+    // device memory for a set of arrays of one kind, all or none, under the
+    // set-up mutex (which the caller holds)
+    bool alloc_all(void **p, const size_t *bytes, int n);
     // per-cell face slots of the FP32 kernels (k32->sl_*), on first use
     bool slots_failed = false;
     bool ensure_slots32();
