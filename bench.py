@@ -118,9 +118,9 @@ def launch_plan(prm, nstages):
         plan["cfl_dt"] = (1, f"cfl_dt_cells<{D}, {mode}>")
     if visc or S == 2:
         # FP32 3D gradients read the face slots (the kernel's last parameter)
-        slots = f", {str(D == 3).lower()}" if fp32 else ""
+        slots = f", {str(D == 3).lower()}" if fp32 else ">"
         plan["grad_vis"] = (nstages, f"grad_vis{sfx}<{D}, {2 if rg else 0}, {str(visc).lower()}, "
-                                     f"{str(S == 2).lower()}{slots}>")
+                                     f"{str(S == 2).lower()}{slots}")
     return plan
 
 

@@ -152,7 +152,7 @@ static int batch_set_locked(Batch *b, lfm_solver *const *hs, int n) {
         b->members.push_back(s);
         args.push_back(*s->k32);
         args.back().q_alt = s->q_alt32;
-        fused = fused && s->fused_ok && s->q_alt32 && s->k32->sl_nb && !s->post_forces;
+        fused = fused && s->fused_ok && s->q_alt32 && !s->post_forces;
         auto add = [&](std::vector<int32_t> &req, std::vector<int32_t> &first, long count) {
             first.push_back((int32_t)req.size());
             const long nb = (count + 255) / 256;

@@ -5,7 +5,7 @@
 // with the deviation formed algebraically, never by subtracting two
 // freestream-sized numbers:
 //   u' = (m' - u_inf rho') / rho
-//   p' = (g-1) [ (rhoE)' - 1/2 (rho' |u|^2 + rho_inf u'.(2 u_inf + u')) ]
+//   p' = (g-1) [ (rhoE)' - 1/2 (rho' |u_inf|^2 + rho u'.(2 u_inf + u')) ]
 //   Rpsi' = (p' - Rpsi_inf rho') / rho
 // Subtracting F(q_inf).S face by face leaves every closed cell's sum unchanged
 // in exact arithmetic (sum of S over a closed cell is zero) and removes the
@@ -52,22 +52,40 @@ struct KArgs32 {
     double *d_cfl, *d_dtmin;  // this solver's FP64 CFL / dt-min scalars
     int nblk_cells;           // blocks of 256 over the cells (reduction partials)
     // per-cell face slots of the one-launch stage and the 3D gradient kernel
-    // (the first GatherUnroll gather entries of each cell, stored as
-    // slot_at places them): the face's other cell (~other where the cell is
-    // the face's N; the cell itself past its last entry), its area vector
-    // (face orientation) and weight; nullptr until built
+    // (the first GatherUnroll gather entries of each cell): either packed
+    // words (pk_at; the other cell in the low pk_shift bits, above them the
+    // face's record in the geometry table pk_tab) or, where the mesh has too
+    // many distinct records, the other cell, the area vector out of the cell
+    // and the cell's own weight (sl_*, as slot_at places them).  A slot past
+    // the cell's last entry holds the cell itself with zero area, so its flux
+    // is zero.  more_faces: some cell has entries beyond the slots.
+    const uint32_t *pk;
+    const float *pk_tab;
+    int pk_shift, pk_half;  // pk_half: every weight in the table is 1/2
     const int32_t *sl_nb;
     const float *sl_S, *sl_w;
+    int more_faces;
     // the second state buffer, in a batch's copy of a member's arguments
     // (the solver's own copy leaves it null)
     float *q_alt;
     float gamma, gm1, gog, R_inv, mu, cp, pr_inv;
     float rho_inf, p_inf, T_inf, Rpsi_inf, E_inf, H_inf, G_inf, c_inf;
-    float uinf[3], minf[3];
+    float uinf[3], minf[3], uinf2;  // uinf2: |u_inf|^2
     double rho_inf_d, m_inf_d[3], rhoE_inf_d;
 };
 
 #define LERP32(w, a, b) ((w) * (a) + (1.0f - (w)) * (b))
+
+// A face value from its two cells, wc c + wo o, with both products rounded
+// before the sum: exchanging the cells gives the same bits, so a face seen
+// from either side has one value (also where the products are subnormal).
+__device__ __forceinline__ float face_value32(float wc, float c, float wo, float o) {
+#pragma clang fp contract(off)
+    const float x = wc * c, y = wo * o;
+    return x + y;
+}
+// M2's midpoint
+__device__ __forceinline__ float midpoint32(float c, float o) { return 0.5f * (c + o); }
 
 // FP32 reciprocal, quotient, square root and reciprocal square root on the
 // hardware instructions (v_rcp_f32, v_sqrt_f32, v_rsq_f32: 1 ulp).  Spelled
@@ -95,7 +113,7 @@ __device__ __forceinline__ void load_S32(const float *S, int f, float (&s)[D]) {
 
 template <int D>
 struct Prim32 {
-    float rp, rho, ri, up[D], u[D], pp, Rp, R;
+    float rp, rho, ri, up[D], u[D], du2, pp, Rp, R;  // du2 = |u|^2 - |u_inf|^2
 };
 
 template <int D>
@@ -104,15 +122,15 @@ __device__ __forceinline__ Prim32<D> prim32(const KArgs32 &a, const float *q) {
     s.rp = q[0];
     s.rho = a.rho_inf + s.rp;
     s.ri = rcp32(s.rho);
-    float u2 = 0.f, du2 = 0.f;
+    s.du2 = 0.f;
 #pragma unroll
     for (int k = 0; k < D; k++) {
         s.up[k] = (q[k + 1] - a.uinf[k] * s.rp) * s.ri;
         s.u[k] = a.uinf[k] + s.up[k];
-        u2 += s.u[k] * s.u[k];
-        du2 += s.up[k] * (2.f * a.uinf[k] + s.up[k]);
+        s.du2 += s.up[k] * (2.f * a.uinf[k] + s.up[k]);
     }
-    s.pp = a.gm1 * (q[D + 1] - 0.5f * (s.rp * u2 + a.rho_inf * du2));
+    // rho' |u|^2 + rho_inf (|u|^2 - |u_inf|^2) = rho' |u_inf|^2 + rho du2
+    s.pp = a.gm1 * (q[D + 1] - 0.5f * (s.rp * a.uinf2 + s.rho * s.du2));
     s.Rp = (s.pp - a.Rpsi_inf * s.rp) * s.ri;
     s.R = a.Rpsi_inf + s.Rp;
     return s;
@@ -343,47 +361,63 @@ inline int grad_record_stride(int D, bool rg) {
     return (n + 1) / 2 * 2;
 }
 
-// Gather entries whose loads the FP32 gradient and update kernels issue
-// together before any arithmetic (the gradient kernel takes any further
-// entries one at a time, the update in further groups of the same size).
-// Fewer in flight is slower: O-grid gradients 0.97 -> 1.54 ms per step
-// with three, 1.89 with two.
+// 2D packed words lie together per cell (one 16-byte load), 3D ones as slots do
 template <int D>
-struct GradUnroll32 {
-    static constexpr int value = GatherUnroll<D>::value;
-};
-template <int D>
-struct UpdateUnroll32 {
-    static constexpr int value = GatherUnroll<D>::value;
-};
-
-// gather entry j of cell c (entry e of the list): its side, other cell,
-// weight and area vector.  SL: from the per-cell face slots for the first
-// GatherUnroll entries (streamed, no face index to chase); otherwise, and
-// beyond them, from the gather list and the face arrays.
-template <int D, bool SL>
-__device__ __forceinline__ void gather_entry32(const KArgs32 &a, const int c, const int e, const int j, bool &isP,
-                                               int &other, float &w, float (&S)[D]) {
-    if (SL && j < GatherUnroll<D>::value) {
-        const int key = ld_once<D, 1>(a.sl_nb + slot_at<D, 1>(a.nc, j, 0, c));
-        isP = key >= 0;
-        other = isP ? key : ~key;
-        w = ld_once<D, 1>(a.sl_w + slot_at<D, 1>(a.nc, j, 0, c));
-#pragma unroll
-        for (int k = 0; k < D; k++) S[k] = ld_once<D, 1>(a.sl_S + slot_at<D, D>(a.nc, j, k, c));
-        return;
-    }
-    const int ent = a.g_ent[e];
-    isP = ent >= 0;
-    const int f = isP ? (ent & kFaceMask) : ~ent;
-    other = isP ? a.fN[f] : a.fP[f];
-    w = a.w[f];
-    load_S32<D>(a.S, f, S);
+__device__ __forceinline__ size_t pk_at(int nc, int j, int c) {
+    if constexpr (D == 2) return (size_t)GatherUnroll<2>::value * c + j;
+    return slot_at<D, 1>(nc, j, 0, c);
 }
+inline size_t pk_len(int D, int nc, int U) { return D == 2 ? (size_t)U * nc : slot_array_len(nc, U, 1); }
+
+// one face as one of its cells sees it: the other cell, the area vector out
+// of the cell and the cell's weight (the other's is 1 - wc, exactly:
+// canonical_w)
+template <int D, bool PK>
+struct FaceOf32 {
+    int other;
+    float S[D], wc;
+    // key: the packed word, or the slot's other cell
+    __device__ __forceinline__ static int load_key(const KArgs32 &a, const int j, const int c) {
+        if constexpr (PK) return (int)ld_once<D, 1>(a.pk + pk_at<D>(a.nc, j, c));
+        return ld_once<D, 1>(a.sl_nb + slot_at<D, 1>(a.nc, j, 0, c));
+    }
+    __device__ __forceinline__ static int other_of(const KArgs32 &a, const int key) {
+        if constexpr (PK) return (int)((uint32_t)key & ((1u << a.pk_shift) - 1u));
+        return key;
+    }
+    __device__ __forceinline__ void load(const KArgs32 &a, const int j, const int c, const int key) {
+        other = other_of(a, key);
+        if constexpr (PK) {
+            const float4 v = reinterpret_cast<const float4 *>(a.pk_tab)[(uint32_t)key >> a.pk_shift];
+            const float r[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int k = 0; k < D; k++) S[k] = r[k];
+            wc = r[D];
+        } else {
+#pragma unroll
+            for (int k = 0; k < D; k++) S[k] = ld_once<D, 1>(a.sl_S + slot_at<D, D>(a.nc, j, k, c));
+            wc = ld_once<D, 1>(a.sl_w + slot_at<D, 1>(a.nc, j, 0, c));
+        }
+    }
+    // an entry of the gather list
+    __device__ __forceinline__ void load_list(const KArgs32 &a, const int ent) {
+        const bool isP = ent >= 0;
+        const int f = isP ? (ent & kFaceMask) : ~ent;
+        other = isP ? a.fN[f] : a.fP[f];
+        const float w = a.w[f];
+        load_S32<D>(a.S, f, S);
+#pragma unroll
+        for (int k = 0; k < D; k++) S[k] = isP ? S[k] : -S[k];
+        wc = isP ? w : 1.0f - w;
+    }
+};
 
 // Green-Gauss sums of one cell over its faces in gather order; returns the
-// cell's own primitive state
-template <int D, int GRAD, bool VISC, bool SL>
+// cell's own primitive state.  SL: every entry from the slots (3D); otherwise
+// from the gather list.  Each face's sums sit in a branch of their own: in one
+// block the compiler interleaves all six faces' arithmetic (124 VGPRs instead
+// of 96, 4 waves per SIMD instead of 5).
+template <int D, int GRAD, bool VISC, bool SL, bool PK>
 __device__ __forceinline__ Prim32<D> grad32_sums(const KArgs32 &a, const int c, float (&dudx)[D][D],
                                                   float (&dTdx)[D], float (&rg)[D], float (&pg)[D],
                                                   float (&ug)[D][D]) {
@@ -397,18 +431,18 @@ __device__ __forceinline__ Prim32<D> grad32_sums(const KArgs32 &a, const int c, 
     float qc0[D + 2];
     load_q32<D>(a, c, qc0);
     const Prim32<D> own = prim32<D>(a, qc0);
-    // one face's contribution (the face values use the face's own P/N order)
-    auto add = [&](const bool isP, const float w, const float (&S)[D], const float (&qo)[D + 2]) {
+    using F = FaceOf32<D, PK>;
+    // one face's contribution
+    auto add = [&](const F &f, const float (&qo)[D + 2]) {
         const Prim32<D> so = prim32<D>(a, qo);
-        const Prim32<D> &sp = isP ? own : so;
-        const Prim32<D> &sn = isP ? so : own;
+        const float wo = 1.0f - f.wc;
         float sv[D];
 #pragma unroll
-        for (int k = 0; k < D; k++) sv[k] = isP ? S[k] * vinv : -S[k] * vinv;
+        for (int k = 0; k < D; k++) sv[k] = f.S[k] * vinv;
         float fU[D];
 #pragma unroll
-        for (int k = 0; k < D; k++) fU[k] = LERP32(w, sp.up[k], sn.up[k]);
-        const float fT = VISC ? LERP32(w, sp.Rp, sn.Rp) * a.R_inv : 0.f;
+        for (int k = 0; k < D; k++) fU[k] = face_value32(f.wc, own.up[k], wo, so.up[k]);
+        const float fT = VISC ? face_value32(f.wc, own.Rp, wo, so.Rp) * a.R_inv : 0.f;
 #pragma unroll
         for (int i = 0; i < D; i++) {
 #pragma unroll
@@ -416,8 +450,8 @@ __device__ __forceinline__ Prim32<D> grad32_sums(const KArgs32 &a, const int c, 
             if (VISC) dTdx[i] += fT * sv[i];
         }
         if (GRAD == 2) {
-            const float rf = LERP32(w, sp.rp, sn.rp);
-            const float pf = LERP32(w, sp.pp, sn.pp);
+            const float rf = face_value32(f.wc, own.rp, wo, so.rp);
+            const float pf = face_value32(f.wc, own.pp, wo, so.pp);
 #pragma unroll
             for (int i = 0; i < D; i++) {
                 pg[i] += pf * sv[i];
@@ -427,42 +461,46 @@ __device__ __forceinline__ Prim32<D> grad32_sums(const KArgs32 &a, const int c, 
             }
         }
     };
-    // every entry in the slots (3D): the gather list's offsets are not read,
-    // a placeholder is known by its other cell, the cell itself
-    constexpr bool kAll = SL && GatherUnroll<D>::value >= kMaxFaces;
-    const int e0 = kAll ? 0 : a.g_off[c], ne = kAll ? kMaxFaces : a.g_off[c + 1] - e0;
+    constexpr int U = GatherUnroll<D>::value;
+    F f[U];
+    float qo[U][D + 2];
+    if constexpr (SL) {
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            f[j].load(a, j, c, F::load_key(a, j, c));
+            load_q32<D>(a, f[j].other, qo[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < U; j++)
+            if (f[j].other != c) add(f[j], qo[j]);  // not a placeholder's
+        return own;
+    }
     // the first faces: every load issued before the sums (a short list
-    // repeats its last face, whose terms are then not added)
-    constexpr int U = GradUnroll32<D>::value;
-    bool isP[U], valid[U];
-    float w[U], S[U][D], qo[U][D + 2];
+    // repeats its last face, whose terms are then not added).  Fewer in
+    // flight is slower: O-grid gradients 0.97 -> 1.54 ms per step with three,
+    // 1.89 with two.
+    const int e0 = a.g_off[c], ne = a.g_off[c + 1] - e0;
 #pragma unroll
     for (int j = 0; j < U; j++) {
-        // past the cell's last entry: the last entry again (list) or the
-        // slot's placeholder (slots), not added
-        const int jj = j < ne ? j : ne - 1;
-        int other;
-        gather_entry32<D, SL>(a, c, e0 + jj, SL ? j : jj, isP[j], other, w[j], S[j]);
-        valid[j] = kAll ? !(isP[j] && other == c) : j < ne;
-        load_q32<D>(a, other, qo[j]);
+        f[j].load_list(a, a.g_ent[e0 + (j < ne ? j : ne - 1)]);
+        load_q32<D>(a, f[j].other, qo[j]);
     }
 #pragma unroll
     for (int j = 0; j < U; j++)
-        if (valid[j]) add(isP[j], w[j], S[j], qo[j]);
+        if (j < ne) add(f[j], qo[j]);
     for (int e = e0 + U; e < e0 + ne; e++) {
-        bool p;
-        int other;
-        float wf, Sf[D], q[D + 2];
-        gather_entry32<D, SL>(a, c, e, e - e0, p, other, wf, Sf);
-        load_q32<D>(a, other, q);
-        add(p, wf, Sf, q);
+        F g;
+        float q[D + 2];
+        g.load_list(a, a.g_ent[e]);
+        load_q32<D>(a, g.other, q);
+        add(g, q);
     }
     return own;
 }
 
 // every thread of the block must call this (the block's records are written
 // through LDS); c = the block's first cell + threadIdx.x
-template <int D, int GRAD, bool VISC, bool RG, bool SL = false>
+template <int D, int GRAD, bool VISC, bool RG, bool SL = false, bool PK = false>
 __device__ __forceinline__ void grad_vis32_body(const KArgs32 &a, const int c) {
     using R = GradRec32<D, RG>;
     const bool valid = c < a.nc;
@@ -471,7 +509,7 @@ __device__ __forceinline__ void grad_vis32_body(const KArgs32 &a, const int c) {
     for (int k = 0; k < R::kStride; k++) r[k] = 0.f;
     if (valid) {
         float dudx[D][D], dTdx[D], rg[D], pg[D], ug[D][D];
-        const Prim32<D> own = grad32_sums<D, GRAD, VISC, SL>(a, c, dudx, dTdx, rg, pg, ug);
+        const Prim32<D> own = grad32_sums<D, GRAD, VISC, SL, PK>(a, c, dudx, dTdx, rg, pg, ug);
         // tauMC / sigmaU stored only where a halo payload needs them (otherwise
         // each face recomputes them from dudx); U_grad equals dudx bit for bit
         // (same face velocity, same sums) and shares its storage unless a halo
@@ -579,9 +617,69 @@ struct GradGlobal32 {
 // ---------------------------------------------------------------------------
 // face fluxes minus the freestream flux, one thread per face
 // ---------------------------------------------------------------------------
+// The convective flux of one face (M1 cfd_v0.cpp:2590-2637, M2 1968-2023)
+// seen from one of its cells: c the cell, o the other, S out of the cell.
+// Every face value is the same from both sides and every other term changes
+// sign with S, so the flux from N is P's negated, bit for bit, and the
+// one-launch stage forms a face from either side without selecting.
+template <int D>
+struct Conv32 {
+    float rp, rho, mp[D], phip, phi, pp, Gdev;
+};
+template <int D, int SOLVER, bool HALF>
+__device__ __forceinline__ Conv32<D> conv32(const KArgs32 &a, const float (&qc)[D + 2], const Prim32<D> &sc,
+                                            const float (&qo)[D + 2], const Prim32<D> &so, const float (&S)[D],
+                                            const float wc, const float wo) {
+    Conv32<D> f;
+    auto face = [&](const float c, const float o) {
+        if constexpr (SOLVER != 0) return midpoint32(c, o);
+        // every weight 1/2: the cell's own products are formed once per cell
+        if constexpr (HALF) return face_value32(0.5f, c, 0.5f, o);
+        return face_value32(wc, c, wo, o);
+    };
+    f.rp = face(qc[0], qo[0]);
+    f.rho = a.rho_inf + f.rp;
+    const float ri = rcp32(f.rho);
+    float phi_inf = 0.f, du2 = 0.f;
+    f.phip = 0.f;
+#pragma unroll
+    for (int k = 0; k < D; k++) {
+        phi_inf += a.uinf[k] * S[k];
+        f.mp[k] = face(qc[k + 1], qo[k + 1]);
+        const float up = (f.mp[k] - a.uinf[k] * f.rp) * ri;
+        f.phip += up * S[k];
+        if (SOLVER == 0) du2 += up * (2.f * a.uinf[k] + up);
+    }
+    f.phi = phi_inf + f.phip;
+    const float Rp = face(sc.Rp, so.Rp);
+    f.pp = f.rp * a.Rpsi_inf + f.rho * Rp;
+    // M1: G = rhoE + p = rho (g/(g-1) Rpsi + |u|^2/2) of the face state; M2:
+    // rho times the average of the cells' H = rhoE/rho + Rpsi
+    float Hp;
+    if constexpr (SOLVER == 0) {
+        Hp = a.gog * Rp + 0.5f * du2;
+    } else {
+        const float hc = a.gog * sc.Rp + 0.5f * sc.du2, ho = a.gog * so.Rp + 0.5f * so.du2;
+        Hp = midpoint32(hc, ho);
+    }
+    f.Gdev = f.rp * a.H_inf + f.rho * Hp;
+    return f;
+}
+// the face's rhs from its convective parts and pressure
+template <int D>
+__device__ __forceinline__ void conv_rhs32(const KArgs32 &a, const Conv32<D> &f, const float pp, const float (&S)[D],
+                                           float (&rhs)[D + 2]) {
+    float mS = 0.f;
+#pragma unroll
+    for (int k = 0; k < D; k++) mS += f.mp[k] * S[k];
+    rhs[0] = -mS;
+#pragma unroll
+    for (int k = 0; k < D; k++) rhs[k + 1] = -(f.phip * a.minf[k] + f.phi * f.mp[k] + pp * S[k]);
+    rhs[D + 1] = -(f.phip * a.G_inf + f.phi * f.Gdev);
+}
+
 // the flux of face f from its cells' states and primitives (qP, sp of P;
-// qN, sn of N), whoever loaded them: the face kernel loads both, the
-// one-launch stage holds its own cell's and loads the other
+// qN, sn of N)
 template <int D, int SOLVER, bool VISC, bool STORED, class GA>
 __device__ __forceinline__ void face_flux32_states(const KArgs32 &a, const int f, const int P, const int N,
                                                    const float (&qP)[D + 2], const float (&qN)[D + 2],
@@ -604,149 +702,86 @@ __device__ __forceinline__ void face_flux32_states(const KArgs32 &a, const int f
 #pragma unroll
     for (int k = 0; k < D; k++) Sm2 += S[k] * S[k];
     const float Sm = sqrt32(Sm2);
-    float phi_inf = 0.f;
+    const Conv32<D> cv = conv32<D, SOLVER, false>(a, qP, sp, qN, sn, S, w, 1.0f - w);
+    float pp = cv.pp;
+    if (SOLVER == 2) {
+        const float phi_inf = cv.phi - cv.phip;
+        const float cP = sqrt32(a.gamma * sp.R), cN = sqrt32(a.gamma * sn.R);
+        const float cavg = 0.5f * (cP + cN);
+        float cdiv = 0.f, ndiv = 0.f, ccurl = 0.f, ncurl = 0.f, unP = 0.f, unN = 0.f;
+        float cdu[D][D], ndu[D][D];
 #pragma unroll
-    for (int k = 0; k < D; k++) phi_inf += a.uinf[k] * S[k];
-
-    if (SOLVER == 0) {
-        // reconstructed state (cfd_v0.cpp:2590-2637): conservatives, Rpsi
-        // (hence p and e = Rpsi/(g-1)) interpolated linearly
-        const float rp = LERP32(w, qP[0], qN[0]);
-        const float rho = a.rho_inf + rp;
-        const float ri = rcp32(rho);
-        float mp[D], up[D];
-        float phip = 0.f, du2 = 0.f;
+        for (int i = 0; i < D; i++)
 #pragma unroll
-        for (int k = 0; k < D; k++) {
-            mp[k] = LERP32(w, qP[k + 1], qN[k + 1]);
-            up[k] = (mp[k] - a.uinf[k] * rp) * ri;
-            phip += up[k] * S[k];
-            du2 += up[k] * (2.f * a.uinf[k] + up[k]);
-        }
-        const float phi = phi_inf + phip;
-        const float Rp = LERP32(w, sp.Rp, sn.Rp);
-        const float pp = rp * a.Rpsi_inf + rho * Rp;
-        // G = rhoE + p = rho (g/(g-1) Rpsi + |u|^2/2), e = Rpsi/(g-1) per cell
-        float uinf2 = 0.f;
-#pragma unroll
-        for (int k = 0; k < D; k++) uinf2 += a.uinf[k] * a.uinf[k];
-        const float Gdev = rp * (a.gog * a.Rpsi_inf + 0.5f * uinf2) + rho * (a.gog * Rp + 0.5f * du2);
-        float mS = 0.f;
-#pragma unroll
-        for (int k = 0; k < D; k++) mS += mp[k] * S[k];
-        rhs[0] = -mS;
-#pragma unroll
-        for (int k = 0; k < D; k++) rhs[k + 1] = -(phip * a.minf[k] + phi * mp[k] + pp * S[k]);
-        rhs[D + 1] = -(phip * a.G_inf + phi * Gdev);
-    } else {
-        // midpoint averages (cfd_v0.cpp:1968-2023)
-        const float rp = 0.5f * (qP[0] + qN[0]);
-        const float rho = a.rho_inf + rp;
-        const float ri = rcp32(rho);
-        float mp[D], up[D];
-        float phip = 0.f;
-#pragma unroll
-        for (int k = 0; k < D; k++) {
-            mp[k] = 0.5f * (qP[k + 1] + qN[k + 1]);
-            up[k] = (mp[k] - a.uinf[k] * rp) * ri;
-            phip += up[k] * S[k];
-        }
-        const float phi = phi_inf + phip;
-        const float Rp = 0.5f * (sp.Rp + sn.Rp);
-        float pp = rp * a.Rpsi_inf + rho * Rp;
-        // H = rhoE/rho + Rpsi = g/(g-1) Rpsi + |u|^2/2 per cell, averaged
-        float duP = 0.f, duN = 0.f;
-#pragma unroll
-        for (int k = 0; k < D; k++) {
-            duP += sp.up[k] * (2.f * a.uinf[k] + sp.up[k]);
-            duN += sn.up[k] * (2.f * a.uinf[k] + sn.up[k]);
-        }
-        const float Hp = 0.5f * ((a.gog * sp.Rp + 0.5f * duP) + (a.gog * sn.Rp + 0.5f * duN));
-        const float Gdev = rp * a.H_inf + rho * Hp;
-        if (SOLVER == 2) {
-            const float cP = sqrt32(a.gamma * sp.R), cN = sqrt32(a.gamma * sn.R);
-            const float cavg = 0.5f * (cP + cN);
-            float cdiv = 0.f, ndiv = 0.f, ccurl = 0.f, ncurl = 0.f, unP = 0.f, unN = 0.f;
-            float cdu[D][D], ndu[D][D];
-#pragma unroll
-            for (int i = 0; i < D; i++)
-#pragma unroll
-                for (int j = 0; j < D; j++) {
-                    cdu[i][j] = gr[0][i * D + j];
-                    ndu[i][j] = gr[1][i * D + j];
-                }
-#pragma unroll
-            for (int p = 0; p < D; p++) {
-                cdiv += cdu[p][p];
-                ndiv += ndu[p][p];
-#pragma unroll
-                for (int b = p + 1; b < D; b++) {
-                    ccurl += (cdu[p][b] - cdu[b][p]) * (cdu[p][b] - cdu[b][p]);
-                    ncurl += (ndu[p][b] - ndu[b][p]) * (ndu[p][b] - ndu[b][p]);
-                }
-                float gc[D], gn[D];
-#pragma unroll
-                for (int k = 0; k < D; k++) {
-                    gc[k] = ga.ug(gr[0], gP, p, k);
-                    gn[k] = ga.ug(gr[1], gN, p, k);
-                }
-                unP += minmod32<D>(sp.up[p], sn.up[p], gc, d, w, 1.0f) * S[p];
-                unN += minmod32<D>(sp.up[p], sn.up[p], gn, d, w, -1.0f) * S[p];
+            for (int j = 0; j < D; j++) {
+                cdu[i][j] = gr[0][i * D + j];
+                ndu[i][j] = gr[1][i * D + j];
             }
-            const float cth0 = -cdiv * rsq32(cdiv * cdiv + ccurl + 4e-2f);
-            const float nth0 = -ndiv * rsq32(ndiv * ndiv + ncurl + 4e-2f);
-            const float tha = 0.5f * (((cth0 < 0.f) ? 0.f : cth0) + ((nth0 < 0.f) ? 0.f : nth0));
-            float gc[D], gn[D], hc[D], hn[D];
+#pragma unroll
+        for (int p = 0; p < D; p++) {
+            cdiv += cdu[p][p];
+            ndiv += ndu[p][p];
+#pragma unroll
+            for (int b = p + 1; b < D; b++) {
+                ccurl += (cdu[p][b] - cdu[b][p]) * (cdu[p][b] - cdu[b][p]);
+                ncurl += (ndu[p][b] - ndu[b][p]) * (ndu[p][b] - ndu[b][p]);
+            }
+            float gc[D], gn[D];
 #pragma unroll
             for (int k = 0; k < D; k++) {
-                gc[k] = gr[0][R::kRG + k];
-                gn[k] = gr[1][R::kRG + k];
-                hc[k] = gr[0][R::kPG + k];
-                hn[k] = gr[1][R::kPG + k];
+                gc[k] = ga.ug(gr[0], gP, p, k);
+                gn[k] = ga.ug(gr[1], gN, p, k);
             }
-            const float rhoPos = a.rho_inf + minmod32<D>(sp.rp, sn.rp, gc, d, w, 1.0f);
-            const float rhoNeg = a.rho_inf + minmod32<D>(sp.rp, sn.rp, gn, d, w, -1.0f);
-            const float pPd = minmod32<D>(sp.pp, sn.pp, hc, d, w, 1.0f);
-            const float pNd = minmod32<D>(sp.pp, sn.pp, hn, d, w, -1.0f);
-            const float unPf = phi_inf + unP, unNf = phi_inf + unN;
-            const float rSc = rcp32(Sm * cavg);
-            const float MP = unPf * rSc;
-            const float MN = unNf * rSc;
-            const float Msq = 0.5f * (MP * MP + MN * MN);
-            const float Minf = 0.2f;
-            const float mx = (Msq < Minf * Minf) ? Minf * Minf : Msq;
-            const float M0 = sqrt32((mx < 1.0f) ? mx : 1.0f);
-            const float fa = M0 * (2.0f - M0);
-            const float alpha = 3.0f * (5.0f * fa * fa - 4.0f) / 16.0f;
-            const float dN = p5pos32(MN, alpha) - p5neg32(MN, alpha);
-            const float dP = p5pos32(MP, alpha) - p5neg32(MP, alpha);
-            // p_half = pN dN - pP dP = p_inf (dN - dP) + pN' dN - pP' dP.  For
-            // |M| < 1, P5+(M) - P5-(M) = M (3 - M^2)/2 + 2 alpha M (1 - M^2)^2, so
-            // dN - dP is formed as (MN - MP) times its divided difference, with
-            // MN - MP from the normal-velocity deviations (no cancellation).
-            float dNP;
-            if (fabsf(MN) < 1.f && fabsf(MP) < 1.f) {
-                const float s2 = MN * MN + MN * MP + MP * MP;
-                const float s4 = MN * MN * MN * MN + MN * MN * MN * MP + MN * MN * MP * MP + MN * MP * MP * MP +
-                                 MP * MP * MP * MP;
-                const float dd = 0.5f * (3.f - s2) + 2.f * alpha * (1.f - 2.f * s2 + s4);
-                dNP = (unN - unP) * rSc * dd;
-            } else {
-                dNP = dN - dP;
-            }
-            const float phalf = a.p_inf * dNP + pNd * dN - pPd * dP;
-            const float pu = -0.75f * p5pos32(MP, alpha) * p5neg32(MN, alpha) * (rhoPos + rhoNeg) * cavg * fa *
-                             (unN - unP);
-            pp += tha * (pu - 0.5f * phalf);
+            unP += minmod32<D>(sp.up[p], sn.up[p], gc, d, w, 1.0f) * S[p];
+            unN += minmod32<D>(sp.up[p], sn.up[p], gn, d, w, -1.0f) * S[p];
         }
-        float mS = 0.f;
+        const float cth0 = -cdiv * rsq32(cdiv * cdiv + ccurl + 4e-2f);
+        const float nth0 = -ndiv * rsq32(ndiv * ndiv + ncurl + 4e-2f);
+        const float tha = 0.5f * (((cth0 < 0.f) ? 0.f : cth0) + ((nth0 < 0.f) ? 0.f : nth0));
+        float gc[D], gn[D], hc[D], hn[D];
 #pragma unroll
-        for (int k = 0; k < D; k++) mS += mp[k] * S[k];
-        rhs[0] = -mS;
-#pragma unroll
-        for (int k = 0; k < D; k++) rhs[k + 1] = -(phip * a.minf[k] + phi * mp[k] + pp * S[k]);
-        rhs[D + 1] = -(phip * a.G_inf + phi * Gdev);
+        for (int k = 0; k < D; k++) {
+            gc[k] = gr[0][R::kRG + k];
+            gn[k] = gr[1][R::kRG + k];
+            hc[k] = gr[0][R::kPG + k];
+            hn[k] = gr[1][R::kPG + k];
+        }
+        const float rhoPos = a.rho_inf + minmod32<D>(sp.rp, sn.rp, gc, d, w, 1.0f);
+        const float rhoNeg = a.rho_inf + minmod32<D>(sp.rp, sn.rp, gn, d, w, -1.0f);
+        const float pPd = minmod32<D>(sp.pp, sn.pp, hc, d, w, 1.0f);
+        const float pNd = minmod32<D>(sp.pp, sn.pp, hn, d, w, -1.0f);
+        const float unPf = phi_inf + unP, unNf = phi_inf + unN;
+        const float rSc = rcp32(Sm * cavg);
+        const float MP = unPf * rSc;
+        const float MN = unNf * rSc;
+        const float Msq = 0.5f * (MP * MP + MN * MN);
+        const float Minf = 0.2f;
+        const float mx = (Msq < Minf * Minf) ? Minf * Minf : Msq;
+        const float M0 = sqrt32((mx < 1.0f) ? mx : 1.0f);
+        const float fa = M0 * (2.0f - M0);
+        const float alpha = 3.0f * (5.0f * fa * fa - 4.0f) / 16.0f;
+        const float dN = p5pos32(MN, alpha) - p5neg32(MN, alpha);
+        const float dP = p5pos32(MP, alpha) - p5neg32(MP, alpha);
+        // p_half = pN dN - pP dP = p_inf (dN - dP) + pN' dN - pP' dP.  For
+        // |M| < 1, P5+(M) - P5-(M) = M (3 - M^2)/2 + 2 alpha M (1 - M^2)^2, so
+        // dN - dP is formed as (MN - MP) times its divided difference, with
+        // MN - MP from the normal-velocity deviations (no cancellation).
+        float dNP;
+        if (fabsf(MN) < 1.f && fabsf(MP) < 1.f) {
+            const float s2 = MN * MN + MN * MP + MP * MP;
+            const float s4 = MN * MN * MN * MN + MN * MN * MN * MP + MN * MN * MP * MP + MN * MP * MP * MP +
+                             MP * MP * MP * MP;
+            const float dd = 0.5f * (3.f - s2) + 2.f * alpha * (1.f - 2.f * s2 + s4);
+            dNP = (unN - unP) * rSc * dd;
+        } else {
+            dNP = dN - dP;
+        }
+        const float phalf = a.p_inf * dNP + pNd * dN - pPd * dP;
+        const float pu = -0.75f * p5pos32(MP, alpha) * p5neg32(MN, alpha) * (rhoPos + rhoNeg) * cavg * fa *
+                         (unN - unP);
+        pp += tha * (pu - 0.5f * phalf);
     }
+    conv_rhs32<D>(a, cv, pp, S, rhs);
 
     // viscous terms (cfd_v0.cpp:2682-2790) on velocity / temperature deviations
     if (VISC) {
@@ -875,129 +910,24 @@ __device__ __forceinline__ void face_flux32_body(const KArgs32 &a, const int f) 
 // ---------------------------------------------------------------------------
 // ordered gather of face fluxes, sponge, RK update (deviations)
 // ---------------------------------------------------------------------------
-// What the ordered gather of a cell (cell_update32_cell) asks of its source
-// of face data, for the cell's j-th gather entry e (j < kMaxFaces, known at
-// compile time wherever the gather calls these):
-//   key(e, j, c)       an entry key, >= 0 where the cell is the face's P;
-//   ghost(key)         the boundary ghost behind a P entry, else -1;
-//   get(e, j, key, r)  the face's flux;
-//   area(e, j, c, S)   the face's area vector, negated on N entries.
-// kUnroll entries have their loads issued together.  FaceList32 reads the
-// gather list (key = the signed face index with the ghost flag);
-// FluxGlobal32 adds the stored face fluxes.
+// the cell's RK register as the last stage left it, zero at a step's first
+// stage: every component's load issued before any is used (a choice per
+// component compiles to a branch and a wait each)
 template <int D>
-struct FaceList32 {
-    const KArgs32 &a;
-    static constexpr int kUnroll = UpdateUnroll32<D>::value;
-    static constexpr bool kAllSlots = false;
-    static constexpr bool kSlotsFirst = false;
-    __device__ __forceinline__ static bool valid(int key, int c) { return (void)key, (void)c, true; }
-    __device__ __forceinline__ void begin_cell(int c) const { (void)c; }
-    __device__ __forceinline__ int key(int e, int j, int c) const {
-        (void)j;
-        (void)c;
-        return a.g_ent[e];
-    }
-    __device__ __forceinline__ int ghost(int key) const {
-        return (key >= 0 && (key & kGhostFaceFlag)) ? a.fN[key & kFaceMask] - a.nc : -1;
-    }
-    __device__ __forceinline__ static int face(int key) { return key >= 0 ? (key & kFaceMask) : ~key; }
-    __device__ __forceinline__ void area(int e, int j, int c, float (&S)[D]) const {
-        const int key = this->key(e, j, c);
-        load_S32<D>(a.S, face(key), S);
+__device__ __forceinline__ void load_dq32(const KArgs32 &a, const int zero_dq, const int c, float (&dq)[D + 2]) {
 #pragma unroll
-        for (int k = 0; k < D; k++) S[k] = key >= 0 ? S[k] : -S[k];
+    for (int k = 0; k < D + 2; k++) dq[k] = 0.f;
+    if (!zero_dq) {
+#pragma unroll
+        for (int k = 0; k < D + 2; k++) dq[k] = ld_once<D, 2>(a.dq + (size_t)k * a.nc + c);
     }
-};
+}
 
+// sponge, RK update and stores of one cell: q its state (the updated one on
+// return), dq its accumulated register
 template <int D>
-struct FluxGlobal32 : FaceList32<D> {
-    using FaceList32<D>::a;
-    using FaceList32<D>::face;
-    // the flux of gather entry e
-    __device__ __forceinline__ void get(int e, int j, int key, float (&r)[D + 2]) const {
-        (void)e;
-        (void)j;
-        const int f = face(key);
-        const float4 v = reinterpret_cast<const float4 *>(a.frhs)[f];
-        r[0] = v.x;
-        r[1] = v.y;
-        r[2] = v.z;
-        r[3] = v.w;
-        if (D == 3) r[D + 1] = a.frhs[(size_t)4 * a.nf + f];
-    }
-};
-// ordered gather of one cell's face fluxes, sponge and RK update from the
-// state in a.q, written to qout (a.q itself for the in-place update) with
-// the cell's boundary ghosts refreshed there; res receives the residual, q
-// the updated state
-template <int D, bool RES, class FA>
-__device__ __forceinline__ void cell_update32_cell(const KArgs32 &a, const FA &fa, float A, float B, int zero_dq,
-                                                   const int c, float *qout, float (&res)[D + 2],
-                                                   float (&q)[D + 2], float &vinv) {
-    const float dt = (float)(*a.dt);
-    vinv = ld_once<D, 3>(a.vinv + c);
-    float dq[D + 2];
-#pragma unroll
-    for (int k = 0; k < D + 2; k++) {
-        dq[k] = zero_dq ? 0.f : ld_once<D, 2>(a.dq + (size_t)k * a.nc + c) * A;
-        res[k] = 0.f;
-    }
-    // kAllSlots: every entry is in the face slots (placeholders past the
-    // last), so the gather list's offsets are not read; the group count is
-    // then kept opaque to the compiler, which would otherwise set up every
-    // group's addresses at once and spill
-    int e0, ne;
-    if constexpr (FA::kAllSlots) {
-        e0 = 0;
-        ne = kMaxFaces;
-        asm volatile("" : "+s"(ne));
-    } else {
-        e0 = a.g_off[c];
-        ne = a.g_off[c + 1] - e0;
-    }
-    unsigned gmask = 0;  // bit j: entry j leads to a boundary ghost
-    // entry j's flux added (valid: j is one of the cell's entries; an
-    // invalid one is selected away, not branched around, so that the loads
-    // of a group stay together)
-    auto add = [&](const int j, const bool valid, const int key, const float (&fr)[D + 2]) {
-        gmask |= valid && fa.ghost(key) >= 0 ? 1u << j : 0u;
-        const float sg = key >= 0 ? 1.f : -1.f;
-#pragma unroll
-        for (int k = 0; k < D + 2; k++) {
-            const float r = valid ? sg * fr[k] : 0.f;
-            if (RES) res[k] = valid ? res[k] + r : res[k];
-            dq[k] = valid ? dq[k] + dt * r * vinv : dq[k];
-        }
-    };
-    // the faces in gather order, kUnroll at a time with their loads issued
-    // together (a cell has at most kMaxFaces).  Within a group no branch: an
-    // entry past the cell's last reads the last entry again (list) or the
-    // slot's placeholder, and is not added.
-    constexpr int U = FA::kUnroll;
-    fa.begin_cell(c);
-#pragma unroll
-    for (int j0 = 0; j0 < kMaxFaces; j0 += U) {
-        // every cell has a first group: where its loads do not address
-        // through the gather list, they need not wait for ne
-        if ((j0 == 0 && FA::kSlotsFirst) || j0 < ne) {
-            int key[U];
-            float fr[U][D + 2];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int j = j0 + u;
-                if (j < kMaxFaces) {
-                    const int e = e0 + (j < ne ? j : ne - 1);
-                    key[u] = fa.key(e, j, c);
-                    fa.get(e, j, key[u], fr[u]);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++)
-                if (j0 + u < kMaxFaces) add(j0 + u, FA::kAllSlots ? fa.valid(key[u], c) : j0 + u < ne, key[u], fr[u]);
-        }
-    }
-    load_q32<D>(a, c, q);
+__device__ __forceinline__ void finish_cell32(const KArgs32 &a, const int c, const float dt, const float B, float *qout,
+                                              float (&q)[D + 2], float (&dq)[D + 2]) {
     // sponge: sigma (q_inf - q) = -sigma q' (no sigma array, and no term,
     // where the case has no sponge layer and every sigma is zero)
     const float sgm = a.sigma ? ld_once<D, 3>(a.sigma + c) : 0.f;
@@ -1008,18 +938,86 @@ __device__ __forceinline__ void cell_update32_cell(const KArgs32 &a, const FA &f
         st_once<D, 2>(a.dq + (size_t)k * a.nc + c, dq[k]);
     }
     store_q32<D>(qout, a.ntot, c, q);
-    // refresh this cell's boundary ghosts for the next stage
-    for (unsigned m = gmask; m; m &= m - 1) {
-        const int j = __builtin_ctz(m);
-        const int g = fa.ghost(fa.key(e0 + j, j, c));
-        float qg[D + 2];
-        if (!ghost_state32<D>(a, a.ghost_role[g], q, qg)) {
-            if (qout == a.q) continue;
-            load_q32<D>(a, a.nc + g, qg);  // an unset patch's ghost keeps its state
-        }
-        store_q32<D>(qout, a.ntot, a.nc + g, qg);
-    }
 }
+// boundary ghost g of a cell whose updated state is q, written for the next
+// stage
+template <int D>
+__device__ __forceinline__ void refresh_ghost32(const KArgs32 &a, const int g, float *qout, const float (&q)[D + 2]) {
+    float qg[D + 2];
+    if (!ghost_state32<D>(a, a.ghost_role[g], q, qg)) {
+        if (qout == a.q) return;
+        load_q32<D>(a, a.nc + g, qg);  // an unset patch's ghost keeps its state
+    }
+    store_q32<D>(qout, a.ntot, a.nc + g, qg);
+}
+
+// ordered gather of one cell's stored face fluxes, sponge and RK update in
+// place, with the cell's boundary ghosts refreshed; res receives the
+// residual, q the updated state
+template <int D, bool RES>
+__device__ __forceinline__ void cell_update32_cell(const KArgs32 &a, float A, float B, int zero_dq, const int c,
+                                                   float (&res)[D + 2], float (&q)[D + 2], float &vinv) {
+    const float dt = (float)(*a.dt);
+    vinv = ld_once<D, 3>(a.vinv + c);
+    const float sP = dt * vinv;
+    float dq[D + 2];
+    load_dq32<D>(a, zero_dq, c, dq);
+#pragma unroll
+    for (int k = 0; k < D + 2; k++) res[k] = 0.f;
+    load_q32<D>(a, c, q);
+    const int e0 = a.g_off[c], ne = a.g_off[c + 1] - e0;
+    unsigned gmask = 0;  // bit j: entry j leads to a boundary ghost
+    // the faces in gather order, U at a time with their loads issued
+    // together (a cell has at most kMaxFaces).  Within a group no branch: an
+    // entry past the cell's last reads the last entry again and is selected
+    // away.
+    constexpr int U = GatherUnroll<D>::value;
+#pragma unroll
+    for (int j0 = 0; j0 < kMaxFaces; j0 += U) {
+        if (j0 < ne) {
+            int key[U];
+            float fr[U][D + 2];
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (j0 + u < kMaxFaces) key[u] = a.g_ent[e0 + (j0 + u < ne ? j0 + u : ne - 1)];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (j0 + u < kMaxFaces) {
+                    const int f = key[u] >= 0 ? (key[u] & kFaceMask) : ~key[u];
+                    const float4 v = reinterpret_cast<const float4 *>(a.frhs)[f];
+                    fr[u][0] = v.x;
+                    fr[u][1] = v.y;
+                    fr[u][2] = v.z;
+                    fr[u][3] = v.w;
+                    if (D == 3) fr[u][D + 1] = a.frhs[(size_t)4 * a.nf + f];
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < D + 2; k++) dq[k] = j0 == 0 ? dq[k] * A : dq[k];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (j0 + u < kMaxFaces) {
+                    const bool valid = j0 + u < ne;
+                    gmask |= valid && key[u] >= 0 && (key[u] & kGhostFaceFlag) ? 1u << (j0 + u) : 0u;
+                    const float sg = key[u] >= 0 ? sP : -sP;
+#pragma unroll
+                    for (int k = 0; k < D + 2; k++) {
+                        if (RES) res[k] = valid ? res[k] + (key[u] >= 0 ? fr[u][k] : -fr[u][k]) : res[k];
+                        dq[k] = valid ? dq[k] + sg * fr[u][k] : dq[k];
+                    }
+                }
+            }
+        }
+    }
+    finish_cell32<D>(a, c, dt, B, a.q, q, dq);
+    // refresh this cell's boundary ghosts for the next stage
+    for (unsigned m = gmask; m; m &= m - 1)
+        refresh_ghost32<D>(a, a.fN[a.g_ent[e0 + __builtin_ctz(m)] & kFaceMask] - a.nc, a.q, q);
+}
+
+template <int D, int MODE>
+__device__ __forceinline__ double cfl_cell32(const KArgs32 &a, const int c, const float (&qc)[D + 2], float vinv,
+                                             double param);
 
 template <int D, int MODE, class FA>
 __device__ __forceinline__ double cfl_cell32(const KArgs32 &a, const FA &fa, const int c, const float (&qc)[D + 2],
@@ -1028,9 +1026,9 @@ __device__ __forceinline__ double cfl_cell32(const KArgs32 &a, const FA &fa, con
 // every thread of the block must call this (block-wide reductions when RES
 // or CFL).  CFL >= 0 (the last stage of a step): the step's compute_dt (0) /
 // compute_cfl (1) of the updated cells, per-block extrema into a.partial.
-template <int D, bool RES, int CFL, class FA>
-__device__ __forceinline__ void cell_update32_body(const KArgs32 &a, const FA &fa, float *qout, float A, float B,
-                                                   int zero_dq, const int c, const int lblk, double cfl_param) {
+template <int D, bool RES, int CFL>
+__device__ __forceinline__ void cell_update32_body(const KArgs32 &a, float A, float B, int zero_dq, const int c,
+                                                   const int lblk, double cfl_param) {
     static_assert(!(RES && CFL >= 0), "the residual and the CFL share a.partial");
     __shared__ double red[256 / 64][D + 2];
     double rsq[D + 2];
@@ -1039,8 +1037,8 @@ __device__ __forceinline__ void cell_update32_body(const KArgs32 &a, const FA &f
     for (int k = 0; k < D + 2; k++) rsq[k] = 0.0;
     if (c < a.nc) {
         float res[D + 2], q[D + 2], vinv;
-        cell_update32_cell<D, RES>(a, fa, A, B, zero_dq, c, qout, res, q, vinv);
-        if constexpr (CFL >= 0) cv = cfl_cell32<D, CFL>(a, fa, c, q, vinv, cfl_param);
+        cell_update32_cell<D, RES>(a, A, B, zero_dq, c, res, q, vinv);
+        if constexpr (CFL >= 0) cv = cfl_cell32<D, CFL>(a, c, q, vinv, cfl_param);
         if (RES) {
 #pragma unroll
             for (int k = 0; k < D + 2; k++) {
@@ -1071,46 +1069,58 @@ __device__ __forceinline__ void cell_update32_body(const KArgs32 &a, const FA &f
 }
 
 // compute_dt / compute_cfl (cfd_v0.cpp:2887-2942) of one cell from its FP32
-// deviations q: the face terms |m.S| (compute_cfl) or |m.S|/|S| (compute_dt)
+// deviations: the face terms |m.S| (compute_cfl) or |m.S|/|S| (compute_dt)
 // summed in FP32 over the cell's faces in gather order (the update's own
-// list, whose entries and area vectors it has just read; the FP64 path keeps
-// the reference's slot order), then dt_c (MODE 0) or cfl_c (MODE 1) in FP64,
-// combined with the block's starting value so a NaN never wins; vinv:
-// the cell's 1/V, as the update read it
-template <int D, int MODE, class FA>
-__device__ __forceinline__ double cfl_cell32(const KArgs32 &a, const FA &fa, const int c, const float (&qc)[D + 2],
-                                             float vinv_c, double param) {
-    float m[D];
+// order; the FP64 path keeps the reference's slot order), then dt_c (MODE 0)
+// or cfl_c (MODE 1) in FP64, combined with the block's starting value so a
+// NaN never wins; vinv: the cell's 1/V, as the update read it
+template <int D, int MODE>
+struct CflSum32 {
+    float m[D], sum = 0.f;
+    __device__ __forceinline__ CflSum32(const KArgs32 &a, const float (&qc)[D + 2]) {
 #pragma unroll
-    for (int k = 0; k < D; k++) m[k] = a.minf[k] + qc[k + 1];
-    // kAllSlots: every entry in the slots, a placeholder known by its zero
-    // area vector (a face has a nonzero one)
-    const int e0 = FA::kAllSlots ? 0 : a.g_off[c];
-    const int ne = FA::kAllSlots ? kMaxFaces : a.g_off[c + 1] - e0;
-    float sum = 0.f;
-#pragma unroll
-    for (int j = 0; j < kMaxFaces; j++) {
-        float S[D];
-        fa.area(e0 + (j < ne ? j : ne - 1), j, c, S);
+        for (int k = 0; k < D; k++) m[k] = a.minf[k] + qc[k + 1];
+    }
+    // a face of either orientation; valid: false leaves the sum
+    __device__ __forceinline__ void add(const float (&S)[D], const bool valid) {
         float fl = 0.f, s2 = 0.f;
 #pragma unroll
         for (int k = 0; k < D; k++) fl += m[k] * S[k];
+        if (MODE == 0) {
 #pragma unroll
-        for (int k = 0; k < D; k++) s2 += S[k] * S[k];
-        if (MODE == 0) fl *= rsq32(s2);
-        sum = (FA::kAllSlots ? s2 > 0.f : j < ne) ? sum + fabsf(fl) : sum;
+            for (int k = 0; k < D; k++) s2 += S[k] * S[k];
+            fl *= rsq32(s2);
+        }
+        sum = valid ? sum + fabsf(fl) : sum;
     }
-    const double rho = a.rho_inf_d + (double)qc[0];
-    const double vinv = (double)vinv_c;
-    double v = MODE == 0 ? 100.0 : 0.0;
-    if (MODE == 0) {
-        const double dtc = param * rho * 2.0 / (vinv * (double)sum);
-        if (v > dtc) v = dtc;
-    } else {
-        const double cfl = (double)sum * ((1.0 / rho) * vinv * param);
-        if (v < cfl) v = cfl;
+    __device__ __forceinline__ double value(const KArgs32 &a, const float rp, const float vinv_c,
+                                            const double param) const {
+        const double rho = a.rho_inf_d + (double)rp;
+        const double vinv = (double)vinv_c;
+        double v = MODE == 0 ? 100.0 : 0.0;
+        if (MODE == 0) {
+            const double dtc = param * rho * 2.0 / (vinv * (double)sum);
+            if (v > dtc) v = dtc;
+        } else {
+            const double cfl = (double)sum * ((1.0 / rho) * vinv * param);
+            if (v < cfl) v = cfl;
+        }
+        return v;
     }
-    return v;
+};
+template <int D, int MODE>
+__device__ __forceinline__ double cfl_cell32(const KArgs32 &a, const int c, const float (&qc)[D + 2], float vinv,
+                                             double param) {
+    CflSum32<D, MODE> t(a, qc);
+    const int e0 = a.g_off[c], ne = a.g_off[c + 1] - e0;
+#pragma unroll
+    for (int j = 0; j < kMaxFaces; j++) {
+        const int ent = a.g_ent[e0 + (j < ne ? j : ne - 1)];
+        float S[D];
+        load_S32<D>(a.S, ent >= 0 ? (ent & kFaceMask) : ~ent, S);
+        t.add(S, j < ne);
+    }
+    return t.value(a, qc[0], vinv, param);
 }
 
 // compute_dt / compute_cfl as their own launch (every thread of the block
@@ -1121,7 +1131,7 @@ __device__ __forceinline__ void cfl_dt_cells32_body(const KArgs32 &a, double par
     if (c < a.nc) {
         float q[D + 2];
         load_q32<D>(a, c, q);
-        v = cfl_cell32<D, MODE>(a, FaceList32<D>{a}, c, q, a.vinv[c], param);
+        v = cfl_cell32<D, MODE>(a, c, q, a.vinv[c], param);
     }
     block_extremum<MODE>(v, a.partial + lblk);
 }
@@ -1179,7 +1189,7 @@ __global__ void __launch_bounds__(256) bc_fill32(KArgs32 a) {
 // fin_nblk > 0: one block more, the last, reduces the previous step's
 // fin_nblk per-block CFL maxima in a.partial into *a.d_cfl (as the one-launch
 // stage does)
-template <int D, int GRAD, bool VISC, bool RG, bool SL>
+template <int D, int GRAD, bool VISC, bool RG, bool SL, bool PK>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 3 && SL && !RG ? 5 : 1)))
 grad_vis32(KArgs32 a, int fin_nblk) {
     int nb = (int)gridDim.x;
@@ -1190,7 +1200,7 @@ grad_vis32(KArgs32 a, int fin_nblk) {
             return;
         }
     }
-    grad_vis32_body<D, GRAD, VISC, RG, SL>(a, xcd_block((int)blockIdx.x, nb) * (int)blockDim.x + (int)threadIdx.x);
+    grad_vis32_body<D, GRAD, VISC, RG, SL, PK>(a, xcd_block((int)blockIdx.x, nb) * (int)blockDim.x + (int)threadIdx.x);
 }
 // 3D M1 / M2 faces: 5 waves per SIMD fit in 96 VGPRs without spills (97
 // would allow 4): O-grid face kernel 1.107 -> 1.033 ms per step.  Forcing
@@ -1202,148 +1212,188 @@ face_flux32(KArgs32 a) {
 }
 template <int D, bool RES, int CFL>
 __global__ void __launch_bounds__(256) cell_update32(KArgs32 a, float A, float B, int zero_dq, double cfl_param) {
-    cell_update32_body<D, RES, CFL>(a, FluxGlobal32<D>{a}, a.q, A, B, zero_dq, LFM_TID(blockIdx.x), LFM_BLK(),
-                                    cfl_param);
+    cell_update32_body<D, RES, CFL>(a, A, B, zero_dq, LFM_TID(blockIdx.x), LFM_BLK(), cfl_param);
 }
-// Where a fused stage takes a face's flux: computed where it is gathered, by
-// the face kernel's own function, from the stage's input state a.q
-// (inviscid M1 / M2: no gradients), with the gathering cell's state and
-// primitives loaded and formed once per cell.  The face data come from the
-// cell's slots (a.sl_*: streamed, one per gather entry) for its first
-// GatherUnroll entries (all of a 3D cell's) and from the face arrays beyond
-// them.  Each interior
-// face is computed by both of its cells, to the same bits as the face
-// kernel's (the same function of the same values).
-template <int D, int SOLVER>
-struct FluxSlots32 {
-    const KArgs32 &a;
-    // LDS for the slots' area vectors, oriented out of the cell, kept for
-    // the CFL/dt sums after the update ([U][D][256] per block; nullptr: not
-    // kept)
-    float *keep_S;
-    static constexpr int U = GatherUnroll<D>::value;  // the slots per cell
-    // 3D: two faces' loads issued together, which leaves 63 VGPRs and 8
-    // waves per SIMD (all six at 4 waves, or three, were slower)
-    static constexpr int kUnroll = D == 3 ? 2 : U;
-    // a 3D cell's entries all fit the slots (kMaxFaces of them)
-    static constexpr bool kAllSlots = U >= kMaxFaces;
-    // the first kUnroll entries are slots, addressed by the cell alone, so
-    // their loads can issue before the entry count arrives (2D: 0.0271 ->
-    // 0.0263 ms per 65 k-cell step; the 3D box showed no gain)
-    static constexpr bool kSlotsFirst = D == 2;
-    // a slot past the cell's last entry holds the cell itself
-    __device__ __forceinline__ static bool valid(int key, int c) { return key != c; }
-    mutable float qc[D + 2];
-    mutable Prim32<D> pc;
-    mutable int c_ = 0;
-    __device__ __forceinline__ void begin_cell(int c) const {
-        c_ = c;
+// ---------------------------------------------------------------------------
+// One RK stage in one launch for inviscid M1 / M2: each cell forms its faces'
+// fluxes from its own and the other cells' states as it gathers them (every
+// interior face by both of its cells, to the face kernel's bits: conv32),
+// adds sponge and RK update and writes the new state and its boundary ghosts
+// to qout, another buffer.  c: the thread's cell.
+// ---------------------------------------------------------------------------
+// Bound: HBM in 3D (box of 4.1 M cells: 108 B per cell and stage where a
+// face's own data take 204; 821 -> 572 us per step), latency in 2D.  Faces
+// whose loads are issued together in 3D: two (box one 637, two 577, three 649
+// us per step); in 2D all four, since a 2D stage is bound by the latency of
+// its dependent loads.
+constexpr int kFusedGroup32 = 2;
+template <int D, int SOLVER, int CFL, bool PK, bool HALF>
+__device__ __forceinline__ void stage32_body(const KArgs32 &a, float *qout, float A, float B, int zero_dq, const int c,
+                                             const int lblk, double cfl_param) {
+    constexpr int U = GatherUnroll<D>::value;
+    constexpr int G = D == 3 ? kFusedGroup32 : U;
+    using F = FaceOf32<D, PK>;
+    // a face's own data are kept for the CFL/dt sums after the update; from
+    // the table they are read again
+    constexpr bool kKeep = CFL >= 0 && !PK;
+    __shared__ float keep[kKeep ? U * D * 256 : 1];
+    double cv = CFL == 0 ? 100.0 : 0.0;
+    if (c < a.nc) {
+        int key[G];
+        if constexpr (PK && D == 2) {
+            const uint4 v = reinterpret_cast<const uint4 *>(a.pk)[c];
+            key[0] = (int)v.x;
+            key[1] = (int)v.y;
+            key[2] = (int)v.z;
+            key[3] = (int)v.w;
+        } else {
+#pragma unroll
+            for (int u = 0; u < G; u++) key[u] = F::load_key(a, u, c);
+        }
+        float qc[D + 2], dq[D + 2];
         load_q32<D>(a, c, qc);
-        pc = prim32<D>(a, qc);
-    }
-    // key: the face's other cell, ~other where the cell is the face's N;
-    // from the slots up to U, from the face arrays beyond
-    __device__ __forceinline__ int key(int e, int j, int c) const {
-        if (j < U) return ld_once<D, 1>(a.sl_nb + slot_at<D, 1>(a.nc, j, 0, c));
-        const int ent = a.g_ent[e];
-        return ent >= 0 ? a.fN[ent & kFaceMask] : ~a.fP[~ent];
-    }
-    // boundary ghosts sit after the cells (no halo ghosts on this path)
-    __device__ __forceinline__ int ghost(int key) const { return key >= a.nc ? key - a.nc : -1; }
-    __device__ __forceinline__ void flux(int key, const float (&S)[D], float w, float (&r)[D + 2]) const {
-        const bool isP = key >= 0;
-        const int o = isP ? key : ~key;
-        float qo[D + 2], qP[D + 2], qN[D + 2];
-        load_q32<D>(a, o, qo);
-        const Prim32<D> po = prim32<D>(a, qo);
+        const float vinv = ld_once<D, 3>(a.vinv + c);
+        load_dq32<D>(a, zero_dq, c, dq);
+        const float dt = (float)(*a.dt);
+        const Prim32<D> sc = prim32<D>(a, qc);
+        const float s = dt * vinv;
+        auto add = [&](const F &f, const float (&qo)[D + 2]) {
+            const Prim32<D> so = prim32<D>(a, qo);
+            const Conv32<D> cf = conv32<D, SOLVER, HALF>(a, qc, sc, qo, so, f.S, f.wc, 1.0f - f.wc);
+            float r[D + 2];
+            conv_rhs32<D>(a, cf, cf.pp, f.S, r);
 #pragma unroll
-        for (int k = 0; k < D + 2; k++) {
-            qP[k] = isP ? qc[k] : qo[k];
-            qN[k] = isP ? qo[k] : qc[k];
+            for (int k = 0; k < D + 2; k++) dq[k] += s * r[k];
+        };
+        // groups of G faces in a rolled loop, the next group's keys loaded a
+        // group ahead
+#pragma unroll 1
+        for (int j0 = 0; j0 < U; j0 += G) {
+            F f[G];
+            float qo[G][D + 2];
+            int next[G];
+#pragma unroll
+            for (int u = 0; u < G; u++) {
+                f[u].load(a, j0 + u, c, key[u]);
+                load_q32<D>(a, f[u].other, qo[u]);
+                if (G < U) next[u] = F::load_key(a, j0 + G < U ? j0 + G + u : u, c);
+                if constexpr (kKeep)
+#pragma unroll
+                    for (int k = 0; k < D; k++) keep[((j0 + u) * D + k) * 256 + threadIdx.x] = f[u].S[k];
+            }
+            if (j0 == 0)
+#pragma unroll
+                for (int k = 0; k < D + 2; k++) dq[k] *= A;
+#pragma unroll
+            for (int u = 0; u < G; u++) {
+                add(f[u], qo[u]);
+                if (G < U) key[u] = next[u];
+            }
         }
-        const Prim32<D> sp = isP ? pc : po, sn = isP ? po : pc;
-        face_flux32_states<D, SOLVER, false, false>(a, 0, 0, 0, qP, qN, sp, sn, S, w, GradGlobal32<D, false>{a}, 0,
-                                                     0, r);
-    }
-    // area vector and weight of entry j
-    __device__ __forceinline__ void data(int e, int j, float (&S)[D], float &w) const {
-        if (j < U) {
-#pragma unroll
-            for (int k = 0; k < D; k++) S[k] = ld_once<D, 1>(a.sl_S + slot_at<D, D>(a.nc, j, k, c_));
-            w = ld_once<D, 1>(a.sl_w + slot_at<D, 1>(a.nc, j, 0, c_));
-            return;
+        int e1 = 0, e2 = 0;  // gather entries beyond the slots
+        if (U < kMaxFaces && a.more_faces) {
+            e1 = a.g_off[c] + U;
+            e2 = a.g_off[c + 1];
+            for (int e = e1; e < e2; e++) {
+                F f;
+                float qo[D + 2];
+                f.load_list(a, a.g_ent[e]);
+                load_q32<D>(a, f.other, qo);
+                add(f, qo);
+            }
         }
-        const int ent = a.g_ent[e];
-        const int f = ent >= 0 ? (ent & kFaceMask) : ~ent;
-        load_S32<D>(a.S, f, S);
-        w = a.w[f];
-    }
-    __device__ __forceinline__ void get(int e, int j, int key, float (&r)[D + 2]) const {
-        float S[D], w;
-        data(e, j, S, w);
-        if (keep_S && j < U) {
+        float q[D + 2];
 #pragma unroll
-            for (int k = 0; k < D; k++) keep_S[(j * D + k) * 256 + threadIdx.x] = key >= 0 ? S[k] : -S[k];
+        for (int k = 0; k < D + 2; k++) q[k] = qc[k];
+        finish_cell32<D>(a, c, dt, B, qout, q, dq);
+        // the boundary ghosts of this cell (only cells of the boundary
+        // submesh have any) for the next stage
+        if (c < a.nsm0) {
+#pragma unroll 1
+            for (int j = 0; j < U; j++) {
+                const int o = F::other_of(a, F::load_key(a, j, c));
+                if (o >= a.nc) refresh_ghost32<D>(a, o - a.nc, qout, q);
+            }
+            for (int e = e1; U < kMaxFaces && e < e2; e++) {
+                const int ent = a.g_ent[e];
+                if (ent >= 0 && (ent & kGhostFaceFlag)) refresh_ghost32<D>(a, a.fN[ent & kFaceMask] - a.nc, qout, q);
+            }
         }
-        flux(key, S, w, r);
-    }
-    __device__ __forceinline__ void area(int e, int j, int c, float (&S)[D]) const {
-        if (keep_S && j < U) {
+        if constexpr (CFL >= 0) {
+            CflSum32<D, CFL> t(a, q);
 #pragma unroll
-            for (int k = 0; k < D; k++) S[k] = keep_S[(j * D + k) * 256 + threadIdx.x];
-            return;
+            for (int j = 0; j < U; j++) {
+                float S[D];
+                if constexpr (kKeep) {
+#pragma unroll
+                    for (int k = 0; k < D; k++) S[k] = keep[(j * D + k) * 256 + threadIdx.x];
+                } else {
+                    F f;
+                    f.load(a, j, c, F::load_key(a, j, c));
+#pragma unroll
+                    for (int k = 0; k < D; k++) S[k] = f.S[k];
+                }
+                // a placeholder's zero area adds zero to the CFL sum
+                bool valid = true;
+                if constexpr (CFL == 0) {
+                    float s2 = 0.f;
+#pragma unroll
+                    for (int k = 0; k < D; k++) s2 += S[k] * S[k];
+                    valid = s2 > 0.f;
+                }
+                t.add(S, valid);
+            }
+            for (int e = e1; U < kMaxFaces && e < e2; e++) {
+                F f;
+                f.load_list(a, a.g_ent[e]);
+                t.add(f.S, true);
+            }
+            cv = t.value(a, q[0], vinv, cfl_param);
         }
-        float w;
-        data(e, j, S, w);
-        const bool isP = key(e, j, c) >= 0;
-#pragma unroll
-        for (int k = 0; k < D; k++) S[k] = isP ? S[k] : -S[k];
     }
-};
+    if constexpr (CFL >= 0) block_extremum<CFL>(cv, a.partial + lblk);
+}
 
-// the one-launch stage's face slots from the gather list: slot j of cell c
-// holds its j-th gather entry's other cell (~other on N entries), area
-// vector and weight
+// the face slots from the gather list: slot j of cell c holds its j-th gather
+// entry's other cell, area vector out of the cell and weight, or with
+// face_rec the other cell and the face's record number in the geometry table
+// (2 face_rec + 1 from the N side; none: a placeholder's record)
 template <int D>
-__global__ void __launch_bounds__(256) build_slots32(KArgs32 a, int32_t *nb, float *S, float *w) {
+__global__ void __launch_bounds__(256) build_slots32(KArgs32 a, const uint16_t *face_rec, int none, uint32_t *pk,
+                                                     int32_t *nb, float *S, float *w) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= a.nc) return;
     const int e0 = a.g_off[c], ne = a.g_off[c + 1] - e0;
     constexpr int U = GatherUnroll<D>::value;
     for (int j = 0; j < U; j++) {
-        if (j >= ne) {
-            // placeholder past the cell's last entry: the cell itself, zero
-            // area (read by unbranched gathers, never added)
-            nb[slot_at<D, 1>(a.nc, j, 0, c)] = c;
-#pragma unroll
-            for (int k = 0; k < D; k++) S[slot_at<D, D>(a.nc, j, k, c)] = 0.f;
-            w[slot_at<D, 1>(a.nc, j, 0, c)] = 0.5f;
+        FaceOf32<D, false> f;
+        f.other = c;
+        f.wc = 0.5f;
+        for (int k = 0; k < D; k++) f.S[k] = 0.f;
+        int rec = none;
+        if (j < ne) {
+            const int ent = a.g_ent[e0 + j];
+            f.load_list(a, ent);
+            if (pk) rec = 2 * face_rec[ent >= 0 ? (ent & kFaceMask) : ~ent] + (ent >= 0 ? 0 : 1);
+        }
+        if (pk) {
+            pk[pk_at<D>(a.nc, j, c)] = (uint32_t)f.other | (uint32_t)rec << a.pk_shift;
             continue;
         }
-        const int ent = a.g_ent[e0 + j];
-        const int f = ent >= 0 ? (ent & kFaceMask) : ~ent;
-        nb[slot_at<D, 1>(a.nc, j, 0, c)] = ent >= 0 ? a.fN[f] : ~a.fP[f];
+        nb[slot_at<D, 1>(a.nc, j, 0, c)] = f.other;
 #pragma unroll
-        for (int k = 0; k < D; k++) S[slot_at<D, D>(a.nc, j, k, c)] = a.S[(size_t)f * D + k];
-        w[slot_at<D, 1>(a.nc, j, 0, c)] = a.w[f];
+        for (int k = 0; k < D; k++) S[slot_at<D, D>(a.nc, j, k, c)] = f.S[k];
+        w[slot_at<D, 1>(a.nc, j, 0, c)] = f.wc;
     }
 }
 
-// One RK stage in one launch for inviscid M1 / M2: the face fluxes, the
-// ordered gather, sponge and update of cell_update32, reading the state in
-// a.q and writing the new state and boundary ghosts to qout (another buffer).
-// 3D: at least 7 waves per SIMD (6 for the last stage, whose CFL/dt sums
-// keep more live; both compile to 8), with two faces' loads in flight per
-// wave (kUnroll).
 // fin_nblk > 0 (a stage without CFL/dt sums): the grid has one block more,
 // the last, which reduces the fin_nblk per-block CFL maxima that an earlier
 // launch left in a.partial into *a.d_cfl (the final reduction of the
 // previous step, whose result no stage of this step reads).
-template <int D, int SOLVER, int CFL>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 3 ? (CFL < 0 ? 7 : 6) : 1)))
-stage_fused32(KArgs32 a, float *qout, float A, float B, int zero_dq, double cfl_param, int fin_nblk) {
-    // the last stage keeps its cells' area vectors in LDS for the CFL/dt sums
-    __shared__ float keep[CFL >= 0 ? GatherUnroll<D>::value * D * 256 : 1];
+template <int D, int SOLVER, int CFL, bool PK, bool HALF>
+__global__ void __launch_bounds__(256) stage_fused32(KArgs32 a, float *qout, float A, float B, int zero_dq,
+                                                     double cfl_param, int fin_nblk) {
     int nb = (int)gridDim.x;
     if constexpr (CFL < 0) {
         if (fin_nblk > 0) {
@@ -1357,8 +1407,8 @@ stage_fused32(KArgs32 a, float *qout, float A, float B, int zero_dq, double cfl_
         (void)fin_nblk;
     }
     const int blk = xcd_block((int)blockIdx.x, nb);
-    cell_update32_body<D, false, CFL>(a, FluxSlots32<D, SOLVER>{a, CFL >= 0 ? keep : nullptr}, qout, A, B, zero_dq,
-                                      blk * (int)blockDim.x + (int)threadIdx.x, blk, cfl_param);
+    stage32_body<D, SOLVER, CFL, PK, HALF>(a, qout, A, B, zero_dq, blk * (int)blockDim.x + (int)threadIdx.x, blk,
+                                           cfl_param);
 }
 template <int D, int MODE>
 __global__ void __launch_bounds__(256) cfl_dt_cells32(KArgs32 a, double param) {
@@ -1425,23 +1475,26 @@ __global__ void __launch_bounds__(256) cell_update32_b(const KArgs32 *args, Batc
     int r, lb;
     batch_slot(m, r, lb);
     const KArgs32 &a = args[r];
-    cell_update32_body<D, false, CFL>(a, FluxGlobal32<D>{a}, a.q, A, B, zero_dq, lb * 256 + threadIdx.x, lb,
-                                      CFL >= 0 ? *a.dt : 0.0);
+    cell_update32_body<D, false, CFL>(a, A, B, zero_dq, lb * 256 + threadIdx.x, lb, CFL >= 0 ? *a.dt : 0.0);
 }
 // one-launch stage over a batch (inviscid M1 / M2), each member from one
 // of its state buffers into the other: flip 0 from a.q into a.q_alt, flip 1
 // back
 template <int D, int SOLVER, int CFL>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 3 ? (CFL < 0 ? 7 : 6) : 1)))
-stage_fused32_b(const KArgs32 *args, BatchMap m, float A, float B, int zero_dq, int flip) {
-    __shared__ float keep[CFL >= 0 ? GatherUnroll<D>::value * D * 256 : 1];
+__global__ void __launch_bounds__(256) stage_fused32_b(const KArgs32 *args, BatchMap m, float A, float B, int zero_dq,
+                                                       int flip) {
     int r, lb;
     batch_slot(m, r, lb);
     KArgs32 a = args[r];
     float *qout = flip ? a.q : a.q_alt;
     if (flip) a.q = a.q_alt;
-    cell_update32_body<D, false, CFL>(a, FluxSlots32<D, SOLVER>{a, CFL >= 0 ? keep : nullptr}, qout, A, B, zero_dq,
-                                      lb * 256 + threadIdx.x, lb, CFL >= 0 ? *a.dt : 0.0);
+    const int c = lb * 256 + threadIdx.x;
+    const double dt = CFL >= 0 ? *a.dt : 0.0;
+    // members may hold either slot form
+    if (a.pk)
+        stage32_body<D, SOLVER, CFL, true, false>(a, qout, A, B, zero_dq, c, lb, dt);
+    else
+        stage32_body<D, SOLVER, CFL, false, false>(a, qout, A, B, zero_dq, c, lb, dt);
 }
 // one block per solver: max of its partials into its CFL scalar
 static __global__ void __launch_bounds__(256) cfl_final32_b(const KArgs32 *args) {
@@ -1476,7 +1529,8 @@ void launch_update32(Solver *s, double A, double B, bool zero_dq, bool res, bool
 template <int D>
 void launch_cfl_dt32(Solver *s, int mode, double param, double *out, double *dt_dst);
 template <int D>
-void launch_build_slots32(Solver *s, int32_t *nb, float *S, float *w);
+void launch_build_slots32(Solver *s, const uint16_t *face_rec, int none, uint32_t *pk, int32_t *nb, float *S,
+                          float *w);
 template <int D>
 void launch_stage_fused32(Solver *s, double A, double B, bool zero_dq, const float *qin, float *qout,
                           const Solver::CflJob *cfl, bool fin);

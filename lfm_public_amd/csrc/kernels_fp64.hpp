@@ -1052,6 +1052,19 @@ __device__ __forceinline__ void block_extremum(double v, double *dst) {
     }
 }
 
+// the cell's RK register as the last stage left it, zero at a step's first
+// stage: every component's load issued before any is used (a choice per
+// component compiles to a branch and a wait each)
+template <int D, int NT = kStreamNT64<D>>
+__device__ __forceinline__ void load_dq64(const KArgs &a, const int zero_dq, const int c, double (&dq)[D + 2]) {
+#pragma unroll
+    for (int k = 0; k < D + 2; k++) dq[k] = 0.0;
+    if (!zero_dq) {
+#pragma unroll
+        for (int k = 0; k < D + 2; k++) dq[k] = ld64_once<D, 2, NT>(a.dq + (size_t)k * a.nc + c);
+    }
+}
+
 // the sponge term of one cell (cfd_v0.cpp:2808-2811)
 template <int D, int NT = kStreamNT64<D>>
 __device__ __forceinline__ void sponge64(const KArgs &a, const int c, const double dt, const double (&q)[D + 2],
@@ -1082,12 +1095,11 @@ __global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, 
     if (c < a.nc) {
         const double dt = *a.dt;
         const double vinv = ld64_once<D, 3>(a.vinv + c);
-        double dq[D + 2], res[D + 2];
+        double dq[D + 2], res[D + 2], q[D + 2];
+        load_dq64<D>(a, zero_dq, c, dq);
 #pragma unroll
-        for (int k = 0; k < D + 2; k++) {
-            dq[k] = zero_dq ? 0.0 : ld64_once<D, 2>(a.dq + (size_t)k * a.nc + c) * A;
-            res[k] = 0.0;
-        }
+        for (int k = 0; k < D + 2; k++) res[k] = 0.0;
+        load_q<D>(a, c, q);
         const int e0 = a.g_off[c], ne = a.g_off[c + 1] - e0;
         int gface[kMaxFaces], ngf = 0;
         // owner side adds, neighbour side subtracts (cfd_v0.cpp:2800-2806)
@@ -1112,11 +1124,14 @@ __global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, 
         int ent[U];
         double fr[U][D + 2];
 #pragma unroll
+        for (int j = 0; j < U; j++) ent[j] = a.g_ent[e0 + (j < ne ? j : ne - 1)];
+#pragma unroll
         for (int j = 0; j < U; j++) {
-            ent[j] = a.g_ent[e0 + (j < ne ? j : ne - 1)];
             const int f = ent[j] >= 0 ? (ent[j] & kFaceMask) : ~ent[j];
             load_frhs<D>(a, f, fr[j]);
         }
+#pragma unroll
+        for (int k = 0; k < D + 2; k++) dq[k] *= A;
 #pragma unroll
         for (int j = 0; j < U; j++)
             if (j < ne) add(ent[j], fr[j]);
@@ -1127,8 +1142,6 @@ __global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, 
             load_frhs<D>(a, f, f1);
             add(en, f1);
         }
-        double q[D + 2];
-        load_q<D>(a, c, q);
         if (a.sigma) sponge64<D>(a, c, dt, q, dq);
 #pragma unroll
         for (int k = 0; k < D + 2; k++) {
@@ -1377,10 +1390,9 @@ __global__ void __launch_bounds__(256) stage_fused64(KArgs a, double *qout, doub
         for (int u = 0; u < G; u++) key[u] = F::load_key(a, u, c);
         double qc[D + 2], dq[D + 2];
         load_q<D>(a, c, qc);
-        const double dt = *a.dt;
         const double vinv = ld64_once<D, 3, NT>(a.vinv + c);
-#pragma unroll
-        for (int k = 0; k < D + 2; k++) dq[k] = zero_dq ? 0.0 : ld64_once<D, 2, NT>(a.dq + (size_t)k * a.nc + c) * A;
+        load_dq64<D, NT>(a, zero_dq, c, dq);
+        const double dt = *a.dt;
         const Prim64<D> sc = prim64<D, SOLVER>(a, qc);
         unsigned gmask = 0;  // bit j: slot j leads to a boundary ghost
         // a rolled loop over groups of G faces, the next group's keys loaded a
@@ -1397,6 +1409,9 @@ __global__ void __launch_bounds__(256) stage_fused64(KArgs a, double *qout, doub
                 load_q<D>(a, f[u].other, qo[u]);
                 next[u] = F::load_key(a, j0 + G < U ? j0 + G + u : u, c);
             }
+            if (j0 == 0)
+#pragma unroll
+                for (int k = 0; k < D + 2; k++) dq[k] *= A;
 #pragma unroll
             for (int u = 0; u < G; u++) {
                 if (f[u].other != c) {

@@ -446,6 +446,22 @@ void Solver::end_step(bool own_dt) {
     if (prm.have_res) res_valid = true;
 }
 
+// a face table's record numbers on the device (freed by the caller), nullptr
+// where memory cannot be had
+static void *upload_records(const std::vector<uint16_t> &rec) {
+    void *p = nullptr;
+    if (hipMalloc(&p, rec.size() * sizeof(uint16_t)) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (hipMemcpy(p, rec.data(), rec.size() * sizeof(uint16_t), hipMemcpyHostToDevice) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipFree(p);
+        return nullptr;
+    }
+    return p;
+}
+
 // the per-cell face slots (each cell's first GatherUnroll gather entries:
 // other cell, area vector, weight), read by the one-launch stages and the
 // FP32 gradient kernel; allocated on first use (under the set-up mutex, as a
@@ -454,28 +470,56 @@ void Solver::end_step(bool own_dt) {
 // gather list and the face arrays, which gives the same bits.
 bool Solver::ensure_slots32() {
     if (!fp32 || slots_failed) return false;
-    if (k32->sl_nb) return true;
-    const int U = L.D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value;
+    if (k32->pk || k32->sl_nb) return true;
+    const int D = L.D, U = D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value, nt = table32.n;
     std::lock_guard<std::mutex> lock(device_setup_mutex());
-    void *p[3] = {nullptr, nullptr, nullptr};
-    const size_t bytes[3] = {slot_array_len(L.nc, U, 1) * sizeof(int32_t),
-                             slot_array_len(L.nc, U, L.D) * sizeof(float), slot_array_len(L.nc, U, 1) * sizeof(float)};
-    for (int i = 0; i < 3; i++)
-        if (hipMalloc(&p[i], bytes[i]) != hipSuccess) {
+    void *p[3] = {nullptr, nullptr, nullptr}, *rec = nullptr;
+    slots_failed = true;
+    if (nt) {
+        // each record as P sees it, then as N does, and a placeholder's
+        std::vector<float> tab((size_t)(2 * nt + 1) * 4, 0.f);
+        bool half = true;
+        for (int i = 0; i < 2 * nt; i++) {
+            const float w = canonical_w(table32.w[i / 2]);
+            for (int k = 0; k < D; k++) {
+                const float x = table32.S[(size_t)(i / 2) * D + k];
+                tab[(size_t)i * 4 + k] = i % 2 ? -x : x;
+            }
+            tab[(size_t)i * 4 + D] = i % 2 ? 1.0f - w : w;
+            half = half && w == 0.5f;
+        }
+        tab[(size_t)2 * nt * 4 + D] = 0.5f;
+        const size_t bytes[2] = {pk_len(D, L.nc, U) * sizeof(uint32_t), tab.size() * sizeof(float)};
+        if (!alloc_all(p, bytes, 2)) return false;
+        rec = upload_records(table32.rec);
+        if (!rec || hipMemcpy(p[1], tab.data(), bytes[1], hipMemcpyHostToDevice) != hipSuccess) {
             (void)hipGetLastError();
-            for (int k = 0; k < i; k++) (void)hipFree(p[k]);
-            slots_failed = true;
+            if (rec) (void)hipFree(rec);
             return false;
         }
-    for (int i = 0; i < 3; i++) {
-        allocs.push_back(p[i]);
-        device_bytes += (int64_t)bytes[i];
+        k32->pk_half = half;
+    } else {
+        const size_t bytes[3] = {slot_array_len(L.nc, U, 1) * sizeof(int32_t),
+                                 slot_array_len(L.nc, U, D) * sizeof(float),
+                                 slot_array_len(L.nc, U, 1) * sizeof(float)};
+        if (!alloc_all(p, bytes, 3)) return false;
     }
-    LFM_DISPATCH_D(this, launch_build_slots32<2>(this, (int32_t *)p[0], (float *)p[1], (float *)p[2]),
-                   launch_build_slots32<3>(this, (int32_t *)p[0], (float *)p[1], (float *)p[2]));
-    k32->sl_nb = (const int32_t *)p[0];
-    k32->sl_S = (const float *)p[1];
-    k32->sl_w = (const float *)p[2];
+    uint32_t *pk = nt ? (uint32_t *)p[0] : nullptr;
+    int32_t *nb = nt ? nullptr : (int32_t *)p[0];
+    float *sS = nt ? nullptr : (float *)p[1], *sw = nt ? nullptr : (float *)p[2];
+    LFM_DISPATCH_D(this, launch_build_slots32<2>(this, (const uint16_t *)rec, 2 * nt, pk, nb, sS, sw),
+                   launch_build_slots32<3>(this, (const uint16_t *)rec, 2 * nt, pk, nb, sS, sw));
+    if (rec) {
+        (void)hipStreamSynchronize(stream);
+        (void)hipFree(rec);
+    }
+    table32 = FaceTable<float>();
+    k32->pk = pk;
+    k32->pk_tab = nt ? (const float *)p[1] : nullptr;
+    k32->sl_nb = nb;
+    k32->sl_S = sS;
+    k32->sl_w = sw;
+    slots_failed = false;
     return true;
 }
 
@@ -536,10 +580,8 @@ bool Solver::ensure_slots64() {
         r[D + 1] = r[D + 2] = 0.5;
         const size_t bytes[3] = {words, tab.size() * sizeof(double), perm};
         if (!alloc_all(p, bytes, 3)) return false;
-        if (hipMalloc(&rec, table64.rec.size() * sizeof(uint16_t)) != hipSuccess ||
-            hipMemcpy(rec, table64.rec.data(), table64.rec.size() * sizeof(uint16_t), hipMemcpyHostToDevice) !=
-                hipSuccess ||
-            hipMemcpy(p[1], tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
+        rec = upload_records(table64.rec);
+        if (!rec || hipMemcpy(p[1], tab.data(), bytes[1], hipMemcpyHostToDevice) != hipSuccess) {
             (void)hipGetLastError();
             if (rec) (void)hipFree(rec);
             return false;

@@ -1,6 +1,7 @@
 // solver_fp32p.hip -- creation and launches of the FP32-perturbation path.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -10,6 +11,9 @@
 
 namespace lfm {
 
+// records of the FP32 geometry table: both orientations of them are at most
+// 128 KiB, which stay in an XCD's 4 MiB L2 beside the gathered states
+static constexpr int kMaxTable32 = 4096;
 static constexpr int kBlock = 256;
 static inline int nblocks(long n) { return (int)((n + kBlock - 1) / kBlock); }
 
@@ -77,6 +81,7 @@ int create_fp32p(Solver *s) {
         a.minf[k] = k < D ? (float)m_inf[k] : 0.f;
         a.m_inf_d[k] = k < D ? m_inf[k] : 0.0;
     }
+    a.uinf2 = (float)uinf2;
     a.rho_inf_d = g.rho_inf;
     a.rhoE_inf_d = rhoE_inf;
 
@@ -89,6 +94,7 @@ int create_fp32p(Solver *s) {
         for (size_t f = 0; f < nf; f++)
             for (int k = 0; k < D; k++) S[f * D + k] = (float)L.S[(size_t)k * nf + f];
         auto d = to_f32(L.d), w = to_f32(L.w);
+        for (float &x : w) x = canonical_w(x);
         rc |= up(s, (float **)&a.S, S.data(), S.size());
         rc |= up(s, (float **)&a.d, d.data(), d.size());
         rc |= up(s, (float **)&a.w, w.data(), w.size());
@@ -124,6 +130,14 @@ int create_fp32p(Solver *s) {
         // step that uses it; its unset-patch ghosts are copied from q by the
         // first fused stage)
         s->fused_ok = !s->visc && s->prm.solver < 2 && L.halo.empty();
+        a.more_faces = L.max_faces > (D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value);
+        // slots are read by the one-launch stage and by 3D gradients (a halo
+        // face has its weight only after the import: no table there)
+        if (s->fused_ok || (D == 3 && L.halo.empty())) {
+            a.pk_shift = index_bits((long)ntot);
+            const long fit = ((1L << (32 - a.pk_shift)) - 1) / 2;
+            s->table32 = face_table<float>(L, (int)std::min<long>(fit, kMaxTable32));
+        }
     }
     rc |= up(s, &a.dq, (float *)nullptr, (size_t)(D + 2) * nc);
     rc |= up(s, &a.res_cell, (float *)nullptr, (size_t)(D + 2) * nc);
@@ -172,17 +186,17 @@ void launch_bc32(Solver *s) {
     if (s->L.ng) hipLaunchKernelGGL(bc_fill32<D>, dim3(nblocks(s->L.ng)), dim3(kBlock), 0, s->stream, *s->k32);
 }
 
-template <int D, bool V, bool SL>
+template <int D, bool V, bool SL, bool PK>
 static void launch_gradvis32_v(Solver *s, bool fin) {
     const int nb = nblocks(s->L.nc);
     const dim3 grid(nb + (fin ? 1 : 0));
     const int fb = fin ? nb : 0;
     if (s->prm.solver == 2 && s->prm.minmod)
-        hipLaunchKernelGGL((grad_vis32<D, 2, V, true, SL>), grid, dim3(kBlock), 0, s->stream, *s->k32, fb);
+        hipLaunchKernelGGL((grad_vis32<D, 2, V, true, SL, PK>), grid, dim3(kBlock), 0, s->stream, *s->k32, fb);
     else if (s->prm.solver == 2)
-        hipLaunchKernelGGL((grad_vis32<D, 0, V, true, SL>), grid, dim3(kBlock), 0, s->stream, *s->k32, fb);
+        hipLaunchKernelGGL((grad_vis32<D, 0, V, true, SL, PK>), grid, dim3(kBlock), 0, s->stream, *s->k32, fb);
     else
-        hipLaunchKernelGGL((grad_vis32<D, 0, V, false, SL>), grid, dim3(kBlock), 0, s->stream, *s->k32, fb);
+        hipLaunchKernelGGL((grad_vis32<D, 0, V, false, SL, PK>), grid, dim3(kBlock), 0, s->stream, *s->k32, fb);
 }
 
 // 3D gradients read the face slots (same bits as the gather list; 4.2 M-cell
@@ -197,11 +211,14 @@ void launch_gradvis32(Solver *s, bool full, bool fin) {
     const bool V = full || s->visc;
     if constexpr (D == 3) {
         if (s->ensure_slots32()) {
-            V ? launch_gradvis32_v<D, true, true>(s, fin) : launch_gradvis32_v<D, false, true>(s, fin);
+            if (s->k32->pk)
+                V ? launch_gradvis32_v<D, true, true, true>(s, fin) : launch_gradvis32_v<D, false, true, true>(s, fin);
+            else
+                V ? launch_gradvis32_v<D, true, true, false>(s, fin) : launch_gradvis32_v<D, false, true, false>(s, fin);
             return;
         }
     }
-    V ? launch_gradvis32_v<D, true, false>(s, fin) : launch_gradvis32_v<D, false, false>(s, fin);
+    V ? launch_gradvis32_v<D, true, false, false>(s, fin) : launch_gradvis32_v<D, false, false, false>(s, fin);
 }
 
 template <int D, bool V, bool ST>
@@ -245,20 +262,20 @@ void launch_update32(Solver *s, double A, double B, bool zero_dq, bool res, bool
 
 // fin: one block more reduces the CFL maxima of the previous step's last
 // stage (left in a.partial) into a.d_cfl
-template <int D, int SOLVER>
+template <int D, int SOLVER, bool PK, bool HALF>
 static void launch_fused32_v(Solver *s, float A, float B, int zero_dq, const KArgs32 &a, float *qout,
                              const Solver::CflJob *cfl, bool fin) {
     const int nb = nblocks(s->L.nc);
     if (!cfl) {
-        hipLaunchKernelGGL((stage_fused32<D, SOLVER, -1>), dim3(nb + (fin ? 1 : 0)), dim3(kBlock), 0, s->stream, a,
+        hipLaunchKernelGGL((stage_fused32<D, SOLVER, -1, PK, HALF>), dim3(nb + (fin ? 1 : 0)), dim3(kBlock), 0, s->stream, a,
                            qout, A, B, zero_dq, 0.0, fin ? nb : 0);
         return;
     }
     if (cfl->mode == 0)
-        hipLaunchKernelGGL((stage_fused32<D, SOLVER, 0>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
+        hipLaunchKernelGGL((stage_fused32<D, SOLVER, 0, PK, HALF>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
                            zero_dq, cfl->param, 0);
     else
-        hipLaunchKernelGGL((stage_fused32<D, SOLVER, 1>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
+        hipLaunchKernelGGL((stage_fused32<D, SOLVER, 1, PK, HALF>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
                            zero_dq, cfl->param, 0);
 }
 
@@ -267,15 +284,23 @@ void launch_stage_fused32(Solver *s, double A, double B, bool zero_dq, const flo
                           const Solver::CflJob *cfl, bool fin) {
     KArgs32 a = *s->k32;
     a.q = const_cast<float *>(qin);
-    if (s->prm.solver == 0)
-        launch_fused32_v<D, 0>(s, (float)A, (float)B, (int)zero_dq, a, qout, cfl, fin);
+    const float fA = (float)A, fB = (float)B;
+    const int z = (int)zero_dq;
+    if (s->prm.solver == 1)
+        a.pk ? launch_fused32_v<D, 1, true, true>(s, fA, fB, z, a, qout, cfl, fin)
+             : launch_fused32_v<D, 1, false, true>(s, fA, fB, z, a, qout, cfl, fin);
+    else if (a.pk)
+        a.pk_half ? launch_fused32_v<D, 0, true, true>(s, fA, fB, z, a, qout, cfl, fin)
+                  : launch_fused32_v<D, 0, true, false>(s, fA, fB, z, a, qout, cfl, fin);
     else
-        launch_fused32_v<D, 1>(s, (float)A, (float)B, (int)zero_dq, a, qout, cfl, fin);
+        launch_fused32_v<D, 0, false, false>(s, fA, fB, z, a, qout, cfl, fin);
 }
 
 template <int D>
-void launch_build_slots32(Solver *s, int32_t *nb, float *S, float *w) {
-    hipLaunchKernelGGL(build_slots32<D>, dim3(nblocks(s->L.nc)), dim3(kBlock), 0, s->stream, *s->k32, nb, S, w);
+void launch_build_slots32(Solver *s, const uint16_t *face_rec, int none, uint32_t *pk, int32_t *nb, float *S,
+                          float *w) {
+    hipLaunchKernelGGL(build_slots32<D>, dim3(nblocks(s->L.nc)), dim3(kBlock), 0, s->stream, *s->k32, face_rec, none, pk,
+                       nb, S, w);
 }
 
 template <int D>
@@ -412,8 +437,8 @@ template void launch_stage_fused32<2>(Solver *, double, double, bool, const floa
                                      const Solver::CflJob *, bool);
 template void launch_stage_fused32<3>(Solver *, double, double, bool, const float *, float *,
                                      const Solver::CflJob *, bool);
-template void launch_build_slots32<2>(Solver *, int32_t *, float *, float *);
-template void launch_build_slots32<3>(Solver *, int32_t *, float *, float *);
+template void launch_build_slots32<2>(Solver *, const uint16_t *, int, uint32_t *, int32_t *, float *, float *);
+template void launch_build_slots32<3>(Solver *, const uint16_t *, int, uint32_t *, int32_t *, float *, float *);
 template void launch_cfl_dt32<2>(Solver *, int, double, double *, double *);
 template void launch_cfl_dt32<3>(Solver *, int, double, double *, double *);
 

@@ -162,13 +162,15 @@ struct Solver {
     // the FP64 one-launch stage's slots (k64.pk or k64.sl_*, k64.s_perm), on
     // first use; the distinct face records found when the handle was created
     FaceTable<double> table64;
+    FaceTable<float> table32;  // of the FP32 slots (canonical_w weights)
     bool ensure_slots64();
     bool stream_nt = true;  // the stage outgrows the Infinity Cache (stream_once)
     bool sym64 = false;  // every record's weights allow flux_m1_sym
     // device memory for a set of arrays of one kind, all or none, under the
     // set-up mutex (which the caller holds)
     bool alloc_all(void **p, const size_t *bytes, int n);
-    // per-cell face slots of the FP32 kernels (k32->sl_*), on first use
+    // per-cell face slots of the FP32 kernels (k32->pk or k32->sl_*), on
+    // first use
     bool slots_failed = false;
     bool ensure_slots32();
     int fused_from() const;
@@ -196,6 +198,12 @@ struct Solver {
     // device scratch instead of an allocated counter
     int check_finite_noalloc(int64_t *n_bad);
 };
+
+// The FP32 path's weights are rounded to those whose complement is exact, so
+// that w and 1 - w, formed from either cell's side, are the same two numbers
+// (a change of at most 2^-25 to weights below one half, what rounding 1 - w
+// takes from them anyway).
+inline float canonical_w(float w) { return 1.0f - (1.0f - w); }
 
 int create_fp32p(Solver *s);
 void free_k32(KArgs32 *k);
