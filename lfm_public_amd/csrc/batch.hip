@@ -42,54 +42,62 @@ struct Batch {
     }
 };
 
-template <int D, int SOLVER>
+template <int D, int SOLVER, bool NT>
 static void enqueue_fused(Batch *b, int rk, int flip) {
     const dim3 blk(256);
     if (rk == b->nstages - 1)
-        hipLaunchKernelGGL((stage_fused32_b<D, SOLVER, 1>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
+        hipLaunchKernelGGL((stage_fused32_b<D, SOLVER, 1, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
                            b->map_cells, (float)b->A[rk], (float)b->B[rk], rk == 0 ? 1 : 0, flip);
     else
-        hipLaunchKernelGGL((stage_fused32_b<D, SOLVER, -1>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
+        hipLaunchKernelGGL((stage_fused32_b<D, SOLVER, -1, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
                            b->map_cells, (float)b->A[rk], (float)b->B[rk], rk == 0 ? 1 : 0, flip);
 }
 
-template <int D, bool V>
-static void enqueue_step(Batch *b) {
+template <int D, bool V, bool NT>
+static void enqueue_step_nt(Batch *b) {
     const dim3 blk(256);
     for (int rk = 0; rk < b->nstages; rk++) {
         if (b->fused && rk >= b->separate) {
             // an even number of one-launch stages: each step ends in a.q
             const int flip = (rk - b->separate) & 1;
-            b->solver == 0 ? enqueue_fused<D, 0>(b, rk, flip) : enqueue_fused<D, 1>(b, rk, flip);
+            b->solver == 0 ? enqueue_fused<D, 0, NT>(b, rk, flip) : enqueue_fused<D, 1, NT>(b, rk, flip);
             continue;
         }
         // ghosts are refreshed by the update kernel (members join with fresh ghosts);
         // without viscosity solvers 0/1 consume no gradient or tensor
         if (V || b->solver == 2) {
             if (b->solver == 2 && b->minmod)
-                hipLaunchKernelGGL((grad_vis32_b<D, 2, V, true>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
+                hipLaunchKernelGGL((grad_vis32_b<D, 2, V, true, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
                                    b->map_cells);
             else if (b->solver == 2)
-                hipLaunchKernelGGL((grad_vis32_b<D, 0, V, true>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
+                hipLaunchKernelGGL((grad_vis32_b<D, 0, V, true, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
                                    b->map_cells);
             else
-                hipLaunchKernelGGL((grad_vis32_b<D, 0, V, false>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
+                hipLaunchKernelGGL((grad_vis32_b<D, 0, V, false, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
                                    b->map_cells);
         }
         switch (b->solver) {
-        case 0: hipLaunchKernelGGL((face_flux32_b<D, 0, V>), dim3(b->nb_faces), blk, 0, b->stream, b->d_args, b->map_faces); break;
-        case 1: hipLaunchKernelGGL((face_flux32_b<D, 1, V>), dim3(b->nb_faces), blk, 0, b->stream, b->d_args, b->map_faces); break;
-        default: hipLaunchKernelGGL((face_flux32_b<D, 2, V>), dim3(b->nb_faces), blk, 0, b->stream, b->d_args, b->map_faces); break;
+        case 0: hipLaunchKernelGGL((face_flux32_b<D, 0, V, NT>), dim3(b->nb_faces), blk, 0, b->stream, b->d_args, b->map_faces); break;
+        case 1: hipLaunchKernelGGL((face_flux32_b<D, 1, V, NT>), dim3(b->nb_faces), blk, 0, b->stream, b->d_args, b->map_faces); break;
+        default: hipLaunchKernelGGL((face_flux32_b<D, 2, V, NT>), dim3(b->nb_faces), blk, 0, b->stream, b->d_args, b->map_faces); break;
         }
         // the last stage's update also forms the step's compute_cfl partials
         if (rk == b->nstages - 1)
-            hipLaunchKernelGGL((cell_update32_b<D, 1>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
+            hipLaunchKernelGGL((cell_update32_b<D, 1, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
                                b->map_cells, (float)b->A[rk], (float)b->B[rk], rk == 0 ? 1 : 0);
         else
-            hipLaunchKernelGGL((cell_update32_b<D, -1>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
+            hipLaunchKernelGGL((cell_update32_b<D, -1, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
                                b->map_cells, (float)b->A[rk], (float)b->B[rk], rk == 0 ? 1 : 0);
     }
     hipLaunchKernelGGL(cfl_final32_b, dim3((unsigned)b->members.size()), blk, 0, b->stream, b->d_args);
+}
+
+// one launch walks every member: NT by what they touch together
+template <int D, bool V>
+static void enqueue_step(Batch *b) {
+    size_t bytes = 0;
+    for (const Solver *s : b->members) bytes += s->stage_bytes;
+    outgrows_cache(bytes) ? enqueue_step_nt<D, V, true>(b) : enqueue_step_nt<D, V, false>(b);
 }
 
 static int batch_set_locked(Batch *b, lfm_solver *const *hs, int n);

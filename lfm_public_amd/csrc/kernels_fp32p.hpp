@@ -143,35 +143,12 @@ __host__ __device__ __forceinline__ size_t q32_index(int k, size_t i, size_t nto
     return k < 4 ? 4 * i + (size_t)k : 4 * ntot + i;
 }
 
-// loads and stores of data a kernel touches once, marked non-temporal so
-// that they do not displace the gathered neighbour states in L2: level 1 the
-// face slots, 2 the RK register, 3 the other streams (new states, face
-// lists and geometry of the face kernel, face fluxes, gradient records,
-// 1/V and sponge).  3D uses every level (256^3 box 3.70 -> 3.35 ms per
-// step, 4.2 M-cell O-grid 2.75 -> 2.51).  2D uses level 1 only: a 2D
-// solve's arrays fit in the 256 MB Infinity Cache, where the next kernel
-// finds what this one wrote unless it was written non-temporally (1 M-cell
-// annulus 0.32 -> 0.40 ms per step with every level).
-template <int D>
-constexpr int kStreamNT = D == 3 ? 3 : 1;
 using f4v = float __attribute__((ext_vector_type(4)));
-template <int D, int LEVEL, class T>
-__device__ __forceinline__ T ld_once(const T *p) {
-    if constexpr (kStreamNT<D> >= LEVEL) return __builtin_nontemporal_load(p);
-    return *p;
-}
-template <int D, int LEVEL, class T>
-__device__ __forceinline__ void st_once(T *p, T v) {
-    if constexpr (kStreamNT<D> >= LEVEL)
-        __builtin_nontemporal_store(v, p);
-    else
-        *p = v;
-}
 // a 16-byte record
-template <int D, int LEVEL>
+template <bool NT>
 __device__ __forceinline__ void st4_once(float *p, float x, float y, float z, float w) {
     const f4v v = {x, y, z, w};
-    st_once<D, LEVEL>(reinterpret_cast<f4v *>(p), v);
+    st_once<NT>(reinterpret_cast<f4v *>(p), v);
 }
 
 template <int D>
@@ -184,10 +161,10 @@ __device__ __forceinline__ void load_q32(const KArgs32 &a, int i, float *q) {
     if (D == 3) q[4] = a.q[(size_t)4 * a.ntot + i];
 }
 
-template <int D>
+template <int D, bool NT>
 __device__ __forceinline__ void store_q32(float *qv, size_t ntot, int i, const float *q) {
-    st4_once<D, 3>(qv + 4 * (size_t)i, q[0], q[1], q[2], q[3]);
-    if (D == 3) st_once<D, 3>(qv + 4 * ntot + i, q[4]);
+    st4_once<NT>(qv + 4 * (size_t)i, q[0], q[1], q[2], q[3]);
+    if (D == 3) st_once<NT>(qv + 4 * ntot + i, q[4]);
 }
 
 template <int D>
@@ -285,7 +262,7 @@ __device__ __forceinline__ void bc_fill32_body(const KArgs32 &a, const int g) {
     load_q32<D>(a, a.ghost_cell[g], qi);
     if (!ghost_state32<D>(a, a.ghost_role[g], qi, qg)) return;
     const int gi = a.nc + g;
-    store_q32<D>(a.q, a.ntot, gi, qg);
+    store_q32<D, false>(a.q, a.ntot, gi, qg);
 }
 
 // ---------------------------------------------------------------------------
@@ -372,14 +349,14 @@ inline size_t pk_len(int D, int nc, int U) { return D == 2 ? (size_t)U * nc : sl
 // one face as one of its cells sees it: the other cell, the area vector out
 // of the cell and the cell's weight (the other's is 1 - wc, exactly:
 // canonical_w)
-template <int D, bool PK>
+template <int D, bool PK, bool NT>
 struct FaceOf32 {
     int other;
     float S[D], wc;
     // key: the packed word, or the slot's other cell
     __device__ __forceinline__ static int load_key(const KArgs32 &a, const int j, const int c) {
-        if constexpr (PK) return (int)ld_once<D, 1>(a.pk + pk_at<D>(a.nc, j, c));
-        return ld_once<D, 1>(a.sl_nb + slot_at<D, 1>(a.nc, j, 0, c));
+        if constexpr (PK) return (int)ld_once<NT>(a.pk + pk_at<D>(a.nc, j, c));
+        return ld_once<NT>(a.sl_nb + slot_at<D, 1>(a.nc, j, 0, c));
     }
     __device__ __forceinline__ static int other_of(const KArgs32 &a, const int key) {
         if constexpr (PK) return (int)((uint32_t)key & ((1u << a.pk_shift) - 1u));
@@ -395,8 +372,8 @@ struct FaceOf32 {
             wc = r[D];
         } else {
 #pragma unroll
-            for (int k = 0; k < D; k++) S[k] = ld_once<D, 1>(a.sl_S + slot_at<D, D>(a.nc, j, k, c));
-            wc = ld_once<D, 1>(a.sl_w + slot_at<D, 1>(a.nc, j, 0, c));
+            for (int k = 0; k < D; k++) S[k] = ld_once<NT>(a.sl_S + slot_at<D, D>(a.nc, j, k, c));
+            wc = ld_once<NT>(a.sl_w + slot_at<D, 1>(a.nc, j, 0, c));
         }
     }
     // an entry of the gather list
@@ -417,7 +394,7 @@ struct FaceOf32 {
 // from the gather list.  Each face's sums sit in a branch of their own: in one
 // block the compiler interleaves all six faces' arithmetic (124 VGPRs instead
 // of 96, 4 waves per SIMD instead of 5).
-template <int D, int GRAD, bool VISC, bool SL, bool PK>
+template <int D, int GRAD, bool VISC, bool SL, bool PK, bool NT>
 __device__ __forceinline__ Prim32<D> grad32_sums(const KArgs32 &a, const int c, float (&dudx)[D][D],
                                                   float (&dTdx)[D], float (&rg)[D], float (&pg)[D],
                                                   float (&ug)[D][D]) {
@@ -431,7 +408,7 @@ __device__ __forceinline__ Prim32<D> grad32_sums(const KArgs32 &a, const int c, 
     float qc0[D + 2];
     load_q32<D>(a, c, qc0);
     const Prim32<D> own = prim32<D>(a, qc0);
-    using F = FaceOf32<D, PK>;
+    using F = FaceOf32<D, PK, NT>;
     // one face's contribution
     auto add = [&](const F &f, const float (&qo)[D + 2]) {
         const Prim32<D> so = prim32<D>(a, qo);
@@ -500,7 +477,7 @@ __device__ __forceinline__ Prim32<D> grad32_sums(const KArgs32 &a, const int c, 
 
 // every thread of the block must call this (the block's records are written
 // through LDS); c = the block's first cell + threadIdx.x
-template <int D, int GRAD, bool VISC, bool RG, bool SL = false, bool PK = false>
+template <int D, int GRAD, bool VISC, bool RG, bool SL, bool PK, bool NT>
 __device__ __forceinline__ void grad_vis32_body(const KArgs32 &a, const int c) {
     using R = GradRec32<D, RG>;
     const bool valid = c < a.nc;
@@ -509,7 +486,7 @@ __device__ __forceinline__ void grad_vis32_body(const KArgs32 &a, const int c) {
     for (int k = 0; k < R::kStride; k++) r[k] = 0.f;
     if (valid) {
         float dudx[D][D], dTdx[D], rg[D], pg[D], ug[D][D];
-        const Prim32<D> own = grad32_sums<D, GRAD, VISC, SL, PK>(a, c, dudx, dTdx, rg, pg, ug);
+        const Prim32<D> own = grad32_sums<D, GRAD, VISC, SL, PK, NT>(a, c, dudx, dTdx, rg, pg, ug);
         // tauMC / sigmaU stored only where a halo payload needs them (otherwise
         // each face recomputes them from dudx); U_grad equals dudx bit for bit
         // (same face velocity, same sums) and shares its storage unless a halo
@@ -572,7 +549,7 @@ __device__ __forceinline__ void grad_vis32_body(const KArgs32 &a, const int c) {
         float *dst = a.dudx + (size_t)c0 * S;
         const int n = nrec * S, n4 = n / 4;
         for (int j = t; j < n4; j += blockDim.x)
-            st_once<D, 3>(reinterpret_cast<f4v *>(dst) + j, reinterpret_cast<const f4v *>(st)[j]);
+            st_once<NT>(reinterpret_cast<f4v *>(dst) + j, reinterpret_cast<const f4v *>(st)[j]);
         for (int j = 4 * n4 + t; j < n; j += blockDim.x) dst[j] = st[j];
     }
 }
@@ -680,7 +657,7 @@ __device__ __forceinline__ void conv_rhs32(const KArgs32 &a, const Conv32<D> &f,
 
 // the flux of face f from its cells' states and primitives (qP, sp of P;
 // qN, sn of N)
-template <int D, int SOLVER, bool VISC, bool STORED, class GA>
+template <int D, int SOLVER, bool VISC, bool STORED, bool NT, class GA>
 __device__ __forceinline__ void face_flux32_states(const KArgs32 &a, const int f, const int P, const int N,
                                                    const float (&qP)[D + 2], const float (&qN)[D + 2],
                                                    const Prim32<D> &sp, const Prim32<D> &sn,
@@ -697,7 +674,7 @@ __device__ __forceinline__ void face_flux32_states(const KArgs32 &a, const int f
     const size_t nt = a.ntot;
     float d[D];
 #pragma unroll
-    for (int k = 0; k < D; k++) d[k] = ld_once<D, 3>(a.d + (size_t)k * a.nf + f);
+    for (int k = 0; k < D; k++) d[k] = ld_once<NT>(a.d + (size_t)k * a.nf + f);
     float Sm2 = 0.f;
 #pragma unroll
     for (int k = 0; k < D; k++) Sm2 += S[k] * S[k];
@@ -883,28 +860,28 @@ __device__ __forceinline__ void face_flux32_states(const KArgs32 &a, const int f
     }
 }
 
-template <int D, int SOLVER, bool VISC, bool STORED, class GA>
+template <int D, int SOLVER, bool VISC, bool STORED, bool NT, class GA>
 __device__ __forceinline__ void face_flux32_rhs(const KArgs32 &a, const int f, const GA &ga, const int gP,
                                                 const int gN, float (&rhs)[D + 2]) {
-    const int P = ld_once<D, 3>(a.fP + f), N = ld_once<D, 3>(a.fN + f);
+    const int P = ld_once<NT>(a.fP + f), N = ld_once<NT>(a.fN + f);
     float qP[D + 2], qN[D + 2];
     load_q32<D>(a, P, qP);
     load_q32<D>(a, N, qN);
     const Prim32<D> sp = prim32<D>(a, qP), sn = prim32<D>(a, qN);
     float S[D];
 #pragma unroll
-    for (int k = 0; k < D; k++) S[k] = ld_once<D, 3>(a.S + (size_t)f * D + k);
-    face_flux32_states<D, SOLVER, VISC, STORED>(a, f, P, N, qP, qN, sp, sn, S, ld_once<D, 3>(a.w + f), ga, gP, gN,
+    for (int k = 0; k < D; k++) S[k] = ld_once<NT>(a.S + (size_t)f * D + k);
+    face_flux32_states<D, SOLVER, VISC, STORED, NT>(a, f, P, N, qP, qN, sp, sn, S, ld_once<NT>(a.w + f), ga, gP, gN,
                                                  rhs);
 }
 
-template <int D, int SOLVER, bool VISC, bool STORED>
+template <int D, int SOLVER, bool VISC, bool STORED, bool NT>
 __device__ __forceinline__ void face_flux32_body(const KArgs32 &a, const int f) {
     if (f >= a.nf) return;
     float rhs[D + 2];
-    face_flux32_rhs<D, SOLVER, VISC, STORED>(a, f, GradGlobal32<D, SOLVER == 2>{a}, a.fP[f], a.fN[f], rhs);
-    st4_once<D, 3>(a.frhs + 4 * (size_t)f, rhs[0], rhs[1], rhs[2], rhs[3]);
-    if (D == 3) st_once<D, 3>(a.frhs + (size_t)4 * a.nf + f, rhs[D + 1]);
+    face_flux32_rhs<D, SOLVER, VISC, STORED, NT>(a, f, GradGlobal32<D, SOLVER == 2>{a}, a.fP[f], a.fN[f], rhs);
+    st4_once<NT>(a.frhs + 4 * (size_t)f, rhs[0], rhs[1], rhs[2], rhs[3]);
+    if (D == 3) st_once<NT>(a.frhs + (size_t)4 * a.nf + f, rhs[D + 1]);
 }
 
 // ---------------------------------------------------------------------------
@@ -913,55 +890,55 @@ __device__ __forceinline__ void face_flux32_body(const KArgs32 &a, const int f) 
 // the cell's RK register as the last stage left it, zero at a step's first
 // stage: every component's load issued before any is used (a choice per
 // component compiles to a branch and a wait each)
-template <int D>
+template <int D, bool NT>
 __device__ __forceinline__ void load_dq32(const KArgs32 &a, const int zero_dq, const int c, float (&dq)[D + 2]) {
 #pragma unroll
     for (int k = 0; k < D + 2; k++) dq[k] = 0.f;
     if (!zero_dq) {
 #pragma unroll
-        for (int k = 0; k < D + 2; k++) dq[k] = ld_once<D, 2>(a.dq + (size_t)k * a.nc + c);
+        for (int k = 0; k < D + 2; k++) dq[k] = ld_once<NT>(a.dq + (size_t)k * a.nc + c);
     }
 }
 
 // sponge, RK update and stores of one cell: q its state (the updated one on
 // return), dq its accumulated register
-template <int D>
+template <int D, bool NT>
 __device__ __forceinline__ void finish_cell32(const KArgs32 &a, const int c, const float dt, const float B, float *qout,
                                               float (&q)[D + 2], float (&dq)[D + 2]) {
     // sponge: sigma (q_inf - q) = -sigma q' (no sigma array, and no term,
     // where the case has no sponge layer and every sigma is zero)
-    const float sgm = a.sigma ? ld_once<D, 3>(a.sigma + c) : 0.f;
+    const float sgm = a.sigma ? ld_once<NT>(a.sigma + c) : 0.f;
 #pragma unroll
     for (int k = 0; k < D + 2; k++) {
         if (a.sigma) dq[k] -= dt * sgm * q[k];
         q[k] += B * dq[k];
-        st_once<D, 2>(a.dq + (size_t)k * a.nc + c, dq[k]);
+        st_once<NT>(a.dq + (size_t)k * a.nc + c, dq[k]);
     }
-    store_q32<D>(qout, a.ntot, c, q);
+    store_q32<D, NT>(qout, a.ntot, c, q);
 }
 // boundary ghost g of a cell whose updated state is q, written for the next
 // stage
-template <int D>
+template <int D, bool NT>
 __device__ __forceinline__ void refresh_ghost32(const KArgs32 &a, const int g, float *qout, const float (&q)[D + 2]) {
     float qg[D + 2];
     if (!ghost_state32<D>(a, a.ghost_role[g], q, qg)) {
         if (qout == a.q) return;
         load_q32<D>(a, a.nc + g, qg);  // an unset patch's ghost keeps its state
     }
-    store_q32<D>(qout, a.ntot, a.nc + g, qg);
+    store_q32<D, NT>(qout, a.ntot, a.nc + g, qg);
 }
 
 // ordered gather of one cell's stored face fluxes, sponge and RK update in
 // place, with the cell's boundary ghosts refreshed; res receives the
 // residual, q the updated state
-template <int D, bool RES>
+template <int D, bool RES, bool NT>
 __device__ __forceinline__ void cell_update32_cell(const KArgs32 &a, float A, float B, int zero_dq, const int c,
                                                    float (&res)[D + 2], float (&q)[D + 2], float &vinv) {
     const float dt = (float)(*a.dt);
-    vinv = ld_once<D, 3>(a.vinv + c);
+    vinv = ld_once<NT>(a.vinv + c);
     const float sP = dt * vinv;
     float dq[D + 2];
-    load_dq32<D>(a, zero_dq, c, dq);
+    load_dq32<D, NT>(a, zero_dq, c, dq);
 #pragma unroll
     for (int k = 0; k < D + 2; k++) res[k] = 0.f;
     load_q32<D>(a, c, q);
@@ -1009,10 +986,10 @@ __device__ __forceinline__ void cell_update32_cell(const KArgs32 &a, float A, fl
             }
         }
     }
-    finish_cell32<D>(a, c, dt, B, a.q, q, dq);
+    finish_cell32<D, NT>(a, c, dt, B, a.q, q, dq);
     // refresh this cell's boundary ghosts for the next stage
     for (unsigned m = gmask; m; m &= m - 1)
-        refresh_ghost32<D>(a, a.fN[a.g_ent[e0 + __builtin_ctz(m)] & kFaceMask] - a.nc, a.q, q);
+        refresh_ghost32<D, NT>(a, a.fN[a.g_ent[e0 + __builtin_ctz(m)] & kFaceMask] - a.nc, a.q, q);
 }
 
 template <int D, int MODE>
@@ -1026,7 +1003,7 @@ __device__ __forceinline__ double cfl_cell32(const KArgs32 &a, const FA &fa, con
 // every thread of the block must call this (block-wide reductions when RES
 // or CFL).  CFL >= 0 (the last stage of a step): the step's compute_dt (0) /
 // compute_cfl (1) of the updated cells, per-block extrema into a.partial.
-template <int D, bool RES, int CFL>
+template <int D, bool RES, int CFL, bool NT>
 __device__ __forceinline__ void cell_update32_body(const KArgs32 &a, float A, float B, int zero_dq, const int c,
                                                    const int lblk, double cfl_param) {
     static_assert(!(RES && CFL >= 0), "the residual and the CFL share a.partial");
@@ -1037,7 +1014,7 @@ __device__ __forceinline__ void cell_update32_body(const KArgs32 &a, float A, fl
     for (int k = 0; k < D + 2; k++) rsq[k] = 0.0;
     if (c < a.nc) {
         float res[D + 2], q[D + 2], vinv;
-        cell_update32_cell<D, RES>(a, A, B, zero_dq, c, res, q, vinv);
+        cell_update32_cell<D, RES, NT>(a, A, B, zero_dq, c, res, q, vinv);
         if constexpr (CFL >= 0) cv = cfl_cell32<D, CFL>(a, c, q, vinv, cfl_param);
         if (RES) {
 #pragma unroll
@@ -1189,7 +1166,7 @@ __global__ void __launch_bounds__(256) bc_fill32(KArgs32 a) {
 // fin_nblk > 0: one block more, the last, reduces the previous step's
 // fin_nblk per-block CFL maxima in a.partial into *a.d_cfl (as the one-launch
 // stage does)
-template <int D, int GRAD, bool VISC, bool RG, bool SL, bool PK>
+template <int D, int GRAD, bool VISC, bool RG, bool SL, bool PK, bool NT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 3 && SL && !RG ? 5 : 1)))
 grad_vis32(KArgs32 a, int fin_nblk) {
     int nb = (int)gridDim.x;
@@ -1200,19 +1177,19 @@ grad_vis32(KArgs32 a, int fin_nblk) {
             return;
         }
     }
-    grad_vis32_body<D, GRAD, VISC, RG, SL, PK>(a, xcd_block((int)blockIdx.x, nb) * (int)blockDim.x + (int)threadIdx.x);
+    grad_vis32_body<D, GRAD, VISC, RG, SL, PK, NT>(a, xcd_block((int)blockIdx.x, nb) * (int)blockDim.x + (int)threadIdx.x);
 }
 // 3D M1 / M2 faces: 5 waves per SIMD fit in 96 VGPRs without spills (97
 // would allow 4): O-grid face kernel 1.107 -> 1.033 ms per step.  Forcing
 // more waves on the update and gradient kernels was measured slower.
-template <int D, int SOLVER, bool VISC, bool STORED>
+template <int D, int SOLVER, bool VISC, bool STORED, bool NT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 3 && SOLVER < 2 ? 5 : 1)))
 face_flux32(KArgs32 a) {
-    face_flux32_body<D, SOLVER, VISC, STORED>(a, LFM_TID(blockIdx.x));
+    face_flux32_body<D, SOLVER, VISC, STORED, NT>(a, LFM_TID(blockIdx.x));
 }
-template <int D, bool RES, int CFL>
+template <int D, bool RES, int CFL, bool NT>
 __global__ void __launch_bounds__(256) cell_update32(KArgs32 a, float A, float B, int zero_dq, double cfl_param) {
-    cell_update32_body<D, RES, CFL>(a, A, B, zero_dq, LFM_TID(blockIdx.x), LFM_BLK(), cfl_param);
+    cell_update32_body<D, RES, CFL, NT>(a, A, B, zero_dq, LFM_TID(blockIdx.x), LFM_BLK(), cfl_param);
 }
 // ---------------------------------------------------------------------------
 // One RK stage in one launch for inviscid M1 / M2: each cell forms its faces'
@@ -1227,12 +1204,12 @@ __global__ void __launch_bounds__(256) cell_update32(KArgs32 a, float A, float B
 // us per step); in 2D all four, since a 2D stage is bound by the latency of
 // its dependent loads.
 constexpr int kFusedGroup32 = 2;
-template <int D, int SOLVER, int CFL, bool PK, bool HALF>
+template <int D, int SOLVER, int CFL, bool PK, bool HALF, bool NT>
 __device__ __forceinline__ void stage32_body(const KArgs32 &a, float *qout, float A, float B, int zero_dq, const int c,
                                              const int lblk, double cfl_param) {
     constexpr int U = GatherUnroll<D>::value;
     constexpr int G = D == 3 ? kFusedGroup32 : U;
-    using F = FaceOf32<D, PK>;
+    using F = FaceOf32<D, PK, NT>;
     // a face's own data are kept for the CFL/dt sums after the update; from
     // the table they are read again
     constexpr bool kKeep = CFL >= 0 && !PK;
@@ -1252,8 +1229,8 @@ __device__ __forceinline__ void stage32_body(const KArgs32 &a, float *qout, floa
         }
         float qc[D + 2], dq[D + 2];
         load_q32<D>(a, c, qc);
-        const float vinv = ld_once<D, 3>(a.vinv + c);
-        load_dq32<D>(a, zero_dq, c, dq);
+        const float vinv = ld_once<NT>(a.vinv + c);
+        load_dq32<D, NT>(a, zero_dq, c, dq);
         const float dt = (float)(*a.dt);
         const Prim32<D> sc = prim32<D>(a, qc);
         const float s = dt * vinv;
@@ -1305,18 +1282,18 @@ __device__ __forceinline__ void stage32_body(const KArgs32 &a, float *qout, floa
         float q[D + 2];
 #pragma unroll
         for (int k = 0; k < D + 2; k++) q[k] = qc[k];
-        finish_cell32<D>(a, c, dt, B, qout, q, dq);
+        finish_cell32<D, NT>(a, c, dt, B, qout, q, dq);
         // the boundary ghosts of this cell (only cells of the boundary
         // submesh have any) for the next stage
         if (c < a.nsm0) {
 #pragma unroll 1
             for (int j = 0; j < U; j++) {
                 const int o = F::other_of(a, F::load_key(a, j, c));
-                if (o >= a.nc) refresh_ghost32<D>(a, o - a.nc, qout, q);
+                if (o >= a.nc) refresh_ghost32<D, NT>(a, o - a.nc, qout, q);
             }
             for (int e = e1; U < kMaxFaces && e < e2; e++) {
                 const int ent = a.g_ent[e];
-                if (ent >= 0 && (ent & kGhostFaceFlag)) refresh_ghost32<D>(a, a.fN[ent & kFaceMask] - a.nc, qout, q);
+                if (ent >= 0 && (ent & kGhostFaceFlag)) refresh_ghost32<D, NT>(a, a.fN[ent & kFaceMask] - a.nc, qout, q);
             }
         }
         if constexpr (CFL >= 0) {
@@ -1366,7 +1343,7 @@ __global__ void __launch_bounds__(256) build_slots32(KArgs32 a, const uint16_t *
     const int e0 = a.g_off[c], ne = a.g_off[c + 1] - e0;
     constexpr int U = GatherUnroll<D>::value;
     for (int j = 0; j < U; j++) {
-        FaceOf32<D, false> f;
+        FaceOf32<D, false, false> f;
         f.other = c;
         f.wc = 0.5f;
         for (int k = 0; k < D; k++) f.S[k] = 0.f;
@@ -1391,7 +1368,7 @@ __global__ void __launch_bounds__(256) build_slots32(KArgs32 a, const uint16_t *
 // the last, which reduces the fin_nblk per-block CFL maxima that an earlier
 // launch left in a.partial into *a.d_cfl (the final reduction of the
 // previous step, whose result no stage of this step reads).
-template <int D, int SOLVER, int CFL, bool PK, bool HALF>
+template <int D, int SOLVER, int CFL, bool PK, bool HALF, bool NT>
 __global__ void __launch_bounds__(256) stage_fused32(KArgs32 a, float *qout, float A, float B, int zero_dq,
                                                      double cfl_param, int fin_nblk) {
     int nb = (int)gridDim.x;
@@ -1407,7 +1384,7 @@ __global__ void __launch_bounds__(256) stage_fused32(KArgs32 a, float *qout, flo
         (void)fin_nblk;
     }
     const int blk = xcd_block((int)blockIdx.x, nb);
-    stage32_body<D, SOLVER, CFL, PK, HALF>(a, qout, A, B, zero_dq, blk * (int)blockDim.x + (int)threadIdx.x, blk,
+    stage32_body<D, SOLVER, CFL, PK, HALF, NT>(a, qout, A, B, zero_dq, blk * (int)blockDim.x + (int)threadIdx.x, blk,
                                            cfl_param);
 }
 template <int D, int MODE>
@@ -1455,32 +1432,32 @@ __device__ __forceinline__ void batch_slot(const BatchMap &m, int &r, int &lblk)
     lblk = b - m.first[r];
 }
 
-template <int D, int GRAD, bool VISC, bool RG>
+template <int D, int GRAD, bool VISC, bool RG, bool NT>
 __global__ void __launch_bounds__(256) grad_vis32_b(const KArgs32 *args, BatchMap m) {
     int r, lb;
     batch_slot(m, r, lb);
-    grad_vis32_body<D, GRAD, VISC, RG>(args[r], lb * 256 + threadIdx.x);
+    grad_vis32_body<D, GRAD, VISC, RG, false, false, NT>(args[r], lb * 256 + threadIdx.x);
 }
 // (batch members are undecomposed: their tensors are never stored)
-template <int D, int SOLVER, bool VISC>
+template <int D, int SOLVER, bool VISC, bool NT>
 __global__ void __launch_bounds__(256) face_flux32_b(const KArgs32 *args, BatchMap m) {
     int r, lb;
     batch_slot(m, r, lb);
-    face_flux32_body<D, SOLVER, VISC, false>(args[r], lb * 256 + threadIdx.x);
+    face_flux32_body<D, SOLVER, VISC, false, NT>(args[r], lb * 256 + threadIdx.x);
 }
 // CFL 1: the last stage, with compute_cfl at each solver's own deltaT
-template <int D, int CFL>
+template <int D, int CFL, bool NT>
 __global__ void __launch_bounds__(256) cell_update32_b(const KArgs32 *args, BatchMap m, float A, float B,
                                                        int zero_dq) {
     int r, lb;
     batch_slot(m, r, lb);
     const KArgs32 &a = args[r];
-    cell_update32_body<D, false, CFL>(a, A, B, zero_dq, lb * 256 + threadIdx.x, lb, CFL >= 0 ? *a.dt : 0.0);
+    cell_update32_body<D, false, CFL, NT>(a, A, B, zero_dq, lb * 256 + threadIdx.x, lb, CFL >= 0 ? *a.dt : 0.0);
 }
 // one-launch stage over a batch (inviscid M1 / M2), each member from one
 // of its state buffers into the other: flip 0 from a.q into a.q_alt, flip 1
 // back
-template <int D, int SOLVER, int CFL>
+template <int D, int SOLVER, int CFL, bool NT>
 __global__ void __launch_bounds__(256) stage_fused32_b(const KArgs32 *args, BatchMap m, float A, float B, int zero_dq,
                                                        int flip) {
     int r, lb;
@@ -1492,9 +1469,9 @@ __global__ void __launch_bounds__(256) stage_fused32_b(const KArgs32 *args, Batc
     const double dt = CFL >= 0 ? *a.dt : 0.0;
     // members may hold either slot form
     if (a.pk)
-        stage32_body<D, SOLVER, CFL, true, false>(a, qout, A, B, zero_dq, c, lb, dt);
+        stage32_body<D, SOLVER, CFL, true, false, NT>(a, qout, A, B, zero_dq, c, lb, dt);
     else
-        stage32_body<D, SOLVER, CFL, false, false>(a, qout, A, B, zero_dq, c, lb, dt);
+        stage32_body<D, SOLVER, CFL, false, false, NT>(a, qout, A, B, zero_dq, c, lb, dt);
 }
 // one block per solver: max of its partials into its CFL scalar
 static __global__ void __launch_bounds__(256) cfl_final32_b(const KArgs32 *args) {

@@ -120,32 +120,29 @@ __device__ __forceinline__ size_t slot_at(int nc, int j, int f, int c) {
 }
 inline size_t slot_array_len(int nc, int U, int NF) { return (size_t)(nc + 63) / 64 * 64 * U * NF; }
 
-// FP64 loads and stores of data a kernel touches once, non-temporal where
-// kStreamNT64 allows (levels as on the FP32 path: 2 the RK register, 3 the
-// new states, the face kernel's face lists and geometry, the face fluxes,
-// the gradient records, 1/V and sponge), so that they do not displace the
-// gathered neighbour records in L2.  Every level in 2D and 3D (FP64 arrays
-// outgrow the Infinity Cache sooner): 256^3 box 11.73 -> 11.38 ms per step,
-// 4.2 M-cell O-grid 5.96 -> 5.65, 1 M-cell annulus 0.880 -> 0.848.
-template <int D>
-constexpr int kStreamNT64 = 3;
-template <int D, int LEVEL, int NT = kStreamNT64<D>, class T>
-__device__ __forceinline__ T ld64_once(const T *p) {
-    if constexpr (NT >= LEVEL) return __builtin_nontemporal_load(p);
+// Loads and stores of data a kernel touches once (face slots, RK register, new
+// states, the face kernel's face lists and geometry, face fluxes, gradient
+// records, 1/V and sponge), non-temporal where NT: that keeps the gathered
+// neighbour records in L2, but what one launch wrote the next then does not
+// find in the 256 MB Infinity Cache.  So NT is chosen by what a stage touches
+// (Solver::stream_nt).
+template <bool NT, class T>
+__device__ __forceinline__ T ld_once(const T *p) {
+    if constexpr (NT) return __builtin_nontemporal_load(p);
     return *p;
 }
-template <int D, int LEVEL, int NT = kStreamNT64<D>, class T>
-__device__ __forceinline__ void st64_once(T *p, T v) {
-    if constexpr (NT >= LEVEL)
+template <bool NT, class T>
+__device__ __forceinline__ void st_once(T *p, T v) {
+    if constexpr (NT)
         __builtin_nontemporal_store(v, p);
     else
         *p = v;
 }
 using d2v = double __attribute__((ext_vector_type(2)));
-template <int D, int LEVEL, int NT = kStreamNT64<D>>
+template <bool NT>
 __device__ __forceinline__ void st64x2_once(double *p, double x, double y) {
     const d2v v = {x, y};
-    st64_once<D, LEVEL, NT>(reinterpret_cast<d2v *>(p), v);
+    st_once<NT>(reinterpret_cast<d2v *>(p), v);
 }
 
 // face f's area vector (one 16-byte load in 2D)
@@ -179,11 +176,11 @@ __device__ __forceinline__ void load_q(const KArgs &a, int i, double *q) {
     if (D == 3) q[4] = a.q[(size_t)4 * a.ntot + i];
 }
 
-template <int D, int NT = kStreamNT64<D>>
+template <int D, bool NT>
 __device__ __forceinline__ void store_q(double *qv, size_t ntot, int i, const double *q) {
-    st64x2_once<D, 3, NT>(qv + 4 * (size_t)i, q[0], q[1]);
-    st64x2_once<D, 3, NT>(qv + 4 * (size_t)i + 2, q[2], q[3]);
-    if (D == 3) st64_once<D, 3, NT>(qv + 4 * ntot + i, q[4]);
+    st64x2_once<NT>(qv + 4 * (size_t)i, q[0], q[1]);
+    st64x2_once<NT>(qv + 4 * (size_t)i + 2, q[2], q[3]);
+    if (D == 3) st_once<NT>(qv + 4 * ntot + i, q[4]);
 }
 
 // One cell's gradients as one record, padded to whole 16-byte words: dudx
@@ -331,7 +328,7 @@ __global__ void __launch_bounds__(256) bc_fill(KArgs a) {
     load_q<D>(a, a.ghost_cell[g], qi);
     if (!ghost_state<D>(a, a.ghost_role[g], qi, qg)) return;
     const int gi = a.nc + g;
-    store_q<D>(a.q, a.ntot, gi, qg);
+    store_q<D, false>(a.q, a.ntot, gi, qg);
 }
 
 // ---------------------------------------------------------------------------
@@ -406,7 +403,7 @@ __device__ __forceinline__ void vis_tensors(const KArgs &a, const double (&dudx)
     for (int i = 0; i < D; i++) sU[i] = dotD<D>(U, tau[i]);
 }
 
-template <int D, int GRAD, bool VISC, bool RG>
+template <int D, int GRAD, bool VISC, bool RG, bool NT>
 __global__ void __launch_bounds__(256) grad_vis(KArgs a) {
     const int c = LFM_TID(blockIdx.x);
     using R = GradRec64<D, RG>;
@@ -557,7 +554,7 @@ __global__ void __launch_bounds__(256) grad_vis(KArgs a) {
         const int c0 = c - t;
         const int nrec = a.nc - c0 < (int)blockDim.x ? a.nc - c0 : (int)blockDim.x;
         d2v *dst = reinterpret_cast<d2v *>(a.dudx + (size_t)c0 * R::kStride);
-        for (int j = t; j < nrec * W; j += blockDim.x) st64_once<D, 3>(dst + j, d2v{st[j].x, st[j].y});
+        for (int j = t; j < nrec * W; j += blockDim.x) st_once<NT>(dst + j, d2v{st[j].x, st[j].y});
     }
 }
 
@@ -707,20 +704,20 @@ __device__ __forceinline__ void flux_m2(const double rhoavg, const double (&rUa)
 // without spills instead of 170 (2 waves), 82 -> 73 us per launch on 1 M
 // cells; in 3D the same bound spills and is slower.
 // ---------------------------------------------------------------------------
-template <int D, int SOLVER, bool VISC, bool STORED>
+template <int D, int SOLVER, bool VISC, bool STORED, bool NT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 2 ? 3 : 2))) face_flux(KArgs a) {
     const int f = LFM_TID(blockIdx.x);
     if (f >= a.nf) return;
-    const int P = ld64_once<D, 3>(a.fP + f), N = ld64_once<D, 3>(a.fN + f);
+    const int P = ld_once<NT>(a.fP + f), N = ld_once<NT>(a.fN + f);
     // is_ghost: boundary ghosts only; halo ghosts carry the neighbour's tensors
     const bool ghost = (unsigned)(N - a.nc) < (unsigned)a.ng_bnd;
-    const double w = ld64_once<D, 3>(a.w + f);
+    const double w = ld_once<NT>(a.w + f);
     const size_t nt = a.ntot;
     double S[D], d[D], qP[D + 2], qN[D + 2];
 #pragma unroll
-    for (int k = 0; k < D; k++) S[k] = ld64_once<D, 3>(a.S + (size_t)f * D + k);
+    for (int k = 0; k < D; k++) S[k] = ld_once<NT>(a.S + (size_t)f * D + k);
 #pragma unroll
-    for (int k = 0; k < D; k++) d[k] = ld64_once<D, 3>(a.d + (size_t)k * a.nf + f);
+    for (int k = 0; k < D; k++) d[k] = ld_once<NT>(a.d + (size_t)k * a.nf + f);
     load_q<D>(a, P, qP);
     load_q<D>(a, N, qN);
     using R = GradRec64<D, SOLVER == 2>;
@@ -933,9 +930,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 2
     const double lapT = kcond * (dm * (aT - cT) * dmi + dotD<D>(K, dT));
     rhs[D + 1] += dotD<D>(sU, S) + lapT;
     }
-    st64x2_once<D, 3>(a.frhs + 4 * (size_t)f, rhs[0], rhs[1]);
-    st64x2_once<D, 3>(a.frhs + 4 * (size_t)f + 2, rhs[2], rhs[3]);
-    if (D == 3) st64_once<D, 3>(a.frhs + (size_t)4 * a.nf + f, rhs[D + 1]);
+    st64x2_once<NT>(a.frhs + 4 * (size_t)f, rhs[0], rhs[1]);
+    st64x2_once<NT>(a.frhs + 4 * (size_t)f + 2, rhs[2], rhs[3]);
+    if (D == 3) st_once<NT>(a.frhs + (size_t)4 * a.nf + f, rhs[D + 1]);
 }
 
 // tauMC and sigmaU of every cell from the stored dudx (field read-back of a
@@ -1055,21 +1052,21 @@ __device__ __forceinline__ void block_extremum(double v, double *dst) {
 // the cell's RK register as the last stage left it, zero at a step's first
 // stage: every component's load issued before any is used (a choice per
 // component compiles to a branch and a wait each)
-template <int D, int NT = kStreamNT64<D>>
+template <int D, bool NT>
 __device__ __forceinline__ void load_dq64(const KArgs &a, const int zero_dq, const int c, double (&dq)[D + 2]) {
 #pragma unroll
     for (int k = 0; k < D + 2; k++) dq[k] = 0.0;
     if (!zero_dq) {
 #pragma unroll
-        for (int k = 0; k < D + 2; k++) dq[k] = ld64_once<D, 2, NT>(a.dq + (size_t)k * a.nc + c);
+        for (int k = 0; k < D + 2; k++) dq[k] = ld_once<NT>(a.dq + (size_t)k * a.nc + c);
     }
 }
 
 // the sponge term of one cell (cfd_v0.cpp:2808-2811)
-template <int D, int NT = kStreamNT64<D>>
+template <int D, bool NT>
 __device__ __forceinline__ void sponge64(const KArgs &a, const int c, const double dt, const double (&q)[D + 2],
                                          double (&dq)[D + 2]) {
-    const double sg = ld64_once<D, 3, NT>(a.sigma + c);
+    const double sg = ld_once<NT>(a.sigma + c);
     dq[0] += dt * sg * (a.rho_inf - q[0]);
 #pragma unroll
     for (int k = 0; k < D; k++) dq[k + 1] += dt * sg * (a.rho_inf * a.U_inf[k] - q[k + 1]);
@@ -1083,7 +1080,7 @@ __device__ __forceinline__ void sponge64(const KArgs &a, const int c, const doub
 // stage of a step): the step's compute_dt (0) / compute_cfl (1) of the
 // updated cells, per-block extrema into a.partial.
 // ---------------------------------------------------------------------------
-template <int D, bool RES, int CFL>
+template <int D, bool RES, int CFL, bool NT>
 __global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, int zero_dq, double cfl_param) {
     static_assert(!(RES && CFL >= 0), "the residual and the CFL share a.partial");
     const int c = LFM_TID(blockIdx.x);
@@ -1094,9 +1091,9 @@ __global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, 
     for (int k = 0; k < D + 2; k++) rsq[k] = 0.0;
     if (c < a.nc) {
         const double dt = *a.dt;
-        const double vinv = ld64_once<D, 3>(a.vinv + c);
+        const double vinv = ld_once<NT>(a.vinv + c);
         double dq[D + 2], res[D + 2], q[D + 2];
-        load_dq64<D>(a, zero_dq, c, dq);
+        load_dq64<D, NT>(a, zero_dq, c, dq);
 #pragma unroll
         for (int k = 0; k < D + 2; k++) res[k] = 0.0;
         load_q<D>(a, c, q);
@@ -1142,19 +1139,19 @@ __global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, 
             load_frhs<D>(a, f, f1);
             add(en, f1);
         }
-        if (a.sigma) sponge64<D>(a, c, dt, q, dq);
+        if (a.sigma) sponge64<D, NT>(a, c, dt, q, dq);
 #pragma unroll
         for (int k = 0; k < D + 2; k++) {
             q[k] += B * dq[k];
-            st64_once<D, 2>(a.dq + (size_t)k * a.nc + c, dq[k]);
+            st_once<NT>(a.dq + (size_t)k * a.nc + c, dq[k]);
         }
-        store_q<D>(a.q, a.ntot, c, q);
+        store_q<D, NT>(a.q, a.ntot, c, q);
         // refresh this cell's boundary ghosts for the next stage
         for (int i = 0; i < ngf; i++) {
             const int g = a.fN[gface[i]] - a.nc;
             double qg[D + 2];
             if (!ghost_state<D>(a, a.ghost_role[g], q, qg)) continue;
-            store_q<D>(a.q, a.ntot, a.nc + g, qg);
+            store_q<D, NT>(a.q, a.ntot, a.nc + g, qg);
         }
         if constexpr (CFL >= 0) cv = cfl_cell<D, CFL>(a, c, q, cfl_param);
         if (RES) {
@@ -1276,14 +1273,14 @@ constexpr int kTabRec64 = 6;
 
 // the face data of gather entry j of cell c as that cell sees them; key: the
 // packed word, or the slot's key
-template <int D, bool PK, int NT>
+template <int D, bool PK, bool NT>
 struct FaceOf64 {
     int other;
     double S[D], Sm, wc, wo;
     __device__ __forceinline__ static int load_key(const KArgs &a, const int j, const int c) {
         const size_t i = slot_at<D, 1>(a.nc, j, 0, c);
-        if constexpr (PK) return (int)ld64_once<D, 1, NT>(a.pk + i);
-        return ld64_once<D, 1, NT>(a.sl_nb + i);
+        if constexpr (PK) return (int)ld_once<NT>(a.pk + i);
+        return ld_once<NT>(a.sl_nb + i);
     }
     __device__ __forceinline__ static int other_of(const KArgs &a, const int key) {
         if constexpr (PK) return (int)((uint32_t)key & ((1u << a.pk_shift) - 1u));
@@ -1317,8 +1314,8 @@ struct FaceOf64 {
         } else {
             double s[D];
 #pragma unroll
-            for (int k = 0; k < D; k++) s[k] = ld64_once<D, 1, NT>(a.sl_S + slot_at<D, D>(a.nc, j, k, c));
-            from_face(key >= 0, s, ld64_once<D, 1, NT>(a.sl_w + slot_at<D, 1>(a.nc, j, 0, c)));
+            for (int k = 0; k < D; k++) s[k] = ld_once<NT>(a.sl_S + slot_at<D, D>(a.nc, j, k, c));
+            from_face(key >= 0, s, ld_once<NT>(a.sl_w + slot_at<D, 1>(a.nc, j, 0, c)));
         }
     }
     // an entry of the gather list (beyond the slots)
@@ -1363,7 +1360,7 @@ __device__ __forceinline__ double cfl_term64(const double (&q)[D + 2], const dou
 // reduces the fin_nblk per-block CFL maxima that the previous step's last
 // stage left in a.partial into *fin_out.
 // SYM: every face's weights allow flux_m1_sym.
-template <int D, int SOLVER, int CFL, bool PK, bool SYM, int NT>
+template <int D, int SOLVER, int CFL, bool PK, bool SYM, bool NT>
 __global__ void __launch_bounds__(256) stage_fused64(KArgs a, double *qout, double A, double B, int zero_dq,
                                                      double cfl_param, int fin_nblk, double *fin_out) {
     int nb = (int)gridDim.x;
@@ -1390,7 +1387,7 @@ __global__ void __launch_bounds__(256) stage_fused64(KArgs a, double *qout, doub
         for (int u = 0; u < G; u++) key[u] = F::load_key(a, u, c);
         double qc[D + 2], dq[D + 2];
         load_q<D>(a, c, qc);
-        const double vinv = ld64_once<D, 3, NT>(a.vinv + c);
+        const double vinv = ld_once<NT>(a.vinv + c);
         load_dq64<D, NT>(a, zero_dq, c, dq);
         const double dt = *a.dt;
         const Prim64<D> sc = prim64<D, SOLVER>(a, qc);
@@ -1446,7 +1443,7 @@ __global__ void __launch_bounds__(256) stage_fused64(KArgs a, double *qout, doub
 #pragma unroll
         for (int k = 0; k < D + 2; k++) {
             q[k] += B * dq[k];
-            st64_once<D, 2, NT>(a.dq + (size_t)k * a.nc + c, dq[k]);
+            st_once<NT>(a.dq + (size_t)k * a.nc + c, dq[k]);
         }
         store_q<D, NT>(qout, a.ntot, c, q);
         // this cell's boundary ghosts for the next stage

@@ -186,15 +186,20 @@ static void launch_bc64(Solver *s) {
     if (s->L.ng) hipLaunchKernelGGL(bc_fill<D>, dim3(nblocks(s->L.ng)), dim3(kBlock), 0, s->stream, s->k64);
 }
 
-template <int D, bool V>
-static void launch_gradvis64_v(Solver *s) {
+template <int D, bool V, bool NT>
+static void launch_gradvis64_nt(Solver *s) {
     const int nb = nblocks(s->L.nc);
     if (s->prm.solver == 2 && s->prm.minmod)
-        hipLaunchKernelGGL((grad_vis<D, 2, V, true>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64);
+        hipLaunchKernelGGL((grad_vis<D, 2, V, true, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64);
     else if (s->prm.solver == 2)
-        hipLaunchKernelGGL((grad_vis<D, 0, V, true>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64);
+        hipLaunchKernelGGL((grad_vis<D, 0, V, true, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64);
     else
-        hipLaunchKernelGGL((grad_vis<D, 0, V, false>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64);
+        hipLaunchKernelGGL((grad_vis<D, 0, V, false, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64);
+}
+
+template <int D, bool V>
+static void launch_gradvis64_v(Solver *s) {
+    s->stream_nt ? launch_gradvis64_nt<D, V, true>(s) : launch_gradvis64_nt<D, V, false>(s);
 }
 
 // full: every tensor calc_VIS forms (the per-stage entry point); otherwise
@@ -207,14 +212,19 @@ static void launch_gradvis64(Solver *s, bool full) {
         launch_gradvis64_v<D, false>(s);
 }
 
-template <int D, bool V, bool ST>
-static void launch_flux64_v(Solver *s) {
+template <int D, bool V, bool ST, bool NT>
+static void launch_flux64_nt(Solver *s) {
     const int nb = nblocks(s->L.nf);
     switch (s->prm.solver) {
-    case 0: hipLaunchKernelGGL((face_flux<D, 0, V, ST>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64); break;
-    case 1: hipLaunchKernelGGL((face_flux<D, 1, V, ST>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64); break;
-    default: hipLaunchKernelGGL((face_flux<D, 2, V, ST>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64); break;
+    case 0: hipLaunchKernelGGL((face_flux<D, 0, V, ST, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64); break;
+    case 1: hipLaunchKernelGGL((face_flux<D, 1, V, ST, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64); break;
+    default: hipLaunchKernelGGL((face_flux<D, 2, V, ST, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64); break;
     }
+}
+
+template <int D, bool V, bool ST>
+static void launch_flux64_v(Solver *s) {
+    s->stream_nt ? launch_flux64_nt<D, V, ST, true>(s) : launch_flux64_nt<D, V, ST, false>(s);
 }
 
 template <int D>
@@ -225,25 +235,32 @@ static void launch_flux64(Solver *s) {
         launch_flux64_v<D, false, false>(s);
 }
 
-template <int D>
-static void launch_update64(Solver *s, double A, double B, bool zero_dq, bool res, bool accumulate_res,
-                            const Solver::CflJob *cfl) {
+template <int D, bool NT>
+static void launch_update64_nt(Solver *s, double A, double B, bool zero_dq, bool res, bool accumulate_res,
+                               const Solver::CflJob *cfl) {
     const int nb = nblocks(s->L.nc);
     if (res) {
-        hipLaunchKernelGGL((cell_update<D, true, -1>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
+        hipLaunchKernelGGL((cell_update<D, true, -1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
                            (int)zero_dq, 0.0);
         hipLaunchKernelGGL(reduce_sum, dim3(1), dim3(kBlock), 0, s->stream, s->k64.partial, nb, D + 2, s->d_res,
                            (int)accumulate_res);
     } else if (cfl && cfl->mode == 0) {
-        hipLaunchKernelGGL((cell_update<D, false, 0>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
+        hipLaunchKernelGGL((cell_update<D, false, 0, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
                            (int)zero_dq, cfl->param);
     } else if (cfl) {
-        hipLaunchKernelGGL((cell_update<D, false, 1>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
+        hipLaunchKernelGGL((cell_update<D, false, 1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
                            (int)zero_dq, cfl->param);
     } else {
-        hipLaunchKernelGGL((cell_update<D, false, -1>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
+        hipLaunchKernelGGL((cell_update<D, false, -1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
                            (int)zero_dq, 0.0);
     }
+}
+
+template <int D>
+static void launch_update64(Solver *s, double A, double B, bool zero_dq, bool res, bool accumulate_res,
+                            const Solver::CflJob *cfl) {
+    s->stream_nt ? launch_update64_nt<D, true>(s, A, B, zero_dq, res, accumulate_res, cfl)
+                 : launch_update64_nt<D, false>(s, A, B, zero_dq, res, accumulate_res, cfl);
 }
 
 template <int D>
@@ -268,7 +285,7 @@ int integrals64(Solver *s, double *out_dev) {
     return 0;
 }
 
-template <int D, int SOLVER, bool PK, bool SYM, int NT>
+template <int D, int SOLVER, bool PK, bool SYM, bool NT>
 static void launch_fused64_nt(Solver *s, double A, double B, int zero_dq, const KArgs &a, double *qout,
                              const Solver::CflJob *cfl, bool fin) {
     const int nb = nblocks(s->L.nc);
@@ -286,8 +303,8 @@ static void launch_fused64_nt(Solver *s, double A, double B, int zero_dq, const 
 template <int D, int SOLVER, bool PK, bool SYM>
 static void launch_fused64_v(Solver *s, double A, double B, int zero_dq, const KArgs &a, double *qout,
                              const Solver::CflJob *cfl, bool fin) {
-    s->stream_nt ? launch_fused64_nt<D, SOLVER, PK, SYM, 3>(s, A, B, zero_dq, a, qout, cfl, fin)
-                 : launch_fused64_nt<D, SOLVER, PK, SYM, 0>(s, A, B, zero_dq, a, qout, cfl, fin);
+    s->stream_nt ? launch_fused64_nt<D, SOLVER, PK, SYM, true>(s, A, B, zero_dq, a, qout, cfl, fin)
+                 : launch_fused64_nt<D, SOLVER, PK, SYM, false>(s, A, B, zero_dq, a, qout, cfl, fin);
 }
 
 // fin: the launch also reduces the previous step's CFL maxima (left in
@@ -523,14 +540,27 @@ bool Solver::ensure_slots32() {
     return true;
 }
 
-// Whether a stage that touches this many bytes marks what a kernel reads or
-// writes once as non-temporal.  Up to about a third more than the 256 MB
-// Infinity Cache the next launch finds part of it there if it is not marked;
-// beyond, marking keeps the gathered neighbour states in L2.  FP64 3D box,
-// one launch per stage, us per step marked / not: 134 MB 313 / 255, 214 MB
-// 460 / 386, 261 MB 553 / 487, 319 MB 654 / 645, 454 MB 903 / 915, 829 MB
-// 1560 / 1607.
-static bool stream_once(size_t bytes) { return bytes > (size_t)340 << 20; }
+// What one RK stage touches, and whether its kernels mark what they touch once
+// as non-temporal.
+void Solver::size_stage() {
+    const size_t D = L.D, w = fp32 ? sizeof(float) : sizeof(double), nc = L.nc, nf = L.nf;
+    const bool grads = visc || prm.solver == 2;
+    const size_t ent = L.g_ent.size() + nc;  // gather list and offsets
+    size_t b = nc * ((2 * (D + 2) + 2) * w);  // state, RK register, 1/V, sponge
+    if (fused_ok) {
+        // second state; slots: one word each, or a face's own data
+        const bool packed = fp32 ? table32.n > 0 : table64.n > 0;
+        const size_t U = D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value;
+        b += nc * ((D + 2) * w + U * (packed ? sizeof(int32_t) : sizeof(int32_t) + (D + 1) * w));
+    } else {
+        // face fluxes, S, d, w, both cells; gather list
+        b += nf * ((3 * D + 3) * w + 2 * sizeof(int32_t)) + ent * sizeof(int32_t);
+    }
+    if (grads) b += nc * (size_t)(fp32 ? k32->gstride : k64.gstride) * w;
+    if (grads && fp32 && D == 3) b += nc * GatherUnroll<3>::value * (sizeof(int32_t) + (D + 1) * w);  // slots
+    stage_bytes = b;
+    stream_nt = outgrows_cache(b);
+}
 
 bool Solver::alloc_all(void **p, const size_t *bytes, int n) {
     for (int i = 0; i < n; i++)
@@ -612,10 +642,6 @@ bool Solver::ensure_slots64() {
     k64.sl_S = sS;
     k64.sl_w = sw;
     k64.s_perm = pm;
-    // what one stage touches: two states, the RK register, the slots, 1/V
-    // and sponge
-    stream_nt = stream_once((size_t)(3 * (D + 2) + 1 + (k64.sigma ? 1 : 0)) * L.nc * sizeof(double) + words +
-                            (nt ? 0 : words / sizeof(int32_t) * (D + 1) * sizeof(double)));
     return true;
 }
 
@@ -796,6 +822,7 @@ int lfm_solver_create_part(const lfm_polymesh *mesh, const lfm_partition *part, 
     HIP_TRY(hipHostMalloc((void **)&s->h_scalar, 64 * sizeof(double), hipHostMallocDefault));
     int rc = s->fp32 ? lfm::create_fp32p(s.get()) : lfm::create_fp64(s.get());
     if (rc) return rc;
+    s->size_stage();
     s->halo_dev.resize(s->L.halo.size());
     for (size_t i = 0; i < s->L.halo.size(); i++) {
         const auto &hn = s->L.halo[i];

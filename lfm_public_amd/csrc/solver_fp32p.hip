@@ -186,17 +186,22 @@ void launch_bc32(Solver *s) {
     if (s->L.ng) hipLaunchKernelGGL(bc_fill32<D>, dim3(nblocks(s->L.ng)), dim3(kBlock), 0, s->stream, *s->k32);
 }
 
-template <int D, bool V, bool SL, bool PK>
-static void launch_gradvis32_v(Solver *s, bool fin) {
+template <int D, bool V, bool SL, bool PK, bool NT>
+static void launch_gradvis32_nt(Solver *s, bool fin) {
     const int nb = nblocks(s->L.nc);
     const dim3 grid(nb + (fin ? 1 : 0));
     const int fb = fin ? nb : 0;
     if (s->prm.solver == 2 && s->prm.minmod)
-        hipLaunchKernelGGL((grad_vis32<D, 2, V, true, SL, PK>), grid, dim3(kBlock), 0, s->stream, *s->k32, fb);
+        hipLaunchKernelGGL((grad_vis32<D, 2, V, true, SL, PK, NT>), grid, dim3(kBlock), 0, s->stream, *s->k32, fb);
     else if (s->prm.solver == 2)
-        hipLaunchKernelGGL((grad_vis32<D, 0, V, true, SL, PK>), grid, dim3(kBlock), 0, s->stream, *s->k32, fb);
+        hipLaunchKernelGGL((grad_vis32<D, 0, V, true, SL, PK, NT>), grid, dim3(kBlock), 0, s->stream, *s->k32, fb);
     else
-        hipLaunchKernelGGL((grad_vis32<D, 0, V, false, SL, PK>), grid, dim3(kBlock), 0, s->stream, *s->k32, fb);
+        hipLaunchKernelGGL((grad_vis32<D, 0, V, false, SL, PK, NT>), grid, dim3(kBlock), 0, s->stream, *s->k32, fb);
+}
+
+template <int D, bool V, bool SL, bool PK>
+static void launch_gradvis32_v(Solver *s, bool fin) {
+    s->stream_nt ? launch_gradvis32_nt<D, V, SL, PK, true>(s, fin) : launch_gradvis32_nt<D, V, SL, PK, false>(s, fin);
 }
 
 // 3D gradients read the face slots (same bits as the gather list; 4.2 M-cell
@@ -221,14 +226,19 @@ void launch_gradvis32(Solver *s, bool full, bool fin) {
     V ? launch_gradvis32_v<D, true, false, false>(s, fin) : launch_gradvis32_v<D, false, false, false>(s, fin);
 }
 
-template <int D, bool V, bool ST>
-static void launch_flux32_v(Solver *s) {
+template <int D, bool V, bool ST, bool NT>
+static void launch_flux32_nt(Solver *s) {
     const int nb = nblocks(s->L.nf);
     switch (s->prm.solver) {
-    case 0: hipLaunchKernelGGL((face_flux32<D, 0, V, ST>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32); break;
-    case 1: hipLaunchKernelGGL((face_flux32<D, 1, V, ST>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32); break;
-    default: hipLaunchKernelGGL((face_flux32<D, 2, V, ST>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32); break;
+    case 0: hipLaunchKernelGGL((face_flux32<D, 0, V, ST, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32); break;
+    case 1: hipLaunchKernelGGL((face_flux32<D, 1, V, ST, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32); break;
+    default: hipLaunchKernelGGL((face_flux32<D, 2, V, ST, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32); break;
     }
+}
+
+template <int D, bool V, bool ST>
+static void launch_flux32_v(Solver *s) {
+    s->stream_nt ? launch_flux32_nt<D, V, ST, true>(s) : launch_flux32_nt<D, V, ST, false>(s);
 }
 
 template <int D>
@@ -239,44 +249,58 @@ void launch_flux32(Solver *s) {
         launch_flux32_v<D, false, false>(s);
 }
 
-template <int D>
-void launch_update32(Solver *s, double A, double B, bool zero_dq, bool res, bool accumulate_res,
-                     const Solver::CflJob *cfl) {
+template <int D, bool NT>
+static void launch_update32_nt(Solver *s, double A, double B, bool zero_dq, bool res, bool accumulate_res,
+                               const Solver::CflJob *cfl) {
     const int nb = nblocks(s->L.nc);
     if (res) {
-        hipLaunchKernelGGL((cell_update32<D, true, -1>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
+        hipLaunchKernelGGL((cell_update32<D, true, -1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
                            (float)B, (int)zero_dq, 0.0);
         hipLaunchKernelGGL(reduce_sum, dim3(1), dim3(kBlock), 0, s->stream, s->k32->partial, nb, D + 2, s->d_res,
                            (int)accumulate_res);
     } else if (cfl && cfl->mode == 0) {
-        hipLaunchKernelGGL((cell_update32<D, false, 0>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
+        hipLaunchKernelGGL((cell_update32<D, false, 0, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
                            (float)B, (int)zero_dq, cfl->param);
     } else if (cfl) {
-        hipLaunchKernelGGL((cell_update32<D, false, 1>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
+        hipLaunchKernelGGL((cell_update32<D, false, 1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
                            (float)B, (int)zero_dq, cfl->param);
     } else {
-        hipLaunchKernelGGL((cell_update32<D, false, -1>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
+        hipLaunchKernelGGL((cell_update32<D, false, -1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
                            (float)B, (int)zero_dq, 0.0);
     }
 }
 
+template <int D>
+void launch_update32(Solver *s, double A, double B, bool zero_dq, bool res, bool accumulate_res,
+                     const Solver::CflJob *cfl) {
+    s->stream_nt ? launch_update32_nt<D, true>(s, A, B, zero_dq, res, accumulate_res, cfl)
+                 : launch_update32_nt<D, false>(s, A, B, zero_dq, res, accumulate_res, cfl);
+}
+
 // fin: one block more reduces the CFL maxima of the previous step's last
 // stage (left in a.partial) into a.d_cfl
-template <int D, int SOLVER, bool PK, bool HALF>
-static void launch_fused32_v(Solver *s, float A, float B, int zero_dq, const KArgs32 &a, float *qout,
+template <int D, int SOLVER, bool PK, bool HALF, bool NT>
+static void launch_fused32_nt(Solver *s, float A, float B, int zero_dq, const KArgs32 &a, float *qout,
                              const Solver::CflJob *cfl, bool fin) {
     const int nb = nblocks(s->L.nc);
     if (!cfl) {
-        hipLaunchKernelGGL((stage_fused32<D, SOLVER, -1, PK, HALF>), dim3(nb + (fin ? 1 : 0)), dim3(kBlock), 0, s->stream, a,
+        hipLaunchKernelGGL((stage_fused32<D, SOLVER, -1, PK, HALF, NT>), dim3(nb + (fin ? 1 : 0)), dim3(kBlock), 0, s->stream, a,
                            qout, A, B, zero_dq, 0.0, fin ? nb : 0);
         return;
     }
     if (cfl->mode == 0)
-        hipLaunchKernelGGL((stage_fused32<D, SOLVER, 0, PK, HALF>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
+        hipLaunchKernelGGL((stage_fused32<D, SOLVER, 0, PK, HALF, NT>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
                            zero_dq, cfl->param, 0);
     else
-        hipLaunchKernelGGL((stage_fused32<D, SOLVER, 1, PK, HALF>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
+        hipLaunchKernelGGL((stage_fused32<D, SOLVER, 1, PK, HALF, NT>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
                            zero_dq, cfl->param, 0);
+}
+
+template <int D, int SOLVER, bool PK, bool HALF>
+static void launch_fused32_v(Solver *s, float A, float B, int zero_dq, const KArgs32 &a, float *qout,
+                             const Solver::CflJob *cfl, bool fin) {
+    s->stream_nt ? launch_fused32_nt<D, SOLVER, PK, HALF, true>(s, A, B, zero_dq, a, qout, cfl, fin)
+                 : launch_fused32_nt<D, SOLVER, PK, HALF, false>(s, A, B, zero_dq, a, qout, cfl, fin);
 }
 
 template <int D>
