@@ -2,9 +2,11 @@
 // reset for a new time step, and the finiteness check.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "kernels_fp32p.hpp"
@@ -63,9 +65,164 @@ FieldRef field_ref64(Solver *s, int which) {
 
 }  // namespace
 
+// ---------------------------------------------------------------------------
+// Read-back.  A kernel gathers the array in original cell order and writes it
+// straight to pinned host memory (no device scratch), so the host only copies
+// or widens consecutive values.  Copies of pageable memory stage through the
+// runtime at 4 (fresh pages) to 18 GB/s where pinned memory takes 56: arrays
+// past kSmallRead go through a pinned ring, each worker with one chunk
+// arriving while it writes out the other.
+// ---------------------------------------------------------------------------
+// values [at, at + n) of the state as [component][original cell]
+template <typename T>
+static __global__ void __launch_bounds__(256) export_state(const T *q, const int32_t *comb, int nc, size_t ntot,
+                                                           size_t at, size_t n, T *out) {
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    const size_t k = (at + t) / (size_t)nc, c = comb[at + t - k * nc];
+    out[t] = q[q64_index((int)k, c, ntot)];
+}
+
+// values [at, at + n) of f x (root: its square root) in original cell order
+static __global__ void __launch_bounds__(256) export_cells(const double *x, const int32_t *comb, double f, int root,
+                                                           size_t at, size_t n, double *out) {
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    const double v = x[comb[at + t]] * f;
+    out[t] = root ? sqrt(v) : v;
+}
+
+struct Solver::ReadRing {
+    static constexpr int kWorkers = 6;
+    static constexpr size_t kChunk = 1 << 20;  // bytes
+    char *buf = nullptr;
+    hipEvent_t ev[2 * kWorkers] = {};
+};
+
+void Solver::free_read_ring() {
+    if (!read_ring) return;
+    for (hipEvent_t e : read_ring->ev)
+        if (e) (void)hipEventDestroy(e);
+    if (read_ring->buf) (void)hipHostFree(read_ring->buf);
+    delete read_ring;
+    read_ring = nullptr;
+}
+
+// n values of T: fill(at, count, dst) enqueues the kernel that writes values
+// [at, at + count) to pinned memory, sink(at, count, src) takes them there;
+// each value once, large arrays from several threads
+template <typename T, class Fill, class Sink>
+int Solver::stream_out(size_t n, const Fill &fill, const Sink &sink) {
+    if (n * sizeof(T) <= kSmallRead) {
+        T *h = reinterpret_cast<T *>(h_scalar + kScalars);
+        fill((size_t)0, n, h);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(stream));
+        sink((size_t)0, n, (const T *)h);
+        return LFM_OK;
+    }
+    using R = ReadRing;
+    constexpr size_t kPart = R::kChunk / sizeof(T);
+    if (!read_ring) {
+        read_ring = new R;
+        hipError_t e = hipHostMalloc((void **)&read_ring->buf, 2 * R::kWorkers * R::kChunk, hipHostMallocDefault);
+        for (hipEvent_t &v : read_ring->ev)
+            if (e == hipSuccess) e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
+        if (e != hipSuccess) {
+            free_read_ring();
+            HIP_TRY(e);
+        }
+    }
+    const size_t parts = (n + kPart - 1) / kPart;
+    hipError_t err[R::kWorkers] = {};
+    // worker w of m: parts w, w + m, ..., the next one on its way while this
+    // one is written out
+    auto work = [&](int w, int m) {
+        auto count = [&](size_t i) { return std::min(kPart, n - i * kPart); };
+        auto slot = [&](int half) { return reinterpret_cast<T *>(read_ring->buf + (2 * w + half) * R::kChunk); };
+        auto start = [&](size_t i, int half) {
+            fill(i * kPart, count(i), slot(half));
+            const hipError_t e = hipGetLastError();
+            return e == hipSuccess ? hipEventRecord(read_ring->ev[2 * w + half], stream) : e;
+        };
+        hipError_t e = hipSetDevice(device);
+        if (e == hipSuccess) e = start(w, 0);
+        int half = 0;
+        for (size_t i = w; i < parts && e == hipSuccess; i += m, half ^= 1) {
+            if (i + m < parts) e = start(i + m, half ^ 1);
+            const hipError_t e2 = hipEventSynchronize(read_ring->ev[2 * w + half]);
+            if (e == hipSuccess) e = e2;
+            if (e == hipSuccess) sink(i * kPart, count(i), (const T *)slot(half));
+        }
+        err[w] = e;
+    };
+    // a thread costs about as much as writing out two parts
+    const int m = (int)std::min<size_t>({(size_t)R::kWorkers, std::max(1u, std::thread::hardware_concurrency() / 2),
+                                         std::max<size_t>(1, parts / 4)});
+    std::vector<std::thread> team;
+    int cur = 0;
+    HIP_TRY(hipGetDevice(&cur));
+    try {
+        for (int w = 1; w < m; w++) team.emplace_back(work, w, m);
+    } catch (const std::exception &) {
+        // fewer threads than asked for: their parts follow on this one
+    }
+    work(0, m);
+    for (int w = (int)team.size() + 1; w < m; w++) work(w, m);
+    for (std::thread &t : team) t.join();
+    if (cur != device) (void)hipSetDevice(cur);
+    for (int w = 0; w < m; w++)
+        if (err[w] != hipSuccess) {
+            (void)hipStreamSynchronize(stream);  // nothing writes to the ring after the return
+            HIP_TRY(err[w]);
+        }
+    return LFM_OK;
+}
+
+int Solver::read_state(double *out) {
+    const size_t nc = L.nc, ntot = nc + L.ng, n = (size_t)(L.D + 2) * nc;
+    auto grid = [](size_t count) { return dim3((unsigned)((count + 255) / 256)); };
+    if (!fp32)
+        return stream_out<double>(
+            n,
+            [&](size_t at, size_t count, double *dst) {
+                hipLaunchKernelGGL(export_state<double>, grid(count), dim3(256), 0, stream, k64.q, d_comb, L.nc, ntot, at,
+                                   count, dst);
+            },
+            [&](size_t at, size_t count, const double *src) { std::memcpy(out + at, src, count * sizeof(double)); });
+    const KArgs32 &a = *k32;
+    double base[5] = {a.rho_inf_d, a.m_inf_d[0], a.m_inf_d[1], a.m_inf_d[2], 0.0};
+    base[L.D + 1] = a.rhoE_inf_d;
+    return stream_out<float>(
+        n,
+        [&](size_t at, size_t count, float *dst) {
+            hipLaunchKernelGGL(export_state<float>, grid(count), dim3(256), 0, stream, a.q, d_comb, L.nc, ntot, at, count,
+                               dst);
+        },
+        [&](size_t i, size_t count, const float *src) {
+            const size_t end = i + count;
+            while (i < end) {
+                const size_t k = i / nc, stop = std::min(end, (k + 1) * nc);
+                const double b = base[k];
+                for (; i < stop; i++) out[i] = b + (double)*src++;
+            }
+        });
+}
+
+int Solver::read_cells(const double *dev, double f, bool root, double *out) {
+    return stream_out<double>(
+        L.nc,
+        [&](size_t at, size_t count, double *dst) {
+            hipLaunchKernelGGL(export_cells, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, dev, d_comb, f,
+                               (int)root, at, count, dst);
+        },
+        [&](size_t at, size_t count, const double *src) { std::memcpy(out + at, src, count * sizeof(double)); });
+}
+
 int Solver::get_field(int which, double *out) {
     const int D = L.D;
     const size_t nc = L.nc;
+    if (which == LFM_FIELD_Q) return read_state(out);
     HIP_TRY(hipStreamSynchronize(stream));
     if (which == LFM_FIELD_PRIM) {
         std::vector<double> q((size_t)(D + 2) * nc);
@@ -109,13 +266,7 @@ int Solver::get_field(int which, double *out) {
         return LFM_OK;
     }
     if (!r.ptr) return fail(LFM_EINVAL, "unknown or unallocated field");
-    const size_t nt = (size_t)L.nc + L.ng;
-    if (r.state) {
-        std::vector<double> tmp((size_t)(D + 2) * nt);
-        HIP_TRY(hipMemcpy(tmp.data(), r.ptr, tmp.size() * sizeof(double), hipMemcpyDeviceToHost));
-        for (int k = 0; k < r.ncomp; k++)
-            for (size_t ci = 0; ci < nc; ci++) out[k * nc + L.orig[ci]] = tmp[q64_index(k, ci, nt)];
-    } else if (r.es == 1) {
+    if (r.es == 1) {
         std::vector<double> tmp(nc);
         for (int k = 0; k < r.ncomp; k++) {
             HIP_TRY(hipMemcpy(tmp.data(), r.ptr + k * r.cs, nc * sizeof(double), hipMemcpyDeviceToHost));

@@ -264,7 +264,8 @@ std::string build_layout(const lfm_polymesh &m, const lfm_partition *part, const
     L.D = D;
     L.nc = nc;
     L.orig.resize(nc);
-    std::vector<int32_t> comb(nc);
+    L.comb.resize(nc);
+    std::vector<int32_t> &comb = L.comb;
     int idx = 0;
     for (int c = 0; c < nc; c++)
         if (sm[c] == 0) { L.orig[idx] = c; comb[c] = idx++; }
@@ -426,6 +427,8 @@ std::string build_layout(const lfm_polymesh &m, const lfm_partition *part, const
 
     // faces in processing order
     std::vector<int32_t> slot_face(slots.size(), -1);
+    L.fP.reserve(slots.size());
+    L.fN.reserve(slots.size());
     for (int ci = 0; ci < nc; ci++)
         for (int s = soff[ci]; s < soff[ci + 1]; s++)
             if (svalid[s]) {
@@ -585,39 +588,67 @@ FaceTable<T> face_table(const SolverLayout &L, int max_n) {
     size_t cap = 16;
     while (cap < 2 * (size_t)(max_n + 1)) cap *= 2;
     std::vector<int32_t> bucket(cap, -1);
+    // a record's bits as words
+    constexpr int kWords = 4 * sizeof(T) / sizeof(uint64_t);
     struct Key {
-        T v[4];
+        uint64_t v[kWords];
+        static uint64_t bits(double x) {
+            uint64_t b;
+            std::memcpy(&b, &x, sizeof b);
+            return b;
+        }
+        static uint64_t bits(float x) {
+            uint32_t b;
+            std::memcpy(&b, &x, sizeof b);
+            return b;
+        }
+        void set(T a, T b, T c, T d) {
+            if constexpr (kWords == 4) {
+                v[0] = bits(a);
+                v[1] = bits(b);
+                v[2] = bits(c);
+                v[3] = bits(d);
+            } else {
+                v[0] = bits(a) | bits(b) << 32;
+                v[1] = bits(c) | bits(d) << 32;
+            }
+        }
+        bool operator==(const Key &o) const {
+            uint64_t d = 0;
+            for (int i = 0; i < kWords; i++) d |= v[i] ^ o.v[i];
+            return d == 0;
+        }
     };
     std::vector<Key> keys;
     t.rec.resize(nf);
     // consecutive cells repeat the previous cells' records: the few last
     // used ones are tried before the hash
     constexpr int kLast = 4;
-    int last[kLast] = {-1, -1, -1, -1}, at = 0;
+    Key last[kLast] = {};
+    int lrec[kLast] = {-1, -1, -1, -1}, at = 0;
+    const double *Sk[3] = {L.S.data(), L.S.data() + nf, D == 3 ? L.S.data() + 2 * nf : nullptr}, *wk = L.w.data();
     for (size_t f = 0; f < nf; f++) {
-        Key k{};
-        for (int i = 0; i < D; i++) k.v[i] = (T)L.S[i * nf + f];
-        k.v[3] = (T)L.w[f];
+        Key k;
+        k.set((T)Sk[0][f], (T)Sk[1][f], D == 3 ? (T)Sk[2][f] : (T)0, (T)wk[f]);
         int r = -1;
         for (int i = 0; i < kLast && r < 0; i++)
-            if (last[i] >= 0 && std::memcmp(&keys[last[i]], &k, sizeof k) == 0) r = last[i];
+            if (last[i] == k) r = lrec[i];
         if (r < 0) {
             uint64_t h = 1469598103934665603ull;
-            for (T x : k.v) {
-                uint64_t b = 0;
-                std::memcpy(&b, &x, sizeof x);
+            for (uint64_t b : k.v) {
                 h = (h ^ b) * 0x9E3779B97F4A7C15ull;
                 h ^= h >> 29;
             }
             size_t i = (size_t)h & (cap - 1);
-            while (bucket[i] >= 0 && std::memcmp(&keys[bucket[i]], &k, sizeof k) != 0) i = (i + 1) & (cap - 1);
+            while (bucket[i] >= 0 && !(keys[bucket[i]] == k)) i = (i + 1) & (cap - 1);
             if (bucket[i] < 0) {
                 if ((int)keys.size() == max_n) return FaceTable<T>();
                 bucket[i] = (int32_t)keys.size();
                 keys.push_back(k);
             }
             r = bucket[i];
-            last[at] = r;
+            last[at] = k;
+            lrec[at] = r;
             at = (at + 1) % kLast;
         }
         t.rec[f] = (uint16_t)r;
@@ -626,8 +657,10 @@ FaceTable<T> face_table(const SolverLayout &L, int max_n) {
     t.S.resize((size_t)t.n * D);
     t.w.resize(t.n);
     for (int i = 0; i < t.n; i++) {
-        for (int k = 0; k < D; k++) t.S[(size_t)i * D + k] = keys[i].v[k];
-        t.w[i] = keys[i].v[3];
+        T rec[4];
+        std::memcpy(rec, &keys[i], sizeof rec);
+        for (int k = 0; k < D; k++) t.S[(size_t)i * D + k] = rec[k];
+        t.w[i] = rec[3];
     }
     return t;
 }

@@ -43,7 +43,7 @@ struct SolverLayout {
     int ng_bnd = 0;                     // boundary ghosts [0, ng_bnd); halo ghosts [ng_bnd, ng)
     int rank = -1;                      // partition rank (-1: undecomposed)
     std::vector<HaloNbr> halo;
-    std::vector<int32_t> orig;          // combined -> original cell id
+    std::vector<int32_t> orig, comb;    // combined -> original cell id, and back
     std::vector<int32_t> fP, fN;        // [nf]
     std::vector<double> S, d, w;        // S,d: [D][nf] SoA; w: [nf]
     std::vector<double> vinv, sigma;    // [nc]

@@ -431,17 +431,9 @@ int lfm_post_average_fields(lfm_solver *h, int32_t n, double *pavg, double *prms
     Solver *s = h->impl.get();
     if (!s->post || !s->post->cfg.have_average) return fail(LFM_ESTATE, "averages not configured");
     if (n <= 0) return fail(LFM_EINVAL, "n must be positive");
-    const size_t nc = s->L.nc;
-    std::vector<double> a(nc), r(nc);
-    HIP_TRY(hipMemcpyAsync(a.data(), s->post->pavg, nc * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(hipMemcpyAsync(r.data(), s->post->prms, nc * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(hipStreamSynchronize(s->stream));
     const double f = 1.0 / n;
-    for (size_t ci = 0; ci < nc; ci++) {
-        pavg[s->L.orig[ci]] = a[ci] * f;
-        prms[s->L.orig[ci]] = std::sqrt(r[ci] * f);
-    }
-    return LFM_OK;
+    const int rc = s->read_cells(s->post->pavg, f, false, pavg);
+    return rc ? rc : s->read_cells(s->post->prms, f, true, prms);
 }
 
 int lfm_post_walls(lfm_solver *h, int32_t *n, int32_t *patches) {

@@ -68,6 +68,7 @@ Solver::~Solver() {
     for (void *p : allocs) (void)hipFree(p);
     if (k32) free_k32(k32);
     free_post(post);
+    free_read_ring();
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (stream) (void)hipStreamDestroy(stream);
@@ -819,9 +820,11 @@ int lfm_solver_create_part(const lfm_polymesh *mesh, const lfm_partition *part, 
     HIP_TRY(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
     HIP_TRY(hipEventCreate(&s->ev0));
     HIP_TRY(hipEventCreate(&s->ev1));
-    HIP_TRY(hipHostMalloc((void **)&s->h_scalar, 64 * sizeof(double), hipHostMallocDefault));
+    HIP_TRY(hipHostMalloc((void **)&s->h_scalar, Solver::kScalars * sizeof(double) + Solver::kSmallRead,
+                          hipHostMallocDefault));
     int rc = s->fp32 ? lfm::create_fp32p(s.get()) : lfm::create_fp64(s.get());
     if (rc) return rc;
+    if (lfm::dev_upload(s.get(), (int32_t **)&s->d_comb, s->L.comb.data(), s->L.comb.size())) return LFM_EDEVICE;
     s->size_stage();
     s->halo_dev.resize(s->L.halo.size());
     for (size_t i = 0; i < s->L.halo.size(); i++) {
@@ -853,6 +856,8 @@ int lfm_solver_destroy(lfm_solver *h) {
 int lfm_get_info(lfm_solver *h, lfm_info *info) {
     if (!h || !info) return fail(LFM_EINVAL, "null argument");
     Solver *s = h->impl.get();
+    // one wait for the stream's work and the scalars behind it
+    HIP_TRY(hipMemcpyAsync(s->h_scalar, s->d_scalar, 16 * sizeof(double), hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
     info->dim = s->L.D;
     info->n_cells = s->L.nc;
@@ -863,7 +868,6 @@ int lfm_get_info(lfm_solver *h, lfm_info *info) {
     info->precision = s->prm.precision;
     info->solver = s->prm.solver;
     info->device_bytes = s->device_bytes;
-    HIP_TRY(hipMemcpy(s->h_scalar, s->d_scalar, 16 * sizeof(double), hipMemcpyDeviceToHost));
     info->dt = s->h_scalar[0];
     info->cfl = s->h_scalar[8];
     info->steps_done = s->steps_done;

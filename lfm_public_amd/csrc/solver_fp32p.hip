@@ -352,7 +352,8 @@ void launch_nonfinite32(Solver *s, unsigned long long *d) {
                        s->L.nc + s->L.ng, d);
 }
 
-// FP32 field access (converted to FP64 values in original cell order)
+// FP32 field access (converted to FP64 values in original cell order); the
+// state has its own path (Solver::read_state)
 int get_field32(Solver *s, int which, double *out) {
     const SolverLayout &L = s->L;
     const int D = L.D;
@@ -362,7 +363,6 @@ int get_field32(Solver *s, int which, double *out) {
     int ncomp = 0;
     size_t stride = nt;
     switch (which) {
-    case LFM_FIELD_Q: ptr = a.q; ncomp = D + 2; break;
     case LFM_FIELD_DQ: ptr = a.dq; ncomp = D + 2; stride = nc; break;
     case LFM_FIELD_DUDX: ptr = a.dudx; ncomp = D * D; break;
     case LFM_FIELD_DTDX: ptr = a.dTdx; ncomp = D; break;
@@ -397,7 +397,7 @@ int get_field32(Solver *s, int which, double *out) {
         return LFM_OK;
     }
     if (!ptr) return fail(LFM_EINVAL, "field not allocated for this solver");
-    const bool in_record = ptr != a.q && ptr != a.dq && ptr != a.res_cell && ptr != a.tauMC && ptr != a.sigmaU &&
+    const bool in_record = ptr != a.dq && ptr != a.res_cell && ptr != a.tauMC && ptr != a.sigmaU &&
                            (ptr != a.U_grad || a.U_grad == a.dudx);
     if (in_record) {
         // component k of cell ci at ptr[ci * gstride + k]
@@ -409,25 +409,11 @@ int get_field32(Solver *s, int which, double *out) {
                 out[k * nc + L.orig[ci]] = (double)recs[ci * a.gstride + off + k];
         return LFM_OK;
     }
-    double qinf[5] = {a.rho_inf_d, a.m_inf_d[0], a.m_inf_d[1], a.m_inf_d[2], 0.0};
-    if (which == LFM_FIELD_Q) {
-        // cell records: components 0-3 interleaved, component 4 after them
-        qinf[D + 1] = a.rhoE_inf_d;
-        std::vector<float> rec((size_t)4 * nc), e4(D == 3 ? nc : 0);
-        HIP_TRY(hipMemcpy(rec.data(), a.q, rec.size() * sizeof(float), hipMemcpyDeviceToHost));
-        if (D == 3) HIP_TRY(hipMemcpy(e4.data(), a.q + 4 * nt, nc * sizeof(float), hipMemcpyDeviceToHost));
-        for (int k = 0; k < D + 2; k++)
-            for (size_t ci = 0; ci < nc; ci++)
-                out[k * nc + L.orig[ci]] = qinf[k] + (double)(k < 4 ? rec[4 * ci + k] : e4[ci]);
-        return LFM_OK;
-    }
-    qinf[D + 1] = a.rhoE_inf_d;
     std::vector<float> tmp(nc);
     for (int k = 0; k < ncomp; k++) {
         HIP_TRY(hipMemcpy(tmp.data(), ptr + k * stride, nc * sizeof(float), hipMemcpyDeviceToHost));
-        const double base = which == LFM_FIELD_Q ? qinf[k] : 0.0;
         double *o = out + k * nc;
-        for (size_t ci = 0; ci < nc; ci++) o[L.orig[ci]] = base + (double)tmp[ci];
+        for (size_t ci = 0; ci < nc; ci++) o[L.orig[ci]] = (double)tmp[ci];
     }
     return LFM_OK;
 }

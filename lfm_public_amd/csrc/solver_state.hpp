@@ -51,7 +51,13 @@ struct Solver {
     int device = 0;  // the HIP device current when the handle was created
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    double *h_scalar = nullptr;   // pinned host scratch (64 doubles)
+    double *h_scalar = nullptr;   // pinned host scratch (kScalars doubles, then kSmallRead bytes)
+    static constexpr size_t kScalars = 64, kSmallRead = 128 << 10;
+    // pinned ring for read-backs larger than kSmallRead, allocated by the
+    // first one: two chunks and their events per worker
+    struct ReadRing;
+    ReadRing *read_ring = nullptr;
+    const int32_t *d_comb = nullptr;  // L.comb on the device
     std::vector<void *> allocs;
     int64_t device_bytes = 0;
 
@@ -196,6 +202,13 @@ struct Solver {
     void zero_state_for_step();
 
     int get_field(int which, double *out);
+    // the state in original cell order, components one after the other
+    int read_state(double *out);
+    // one per-cell array, times f (root: its square root), in that order
+    int read_cells(const double *dev, double f, bool root, double *out);
+    template <typename T, class Fill, class Sink>
+    int stream_out(size_t n, const Fill &fill, const Sink &sink);
+    void free_read_ring();
     int set_field(int which, const double *in);
     int check_finite(int64_t *n_bad);
     // the same count with its per-block partials in the library's static
