@@ -139,6 +139,14 @@ __device__ __forceinline__ void st_once(T *p, T v) {
         *p = v;
 }
 using d2v = double __attribute__((ext_vector_type(2)));
+
+// orders a wave's LDS writes before the reads of its other lanes that follow
+// (LDS serves one wave's accesses in order; this keeps the compiler to it)
+__device__ __forceinline__ void wave_sync_lds() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 template <bool NT>
 __device__ __forceinline__ void st64x2_once(double *p, double x, double y) {
     const d2v v = {x, y};
@@ -403,8 +411,15 @@ __device__ __forceinline__ void vis_tensors(const KArgs &a, const double (&dudx)
     for (int i = 0; i < D; i++) sU[i] = dotD<D>(U, tau[i]);
 }
 
+// Bound: latency (at a few 100 k cells a launch has 2-3 waves per SIMD to hide
+// its dependent loads), so registers decide.  Faces in groups whose loads are
+// issued together: two in 2D (176 k-cell annulus, four 182, three 179, two 177,
+// one 179 us per step), three in 3D at 3 waves per SIMD (193 k-cell O-grid: all
+// six at 2 waves 417, three 404, two 406, one 414).
+template <int D>
+constexpr int kGradGroup64 = D == 2 ? 2 : 3;
 template <int D, int GRAD, bool VISC, bool RG, bool NT>
-__global__ void __launch_bounds__(256) grad_vis(KArgs a) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) grad_vis(KArgs a) {
     const int c = LFM_TID(blockIdx.x);
     using R = GradRec64<D, RG>;
     // every thread reaches the record write-out below (LDS staging)
@@ -429,82 +444,88 @@ __global__ void __launch_bounds__(256) grad_vis(KArgs a) {
     }
     double qself[D + 2];
     load_q<D>(a, c, qself);
-    const double Rself = rpsi<D>(a, qself), riself = 1.0 / qself[0];
-    // one face's contribution, in the face's own P/N order
-    auto add = [&](const bool isP, const double w, const double (&S)[D], const double (&qo)[D + 2]) {
-        double qP[D + 2], qN[D + 2];
-        const double Ro = rpsi<D>(a, qo), rio = 1.0 / qo[0];
+    // what a face needs of a cell: velocities as products with 1/rho (dudx,
+    // dTdx) and, for M2AUSM, as quotients (ug, p), as the reference forms them
+    struct Cell {
+        double R, u[D], v[D], p;
+    };
+    auto cell = [&](const double (&q)[D + 2]) {
+        Cell x;
+        const double ri = 1.0 / q[0];
+        x.R = VISC ? rpsi<D>(a, q) : 0.0;
 #pragma unroll
-        for (int k = 0; k < D + 2; k++) {
-            qP[k] = isP ? qself[k] : qo[k];
-            qN[k] = isP ? qo[k] : qself[k];
+        for (int k = 0; k < D; k++) x.u[k] = q[k + 1] * ri;
+        if (GRAD == 2) {
+            const double r = q[0], E = q[D + 1] / r;
+            double vm = 0.0;
+#pragma unroll
+            for (int k = 0; k < D; k++) {
+                x.v[k] = q[k + 1] / r;
+                vm += x.v[k] * x.v[k];
+            }
+            x.p = r * a.gm1 * (E - 0.5 * vm);
         }
-        const double cR = isP ? Rself : Ro, aR = isP ? Ro : Rself;
-        const double cri = isP ? riself : rio, ari = isP ? rio : riself;
+        return x;
+    };
+    const Cell own = cell(qself);
+    // one face's contribution; INTERP_LINEAR's two products are the same ones
+    // from either side, so the cell's own come first and no side is selected
+    auto add = [&](const bool isP, const double w, const double (&S)[D], const double (&qo)[D + 2]) {
+        const Cell o = cell(qo);
+        const double omw = 1.0 - w, wc = isP ? w : omw, wo = isP ? omw : w;
         double sv[D];
 #pragma unroll
         for (int k = 0; k < D; k++) sv[k] = isP ? S[k] * vinv : -S[k] * vinv;
         if (GRAD == 2) {
-            double UU[D];
-#pragma unroll
-            for (int k = 0; k < D; k++) UU[k] = INTERP_LINEAR(w, qP[k + 1] / qP[0], qN[k + 1] / qN[0]);
-            const double rho = INTERP_LINEAR(w, qP[0], qN[0]);
-            double r = qP[0], E = qP[D + 1] / r, vm = 0.0;
-#pragma unroll
-            for (int k = 0; k < D; k++) vm += (qP[k + 1] / r) * (qP[k + 1] / r);
-            const double cp_ = r * a.gm1 * (E - 0.5 * vm);
-            r = qN[0];
-            E = qN[D + 1] / r;
-            vm = 0.0;
-#pragma unroll
-            for (int k = 0; k < D; k++) vm += (qN[k + 1] / r) * (qN[k + 1] / r);
-            const double np_ = r * a.gm1 * (E - 0.5 * vm);
-            const double pf = INTERP_LINEAR(w, cp_, np_);
+            const double rho = wc * qself[0] + wo * qo[0];
+            const double pf = wc * own.p + wo * o.p;
 #pragma unroll
             for (int i = 0; i < D; i++) {
                 pg[i] += pf * sv[i];
-#pragma unroll
-                for (int j = 0; j < D; j++) ug[j][i] += UU[j] * sv[i];
                 rg[i] += rho * sv[i];
             }
-        }
-        double fU[D];
 #pragma unroll
-        for (int k = 0; k < D; k++) fU[k] = INTERP_LINEAR(w, qP[k + 1] * cri, qN[k + 1] * ari);
-        const double fT = VISC ? INTERP_LINEAR(w, cR, aR) * a.R_inv : 0.0;
+            for (int j = 0; j < D; j++) {
+                const double UU = wc * own.v[j] + wo * o.v[j];
+#pragma unroll
+                for (int i = 0; i < D; i++) ug[j][i] += UU * sv[i];
+            }
+        }
+        const double fT = VISC ? (wc * own.R + wo * o.R) * a.R_inv : 0.0;
 #pragma unroll
         for (int i = 0; i < D; i++) {
+            const double fU = wc * own.u[i] + wo * o.u[i];
 #pragma unroll
-            for (int j = 0; j < D; j++) dudx[i][j] += fU[i] * sv[j];
+            for (int j = 0; j < D; j++) dudx[i][j] += fU * sv[j];
             if (VISC) dTdx[i] += fT * sv[i];
         }
     };
+    // groups of G faces in gather order, their loads issued together
     const int e0 = a.g_off[c], ne = a.g_off[c + 1] - e0;
-    // the first faces' gathers issued together before the sums (a short list
-    // repeats its last face, whose terms are then not added)
-    constexpr int U = GatherUnroll<D>::value;
-    bool isPj[U];
-    double wj[U], Sj[U][D], qj[U][D + 2];
+    constexpr int G = kGradGroup64<D>;
+    int ent[G];
 #pragma unroll
-    for (int j = 0; j < U; j++) {
-        const int ent = a.g_ent[e0 + (j < ne ? j : ne - 1)];
-        isPj[j] = ent >= 0;
-        const int f = isPj[j] ? (ent & kFaceMask) : ~ent;
-        wj[j] = a.w[f];
-        load_S64<D>(a.S, f, Sj[j]);
-        load_q<D>(a, isPj[j] ? a.fN[f] : a.fP[f], qj[j]);
-    }
+    for (int u = 0; u < G; u++) ent[u] = a.g_ent[e0 + (u < ne ? u : ne - 1)];
+#pragma unroll 1
+    for (int j0 = 0; j0 < ne; j0 += G) {
+        bool isPj[G];
+        double wj[G], Sj[G][D], qj[G][D + 2];
+        int next[G];
 #pragma unroll
-    for (int j = 0; j < U; j++)
-        if (j < ne) add(isPj[j], wj[j], Sj[j], qj[j]);
-    for (int e = e0 + U; e < e0 + ne; e++) {
-        const int ent = a.g_ent[e];
-        const bool p = ent >= 0;
-        const int f = p ? (ent & kFaceMask) : ~ent;
-        double Sf[D], q[D + 2];
-        load_S64<D>(a.S, f, Sf);
-        load_q<D>(a, p ? a.fN[f] : a.fP[f], q);
-        add(p, a.w[f], Sf, q);
+        for (int u = 0; u < G; u++) {
+            isPj[u] = ent[u] >= 0;
+            const int f = isPj[u] ? (ent[u] & kFaceMask) : ~ent[u];
+            const int o = isPj[u] ? a.fN[f] : a.fP[f];
+            wj[u] = a.w[f];
+            load_S64<D>(a.S, f, Sj[u]);
+            load_q<D>(a, o, qj[u]);
+            next[u] = a.g_ent[e0 + (j0 + G + u < ne ? j0 + G + u : ne - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < G; u++) {
+            if (j0 + u < ne) add(isPj[u], wj[u], Sj[u], qj[u]);
+            ent[u] = next[u];
+        }
     }
     // refresh of tau / sigmaU / tauMC from the completed dudx (cfd_v0.cpp:1813-1834);
     // stored only where a halo payload needs them (otherwise each face
@@ -542,19 +563,30 @@ __global__ void __launch_bounds__(256) grad_vis(KArgs a) {
     }
     }
     if (VISC) {
-        // the block's records are contiguous from its first cell: staged in
-        // LDS, then written as consecutive 16-byte words (without minmod the
-        // rho / p / U gradient slots are written zero, as they stay)
-        constexpr int W = R::kStride / 2;
-        __shared__ double2 st[256 * W];
-        const int t = threadIdx.x;
-#pragma unroll
-        for (int k = 0; k < W; k++) st[t * W + k] = make_double2(rec[2 * k], rec[2 * k + 1]);
-        __syncthreads();
-        const int c0 = c - t;
-        const int nrec = a.nc - c0 < (int)blockDim.x ? a.nc - c0 : (int)blockDim.x;
+        // the wave's records are contiguous from its first cell: four 16-byte
+        // words of each at a time are staged in LDS and written as 64-byte
+        // runs (without minmod the rho / p / U gradient slots are written
+        // zero, as they stay).  Staging whole records (57 KB per block for 3D
+        // M2AUSM) held the kernel at 2 waves per SIMD.
+        constexpr int W = R::kStride / 2, C = 4;
+        __shared__ double2 stage[256 / 64][64 * C];
+        double2 *st = stage[threadIdx.x >> 6];
+        const int lane = threadIdx.x & 63, c0 = c - lane;
         d2v *dst = reinterpret_cast<d2v *>(a.dudx + (size_t)c0 * R::kStride);
-        for (int j = t; j < nrec * W; j += blockDim.x) st_once<NT>(dst + j, d2v{st[j].x, st[j].y});
+#pragma unroll
+        for (int w0 = 0; w0 < W; w0 += C) {
+            const int n = W - w0 < C ? W - w0 : C;
+#pragma unroll
+            for (int k = 0; k < n; k++) st[lane * n + k] = make_double2(rec[2 * (w0 + k)], rec[2 * (w0 + k) + 1]);
+            wave_sync_lds();
+#pragma unroll
+            for (int i = 0; i < n; i++) {
+                const int j = i * 64 + lane, r = j / n;
+                const double2 v = st[j];
+                if (c0 + r < a.nc) st_once<NT>(dst + r * W + w0 + j % n, d2v{v.x, v.y});
+            }
+            wave_sync_lds();
+        }
     }
 }
 
