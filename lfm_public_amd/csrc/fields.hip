@@ -94,8 +94,12 @@ static __global__ void __launch_bounds__(256) export_cells(const double *x, cons
 
 struct Solver::ReadRing {
     static constexpr int kWorkers = 6;
-    static constexpr size_t kChunk = 1 << 20;  // bytes
+    // bytes: pinning memory takes some 0.2 us per KiB, so a solver's first
+    // read-back pays for the ring (8 solvers of 16 to 260 thousand cells: 5 ms
+    // with chunks of 1 MiB)
+    static constexpr size_t kChunk = 256 << 10;
     char *buf = nullptr;
+    int workers = 0;  // that it has chunks and events for
     hipEvent_t ev[2 * kWorkers] = {};
 };
 
@@ -123,17 +127,22 @@ int Solver::stream_out(size_t n, const Fill &fill, const Sink &sink) {
     }
     using R = ReadRing;
     constexpr size_t kPart = R::kChunk / sizeof(T);
-    if (!read_ring) {
+    const size_t parts = (n + kPart - 1) / kPart;
+    // a thread costs about as much as writing out 2 MiB
+    const int m = (int)std::min<size_t>({(size_t)R::kWorkers, std::max(1u, std::thread::hardware_concurrency() / 2),
+                                         std::max<size_t>(1, parts * R::kChunk >> 22)});
+    if (!read_ring || read_ring->workers < m) {
+        free_read_ring();
         read_ring = new R;
-        hipError_t e = hipHostMalloc((void **)&read_ring->buf, 2 * R::kWorkers * R::kChunk, hipHostMallocDefault);
-        for (hipEvent_t &v : read_ring->ev)
-            if (e == hipSuccess) e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
+        read_ring->workers = m;
+        hipError_t e = hipHostMalloc((void **)&read_ring->buf, 2 * (size_t)m * R::kChunk, hipHostMallocDefault);
+        for (int i = 0; i < 2 * m && e == hipSuccess; i++)
+            e = hipEventCreateWithFlags(&read_ring->ev[i], hipEventDisableTiming);
         if (e != hipSuccess) {
             free_read_ring();
             HIP_TRY(e);
         }
     }
-    const size_t parts = (n + kPart - 1) / kPart;
     hipError_t err[R::kWorkers] = {};
     // worker w of m: parts w, w + m, ..., the next one on its way while this
     // one is written out
@@ -156,9 +165,6 @@ int Solver::stream_out(size_t n, const Fill &fill, const Sink &sink) {
         }
         err[w] = e;
     };
-    // a thread costs about as much as writing out two parts
-    const int m = (int)std::min<size_t>({(size_t)R::kWorkers, std::max(1u, std::thread::hardware_concurrency() / 2),
-                                         std::max<size_t>(1, parts / 4)});
     std::vector<std::thread> team;
     int cur = 0;
     HIP_TRY(hipGetDevice(&cur));

@@ -38,15 +38,33 @@ static constexpr int kMaxTable64 = 2048;
 static constexpr int kBlock = 256;
 static inline int nblocks(long n) { return (int)((n + kBlock - 1) / kBlock); }
 
+int Solver::dev_alloc(void **p, size_t bytes) {
+    constexpr size_t kSlab = 1 << 20, kShare = 128 << 10, kAlign = 256;
+    const size_t need = (bytes + kAlign - 1) / kAlign * kAlign;
+    if (need > kShare) {
+        HIP_TRY(hipMalloc(p, bytes));
+        allocs.push_back(*p);
+    } else {
+        if (need > slab_left) {
+            HIP_TRY(hipMalloc((void **)&slab, kSlab));
+            allocs.push_back(slab);
+            slab_left = kSlab;
+        }
+        *p = slab;
+        slab += need;
+        slab_left -= need;
+    }
+    device_bytes += (int64_t)bytes;
+    return 0;
+}
+
 template <typename T>
 static int dev_upload(Solver *s, T **dst, const T *src, size_t n) {
     if (n == 0) {
         *dst = nullptr;
         return 0;
     }
-    HIP_TRY(hipMalloc((void **)dst, n * sizeof(T)));
-    s->allocs.push_back((void *)*dst);
-    s->device_bytes += (int64_t)(n * sizeof(T));
+    if (int rc = s->dev_alloc((void **)dst, n * sizeof(T))) return rc;
     if (src) HIP_TRY(hipMemcpy(*dst, src, n * sizeof(T), hipMemcpyHostToDevice));
     return 0;
 }
@@ -57,9 +75,7 @@ static int dev_zeros(Solver *s, T **dst, size_t n) {
         *dst = nullptr;
         return 0;
     }
-    HIP_TRY(hipMalloc((void **)dst, n * sizeof(T)));
-    s->allocs.push_back((void *)*dst);
-    s->device_bytes += (int64_t)(n * sizeof(T));
+    if (int rc = s->dev_alloc((void **)dst, n * sizeof(T))) return rc;
     HIP_TRY(hipMemset(*dst, 0, n * sizeof(T)));
     return 0;
 }

@@ -23,9 +23,7 @@ static int up(Solver *s, T **dst, const T *src, size_t n) {
         *dst = nullptr;
         return 0;
     }
-    HIP_TRY(hipMalloc((void **)dst, n * sizeof(T)));
-    s->allocs.push_back((void *)*dst);
-    s->device_bytes += (int64_t)(n * sizeof(T));
+    if (int rc = s->dev_alloc((void **)dst, n * sizeof(T))) return rc;
     if (src)
         HIP_TRY(hipMemcpy(*dst, src, n * sizeof(T), hipMemcpyHostToDevice));
     else

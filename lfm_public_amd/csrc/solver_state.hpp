@@ -60,6 +60,11 @@ struct Solver {
     const int32_t *d_comb = nullptr;  // L.comb on the device
     std::vector<void *> allocs;
     int64_t device_bytes = 0;
+    // device memory of the set-up: small arrays share slabs, so that creating
+    // a small solve does not take one allocation per array
+    int dev_alloc(void **p, size_t bytes);
+    char *slab = nullptr;
+    size_t slab_left = 0;
 
     // device scalars: [0] deltaT, [2..6] residual sums, [8] cfl, [9] dt min
     double *d_scalar = nullptr;
