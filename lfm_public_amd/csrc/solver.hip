@@ -81,6 +81,7 @@ static int dev_zeros(Solver *s, T **dst, size_t n) {
 }
 
 Solver::~Solver() {
+    free_step_graph();
     for (void *p : allocs) (void)hipFree(p);
     if (k32) free_k32(k32);
     free_post(post);
@@ -788,6 +789,116 @@ void Solver::step() {
     // launch, so later launches see the swap)
     if (in_alt) fp32 ? std::swap(k32->q, q_alt32) : std::swap(k64.q, q_alt64);
     end_step(true);
+    eager_launches += nstages * (first < nstages ? 1 : 3) + 1;
+}
+
+// ---------------------------------------------------------------------------
+// Steps as a captured graph.  A launch costs 2.7 us of host time and 3.6 us
+// from one small kernel to the next; inside a graph of 40 kernels or more the
+// next one starts after 1.8 (4 blocks) to 2.4 us (256 blocks).  A graph of one
+// step's five launches gains nothing (3.7 us per kernel), so it holds
+// kGraphSteps steps.  Capturing costs what it saves in some 500 launches: it is
+// done by a run that continues past kGraphAfter of them.
+// ---------------------------------------------------------------------------
+constexpr long kGraphAfter = 512;
+
+struct Solver::StepGraph {
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    // all that the captured launches depend on
+    KArgs k64;
+    KArgs32 k32;
+    const void *alt = nullptr;
+    double dt = 0.0;
+    bool pending = false;
+    int from = 0;
+    void note(const Solver &s) {
+        std::memcpy((void *)&k64, &s.k64, sizeof k64);
+        if (s.k32) std::memcpy((void *)&k32, s.k32, sizeof k32);
+        alt = s.fp32 ? (const void *)s.q_alt32 : (const void *)s.q_alt64;
+        dt = s.dt;
+        pending = s.cfl_pending;
+        from = s.fused_from();
+    }
+    bool matches(const Solver &s) const {
+        return std::memcmp(&k64, &s.k64, sizeof k64) == 0 && (!s.k32 || std::memcmp(&k32, s.k32, sizeof k32) == 0) &&
+               alt == (s.fp32 ? (const void *)s.q_alt32 : (const void *)s.q_alt64) && dt == s.dt &&
+               pending == s.cfl_pending && from == s.fused_from();
+    }
+    ~StepGraph() {
+        if (exec) (void)hipGraphExecDestroy(exec);
+        if (graph) (void)hipGraphDestroy(graph);
+    }
+};
+
+void Solver::free_step_graph() {
+    delete step_graph;
+    step_graph = nullptr;
+}
+
+// whether the next kGraphSteps steps are one graph launch
+bool Solver::graph_ready() {
+    if (post || prof || graph_failed || ghosts_stale || nstages == 0) return false;
+    // a step leaves its CFL reduction to the next one wherever it can: the
+    // steps before the first such step are launched one by one
+    if (!prm.adjust_dt && carry_target() != 0 && !cfl_pending) return false;
+    if (step_graph && step_graph->matches(*this)) {
+        graph_misses = 0;
+        return true;
+    }
+    // an odd number of one-launch stages swaps the buffers each step: the
+    // graph's turn comes with the next one
+    if (step_graph && ++graph_misses < 2) return false;
+    return eager_launches >= kGraphAfter && graph_capture();
+}
+
+bool Solver::graph_capture() {
+    free_step_graph();
+    auto *g = new StepGraph;
+    std::lock_guard<std::mutex> lock(device_setup_mutex());
+    g->note(*this);
+    hipError_t e = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
+    if (e == hipSuccess) {
+        const int64_t done = steps_done;
+        defer_cfl = true;
+        for (int i = 0; i < kGraphSteps; i++) step();
+        steps_done = done;
+        e = hipStreamEndCapture(stream, &g->graph);
+        if (e == hipSuccess) e = hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0);
+    }
+    eager_launches = 0;
+    graph_misses = 0;
+    if (e != hipSuccess || !g->matches(*this)) {
+        // nothing was launched: the steps follow as launches of their own
+        (void)hipGetLastError();
+        delete g;
+        graph_failed = true;
+        return false;
+    }
+    step_graph = g;
+    return true;
+}
+
+int Solver::run_steps(int n, bool with_post) {
+    for (int i = 0; i < n;) {
+        // the run's last step is never in the graph: it reduces its own CFL
+        if (n - i > kGraphSteps && graph_ready()) {
+            HIP_TRY(hipGraphLaunch(step_graph->exec, stream));
+            steps_done += kGraphSteps;
+            if (prm.have_res) res_valid = true;
+            i += kGraphSteps;
+            continue;
+        }
+        defer_cfl = i + 1 < n && !(with_post && post);
+        step();
+        if (with_post && post) {
+            const int rc = post_step();
+            if (rc) return rc;
+        }
+        i++;
+    }
+    flush_cfl();
+    return LFM_OK;
 }
 
 }  // namespace lfm
@@ -983,15 +1094,8 @@ int lfm_run(lfm_solver *h, int nsteps) {
     if (!s->L.halo.empty())
         return fail(LFM_ESTATE, "a partition with processor patches steps through lfm_part_group_run or the "
                                 "per-stage calls with halo exchange");
-    for (int i = 0; i < nsteps; i++) {
-        s->defer_cfl = i + 1 < nsteps && !s->post;
-        s->step();
-        if (s->post) {
-            const int rc = s->post_step();
-            if (rc) return rc;
-        }
-    }
-    s->flush_cfl();
+    const int rc = s->run_steps(nsteps, true);
+    if (rc) return rc;
     HIP_TRY(hipGetLastError());
     return LFM_OK;
 }
@@ -1009,11 +1113,8 @@ int lfm_time_steps(lfm_solver *h, int nsteps, double *ms_out) {
         return fail(LFM_ESTATE, "a partition with processor patches steps through lfm_part_group_run or the "
                                 "per-stage calls with halo exchange");
     HIP_TRY(hipEventRecord(s->ev0, s->stream));
-    for (int i = 0; i < nsteps; i++) {
-        s->defer_cfl = i + 1 < nsteps;
-        s->step();
-    }
-    s->flush_cfl();
+    const int rc = s->run_steps(nsteps, false);
+    if (rc) return rc;
     HIP_TRY(hipEventRecord(s->ev1, s->stream));
     HIP_TRY(hipEventSynchronize(s->ev1));
     float ms = 0.f;

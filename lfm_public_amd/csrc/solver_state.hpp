@@ -204,6 +204,18 @@ struct Solver {
     void final_or_carry(const CflJob &job);
     void flush_cfl();
     void end_step(bool own_dt);
+    // n steps; with_post: the post-processing after each.  Long runs replay
+    // kGraphSteps steps at a time as a captured graph.
+    int run_steps(int n, bool with_post);
+    static constexpr int kGraphSteps = 8;  // even: the state buffers' roles return
+    struct StepGraph;
+    StepGraph *step_graph = nullptr;
+    bool graph_failed = false;
+    int graph_misses = 0;        // steps in a row whose launches were not the graph's
+    long eager_launches = 0;     // since the last capture
+    bool graph_ready();
+    bool graph_capture();
+    void free_step_graph();
     void zero_state_for_step();
 
     int get_field(int which, double *out);
