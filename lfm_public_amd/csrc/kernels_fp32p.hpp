@@ -31,6 +31,9 @@ struct KArgs32 {
     const float *S;  // [nf][D]: a face's area vector as one record
     const float *d, *w;
     const int32_t *g_off, *g_ent;
+    // each cell's first GatherUnroll gather entries and (2D) the cells they
+    // lead to (key_at places them; kNoFace and the cell itself past its last)
+    const int32_t *g_key, *g_oth;
     const int32_t *ghost_cell, *ghost_role;
     const float *vinv;
     const float *sigma;  // nullptr where every cell's sponge sigma is zero
@@ -378,9 +381,13 @@ struct FaceOf32 {
     }
     // an entry of the gather list
     __device__ __forceinline__ void load_list(const KArgs32 &a, const int ent) {
+        load_face(a, ent);
+        other = ent >= 0 ? a.fN[face_of(ent)] : a.fP[face_of(ent)];
+    }
+    // its face's data alone
+    __device__ __forceinline__ void load_face(const KArgs32 &a, const int ent) {
         const bool isP = ent >= 0;
-        const int f = isP ? (ent & kFaceMask) : ~ent;
-        other = isP ? a.fN[f] : a.fP[f];
+        const int f = face_of(ent);
         const float w = a.w[f];
         load_S32<D>(a.S, f, S);
 #pragma unroll
@@ -452,19 +459,33 @@ __device__ __forceinline__ Prim32<D> grad32_sums(const KArgs32 &a, const int c, 
             if (f[j].other != c) add(f[j], qo[j]);  // not a placeholder's
         return own;
     }
-    // the first faces: every load issued before the sums (a short list
-    // repeats its last face, whose terms are then not added).  Fewer in
-    // flight is slower: O-grid gradients 0.97 -> 1.54 ms per step with three,
-    // 1.89 with two.
-    const int e0 = a.g_off[c], ne = a.g_off[c + 1] - e0;
+    // the first faces: every load issued before the sums.  Fewer in flight is
+    // slower: O-grid gradients 0.97 -> 1.54 ms per step with three, 1.89 with
+    // two.
+    int e0 = 0, ne = U, key[U], oth[U];
+    if constexpr (D == 2) {
+        load_keys<D, NT>(a.g_key, a.nc, 0, c, key);
+        load_keys<D, NT>(a.g_oth, a.nc, 0, c, oth);
+    } else {
+        load_keys<D, NT>(a.g_key, a.nc, 0, c, key);
+    }
+    if (a.more_faces) {
+        e0 = a.g_off[c];
+        ne = a.g_off[c + 1] - e0;
+    }
 #pragma unroll
     for (int j = 0; j < U; j++) {
-        f[j].load_list(a, a.g_ent[e0 + (j < ne ? j : ne - 1)]);
+        if constexpr (D == 2) {
+            f[j].load_face(a, key[j]);
+            f[j].other = oth[j];
+        } else {
+            f[j].load_list(a, key[j]);
+        }
         load_q32<D>(a, f[j].other, qo[j]);
     }
 #pragma unroll
     for (int j = 0; j < U; j++)
-        if (j < ne) add(f[j], qo[j]);
+        if (key[j] != kNoFace) add(f[j], qo[j]);
     for (int e = e0 + U; e < e0 + ne; e++) {
         F g;
         float q[D + 2];
@@ -942,54 +963,55 @@ __device__ __forceinline__ void cell_update32_cell(const KArgs32 &a, float A, fl
 #pragma unroll
     for (int k = 0; k < D + 2; k++) res[k] = 0.f;
     load_q32<D>(a, c, q);
-    const int e0 = a.g_off[c], ne = a.g_off[c + 1] - e0;
-    unsigned gmask = 0;  // bit j: entry j leads to a boundary ghost
-    // the faces in gather order, U at a time with their loads issued
-    // together (a cell has at most kMaxFaces).  Within a group no branch: an
-    // entry past the cell's last reads the last entry again and is selected
-    // away.
     constexpr int U = GatherUnroll<D>::value;
+    int key[U];
+    load_keys<D, NT>(a.g_key, a.nc, 0, c, key);
+    unsigned gmask = 0;  // bit j: entry j leads to a boundary ghost
+    auto load = [&](const int ent, float (&fr)[D + 2]) {
+        const int f = face_of(ent);
+        const float4 v = reinterpret_cast<const float4 *>(a.frhs)[f];
+        fr[0] = v.x;
+        fr[1] = v.y;
+        fr[2] = v.z;
+        fr[3] = v.w;
+        if (D == 3) fr[D + 1] = a.frhs[(size_t)4 * a.nf + f];
+    };
+    auto add = [&](const int j, const int ent, const bool valid, const float (&fr)[D + 2]) {
+        gmask |= ent >= 0 && (ent & kGhostFaceFlag) ? 1u << j : 0u;
+        const float sg = ent >= 0 ? sP : -sP;
 #pragma unroll
-    for (int j0 = 0; j0 < kMaxFaces; j0 += U) {
-        if (j0 < ne) {
-            int key[U];
-            float fr[U][D + 2];
+        for (int k = 0; k < D + 2; k++) {
+            if (RES) res[k] = valid ? res[k] + (ent >= 0 ? fr[k] : -fr[k]) : res[k];
+            dq[k] = valid ? dq[k] + sg * fr[k] : dq[k];
+        }
+    };
+    // the faces in gather order, the first U with their loads issued together
+    // and without a branch: a placeholder reads face 0 and is selected away
+    float fr[U][D + 2];
 #pragma unroll
-            for (int u = 0; u < U; u++)
-                if (j0 + u < kMaxFaces) key[u] = a.g_ent[e0 + (j0 + u < ne ? j0 + u : ne - 1)];
+    for (int u = 0; u < U; u++) load(key[u], fr[u]);
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                if (j0 + u < kMaxFaces) {
-                    const int f = key[u] >= 0 ? (key[u] & kFaceMask) : ~key[u];
-                    const float4 v = reinterpret_cast<const float4 *>(a.frhs)[f];
-                    fr[u][0] = v.x;
-                    fr[u][1] = v.y;
-                    fr[u][2] = v.z;
-                    fr[u][3] = v.w;
-                    if (D == 3) fr[u][D + 1] = a.frhs[(size_t)4 * a.nf + f];
-                }
-            }
+    for (int k = 0; k < D + 2; k++) dq[k] *= A;
 #pragma unroll
-            for (int k = 0; k < D + 2; k++) dq[k] = j0 == 0 ? dq[k] * A : dq[k];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                if (j0 + u < kMaxFaces) {
-                    const bool valid = j0 + u < ne;
-                    gmask |= valid && key[u] >= 0 && (key[u] & kGhostFaceFlag) ? 1u << (j0 + u) : 0u;
-                    const float sg = key[u] >= 0 ? sP : -sP;
-#pragma unroll
-                    for (int k = 0; k < D + 2; k++) {
-                        if (RES) res[k] = valid ? res[k] + (key[u] >= 0 ? fr[u][k] : -fr[u][k]) : res[k];
-                        dq[k] = valid ? dq[k] + sg * fr[u][k] : dq[k];
-                    }
-                }
-            }
+    for (int u = 0; u < U; u++) add(u, key[u], key[u] != kNoFace, fr[u]);
+    int e1 = 0, ne = 0;  // entries beyond the first U (a cell has at most kMaxFaces)
+    if (U < kMaxFaces && a.more_faces) {
+        e1 = a.g_off[c] + U;
+        ne = min(a.g_off[c + 1] - e1, kMaxFaces - U);
+        for (int j = 0; j < ne; j++) {
+            const int ent = a.g_ent[e1 + j];
+            float f1[D + 2];
+            load(ent, f1);
+            add(U + j, ent, true, f1);
         }
     }
     finish_cell32<D, NT>(a, c, dt, B, a.q, q, dq);
     // refresh this cell's boundary ghosts for the next stage
-    for (unsigned m = gmask; m; m &= m - 1)
-        refresh_ghost32<D, NT>(a, a.fN[a.g_ent[e0 + __builtin_ctz(m)] & kFaceMask] - a.nc, a.q, q);
+    for (unsigned m = gmask; m; m &= m - 1) {
+        const int j = __builtin_ctz(m);
+        const int ent = U >= kMaxFaces || j < U ? a.g_key[key_at<D>(a.nc, j, c)] : a.g_ent[e1 + j - U];
+        refresh_ghost32<D, NT>(a, a.fN[ent & kFaceMask] - a.nc, a.q, q);
+    }
 }
 
 template <int D, int MODE>
@@ -1089,13 +1111,20 @@ template <int D, int MODE>
 __device__ __forceinline__ double cfl_cell32(const KArgs32 &a, const int c, const float (&qc)[D + 2], float vinv,
                                              double param) {
     CflSum32<D, MODE> t(a, qc);
-    const int e0 = a.g_off[c], ne = a.g_off[c + 1] - e0;
+    constexpr int U = GatherUnroll<D>::value;
+    int key[U];
+    float S[U][D];
+    load_keys<D, false>(a.g_key, a.nc, 0, c, key);
 #pragma unroll
-    for (int j = 0; j < kMaxFaces; j++) {
-        const int ent = a.g_ent[e0 + (j < ne ? j : ne - 1)];
-        float S[D];
-        load_S32<D>(a.S, ent >= 0 ? (ent & kFaceMask) : ~ent, S);
-        t.add(S, j < ne);
+    for (int j = 0; j < U; j++) load_S32<D>(a.S, face_of(key[j]), S[j]);
+#pragma unroll
+    for (int j = 0; j < U; j++) t.add(S[j], key[j] != kNoFace);
+    if (U < kMaxFaces && a.more_faces) {
+        const int e0 = a.g_off[c], ne = min(a.g_off[c + 1] - e0, kMaxFaces);
+        for (int j = U; j < ne; j++) {
+            load_S32<D>(a.S, face_of(a.g_ent[e0 + j]), S[0]);
+            t.add(S[0], true);
+        }
     }
     return t.value(a, qc[0], vinv, param);
 }

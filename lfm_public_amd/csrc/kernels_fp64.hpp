@@ -27,6 +27,9 @@ struct KArgs {
     const double *S;                // [nf][D]: a face's area vector as one record
     const double *d, *w;            // d: [D][nf]
     const int32_t *g_off, *g_ent;   // gather lists
+    // each cell's first GatherUnroll gather entries and the cells they lead
+    // to (key_at places them; kNoFace and the cell itself past its last)
+    const int32_t *g_key, *g_oth;
     const int32_t *s_off, *s_ent;   // slot lists
     const int32_t *ghost_cell, *ghost_role;
     const double *vinv;
@@ -209,6 +212,60 @@ inline int grad_record_stride64(int D, bool rg) {
 }
 
 // face flux record: components 0-3 as 32 bytes per face, component 4 after
+// Gather entries of fixed width.  A kernel that walks the gather list waits for
+// the list's offsets, then the entry, then (gradients) the face's cells before
+// it can ask for the other cell's state; from these arrays the face's data and
+// the other cell's state are asked for as soon as the entry is there, at the
+// same bytes (32 per 2D cell and gradient launch against 30).  Per step, list
+// against these: 2D M2AUSM FP32 50.0 -> 47.6 us (4 k cells), 118 -> 112 (262 k),
+// 1429 -> 1328 (4.2 M); FP64 73.6 -> 68.4 (16 k), 470 -> 447 (640 k); FP32 O-grid
+// 2377 -> 2303 (4 M).
+constexpr int32_t kNoFace = INT32_MIN;
+__device__ __forceinline__ int face_of(const int key) {
+    return key >= 0 ? (key & kFaceMask) : key == kNoFace ? 0 : ~key;
+}
+// 2D: a cell's four together (one 16-byte load); 3D: as slots
+template <int D>
+__device__ __forceinline__ size_t key_at(int nc, int j, int c) {
+    if constexpr (D == 2) return (size_t)GatherUnroll<2>::value * c + j;
+    return slot_at<D, 1>(nc, j, 0, c);
+}
+inline size_t keys_len(int D, int nc) {
+    return D == 2 ? (size_t)GatherUnroll<2>::value * nc : slot_array_len(nc, GatherUnroll<3>::value, 1);
+}
+using i2v = int32_t __attribute__((ext_vector_type(2)));
+using i4v = int32_t __attribute__((ext_vector_type(4)));
+// entries [j0, j0 + N) of cell c (2D: j0 a multiple of N)
+template <int D, bool NT, int N>
+__device__ __forceinline__ void load_keys(const int32_t *p, const int nc, const int j0, const int c, int (&k)[N]) {
+    if constexpr (D == 2 && N == 4) {
+        const i4v v = ld_once<NT>(reinterpret_cast<const i4v *>(p) + c);
+        k[0] = v.x;
+        k[1] = v.y;
+        k[2] = v.z;
+        k[3] = v.w;
+    } else if constexpr (D == 2 && N == 2) {
+        const i2v v = ld_once<NT>(reinterpret_cast<const i2v *>(p) + 2 * (size_t)c + j0 / 2);
+        k[0] = v.x;
+        k[1] = v.y;
+    } else {
+#pragma unroll
+        for (int u = 0; u < N; u++) k[u] = ld_once<NT>(p + key_at<D>(nc, j0 + u, c));
+    }
+}
+template <int D>
+__global__ void __launch_bounds__(256) build_keys(int nc, const int32_t *g_off, const int32_t *g_ent, const int32_t *fP,
+                                                  const int32_t *fN, int32_t *key, int32_t *oth) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= nc) return;
+    const int e0 = g_off[c], ne = g_off[c + 1] - e0;
+    for (int j = 0; j < GatherUnroll<D>::value; j++) {
+        const int ent = j < ne ? g_ent[e0 + j] : kNoFace, f = face_of(ent);
+        key[key_at<D>(nc, j, c)] = ent;
+        if (oth) oth[key_at<D>(nc, j, c)] = j >= ne ? c : ent >= 0 ? fN[f] : fP[f];
+    }
+}
+
 template <int D>
 __device__ __forceinline__ void load_frhs(const KArgs &a, int f, double (&r)[D + 2]) {
     const double2 *p = reinterpret_cast<const double2 *>(a.frhs + 4 * (size_t)f);
@@ -217,7 +274,7 @@ __device__ __forceinline__ void load_frhs(const KArgs &a, int f, double (&r)[D +
     r[1] = v0.y;
     r[2] = v1.x;
     r[3] = v1.y;
-    if (D == 3) r[4] = a.frhs[(size_t)4 * a.nf + f];
+    if constexpr (D == 3) r[4] = a.frhs[(size_t)4 * a.nf + f];
 }
 
 template <int D, bool RG>
@@ -413,11 +470,11 @@ __device__ __forceinline__ void vis_tensors(const KArgs &a, const double (&dudx)
 
 // Bound: latency (at a few 100 k cells a launch has 2-3 waves per SIMD to hide
 // its dependent loads), so registers decide.  Faces in groups whose loads are
-// issued together: two in 2D (176 k-cell annulus, four 182, three 179, two 177,
-// one 179 us per step), three in 3D at 3 waves per SIMD (193 k-cell O-grid: all
-// six at 2 waves 417, three 404, two 406, one 414).
+// issued together: all four in 2D (176 k-cell annulus, four 171, two 176 us per
+// step), two in 3D at 3 waves per SIMD (193 k-cell O-grid: three spill and take
+// 415, two 397, one 397; 1 M cells: two 1531, one 1586).
 template <int D>
-constexpr int kGradGroup64 = D == 2 ? 2 : 3;
+constexpr int kGradGroup64 = D == 2 ? 4 : 2;
 template <int D, int GRAD, bool VISC, bool RG, bool NT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) grad_vis(KArgs a) {
     const int c = LFM_TID(blockIdx.x);
@@ -501,30 +558,42 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) g
         }
     };
     // groups of G faces in gather order, their loads issued together
-    const int e0 = a.g_off[c], ne = a.g_off[c + 1] - e0;
-    constexpr int G = kGradGroup64<D>;
-    int ent[G];
-#pragma unroll
-    for (int u = 0; u < G; u++) ent[u] = a.g_ent[e0 + (u < ne ? u : ne - 1)];
+    constexpr int U = GatherUnroll<D>::value, G = kGradGroup64<D>;
+    static_assert(U % G == 0);
+    int key[G], oth[G], e0 = 0, ne = U;
+    load_keys<D, NT>(a.g_key, a.nc, 0, c, key);
+    load_keys<D, NT>(a.g_oth, a.nc, 0, c, oth);
+    if (a.more_faces) {
+        e0 = a.g_off[c];
+        ne = max(U, a.g_off[c + 1] - e0);
+    }
 #pragma unroll 1
     for (int j0 = 0; j0 < ne; j0 += G) {
-        bool isPj[G];
         double wj[G], Sj[G][D], qj[G][D + 2];
-        int next[G];
+        int nkey[G], noth[G];
 #pragma unroll
         for (int u = 0; u < G; u++) {
-            isPj[u] = ent[u] >= 0;
-            const int f = isPj[u] ? (ent[u] & kFaceMask) : ~ent[u];
-            const int o = isPj[u] ? a.fN[f] : a.fP[f];
+            const int f = face_of(key[u]);
             wj[u] = a.w[f];
             load_S64<D>(a.S, f, Sj[u]);
-            load_q<D>(a, o, qj[u]);
-            next[u] = a.g_ent[e0 + (j0 + G + u < ne ? j0 + G + u : ne - 1)];
+            load_q<D>(a, oth[u], qj[u]);
+        }
+        const int jn = j0 + G;
+        load_keys<D, NT>(a.g_key, a.nc, jn < U ? jn : 0, c, nkey);
+        load_keys<D, NT>(a.g_oth, a.nc, jn < U ? jn : 0, c, noth);
+        if (a.more_faces && jn >= U) {  // entries beyond the first U
+#pragma unroll
+            for (int u = 0; u < G; u++) {
+                nkey[u] = jn + u < ne ? a.g_ent[e0 + jn + u] : kNoFace;
+                const int f = face_of(nkey[u]);
+                noth[u] = nkey[u] >= 0 ? a.fN[f] : a.fP[f];
+            }
         }
 #pragma unroll
         for (int u = 0; u < G; u++) {
-            if (j0 + u < ne) add(isPj[u], wj[u], Sj[u], qj[u]);
-            ent[u] = next[u];
+            if (key[u] != kNoFace) add(key[u] >= 0, wj[u], Sj[u], qj[u]);
+            key[u] = nkey[u];
+            oth[u] = noth[u];
         }
     }
     // refresh of tau / sigmaU / tauMC from the completed dudx (cfd_v0.cpp:1813-1834);
@@ -1129,12 +1198,14 @@ __global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, 
 #pragma unroll
         for (int k = 0; k < D + 2; k++) res[k] = 0.0;
         load_q<D>(a, c, q);
-        const int e0 = a.g_off[c], ne = a.g_off[c + 1] - e0;
-        int gface[kMaxFaces], ngf = 0;
+        constexpr int U = GatherUnroll<D>::value;
+        int key[U];
+        load_keys<D, NT>(a.g_key, a.nc, 0, c, key);
+        unsigned gmask = 0;  // bit j: entry j leads to a boundary ghost
         // owner side adds, neighbour side subtracts (cfd_v0.cpp:2800-2806)
-        auto add = [&](const int ent, const double (&fr)[D + 2]) {
+        auto add = [&](const int j, const int ent, const double (&fr)[D + 2]) {
             if (ent >= 0) {
-                if ((ent & kGhostFaceFlag) && ngf < kMaxFaces) gface[ngf++] = ent & kFaceMask;
+                if (ent & kGhostFaceFlag) gmask |= 1u << j;
 #pragma unroll
                 for (int k = 0; k < D + 2; k++) {
                     if (RES) res[k] += fr[k];
@@ -1149,27 +1220,24 @@ __global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, 
             }
         };
         // the first faces' fluxes fetched together, then added in gather order
-        constexpr int U = GatherUnroll<D>::value;
-        int ent[U];
         double fr[U][D + 2];
 #pragma unroll
-        for (int j = 0; j < U; j++) ent[j] = a.g_ent[e0 + (j < ne ? j : ne - 1)];
-#pragma unroll
-        for (int j = 0; j < U; j++) {
-            const int f = ent[j] >= 0 ? (ent[j] & kFaceMask) : ~ent[j];
-            load_frhs<D>(a, f, fr[j]);
-        }
+        for (int j = 0; j < U; j++) load_frhs<D>(a, face_of(key[j]), fr[j]);
 #pragma unroll
         for (int k = 0; k < D + 2; k++) dq[k] *= A;
 #pragma unroll
         for (int j = 0; j < U; j++)
-            if (j < ne) add(ent[j], fr[j]);
-        for (int e = e0 + U; e < e0 + ne; e++) {
-            const int en = a.g_ent[e];
-            const int f = en >= 0 ? (en & kFaceMask) : ~en;
-            double f1[D + 2];
-            load_frhs<D>(a, f, f1);
-            add(en, f1);
+            if (key[j] != kNoFace) add(j, key[j], fr[j]);
+        int e1 = 0, ne = 0;  // entries beyond the first U
+        if (a.more_faces) {
+            e1 = a.g_off[c] + U;
+            ne = a.g_off[c + 1] - e1;
+            for (int j = 0; j < ne; j++) {
+                const int ent = a.g_ent[e1 + j];
+                double f1[D + 2];
+                load_frhs<D>(a, face_of(ent), f1);
+                add(U + j, ent, f1);
+            }
         }
         if (a.sigma) sponge64<D, NT>(a, c, dt, q, dq);
 #pragma unroll
@@ -1179,8 +1247,10 @@ __global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, 
         }
         store_q<D, NT>(a.q, a.ntot, c, q);
         // refresh this cell's boundary ghosts for the next stage
-        for (int i = 0; i < ngf; i++) {
-            const int g = a.fN[gface[i]] - a.nc;
+        for (unsigned m = gmask; m; m &= m - 1) {
+            const int j = __builtin_ctz(m);
+            const int ent = j < U ? a.g_key[key_at<D>(a.nc, j, c)] : a.g_ent[e1 + j - U];
+            const int g = a.fN[ent & kFaceMask] - a.nc;
             double qg[D + 2];
             if (!ghost_state<D>(a, a.ghost_role[g], q, qg)) continue;
             store_q<D, NT>(a.q, a.ntot, a.nc + g, qg);

@@ -2,6 +2,7 @@
 // layout in the reference's cell and face processing order.
 #pragma once
 
+#include <algorithm>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -98,6 +99,14 @@ struct FaceTable {
 };
 template <typename T>
 FaceTable<T> face_table(const SolverLayout &L, int max_n);
+
+// the most gather entries of a cell (a cell that is its own neighbour has two
+// for each such face)
+inline int max_entries(const SolverLayout &L) {
+    int m = 0;
+    for (int c = 0; c < L.nc; c++) m = std::max(m, L.g_off[c + 1] - L.g_off[c]);
+    return m;
+}
 
 // bits that hold an index below n
 inline int index_bits(long n) {

@@ -80,6 +80,25 @@ static int dev_zeros(Solver *s, T **dst, size_t n) {
     return 0;
 }
 
+// the fixed-width gather entries of an argument block whose lists are on the
+// device (on the null stream, as the uploads of the set-up)
+template <class Args>
+int Solver::build_gather_keys(Args &a, bool others) {
+    const size_t n = keys_len(L.D, L.nc) * sizeof(int32_t);
+    void *key = nullptr, *oth = nullptr;
+    if (int rc = dev_alloc(&key, n)) return rc;
+    if (others)
+        if (int rc = dev_alloc(&oth, n)) return rc;
+    auto build = L.D == 2 ? build_keys<2> : build_keys<3>;
+    hipLaunchKernelGGL(build, dim3(nblocks(L.nc)), dim3(kBlock), 0, nullptr, L.nc, a.g_off, a.g_ent, a.fP, a.fN,
+                       (int32_t *)key, (int32_t *)oth);
+    HIP_TRY(hipGetLastError());
+    a.g_key = (const int32_t *)key;
+    a.g_oth = (const int32_t *)oth;
+    return 0;
+}
+template int Solver::build_gather_keys<KArgs32>(KArgs32 &, bool);
+
 Solver::~Solver() {
     free_step_graph();
     for (void *p : allocs) (void)hipFree(p);
@@ -185,7 +204,8 @@ static int create_fp64(Solver *s) {
     // that walk the list
     s->fused_ok = !s->visc && s->prm.solver < 2 && L.halo.empty();
     for (size_t f = 0; f < nf && s->fused_ok; f++) s->fused_ok = L.fP[f] != L.fN[f];
-    a.more_faces = L.max_faces > (D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value);
+    a.more_faces = max_entries(L) > (D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value);
+    if (s->build_gather_keys(a, true)) return LFM_EDEVICE;
     if (s->fused_ok) {
         // records in both orientations and a placeholder's fit above the
         // cell index; kMaxTable64 keeps the table in an XCD's L2
@@ -563,7 +583,7 @@ bool Solver::ensure_slots32() {
 void Solver::size_stage() {
     const size_t D = L.D, w = fp32 ? sizeof(float) : sizeof(double), nc = L.nc, nf = L.nf;
     const bool grads = visc || prm.solver == 2;
-    const size_t ent = L.g_ent.size() + nc;  // gather list and offsets
+    const size_t keys = keys_len(L.D, L.nc) * sizeof(int32_t);  // gather entries
     size_t b = nc * ((2 * (D + 2) + 2) * w);  // state, RK register, 1/V, sponge
     if (fused_ok) {
         // second state; slots: one word each, or a face's own data
@@ -571,8 +591,9 @@ void Solver::size_stage() {
         const size_t U = D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value;
         b += nc * ((D + 2) * w + U * (packed ? sizeof(int32_t) : sizeof(int32_t) + (D + 1) * w));
     } else {
-        // face fluxes, S, d, w, both cells; gather list
-        b += nf * ((3 * D + 3) * w + 2 * sizeof(int32_t)) + ent * sizeof(int32_t);
+        // face fluxes, S, d, w, both cells; gather entries
+        b += nf * ((3 * D + 3) * w + 2 * sizeof(int32_t)) + keys;
+        if (grads && !(fp32 && D == 3)) b += keys;  // the cells they lead to
     }
     if (grads) b += nc * (size_t)(fp32 ? k32->gstride : k64.gstride) * w;
     if (grads && fp32 && D == 3) b += nc * GatherUnroll<3>::value * (sizeof(int32_t) + (D + 1) * w);  // slots

@@ -108,6 +108,7 @@ int create_fp32p(Solver *s) {
     }
     rc |= up(s, (int32_t **)&a.g_off, L.g_off.data(), nc + 1);
     rc |= up(s, (int32_t **)&a.g_ent, L.g_ent.data(), L.g_ent.size());
+    if (!rc) rc |= s->build_gather_keys(a, D == 2);
     rc |= up(s, (int32_t **)&a.ghost_cell, L.ghost_cell.data(), L.ng);
     rc |= up(s, (int32_t **)&a.ghost_role, L.ghost_role.data(), L.ng);
     rc |= up(s, (double **)&a.vol_d, L.volume.data(), nc);
@@ -128,7 +129,7 @@ int create_fp32p(Solver *s) {
         // step that uses it; its unset-patch ghosts are copied from q by the
         // first fused stage)
         s->fused_ok = !s->visc && s->prm.solver < 2 && L.halo.empty();
-        a.more_faces = L.max_faces > (D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value);
+        a.more_faces = max_entries(L) > (D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value);
         // slots are read by the one-launch stage and by 3D gradients (a halo
         // face has its weight only after the import: no table there)
         if (s->fused_ok || (D == 3 && L.halo.empty())) {

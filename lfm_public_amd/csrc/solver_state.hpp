@@ -63,6 +63,8 @@ struct Solver {
     // device memory of the set-up: small arrays share slabs, so that creating
     // a small solve does not take one allocation per array
     int dev_alloc(void **p, size_t bytes);
+    template <class Args>
+    int build_gather_keys(Args &a, bool others);
     char *slab = nullptr;
     size_t slab_left = 0;
 
