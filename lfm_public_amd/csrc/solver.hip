@@ -38,23 +38,45 @@ static constexpr int kMaxTable64 = 2048;
 static constexpr int kBlock = 256;
 static inline int nblocks(long n) { return (int)((n + kBlock - 1) / kBlock); }
 
+static constexpr size_t kSlab = 1 << 20;
 int Solver::dev_alloc(void **p, size_t bytes) {
-    constexpr size_t kSlab = 1 << 20, kShare = 128 << 10, kAlign = 256;
+    constexpr size_t kShare = 128 << 10, kAlign = 256;
     const size_t need = (bytes + kAlign - 1) / kAlign * kAlign;
     if (need > kShare) {
         HIP_TRY(hipMalloc(p, bytes));
         allocs.push_back(*p);
     } else {
-        if (need > slab_left) {
+        if (!slab || slab_used + need > kSlab) {
+            if (int rc = slab_flush()) return rc;
+            slab = nullptr;
             HIP_TRY(hipMalloc((void **)&slab, kSlab));
             allocs.push_back(slab);
-            slab_left = kSlab;
+            slab_used = slab_copied = 0;
+            slab_host.reset(new char[kSlab]);
         }
-        *p = slab;
-        slab += need;
-        slab_left -= need;
+        *p = slab + slab_used;
+        slab_used += need;
     }
     device_bytes += (int64_t)bytes;
+    return 0;
+}
+
+int Solver::dev_fill(void *p, const void *src, size_t bytes) {
+    const size_t at = (size_t)((char *)p - slab);
+    if (slab && (char *)p >= slab && at >= slab_copied && at + bytes <= slab_used)
+        src ? std::memcpy(slab_host.get() + at, src, bytes) : std::memset(slab_host.get() + at, 0, bytes);
+    else if (src)
+        HIP_TRY(hipMemcpy(p, src, bytes, hipMemcpyHostToDevice));
+    else
+        HIP_TRY(hipMemset(p, 0, bytes));
+    return 0;
+}
+
+int Solver::slab_flush() {
+    if (slab && slab_used > slab_copied)
+        HIP_TRY(hipMemcpy(slab + slab_copied, slab_host.get() + slab_copied, slab_used - slab_copied,
+                          hipMemcpyHostToDevice));
+    slab_copied = slab_used;
     return 0;
 }
 
@@ -65,8 +87,7 @@ static int dev_upload(Solver *s, T **dst, const T *src, size_t n) {
         return 0;
     }
     if (int rc = s->dev_alloc((void **)dst, n * sizeof(T))) return rc;
-    if (src) HIP_TRY(hipMemcpy(*dst, src, n * sizeof(T), hipMemcpyHostToDevice));
-    return 0;
+    return src ? s->dev_fill(*dst, src, n * sizeof(T)) : 0;
 }
 
 template <typename T>
@@ -76,8 +97,7 @@ static int dev_zeros(Solver *s, T **dst, size_t n) {
         return 0;
     }
     if (int rc = s->dev_alloc((void **)dst, n * sizeof(T))) return rc;
-    HIP_TRY(hipMemset(*dst, 0, n * sizeof(T)));
-    return 0;
+    return s->dev_fill(*dst, nullptr, n * sizeof(T));
 }
 
 // the fixed-width gather entries of an argument block whose lists are on the
@@ -89,6 +109,7 @@ int Solver::build_gather_keys(Args &a, bool others) {
     if (int rc = dev_alloc(&key, n)) return rc;
     if (others)
         if (int rc = dev_alloc(&oth, n)) return rc;
+    if (int rc = slab_flush()) return rc;
     auto build = L.D == 2 ? build_keys<2> : build_keys<3>;
     hipLaunchKernelGGL(build, dim3(nblocks(L.nc)), dim3(kBlock), 0, nullptr, L.nc, a.g_off, a.g_ent, a.fP, a.fN,
                        (int32_t *)key, (int32_t *)oth);
@@ -196,9 +217,9 @@ static int create_fp64(Solver *s) {
         std::vector<double> q0((size_t)(D + 2) * ntot, 0.0);
         for (int k = 0; k < D + 2; k++)
             for (size_t c = 0; c < nc; c++) q0[q64_index(k, c, ntot)] = L.q0[(size_t)k * nc + c];
-        HIP_TRY(hipMemcpy(a.q, q0.data(), q0.size() * sizeof(double), hipMemcpyHostToDevice));
+        if (int rc = s->dev_fill(a.q, q0.data(), q0.size() * sizeof(double))) return rc;
     }
-    HIP_TRY(hipMemcpy(s->d_scalar, &s->dt, sizeof(double), hipMemcpyHostToDevice));
+    if (int rc = s->dev_fill(s->d_scalar, &s->dt, sizeof(double))) return rc;
     // one-launch stages; a cell that is its own neighbour (a cyclic pair one
     // cell apart) has more gather entries than slots and keeps the launches
     // that walk the list
@@ -987,6 +1008,9 @@ int lfm_solver_create_part(const lfm_polymesh *mesh, const lfm_partition *part, 
             lfm::dev_zeros(s.get(), &hd.recv_src, gslot.size()))
             return LFM_EDEVICE;
     }
+    if (s->slab_flush()) return LFM_EDEVICE;
+    s->slab_host.reset();
+    s->slab = nullptr;  // what follows is allocated by itself
     HIP_TRY(hipDeviceSynchronize());
     auto *h = new lfm_solver;
     h->impl = std::move(s);

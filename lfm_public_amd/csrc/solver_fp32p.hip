@@ -24,11 +24,7 @@ static int up(Solver *s, T **dst, const T *src, size_t n) {
         return 0;
     }
     if (int rc = s->dev_alloc((void **)dst, n * sizeof(T))) return rc;
-    if (src)
-        HIP_TRY(hipMemcpy(*dst, src, n * sizeof(T), hipMemcpyHostToDevice));
-    else
-        HIP_TRY(hipMemset(*dst, 0, n * sizeof(T)));
-    return 0;
+    return s->dev_fill(*dst, src, n * sizeof(T));
 }
 
 static std::vector<float> to_f32(const std::vector<double> &v) {
@@ -176,7 +172,7 @@ int create_fp32p(Solver *s) {
     a.d_cfl = s->d_cfl;
     a.d_dtmin = s->d_dtmin;
     a.nblk_cells = nblocks((long)nc);
-    HIP_TRY(hipMemcpy(s->d_scalar, &s->dt, sizeof(double), hipMemcpyHostToDevice));
+    if (int rc = s->dev_fill(s->d_scalar, &s->dt, sizeof(double))) return rc;
     return 0;
 }
 

@@ -60,13 +60,17 @@ struct Solver {
     const int32_t *d_comb = nullptr;  // L.comb on the device
     std::vector<void *> allocs;
     int64_t device_bytes = 0;
-    // device memory of the set-up: small arrays share slabs, so that creating
-    // a small solve does not take one allocation per array
+    // device memory of the set-up: small arrays share slabs, each filled on the
+    // host and copied as a whole, so that creating a small solve does not take
+    // an allocation and a copy per array
     int dev_alloc(void **p, size_t bytes);
+    int dev_fill(void *p, const void *src, size_t bytes);  // src null: zeros
+    int slab_flush();  // what was filled so far, before a kernel reads it
     template <class Args>
     int build_gather_keys(Args &a, bool others);
     char *slab = nullptr;
-    size_t slab_left = 0;
+    size_t slab_used = 0, slab_copied = 0;
+    std::unique_ptr<char[]> slab_host;
 
     // device scalars: [0] deltaT, [2..6] residual sums, [8] cfl, [9] dt min
     double *d_scalar = nullptr;
