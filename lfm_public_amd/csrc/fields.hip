@@ -15,21 +15,13 @@
 namespace lfm {
 
 // ISolver::prepare_for_timestep: dq = 0, RES = 0
-static __global__ void __launch_bounds__(256) fill_zero32(float *p, size_t n) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.0f;
-}
-
 void Solver::zero_state_for_step() {
     const size_t n = (size_t)(L.D + 2) * L.nc;
     const int nb = (int)((n + 255) / 256);
-    if (fp32) {
-        hipLaunchKernelGGL(fill_zero32, dim3(nb), dim3(256), 0, stream, k32->dq, n);
-        hipLaunchKernelGGL(fill_zero32, dim3(nb), dim3(256), 0, stream, k32->res_cell, n);
-    } else {
-        hipLaunchKernelGGL(fill_zero, dim3(nb), dim3(256), 0, stream, k64.dq, n);
-        hipLaunchKernelGGL(fill_zero, dim3(nb), dim3(256), 0, stream, k64.res_cell, n);
-    }
+    if (fp32)
+        hipLaunchKernelGGL(fill_zero<float>, dim3(nb), dim3(256), 0, stream, k32->dq, k32->res_cell, n);
+    else
+        hipLaunchKernelGGL(fill_zero<double>, dim3(nb), dim3(256), 0, stream, k64.dq, k64.res_cell, n);
     pending_A = 1.0;
 }
 

@@ -1286,20 +1286,38 @@ __global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, 
     if constexpr (CFL >= 0) block_extremum<CFL>(cv, a.partial + LFM_BLK());
 }
 
-// Sum of per-block partials in fixed order, one block.
+// Sum of per-block partials in fixed order, one block; all components go down
+// the tree together (one after the other took 5.1 us for 256 partials of four).
 static __global__ void __launch_bounds__(256) reduce_sum(const double *partial, int nblk, int ncomp, double *out, int accumulate) {
-    __shared__ double sh[256];
-    for (int k = 0; k < ncomp; k++) {
-        double s = 0.0;
-        for (int i = threadIdx.x; i < nblk; i += blockDim.x) s += partial[(size_t)i * ncomp + k];
-        sh[threadIdx.x] = s;
+    constexpr int kMax = 5;
+    __shared__ double sh[kMax][256];
+    const int t = threadIdx.x;
+    double v[kMax];
+#pragma unroll
+    for (int k = 0; k < kMax; k++) v[k] = 0.0;
+    for (int i = t; i < nblk; i += 256) {
+#pragma unroll
+        for (int k = 0; k < kMax; k++)
+            if (k < ncomp) v[k] += partial[(size_t)i * ncomp + k];
+    }
+#pragma unroll
+    for (int k = 0; k < kMax; k++) sh[k][t] = v[k];
+    for (int st = 128; st >= 64; st >>= 1) {
         __syncthreads();
-        for (int st = blockDim.x / 2; st > 0; st >>= 1) {
-            if ((int)threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-            __syncthreads();
+        if (t < st) {
+#pragma unroll
+            for (int k = 0; k < kMax; k++) sh[k][t] = v[k] = sh[k][t] + sh[k][t + st];
         }
-        if (threadIdx.x == 0) out[k] = accumulate ? out[k] + sh[0] : sh[0];
-        __syncthreads();
+    }
+    if (t >= 64) return;
+    for (int st = 32; st > 0; st >>= 1) {
+#pragma unroll
+        for (int k = 0; k < kMax; k++) v[k] += __shfl_down(v[k], st, 64);
+    }
+    if (t == 0) {
+#pragma unroll
+        for (int k = 0; k < kMax; k++)
+            if (k < ncomp) out[k] = accumulate ? out[k] + v[k] : v[k];
     }
 }
 
@@ -1664,9 +1682,14 @@ __global__ void __launch_bounds__(256) integrals64(KArgs a) {
     }
 }
 
-static __global__ void __launch_bounds__(256) fill_zero(double *p, size_t n) {
+template <typename T>
+static __global__ void __launch_bounds__(256) fill_zero(T *p, T *r, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.0;
+    if (i < n) p[i] = r[i] = 0;
+}
+// n <= 64 device values to pinned host memory: 2 us less than a copy of theirs
+static __global__ void __launch_bounds__(64) export_scalars(const double *x, int n, double *host) {
+    if ((int)threadIdx.x < n) host[threadIdx.x] = x[threadIdx.x];
 }
 
 template <int D>

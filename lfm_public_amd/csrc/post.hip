@@ -52,11 +52,15 @@ __device__ __forceinline__ double qv(const QView<T> &v, int k, int i) {
     return v.base[k] + (double)v.q[q64_index(k, (size_t)i, (size_t)v.ntot)];
 }
 
+// averages of cell i: sums of p and of its squared deviation from the mean
+struct AvgJob {
+    int nc;
+    double n, *pavg, *prms;
+};
 template <int D, typename T>
-__global__ void __launch_bounds__(kPostBlock) avg_accumulate(QView<T> v, int nc, double gm1, double n, double *pavg,
-                                                             double *prms) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nc) return;
+__device__ __forceinline__ void avg_accumulate(const QView<T> &v, const AvgJob &job, const double gm1, const int i) {
+    if (i >= job.nc) return;
+    double *pavg = job.pavg, *prms = job.prms;
     const double r = qv(v, 0, i);
     double velMag = 0.0;
 #pragma unroll
@@ -68,7 +72,7 @@ __global__ void __launch_bounds__(kPostBlock) avg_accumulate(QView<T> v, int nc,
     const double p = (r * gm1) * (E - 0.5 * velMag);
     const double a = pavg[i] + p;
     pavg[i] = a;
-    const double dev = p - a / n;
+    const double dev = p - a / job.n;
     prms[i] += dev * dev;
 }
 
@@ -85,20 +89,41 @@ __global__ void advance_time(double *time, const double *dt) {
     if (threadIdx.x == 0) time[0] += dt[0];
 }
 
-__global__ void write_time(double *row, const double *time_ptr, double time_val) {
-    if (threadIdx.x == 0) row[0] = time_ptr ? time_ptr[0] : time_val;
+// a row without wall patches: the time alone
+__global__ void write_time(double *row, double *time, const double *dt, double time_val) {
+    if (threadIdx.x == 0) {
+        if (time) time[0] += dt[0];
+        row[0] = time ? time[0] : time_val;
+    }
 }
 
-// One block per wall patch; each thread sums a strided share of the patch's
-// entries, then a fixed-shape tree adds the thread sums.
+// Wall forces of one row.  time: the clock this row advances by *dt first
+// (null: the row holds time_val).
+struct ForceJob {
+    const int32_t *off, *cell, *nb;
+    const double *S, *d, *snap;
+    int nw, ne, nsnap;
+    double p_inf, mu, *time, time_val, *row;
+    const double *dt;
+};
+
+// What follows a step, in one launch: blocks [0, nw) form the wall forces, one
+// per wall patch (each thread sums a strided share of the patch's entries,
+// then a fixed-shape tree adds the thread sums), the others the averages.  As
+// launches of their own (clock, averages, forces) they took 7.7 us of a
+// 65 k-cell step's 117 and a launch gap each.
 template <int D, typename T>
-__global__ void __launch_bounds__(kPostBlock) wall_forces(QView<T> v, const int32_t *off, const int32_t *cell,
-                                                          const int32_t *nb, const double *S, const double *d, int ne,
-                                                          const double *snap, int nsnap, double gm1, double p_inf,
-                                                          double mu, const double *time_ptr, double time_val,
-                                                          double *row) {
+__global__ void __launch_bounds__(kPostBlock) post_kernel(QView<T> v, double gm1, ForceJob job, AvgJob avg) {
     __shared__ double red[2 * D][kPostBlock];
     const int w = blockIdx.x, t = threadIdx.x;
+    if (w >= job.nw) {
+        avg_accumulate<D>(v, avg, gm1, (w - job.nw) * kPostBlock + t);
+        return;
+    }
+    const int32_t *off = job.off, *cell = job.cell, *nb = job.nb;
+    const double *S = job.S, *d = job.d, *snap = job.snap, p_inf = job.p_inf, mu = job.mu;
+    const int ne = job.ne, nsnap = job.nsnap;
+    double *row = job.row;
     double acc[2 * D];
 #pragma unroll
     for (int k = 0; k < 2 * D; k++) acc[k] = 0.0;
@@ -172,7 +197,14 @@ __global__ void __launch_bounds__(kPostBlock) wall_forces(QView<T> v, const int3
         __syncthreads();
     }
     if (t < 2 * D) row[1 + w * 2 * D + t] = red[t][0];
-    if (w == 0 && t == 0) row[0] = time_ptr ? time_ptr[0] : time_val;
+    if (w == 0 && t == 0) {
+        double tm = job.time_val;
+        if (job.time) {
+            tm = job.time[0] + job.dt[0];
+            job.time[0] = tm;
+        }
+        row[0] = tm;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -245,8 +277,39 @@ void Solver::post_snapshot() {
     p->snap_valid = true;
 }
 
-// records one force row (time from the device clock when time_ptr is set)
-static int post_record(Solver *s, const double *time_ptr, double time_val) {
+// one launch of post_kernel: a force row where forces.row is set, averages
+// where avg.pavg is
+static int post_launch(Solver *s, const ForceJob &forces, const AvgJob &avg) {
+    const int nb = forces.nw + (avg.pavg ? (avg.nc + kPostBlock - 1) / kPostBlock : 0);
+    if (nb == 0) return LFM_OK;
+    const double gm1 = s->gas.gm1;
+    if (s->L.D == 2) {
+        if (s->fp32)
+            hipLaunchKernelGGL((post_kernel<2, float>), dim3(nb), dim3(kPostBlock), 0, s->stream, qview<float>(s), gm1,
+                               forces, avg);
+        else
+            hipLaunchKernelGGL((post_kernel<2, double>), dim3(nb), dim3(kPostBlock), 0, s->stream, qview<double>(s),
+                               gm1, forces, avg);
+    } else {
+        if (s->fp32)
+            hipLaunchKernelGGL((post_kernel<3, float>), dim3(nb), dim3(kPostBlock), 0, s->stream, qview<float>(s), gm1,
+                               forces, avg);
+        else
+            hipLaunchKernelGGL((post_kernel<3, double>), dim3(nb), dim3(kPostBlock), 0, s->stream, qview<double>(s),
+                               gm1, forces, avg);
+    }
+    HIP_TRY(hipGetLastError());
+    return LFM_OK;
+}
+
+static AvgJob avg_job(Solver *s, int64_t n) {
+    if (n <= 0) return AvgJob{};
+    return AvgJob{s->L.nc, (double)n, s->post->pavg, s->post->prms};
+}
+
+// records one force row (clocked: the device clock advanced by deltaT;
+// otherwise of time_val) and adds to the averages where avg says so
+static int post_record(Solver *s, bool clocked, double time_val, const AvgJob &avg) {
     PostState *p = s->post;
     if (s->ghosts_stale) {
         // the state was set from outside: the ghosts are filled as the
@@ -266,56 +329,17 @@ static int post_record(Solver *s, const double *time_ptr, double time_val) {
         p->rows_dev = 0;
     }
     double *row = p->hist + (size_t)p->rows_dev * p->row_w;
+    double *time = clocked ? s->d_scalar + 15 : nullptr;
     const int nw = (int)p->walls.size();
     const Gas &g = s->gas;
-    if (nw == 0) {
-        // no wall patch: the row is the time alone
-        hipLaunchKernelGGL(write_time, dim3(1), dim3(64), 0, s->stream, row, time_ptr, time_val);
-    } else if (s->L.D == 2) {
-        if (s->fp32)
-            hipLaunchKernelGGL((wall_forces<2, float>), dim3(nw), dim3(kPostBlock), 0, s->stream, qview<float>(s),
-                               p->off, p->cell, p->nb, p->S, p->d, p->ne, p->snap, p->nsnap, g.gm1, g.p_inf, g.mu,
-                               time_ptr, time_val, row);
-        else
-            hipLaunchKernelGGL((wall_forces<2, double>), dim3(nw), dim3(kPostBlock), 0, s->stream, qview<double>(s),
-                               p->off, p->cell, p->nb, p->S, p->d, p->ne, p->snap, p->nsnap, g.gm1, g.p_inf, g.mu,
-                               time_ptr, time_val, row);
-    } else {
-        if (s->fp32)
-            hipLaunchKernelGGL((wall_forces<3, float>), dim3(nw), dim3(kPostBlock), 0, s->stream, qview<float>(s),
-                               p->off, p->cell, p->nb, p->S, p->d, p->ne, p->snap, p->nsnap, g.gm1, g.p_inf, g.mu,
-                               time_ptr, time_val, row);
-        else
-            hipLaunchKernelGGL((wall_forces<3, double>), dim3(nw), dim3(kPostBlock), 0, s->stream, qview<double>(s),
-                               p->off, p->cell, p->nb, p->S, p->d, p->ne, p->snap, p->nsnap, g.gm1, g.p_inf, g.mu,
-                               time_ptr, time_val, row);
-    }
+    ForceJob job{};
+    if (nw == 0)
+        hipLaunchKernelGGL(write_time, dim3(1), dim3(64), 0, s->stream, row, time, dt_ptr(s), time_val);
+    else
+        job = ForceJob{p->off, p->cell, p->nb,    p->S,  p->d, p->snap,  nw,  p->ne,
+                       p->nsnap, g.p_inf, g.mu, time,  time_val, row, dt_ptr(s)};
+    if (int rc = post_launch(s, job, avg)) return rc;
     p->rows_dev++;
-    HIP_TRY(hipGetLastError());
-    return LFM_OK;
-}
-
-static int post_average(Solver *s, int64_t n) {
-    PostState *p = s->post;
-    if (n <= 0) return LFM_OK;
-    const int nc = s->L.nc;
-    const int nb = (nc + kPostBlock - 1) / kPostBlock;
-    const double gm1 = s->gas.gm1, dn = (double)n;
-    if (s->L.D == 2) {
-        if (s->fp32)
-            hipLaunchKernelGGL((avg_accumulate<2, float>), dim3(nb), dim3(kPostBlock), 0, s->stream,
-                               qview<float>(s), nc, gm1, dn, p->pavg, p->prms);
-        else
-            hipLaunchKernelGGL((avg_accumulate<2, double>), dim3(nb), dim3(kPostBlock), 0, s->stream,
-                               qview<double>(s), nc, gm1, dn, p->pavg, p->prms);
-    } else {
-        if (s->fp32)
-            hipLaunchKernelGGL((avg_accumulate<3, float>), dim3(nb), dim3(kPostBlock), 0, s->stream,
-                               qview<float>(s), nc, gm1, dn, p->pavg, p->prms);
-        else
-            hipLaunchKernelGGL((avg_accumulate<3, double>), dim3(nb), dim3(kPostBlock), 0, s->stream,
-                               qview<double>(s), nc, gm1, dn, p->pavg, p->prms);
-    }
     HIP_TRY(hipGetLastError());
     return LFM_OK;
 }
@@ -324,12 +348,11 @@ int Solver::post_step() {
     PostState *p = post;
     if (!p) return LFM_OK;
     p->step++;
+    const AvgJob avg = p->cfg.have_average ? avg_job(this, p->step - p->cfg.average_start) : AvgJob{};
+    if (p->cfg.have_forces && p->step % p->cfg.forces_every == 0) return post_record(this, true, 0.0, avg);
     if (p->cfg.have_forces)
         hipLaunchKernelGGL(advance_time, dim3(1), dim3(64), 0, stream, d_scalar + 15, dt_ptr(this));
-    int rc = LFM_OK;
-    if (p->cfg.have_average) rc = post_average(this, p->step - p->cfg.average_start);
-    if (!rc && p->cfg.have_forces && p->step % p->cfg.forces_every == 0) rc = post_record(this, d_scalar + 15, 0.0);
-    return rc;
+    return post_launch(this, ForceJob{}, avg);
 }
 
 static int post_configure(Solver *s, const lfm_post &cfg) {
@@ -423,7 +446,7 @@ int lfm_post_average(lfm_solver *h, int32_t n) {
     if (!h) return fail(LFM_EINVAL, "null handle");
     Solver *s = h->impl.get();
     if (!s->post || !s->post->cfg.have_average) return fail(LFM_ESTATE, "averages not configured");
-    return lfm::post_average(s, n);
+    return lfm::post_launch(s, lfm::ForceJob{}, lfm::avg_job(s, n));
 }
 
 int lfm_post_average_fields(lfm_solver *h, int32_t n, double *pavg, double *prms) {
@@ -449,7 +472,7 @@ int lfm_post_forces(lfm_solver *h, double time) {
     if (!h) return fail(LFM_EINVAL, "null handle");
     Solver *s = h->impl.get();
     if (!s->post || !s->post->cfg.have_forces) return fail(LFM_ESTATE, "forces not configured");
-    return lfm::post_record(s, nullptr, time);
+    return lfm::post_record(s, false, time, lfm::AvgJob{});
 }
 
 int lfm_post_forces_read(lfm_solver *h, int32_t max_rows, double *rows, int32_t *n_rows) {

@@ -1029,7 +1029,8 @@ int lfm_get_info(lfm_solver *h, lfm_info *info) {
     if (!h || !info) return fail(LFM_EINVAL, "null argument");
     Solver *s = h->impl.get();
     // one wait for the stream's work and the scalars behind it
-    HIP_TRY(hipMemcpyAsync(s->h_scalar, s->d_scalar, 16 * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+    hipLaunchKernelGGL(lfm::export_scalars, dim3(1), dim3(64), 0, s->stream, s->d_scalar, 16, s->h_scalar);
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s->stream));
     info->dim = s->L.D;
     info->n_cells = s->L.nc;
@@ -1065,7 +1066,9 @@ int lfm_prepare_for_rkstep(lfm_solver *h, int rk) {
 
 int lfm_set_boundary_conditions(lfm_solver *h) {
     if (!h) return fail(LFM_EINVAL, "null handle");
-    h->impl->bc();
+    // the update kernel leaves the boundary ghosts as this fill would: it is
+    // launched after the state was set from outside
+    if (h->impl->ghosts_stale) h->impl->bc();
     h->impl->ghosts_stale = false;
     if (h->impl->post_forces) h->impl->post_snapshot();
     HIP_TRY(hipGetLastError());
@@ -1093,9 +1096,13 @@ int lfm_one_rk_step(lfm_solver *h, int rk, double dt, double *res) {
     if (rk < 0 || rk > 4) return fail(LFM_EINVAL, "rk stage out of range");
     if (!s->halo_ready()) return fail(LFM_ESTATE, "halo set-up not imported for every neighbour");
     const double B = s->B[rk];
-    s->h_scalar[0] = dt;
-    HIP_TRY(hipMemcpyAsync(s->d_dt_ptr(), s->h_scalar, sizeof(double), hipMemcpyHostToDevice, s->stream));
-    s->dt = dt;
+    // without adjustTimeStep nothing on the device writes its deltaT, which
+    // is then the last one that was copied there
+    if (s->prm.adjust_dt || !(dt == s->dt)) {
+        s->h_scalar[0] = dt;
+        HIP_TRY(hipMemcpyAsync(s->d_dt_ptr(), s->h_scalar, sizeof(double), hipMemcpyHostToDevice, s->stream));
+        s->dt = dt;
+    }
     const bool want_res = res && rk == 0 && s->prm.have_res;
     s->flux();
     s->update(s->pending_A, B, false, want_res, false);
@@ -1114,9 +1121,8 @@ int lfm_one_rk_step(lfm_solver *h, int rk, double dt, double *res) {
 int lfm_compute_dt(lfm_solver *h, double max_co, double *dt_out) {
     if (!h || !dt_out) return fail(LFM_EINVAL, "null argument");
     Solver *s = h->impl.get();
-    s->cfl_dt(0, max_co, s->d_dtmin, nullptr);
+    s->cfl_dt(0, max_co, s->d_dtmin, s->h_scalar + 9);  // pinned: the kernel writes it there as well
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(s->h_scalar + 9, s->d_dtmin, sizeof(double), hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
     *dt_out = s->h_scalar[9];
     return LFM_OK;
@@ -1125,9 +1131,8 @@ int lfm_compute_dt(lfm_solver *h, double max_co, double *dt_out) {
 int lfm_compute_cfl(lfm_solver *h, double dt, double *cfl_out) {
     if (!h || !cfl_out) return fail(LFM_EINVAL, "null argument");
     Solver *s = h->impl.get();
-    s->cfl_dt(1, dt, s->d_cfl, nullptr);
+    s->cfl_dt(1, dt, s->d_cfl, s->h_scalar + 8);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(s->h_scalar + 8, s->d_cfl, sizeof(double), hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
     *cfl_out = s->h_scalar[8];
     return LFM_OK;
