@@ -30,6 +30,8 @@ struct Batch {
     bool fused = false;
     int separate = 0;
     double A[5]{}, B[5]{};
+    bool drop_dq = false;  // the step being enqueued is followed by another one of its graph
+    int dq_mode(int rk) const { return (rk == 0 ? kDqZero : 0) | (drop_dq && rk == nstages - 1 ? kDqDrop : 0); }
     // one step, and kSteps of them for runs of many.  A graph launch costs
     // some 9 us beside its kernels, so the longer graph saves 8 us per step;
     // capturing it costs 0.6 (6 launches per step) to 1.3 ms (16), what it
@@ -64,10 +66,10 @@ static void enqueue_fused(Batch *b, int rk, int flip) {
     const dim3 blk(256);
     if (rk == b->nstages - 1)
         hipLaunchKernelGGL((stage_fused32_b<D, SOLVER, 1, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
-                           b->map_cells, (float)b->A[rk], (float)b->B[rk], rk == 0 ? 1 : 0, flip);
+                           b->map_cells, (float)b->A[rk], (float)b->B[rk], b->dq_mode(rk), flip);
     else
         hipLaunchKernelGGL((stage_fused32_b<D, SOLVER, -1, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
-                           b->map_cells, (float)b->A[rk], (float)b->B[rk], rk == 0 ? 1 : 0, flip);
+                           b->map_cells, (float)b->A[rk], (float)b->B[rk], b->dq_mode(rk), flip);
 }
 
 template <int D, bool V, bool NT>
@@ -101,10 +103,10 @@ static void enqueue_step_nt(Batch *b) {
         // the last stage's update also forms the step's compute_cfl partials
         if (rk == b->nstages - 1)
             hipLaunchKernelGGL((cell_update32_b<D, 1, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
-                               b->map_cells, (float)b->A[rk], (float)b->B[rk], rk == 0 ? 1 : 0);
+                               b->map_cells, (float)b->A[rk], (float)b->B[rk], b->dq_mode(rk));
         else
             hipLaunchKernelGGL((cell_update32_b<D, -1, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
-                               b->map_cells, (float)b->A[rk], (float)b->B[rk], rk == 0 ? 1 : 0);
+                               b->map_cells, (float)b->A[rk], (float)b->B[rk], b->dq_mode(rk));
     }
     hipLaunchKernelGGL(cfl_final32_b, dim3((unsigned)b->members.size()), blk, 0, b->stream, b->d_args);
 }
@@ -123,6 +125,7 @@ static hipError_t capture(Batch *b, int n, hipGraph_t *graph, hipGraphExec_t *ex
     hipError_t e = hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) {
         for (int i = 0; i < n; i++) {
+            b->drop_dq = i + 1 < n;
             if (b->D == 2)
                 b->visc ? enqueue_step<2, true>(b) : enqueue_step<2, false>(b);
             else

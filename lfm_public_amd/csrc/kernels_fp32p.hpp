@@ -912,20 +912,20 @@ __device__ __forceinline__ void face_flux32_body(const KArgs32 &a, const int f) 
 // stage: every component's load issued before any is used (a choice per
 // component compiles to a branch and a wait each)
 template <int D, bool NT>
-__device__ __forceinline__ void load_dq32(const KArgs32 &a, const int zero_dq, const int c, float (&dq)[D + 2]) {
+__device__ __forceinline__ void load_dq32(const KArgs32 &a, const int dq_mode, const int c, float (&dq)[D + 2]) {
 #pragma unroll
     for (int k = 0; k < D + 2; k++) dq[k] = 0.f;
-    if (!zero_dq) {
+    if (!(dq_mode & kDqZero)) {
 #pragma unroll
         for (int k = 0; k < D + 2; k++) dq[k] = ld_once<NT>(a.dq + (size_t)k * a.nc + c);
     }
 }
 
 // sponge, RK update and stores of one cell: q its state (the updated one on
-// return), dq its accumulated register
+// return), dq its accumulated register (drop: not stored)
 template <int D, bool NT>
-__device__ __forceinline__ void finish_cell32(const KArgs32 &a, const int c, const float dt, const float B, float *qout,
-                                              float (&q)[D + 2], float (&dq)[D + 2]) {
+__device__ __forceinline__ void finish_cell32(const KArgs32 &a, const int c, const float dt, const float B,
+                                              const bool drop, float *qout, float (&q)[D + 2], float (&dq)[D + 2]) {
     // sponge: sigma (q_inf - q) = -sigma q' (no sigma array, and no term,
     // where the case has no sponge layer and every sigma is zero)
     const float sgm = a.sigma ? ld_once<NT>(a.sigma + c) : 0.f;
@@ -933,8 +933,10 @@ __device__ __forceinline__ void finish_cell32(const KArgs32 &a, const int c, con
     for (int k = 0; k < D + 2; k++) {
         if (a.sigma) dq[k] -= dt * sgm * q[k];
         q[k] += B * dq[k];
-        st_once<NT>(a.dq + (size_t)k * a.nc + c, dq[k]);
     }
+    if (!drop)
+#pragma unroll
+        for (int k = 0; k < D + 2; k++) st_once<NT>(a.dq + (size_t)k * a.nc + c, dq[k]);
     store_q32<D, NT>(qout, a.ntot, c, q);
 }
 // boundary ghost g of a cell whose updated state is q, written for the next
@@ -953,13 +955,13 @@ __device__ __forceinline__ void refresh_ghost32(const KArgs32 &a, const int g, f
 // place, with the cell's boundary ghosts refreshed; res receives the
 // residual, q the updated state
 template <int D, bool RES, bool NT>
-__device__ __forceinline__ void cell_update32_cell(const KArgs32 &a, float A, float B, int zero_dq, const int c,
-                                                   float (&res)[D + 2], float (&q)[D + 2], float &vinv) {
+__device__ __forceinline__ void cell_update32_cell(const KArgs32 &a, float A, float B, int dq_mode, const bool drop,
+                                                   const int c, float (&res)[D + 2], float (&q)[D + 2], float &vinv) {
     const float dt = (float)(*a.dt);
     vinv = ld_once<NT>(a.vinv + c);
     const float sP = dt * vinv;
     float dq[D + 2];
-    load_dq32<D, NT>(a, zero_dq, c, dq);
+    load_dq32<D, NT>(a, dq_mode, c, dq);
 #pragma unroll
     for (int k = 0; k < D + 2; k++) res[k] = 0.f;
     load_q32<D>(a, c, q);
@@ -1005,7 +1007,7 @@ __device__ __forceinline__ void cell_update32_cell(const KArgs32 &a, float A, fl
             add(U + j, ent, true, f1);
         }
     }
-    finish_cell32<D, NT>(a, c, dt, B, a.q, q, dq);
+    finish_cell32<D, NT>(a, c, dt, B, drop, a.q, q, dq);
     // refresh this cell's boundary ghosts for the next stage
     for (unsigned m = gmask; m; m &= m - 1) {
         const int j = __builtin_ctz(m);
@@ -1026,7 +1028,7 @@ __device__ __forceinline__ double cfl_cell32(const KArgs32 &a, const FA &fa, con
 // or CFL).  CFL >= 0 (the last stage of a step): the step's compute_dt (0) /
 // compute_cfl (1) of the updated cells, per-block extrema into a.partial.
 template <int D, bool RES, int CFL, bool NT>
-__device__ __forceinline__ void cell_update32_body(const KArgs32 &a, float A, float B, int zero_dq, const int c,
+__device__ __forceinline__ void cell_update32_body(const KArgs32 &a, float A, float B, int dq_mode, const int c,
                                                    const int lblk, double cfl_param) {
     static_assert(!(RES && CFL >= 0), "the residual and the CFL share a.partial");
     __shared__ double red[256 / 64][D + 2];
@@ -1036,7 +1038,7 @@ __device__ __forceinline__ void cell_update32_body(const KArgs32 &a, float A, fl
     for (int k = 0; k < D + 2; k++) rsq[k] = 0.0;
     if (c < a.nc) {
         float res[D + 2], q[D + 2], vinv;
-        cell_update32_cell<D, RES, NT>(a, A, B, zero_dq, c, res, q, vinv);
+        cell_update32_cell<D, RES, NT>(a, A, B, dq_mode, CFL >= 0 && (dq_mode & kDqDrop), c, res, q, vinv);
         if constexpr (CFL >= 0) cv = cfl_cell32<D, CFL>(a, c, q, vinv, cfl_param);
         if (RES) {
 #pragma unroll
@@ -1217,8 +1219,8 @@ face_flux32(KArgs32 a) {
     face_flux32_body<D, SOLVER, VISC, STORED, NT>(a, LFM_TID(blockIdx.x));
 }
 template <int D, bool RES, int CFL, bool NT>
-__global__ void __launch_bounds__(256) cell_update32(KArgs32 a, float A, float B, int zero_dq, double cfl_param) {
-    cell_update32_body<D, RES, CFL, NT>(a, A, B, zero_dq, LFM_TID(blockIdx.x), LFM_BLK(), cfl_param);
+__global__ void __launch_bounds__(256) cell_update32(KArgs32 a, float A, float B, int dq_mode, double cfl_param) {
+    cell_update32_body<D, RES, CFL, NT>(a, A, B, dq_mode, LFM_TID(blockIdx.x), LFM_BLK(), cfl_param);
 }
 // ---------------------------------------------------------------------------
 // One RK stage in one launch for inviscid M1 / M2: each cell forms its faces'
@@ -1234,15 +1236,17 @@ __global__ void __launch_bounds__(256) cell_update32(KArgs32 a, float A, float B
 // its dependent loads.
 constexpr int kFusedGroup32 = 2;
 template <int D, int SOLVER, int CFL, bool PK, bool HALF, bool NT>
-__device__ __forceinline__ void stage32_body(const KArgs32 &a, float *qout, float A, float B, int zero_dq, const int c,
+__device__ __forceinline__ void stage32_body(const KArgs32 &a, float *qout, float A, float B, int dq_mode, const int c,
                                              const int lblk, double cfl_param) {
     constexpr int U = GatherUnroll<D>::value;
     constexpr int G = D == 3 ? kFusedGroup32 : U;
     using F = FaceOf32<D, PK, NT>;
-    // a face's own data are kept for the CFL/dt sums after the update; from
-    // the table they are read again
-    constexpr bool kKeep = CFL >= 0 && !PK;
+    // a face's own data, or its key where they come from the table, are kept
+    // for the CFL/dt sums after the update: read again they come from memory
+    // (4.1 M-cell box: 128 -> 105 us per launch)
+    constexpr bool kKeep = CFL >= 0 && !PK, kKeepKey = CFL >= 0 && PK && G < U;
     __shared__ float keep[kKeep ? U * D * 256 : 1];
+    __shared__ int keys[kKeepKey ? U * 256 : 1];
     double cv = CFL == 0 ? 100.0 : 0.0;
     if (c < a.nc) {
         int key[G];
@@ -1259,7 +1263,7 @@ __device__ __forceinline__ void stage32_body(const KArgs32 &a, float *qout, floa
         float qc[D + 2], dq[D + 2];
         load_q32<D>(a, c, qc);
         const float vinv = ld_once<NT>(a.vinv + c);
-        load_dq32<D, NT>(a, zero_dq, c, dq);
+        load_dq32<D, NT>(a, dq_mode, c, dq);
         const float dt = (float)(*a.dt);
         const Prim32<D> sc = prim32<D>(a, qc);
         const float s = dt * vinv;
@@ -1283,6 +1287,7 @@ __device__ __forceinline__ void stage32_body(const KArgs32 &a, float *qout, floa
                 f[u].load(a, j0 + u, c, key[u]);
                 load_q32<D>(a, f[u].other, qo[u]);
                 if (G < U) next[u] = F::load_key(a, j0 + G < U ? j0 + G + u : u, c);
+                if constexpr (kKeepKey) keys[(j0 + u) * 256 + threadIdx.x] = key[u];
                 if constexpr (kKeep)
 #pragma unroll
                     for (int k = 0; k < D; k++) keep[((j0 + u) * D + k) * 256 + threadIdx.x] = f[u].S[k];
@@ -1311,7 +1316,7 @@ __device__ __forceinline__ void stage32_body(const KArgs32 &a, float *qout, floa
         float q[D + 2];
 #pragma unroll
         for (int k = 0; k < D + 2; k++) q[k] = qc[k];
-        finish_cell32<D, NT>(a, c, dt, B, qout, q, dq);
+        finish_cell32<D, NT>(a, c, dt, B, CFL >= 0 && (dq_mode & kDqDrop), qout, q, dq);
         // the boundary ghosts of this cell (only cells of the boundary
         // submesh have any) for the next stage
         if (c < a.nsm0) {
@@ -1335,7 +1340,7 @@ __device__ __forceinline__ void stage32_body(const KArgs32 &a, float *qout, floa
                     for (int k = 0; k < D; k++) S[k] = keep[(j * D + k) * 256 + threadIdx.x];
                 } else {
                     F f;
-                    f.load(a, j, c, F::load_key(a, j, c));
+                    f.load(a, j, c, kKeepKey ? keys[j * 256 + threadIdx.x] : key[j % G]);
 #pragma unroll
                     for (int k = 0; k < D; k++) S[k] = f.S[k];
                 }
@@ -1398,7 +1403,7 @@ __global__ void __launch_bounds__(256) build_slots32(KArgs32 a, const uint16_t *
 // launch left in a.partial into *a.d_cfl (the final reduction of the
 // previous step, whose result no stage of this step reads).
 template <int D, int SOLVER, int CFL, bool PK, bool HALF, bool NT>
-__global__ void __launch_bounds__(256) stage_fused32(KArgs32 a, float *qout, float A, float B, int zero_dq,
+__global__ void __launch_bounds__(256) stage_fused32(KArgs32 a, float *qout, float A, float B, int dq_mode,
                                                      double cfl_param, int fin_nblk) {
     int nb = (int)gridDim.x;
     if constexpr (CFL < 0) {
@@ -1413,7 +1418,7 @@ __global__ void __launch_bounds__(256) stage_fused32(KArgs32 a, float *qout, flo
         (void)fin_nblk;
     }
     const int blk = xcd_block((int)blockIdx.x, nb);
-    stage32_body<D, SOLVER, CFL, PK, HALF, NT>(a, qout, A, B, zero_dq, blk * (int)blockDim.x + (int)threadIdx.x, blk,
+    stage32_body<D, SOLVER, CFL, PK, HALF, NT>(a, qout, A, B, dq_mode, blk * (int)blockDim.x + (int)threadIdx.x, blk,
                                            cfl_param);
 }
 template <int D, int MODE>
@@ -1477,17 +1482,17 @@ __global__ void __launch_bounds__(256) face_flux32_b(const KArgs32 *args, BatchM
 // CFL 1: the last stage, with compute_cfl at each solver's own deltaT
 template <int D, int CFL, bool NT>
 __global__ void __launch_bounds__(256) cell_update32_b(const KArgs32 *args, BatchMap m, float A, float B,
-                                                       int zero_dq) {
+                                                       int dq_mode) {
     int r, lb;
     batch_slot(m, r, lb);
     const KArgs32 &a = args[r];
-    cell_update32_body<D, false, CFL, NT>(a, A, B, zero_dq, lb * 256 + threadIdx.x, lb, CFL >= 0 ? *a.dt : 0.0);
+    cell_update32_body<D, false, CFL, NT>(a, A, B, dq_mode, lb * 256 + threadIdx.x, lb, CFL >= 0 ? *a.dt : 0.0);
 }
 // one-launch stage over a batch (inviscid M1 / M2), each member from one
 // of its state buffers into the other: flip 0 from a.q into a.q_alt, flip 1
 // back
 template <int D, int SOLVER, int CFL, bool NT>
-__global__ void __launch_bounds__(256) stage_fused32_b(const KArgs32 *args, BatchMap m, float A, float B, int zero_dq,
+__global__ void __launch_bounds__(256) stage_fused32_b(const KArgs32 *args, BatchMap m, float A, float B, int dq_mode,
                                                        int flip) {
     int r, lb;
     batch_slot(m, r, lb);
@@ -1498,9 +1503,9 @@ __global__ void __launch_bounds__(256) stage_fused32_b(const KArgs32 *args, Batc
     const double dt = CFL >= 0 ? *a.dt : 0.0;
     // members may hold either slot form
     if (a.pk)
-        stage32_body<D, SOLVER, CFL, true, false, NT>(a, qout, A, B, zero_dq, c, lb, dt);
+        stage32_body<D, SOLVER, CFL, true, false, NT>(a, qout, A, B, dq_mode, c, lb, dt);
     else
-        stage32_body<D, SOLVER, CFL, false, false, NT>(a, qout, A, B, zero_dq, c, lb, dt);
+        stage32_body<D, SOLVER, CFL, false, false, NT>(a, qout, A, B, dq_mode, c, lb, dt);
 }
 // one block per solver: max of its partials into its CFL scalar
 static __global__ void __launch_bounds__(256) cfl_final32_b(const KArgs32 *args) {
@@ -1530,7 +1535,7 @@ void launch_gradvis32(Solver *s, bool full, bool fin = false);
 template <int D>
 void launch_flux32(Solver *s);
 template <int D>
-void launch_update32(Solver *s, double A, double B, bool zero_dq, bool res, bool accumulate_res,
+void launch_update32(Solver *s, double A, double B, int dq_mode, bool res, bool accumulate_res,
                      const Solver::CflJob *cfl);
 template <int D>
 void launch_cfl_dt32(Solver *s, int mode, double param, double *out, double *dt_dst);
@@ -1538,7 +1543,7 @@ template <int D>
 void launch_build_slots32(Solver *s, const uint16_t *face_rec, int none, uint32_t *pk, int32_t *nb, float *S,
                           float *w);
 template <int D>
-void launch_stage_fused32(Solver *s, double A, double B, bool zero_dq, const float *qin, float *qout,
+void launch_stage_fused32(Solver *s, double A, double B, int dq_mode, const float *qin, float *qout,
                           const Solver::CflJob *cfl, bool fin);
 
 }  // namespace lfm

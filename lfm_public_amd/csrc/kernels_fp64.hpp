@@ -1150,14 +1150,20 @@ __device__ __forceinline__ void block_extremum(double v, double *dst) {
     }
 }
 
+// How a stage treats the RK register: zero before it (a step's first stage),
+// and not stored after it (the last stage of a step that another follows in the
+// same call: nothing reads it before that step starts from zero; 20 of 108 B per
+// 3D FP32 cell and stage).  Looked at only by the launches that form the CFL as
+// well, which a step's last stage is: the choice costs 0.1 us.
+constexpr int kDqZero = 1, kDqDrop = 2;
 // the cell's RK register as the last stage left it, zero at a step's first
 // stage: every component's load issued before any is used (a choice per
 // component compiles to a branch and a wait each)
 template <int D, bool NT>
-__device__ __forceinline__ void load_dq64(const KArgs &a, const int zero_dq, const int c, double (&dq)[D + 2]) {
+__device__ __forceinline__ void load_dq64(const KArgs &a, const int dq_mode, const int c, double (&dq)[D + 2]) {
 #pragma unroll
     for (int k = 0; k < D + 2; k++) dq[k] = 0.0;
-    if (!zero_dq) {
+    if (!(dq_mode & kDqZero)) {
 #pragma unroll
         for (int k = 0; k < D + 2; k++) dq[k] = ld_once<NT>(a.dq + (size_t)k * a.nc + c);
     }
@@ -1176,13 +1182,13 @@ __device__ __forceinline__ void sponge64(const KArgs &a, const int c, const doub
 
 // ---------------------------------------------------------------------------
 // Residual gather, sponge, RK update (cfd_v0.cpp:2792-2822).  dq starts from
-// A_rk * dq (prepare_for_RKstep); zero_dq replaces it by 0 for the first
+// A_rk * dq (prepare_for_RKstep); dq_mode replaces it by 0 for the first
 // stage of a step (prepare_for_timestep zeroed it).  CFL >= 0 (the last
 // stage of a step): the step's compute_dt (0) / compute_cfl (1) of the
 // updated cells, per-block extrema into a.partial.
 // ---------------------------------------------------------------------------
 template <int D, bool RES, int CFL, bool NT>
-__global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, int zero_dq, double cfl_param) {
+__global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, int dq_mode, double cfl_param) {
     static_assert(!(RES && CFL >= 0), "the residual and the CFL share a.partial");
     const int c = LFM_TID(blockIdx.x);
     __shared__ double red[256 / 64][D + 2];
@@ -1194,7 +1200,7 @@ __global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, 
         const double dt = *a.dt;
         const double vinv = ld_once<NT>(a.vinv + c);
         double dq[D + 2], res[D + 2], q[D + 2];
-        load_dq64<D, NT>(a, zero_dq, c, dq);
+        load_dq64<D, NT>(a, dq_mode, c, dq);
 #pragma unroll
         for (int k = 0; k < D + 2; k++) res[k] = 0.0;
         load_q<D>(a, c, q);
@@ -1241,11 +1247,11 @@ __global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, 
         }
         if (a.sigma) sponge64<D, NT>(a, c, dt, q, dq);
 #pragma unroll
-        for (int k = 0; k < D + 2; k++) {
-            q[k] += B * dq[k];
-            st_once<NT>(a.dq + (size_t)k * a.nc + c, dq[k]);
-        }
+        for (int k = 0; k < D + 2; k++) q[k] += B * dq[k];
         store_q<D, NT>(a.q, a.ntot, c, q);
+        if (CFL < 0 || !(dq_mode & kDqDrop))
+#pragma unroll
+            for (int k = 0; k < D + 2; k++) st_once<NT>(a.dq + (size_t)k * a.nc + c, dq[k]);
         // refresh this cell's boundary ghosts for the next stage
         for (unsigned m = gmask; m; m &= m - 1) {
             const int j = __builtin_ctz(m);
@@ -1481,7 +1487,7 @@ __device__ __forceinline__ double cfl_term64(const double (&q)[D + 2], const dou
 // stage left in a.partial into *fin_out.
 // SYM: every face's weights allow flux_m1_sym.
 template <int D, int SOLVER, int CFL, bool PK, bool SYM, bool NT>
-__global__ void __launch_bounds__(256) stage_fused64(KArgs a, double *qout, double A, double B, int zero_dq,
+__global__ void __launch_bounds__(256) stage_fused64(KArgs a, double *qout, double A, double B, int dq_mode,
                                                      double cfl_param, int fin_nblk, double *fin_out) {
     int nb = (int)gridDim.x;
     if constexpr (CFL < 0) {
@@ -1500,6 +1506,10 @@ __global__ void __launch_bounds__(256) stage_fused64(KArgs a, double *qout, doub
     double cv = CFL == 0 ? 100.0 : 0.0;
     // the CFL/dt terms of a cell's faces in slot order (own thread only)
     __shared__ double terms[CFL >= 0 ? kMaxFaces * 256 : 1];
+    // and in 3D its keys, kept for them: read again they come from memory (1.4
+    // M-cell box: 89 -> 85 us per launch; in 2D it gains nothing)
+    constexpr bool kKeepKey = CFL >= 0 && D == 3;
+    __shared__ int keys[kKeepKey ? GatherUnroll<D>::value * 256 : 1];
     if (c < a.nc) {
         constexpr int G = kFusedGroup64;
         int key[G];
@@ -1508,7 +1518,7 @@ __global__ void __launch_bounds__(256) stage_fused64(KArgs a, double *qout, doub
         double qc[D + 2], dq[D + 2];
         load_q<D>(a, c, qc);
         const double vinv = ld_once<NT>(a.vinv + c);
-        load_dq64<D, NT>(a, zero_dq, c, dq);
+        load_dq64<D, NT>(a, dq_mode, c, dq);
         const double dt = *a.dt;
         const Prim64<D> sc = prim64<D, SOLVER>(a, qc);
         unsigned gmask = 0;  // bit j: slot j leads to a boundary ghost
@@ -1522,6 +1532,7 @@ __global__ void __launch_bounds__(256) stage_fused64(KArgs a, double *qout, doub
             int next[G];
 #pragma unroll
             for (int u = 0; u < G; u++) {
+                if constexpr (kKeepKey) keys[(j0 + u) * 256 + threadIdx.x] = key[u];
                 f[u].load(a, j0 + u, c, key[u]);
                 load_q<D>(a, f[u].other, qo[u]);
                 next[u] = F::load_key(a, j0 + G < U ? j0 + G + u : u, c);
@@ -1561,11 +1572,11 @@ __global__ void __launch_bounds__(256) stage_fused64(KArgs a, double *qout, doub
         for (int k = 0; k < D + 2; k++) q[k] = qc[k];
         if (a.sigma) sponge64<D, NT>(a, c, dt, q, dq);
 #pragma unroll
-        for (int k = 0; k < D + 2; k++) {
-            q[k] += B * dq[k];
-            st_once<NT>(a.dq + (size_t)k * a.nc + c, dq[k]);
-        }
+        for (int k = 0; k < D + 2; k++) q[k] += B * dq[k];
         store_q<D, NT>(qout, a.ntot, c, q);
+        if (CFL < 0 || !(dq_mode & kDqDrop))
+#pragma unroll
+            for (int k = 0; k < D + 2; k++) st_once<NT>(a.dq + (size_t)k * a.nc + c, dq[k]);
         // this cell's boundary ghosts for the next stage
         for (unsigned m = gmask; m; m &= m - 1) {
             const int j = __builtin_ctz(m);
@@ -1584,7 +1595,7 @@ __global__ void __launch_bounds__(256) stage_fused64(KArgs a, double *qout, doub
 #pragma unroll
             for (int j = 0; j < U; j++) {
                 F f;
-                f.load(a, j, c, F::load_key(a, j, c));
+                f.load(a, j, c, kKeepKey ? keys[j * 256 + threadIdx.x] : F::load_key(a, j, c));
                 if (f.other != c)
                     terms[((perm >> (3 * j)) & 7) * 256 + threadIdx.x] = cfl_term64<D, CFL>(q, f.S, f.Sm);
             }
@@ -1596,7 +1607,7 @@ __global__ void __launch_bounds__(256) stage_fused64(KArgs a, double *qout, doub
             const int n = (perm >> 18) & 7;
             double sum = 0.0;
             for (int j = 0; j < n; j++) sum += terms[j * 256 + threadIdx.x];
-            cv = cfl_value64<D, CFL>(q[0], a.vinv[c], sum, cfl_param);
+            cv = cfl_value64<D, CFL>(q[0], vinv, sum, cfl_param);
         }
     }
     if constexpr (CFL >= 0) block_extremum<CFL>(cv, a.partial + blk);

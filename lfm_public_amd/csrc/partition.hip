@@ -324,6 +324,7 @@ int lfm_part_group_run(lfm_part_group *g, int nsteps) {
     int rc = exchange(g, LFM_HALO_SOLVARS);  // halo ghosts hold the current state
     const int nst = g->parts[0]->nstages;
     for (int it = 0; it < nsteps && !rc; it++) {
+        for (Solver *p : g->parts) p->drop_dq = it + 1 < nsteps;
         for (int rk = 0; rk < nst && !rc; rk++) {
             for (Solver *p : g->parts) p->stage_a(rk);
             rc = exchange(g, LFM_HALO_VISCOUS);
@@ -340,6 +341,7 @@ int lfm_part_group_run(lfm_part_group *g, int nsteps) {
     hipError_t e = hipEventRecord(g->done, g->stream);
     for (int p = 0; p < n; p++) {
         g->parts[p]->stream = own[p];
+        g->parts[p]->drop_dq = false;
         if (e == hipSuccess) e = hipStreamWaitEvent(own[p], g->done, 0);
     }
     if (rc) return rc;

@@ -295,31 +295,31 @@ static void launch_flux64(Solver *s) {
 }
 
 template <int D, bool NT>
-static void launch_update64_nt(Solver *s, double A, double B, bool zero_dq, bool res, bool accumulate_res,
+static void launch_update64_nt(Solver *s, double A, double B, int dq_mode, bool res, bool accumulate_res,
                                const Solver::CflJob *cfl) {
     const int nb = nblocks(s->L.nc);
     if (res) {
         hipLaunchKernelGGL((cell_update<D, true, -1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
-                           (int)zero_dq, 0.0);
+                           dq_mode, 0.0);
         hipLaunchKernelGGL(reduce_sum, dim3(1), dim3(kBlock), 0, s->stream, s->k64.partial, nb, D + 2, s->d_res,
                            (int)accumulate_res);
     } else if (cfl && cfl->mode == 0) {
         hipLaunchKernelGGL((cell_update<D, false, 0, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
-                           (int)zero_dq, cfl->param);
+                           dq_mode, cfl->param);
     } else if (cfl) {
         hipLaunchKernelGGL((cell_update<D, false, 1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
-                           (int)zero_dq, cfl->param);
+                           dq_mode, cfl->param);
     } else {
         hipLaunchKernelGGL((cell_update<D, false, -1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
-                           (int)zero_dq, 0.0);
+                           dq_mode, 0.0);
     }
 }
 
 template <int D>
-static void launch_update64(Solver *s, double A, double B, bool zero_dq, bool res, bool accumulate_res,
+static void launch_update64(Solver *s, double A, double B, int dq_mode, bool res, bool accumulate_res,
                             const Solver::CflJob *cfl) {
-    s->stream_nt ? launch_update64_nt<D, true>(s, A, B, zero_dq, res, accumulate_res, cfl)
-                 : launch_update64_nt<D, false>(s, A, B, zero_dq, res, accumulate_res, cfl);
+    s->stream_nt ? launch_update64_nt<D, true>(s, A, B, dq_mode, res, accumulate_res, cfl)
+                 : launch_update64_nt<D, false>(s, A, B, dq_mode, res, accumulate_res, cfl);
 }
 
 template <int D>
@@ -345,42 +345,42 @@ int integrals64(Solver *s, double *out_dev) {
 }
 
 template <int D, int SOLVER, bool PK, bool SYM, bool NT>
-static void launch_fused64_nt(Solver *s, double A, double B, int zero_dq, const KArgs &a, double *qout,
+static void launch_fused64_nt(Solver *s, double A, double B, int dq_mode, const KArgs &a, double *qout,
                              const Solver::CflJob *cfl, bool fin) {
     const int nb = nblocks(s->L.nc);
     if (!cfl)
         hipLaunchKernelGGL((stage_fused64<D, SOLVER, -1, PK, SYM, NT>), dim3(nb + (fin ? 1 : 0)), dim3(kBlock), 0, s->stream, a,
-                           qout, A, B, zero_dq, 0.0, fin ? nb : 0, s->d_cfl);
+                           qout, A, B, dq_mode, 0.0, fin ? nb : 0, s->d_cfl);
     else if (cfl->mode == 0)
         hipLaunchKernelGGL((stage_fused64<D, SOLVER, 0, PK, SYM, NT>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
-                           zero_dq, cfl->param, 0, s->d_cfl);
+                           dq_mode, cfl->param, 0, s->d_cfl);
     else
         hipLaunchKernelGGL((stage_fused64<D, SOLVER, 1, PK, SYM, NT>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
-                           zero_dq, cfl->param, 0, s->d_cfl);
+                           dq_mode, cfl->param, 0, s->d_cfl);
 }
 
 template <int D, int SOLVER, bool PK, bool SYM>
-static void launch_fused64_v(Solver *s, double A, double B, int zero_dq, const KArgs &a, double *qout,
+static void launch_fused64_v(Solver *s, double A, double B, int dq_mode, const KArgs &a, double *qout,
                              const Solver::CflJob *cfl, bool fin) {
-    s->stream_nt ? launch_fused64_nt<D, SOLVER, PK, SYM, true>(s, A, B, zero_dq, a, qout, cfl, fin)
-                 : launch_fused64_nt<D, SOLVER, PK, SYM, false>(s, A, B, zero_dq, a, qout, cfl, fin);
+    s->stream_nt ? launch_fused64_nt<D, SOLVER, PK, SYM, true>(s, A, B, dq_mode, a, qout, cfl, fin)
+                 : launch_fused64_nt<D, SOLVER, PK, SYM, false>(s, A, B, dq_mode, a, qout, cfl, fin);
 }
 
 // fin: the launch also reduces the previous step's CFL maxima (left in
 // a.partial) into d_cfl, in one extra block
 template <int D>
-static void launch_stage_fused64(Solver *s, double A, double B, bool zero_dq, const double *qin, double *qout,
+static void launch_stage_fused64(Solver *s, double A, double B, int dq_mode, const double *qin, double *qout,
                                  const Solver::CflJob *cfl, bool fin) {
     KArgs a = s->k64;
     a.q = const_cast<double *>(qin);
     if (s->prm.solver == 1)
-        a.pk ? launch_fused64_v<D, 1, true, false>(s, A, B, zero_dq, a, qout, cfl, fin)
-             : launch_fused64_v<D, 1, false, false>(s, A, B, zero_dq, a, qout, cfl, fin);
+        a.pk ? launch_fused64_v<D, 1, true, false>(s, A, B, dq_mode, a, qout, cfl, fin)
+             : launch_fused64_v<D, 1, false, false>(s, A, B, dq_mode, a, qout, cfl, fin);
     else if (a.pk)
-        s->sym64 ? launch_fused64_v<D, 0, true, true>(s, A, B, zero_dq, a, qout, cfl, fin)
-                 : launch_fused64_v<D, 0, true, false>(s, A, B, zero_dq, a, qout, cfl, fin);
+        s->sym64 ? launch_fused64_v<D, 0, true, true>(s, A, B, dq_mode, a, qout, cfl, fin)
+                 : launch_fused64_v<D, 0, true, false>(s, A, B, dq_mode, a, qout, cfl, fin);
     else
-        launch_fused64_v<D, 0, false, false>(s, A, B, zero_dq, a, qout, cfl, fin);
+        launch_fused64_v<D, 0, false, false>(s, A, B, dq_mode, a, qout, cfl, fin);
 }
 
 // dispatch helpers over dimension
@@ -420,13 +420,13 @@ void Solver::flux() {
     }
 }
 
-void Solver::update(double A, double B, bool zero_dq, bool res, bool accumulate_res, const CflJob *cfl) {
+void Solver::update(double A, double B, int dq_mode, bool res, bool accumulate_res, const CflJob *cfl) {
     if (fp32) {
-        LFM_DISPATCH_D(this, launch_update32<2>(this, A, B, zero_dq, res, accumulate_res, cfl),
-                       launch_update32<3>(this, A, B, zero_dq, res, accumulate_res, cfl));
+        LFM_DISPATCH_D(this, launch_update32<2>(this, A, B, dq_mode, res, accumulate_res, cfl),
+                       launch_update32<3>(this, A, B, dq_mode, res, accumulate_res, cfl));
     } else {
-        LFM_DISPATCH_D(this, launch_update64<2>(this, A, B, zero_dq, res, accumulate_res, cfl),
-                       launch_update64<3>(this, A, B, zero_dq, res, accumulate_res, cfl));
+        LFM_DISPATCH_D(this, launch_update64<2>(this, A, B, dq_mode, res, accumulate_res, cfl),
+                       launch_update64<3>(this, A, B, dq_mode, res, accumulate_res, cfl));
     }
 }
 
@@ -498,13 +498,13 @@ void Solver::stage_b(int rk, bool fuse_cfl, bool own_dt) {
     if (fuse_cfl && rk == nstages - 1 && !res && (fp32 || L.D == 2)) {
         const CflJob job = cfl_job(own_dt);
         prof_mark(5, true);
-        update(A[rk], B[rk], rk == 0, false, false, &job);
+        update(A[rk], B[rk], dq_mode(rk), false, false, &job);
         prof_mark(5, false);
         final_or_carry(job);
         cfl_fused = true;
     } else {
         prof_mark(3, true);
-        update(A[rk], B[rk], rk == 0, res, false);
+        update(A[rk], B[rk], dq_mode(rk), res, false);
         prof_mark(3, false);
     }
 }
@@ -757,13 +757,13 @@ void Solver::stage_fused(int rk, bool from_alt) {
     auto launch = [&](const CflJob *job, bool fin) {
         if (!fp32) {
             double *qin = from_alt ? q_alt64 : k64.q, *qout = from_alt ? k64.q : q_alt64;
-            LFM_DISPATCH_D(this, launch_stage_fused64<2>(this, A[rk], B[rk], rk == 0, qin, qout, job, fin),
-                           launch_stage_fused64<3>(this, A[rk], B[rk], rk == 0, qin, qout, job, fin));
+            LFM_DISPATCH_D(this, launch_stage_fused64<2>(this, A[rk], B[rk], dq_mode(rk), qin, qout, job, fin),
+                           launch_stage_fused64<3>(this, A[rk], B[rk], dq_mode(rk), qin, qout, job, fin));
             return;
         }
         float *qin = from_alt ? q_alt32 : k32->q, *qout = from_alt ? k32->q : q_alt32;
-        LFM_DISPATCH_D(this, launch_stage_fused32<2>(this, A[rk], B[rk], rk == 0, qin, qout, job, fin),
-                       launch_stage_fused32<3>(this, A[rk], B[rk], rk == 0, qin, qout, job, fin));
+        LFM_DISPATCH_D(this, launch_stage_fused32<2>(this, A[rk], B[rk], dq_mode(rk), qin, qout, job, fin),
+                       launch_stage_fused32<3>(this, A[rk], B[rk], dq_mode(rk), qin, qout, job, fin));
     };
     if (rk == nstages - 1) {
         const CflJob job = cfl_job(true);
@@ -902,7 +902,7 @@ bool Solver::graph_capture() {
     hipError_t e = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) {
         const int64_t done = steps_done;
-        defer_cfl = true;
+        defer_cfl = drop_dq = true;
         for (int i = 0; i < kGraphSteps; i++) step();
         steps_done = done;
         e = hipStreamEndCapture(stream, &g->graph);
@@ -932,10 +932,14 @@ int Solver::run_steps(int n, bool with_post) {
             continue;
         }
         defer_cfl = i + 1 < n && !(with_post && post);
+        drop_dq = i + 1 < n;
         step();
         if (with_post && post) {
             const int rc = post_step();
-            if (rc) return rc;
+            if (rc) {
+                drop_dq = false;
+                return rc;
+            }
         }
         i++;
     }
@@ -1105,7 +1109,7 @@ int lfm_one_rk_step(lfm_solver *h, int rk, double dt, double *res) {
     }
     const bool want_res = res && rk == 0 && s->prm.have_res;
     s->flux();
-    s->update(s->pending_A, B, false, want_res, false);
+    s->update(s->pending_A, B, 0, want_res, false);
     s->pending_A = 1.0;
     HIP_TRY(hipGetLastError());
     if (want_res) {

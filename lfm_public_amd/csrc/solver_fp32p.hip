@@ -245,66 +245,66 @@ void launch_flux32(Solver *s) {
 }
 
 template <int D, bool NT>
-static void launch_update32_nt(Solver *s, double A, double B, bool zero_dq, bool res, bool accumulate_res,
+static void launch_update32_nt(Solver *s, double A, double B, int dq_mode, bool res, bool accumulate_res,
                                const Solver::CflJob *cfl) {
     const int nb = nblocks(s->L.nc);
     if (res) {
         hipLaunchKernelGGL((cell_update32<D, true, -1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
-                           (float)B, (int)zero_dq, 0.0);
+                           (float)B, dq_mode, 0.0);
         hipLaunchKernelGGL(reduce_sum, dim3(1), dim3(kBlock), 0, s->stream, s->k32->partial, nb, D + 2, s->d_res,
                            (int)accumulate_res);
     } else if (cfl && cfl->mode == 0) {
         hipLaunchKernelGGL((cell_update32<D, false, 0, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
-                           (float)B, (int)zero_dq, cfl->param);
+                           (float)B, dq_mode, cfl->param);
     } else if (cfl) {
         hipLaunchKernelGGL((cell_update32<D, false, 1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
-                           (float)B, (int)zero_dq, cfl->param);
+                           (float)B, dq_mode, cfl->param);
     } else {
         hipLaunchKernelGGL((cell_update32<D, false, -1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
-                           (float)B, (int)zero_dq, 0.0);
+                           (float)B, dq_mode, 0.0);
     }
 }
 
 template <int D>
-void launch_update32(Solver *s, double A, double B, bool zero_dq, bool res, bool accumulate_res,
+void launch_update32(Solver *s, double A, double B, int dq_mode, bool res, bool accumulate_res,
                      const Solver::CflJob *cfl) {
-    s->stream_nt ? launch_update32_nt<D, true>(s, A, B, zero_dq, res, accumulate_res, cfl)
-                 : launch_update32_nt<D, false>(s, A, B, zero_dq, res, accumulate_res, cfl);
+    s->stream_nt ? launch_update32_nt<D, true>(s, A, B, dq_mode, res, accumulate_res, cfl)
+                 : launch_update32_nt<D, false>(s, A, B, dq_mode, res, accumulate_res, cfl);
 }
 
 // fin: one block more reduces the CFL maxima of the previous step's last
 // stage (left in a.partial) into a.d_cfl
 template <int D, int SOLVER, bool PK, bool HALF, bool NT>
-static void launch_fused32_nt(Solver *s, float A, float B, int zero_dq, const KArgs32 &a, float *qout,
+static void launch_fused32_nt(Solver *s, float A, float B, int dq_mode, const KArgs32 &a, float *qout,
                              const Solver::CflJob *cfl, bool fin) {
     const int nb = nblocks(s->L.nc);
     if (!cfl) {
         hipLaunchKernelGGL((stage_fused32<D, SOLVER, -1, PK, HALF, NT>), dim3(nb + (fin ? 1 : 0)), dim3(kBlock), 0, s->stream, a,
-                           qout, A, B, zero_dq, 0.0, fin ? nb : 0);
+                           qout, A, B, dq_mode, 0.0, fin ? nb : 0);
         return;
     }
     if (cfl->mode == 0)
         hipLaunchKernelGGL((stage_fused32<D, SOLVER, 0, PK, HALF, NT>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
-                           zero_dq, cfl->param, 0);
+                           dq_mode, cfl->param, 0);
     else
         hipLaunchKernelGGL((stage_fused32<D, SOLVER, 1, PK, HALF, NT>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
-                           zero_dq, cfl->param, 0);
+                           dq_mode, cfl->param, 0);
 }
 
 template <int D, int SOLVER, bool PK, bool HALF>
-static void launch_fused32_v(Solver *s, float A, float B, int zero_dq, const KArgs32 &a, float *qout,
+static void launch_fused32_v(Solver *s, float A, float B, int dq_mode, const KArgs32 &a, float *qout,
                              const Solver::CflJob *cfl, bool fin) {
-    s->stream_nt ? launch_fused32_nt<D, SOLVER, PK, HALF, true>(s, A, B, zero_dq, a, qout, cfl, fin)
-                 : launch_fused32_nt<D, SOLVER, PK, HALF, false>(s, A, B, zero_dq, a, qout, cfl, fin);
+    s->stream_nt ? launch_fused32_nt<D, SOLVER, PK, HALF, true>(s, A, B, dq_mode, a, qout, cfl, fin)
+                 : launch_fused32_nt<D, SOLVER, PK, HALF, false>(s, A, B, dq_mode, a, qout, cfl, fin);
 }
 
 template <int D>
-void launch_stage_fused32(Solver *s, double A, double B, bool zero_dq, const float *qin, float *qout,
+void launch_stage_fused32(Solver *s, double A, double B, int dq_mode, const float *qin, float *qout,
                           const Solver::CflJob *cfl, bool fin) {
     KArgs32 a = *s->k32;
     a.q = const_cast<float *>(qin);
     const float fA = (float)A, fB = (float)B;
-    const int z = (int)zero_dq;
+    const int z = dq_mode;
     if (s->prm.solver == 1)
         a.pk ? launch_fused32_v<D, 1, true, true>(s, fA, fB, z, a, qout, cfl, fin)
              : launch_fused32_v<D, 1, false, true>(s, fA, fB, z, a, qout, cfl, fin);
@@ -436,11 +436,11 @@ template void launch_gradvis32<2>(Solver *, bool, bool);
 template void launch_gradvis32<3>(Solver *, bool, bool);
 template void launch_flux32<2>(Solver *);
 template void launch_flux32<3>(Solver *);
-template void launch_update32<2>(Solver *, double, double, bool, bool, bool, const Solver::CflJob *);
-template void launch_update32<3>(Solver *, double, double, bool, bool, bool, const Solver::CflJob *);
-template void launch_stage_fused32<2>(Solver *, double, double, bool, const float *, float *,
+template void launch_update32<2>(Solver *, double, double, int, bool, bool, const Solver::CflJob *);
+template void launch_update32<3>(Solver *, double, double, int, bool, bool, const Solver::CflJob *);
+template void launch_stage_fused32<2>(Solver *, double, double, int, const float *, float *,
                                      const Solver::CflJob *, bool);
-template void launch_stage_fused32<3>(Solver *, double, double, bool, const float *, float *,
+template void launch_stage_fused32<3>(Solver *, double, double, int, const float *, float *,
                                      const Solver::CflJob *, bool);
 template void launch_build_slots32<2>(Solver *, const uint16_t *, int, uint32_t *, int32_t *, float *, float *);
 template void launch_build_slots32<3>(Solver *, const uint16_t *, int, uint32_t *, int32_t *, float *, float *);

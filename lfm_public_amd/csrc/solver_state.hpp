@@ -149,7 +149,7 @@ struct Solver {
     void flux();
     // cfl: the update also forms that reduction from the updated cells (it
     // reads only a cell's own state and its faces' areas); not with res
-    void update(double A, double B, bool zero_dq, bool res, bool accumulate_res, const CflJob *cfl = nullptr);
+    void update(double A, double B, int dq_mode, bool res, bool accumulate_res, const CflJob *cfl = nullptr);
     void cfl_dt(int mode, double param, double *out, double *dt_dst);
     // the final single-block reduction after an update that formed the
     // block extrema of a CFL job
@@ -207,6 +207,9 @@ struct Solver {
     bool defer_cfl = false;
     bool cfl_pending = false;
     int carry_target() const;
+    // the step is followed by another one in the same call
+    bool drop_dq = false;
+    int dq_mode(int rk) const { return (rk == 0 ? kDqZero : 0) | (drop_dq && rk == nstages - 1 ? kDqDrop : 0); }
     void final_or_carry(const CflJob &job);
     void flush_cfl();
     void end_step(bool own_dt);
