@@ -31,8 +31,8 @@ struct KArgs32 {
     const float *S;  // [nf][D]: a face's area vector as one record
     const float *d, *w;
     const int32_t *g_off, *g_ent;
-    // each cell's first GatherUnroll gather entries and (2D) the cells they
-    // lead to (key_at places them; kNoFace and the cell itself past its last)
+    // each cell's first GatherUnroll gather entries and the cells they lead to
+    // (key_at places them; kNoFace and the cell itself past its last)
     const int32_t *g_key, *g_oth;
     const int32_t *ghost_cell, *ghost_role;
     const float *vinv;
@@ -398,7 +398,7 @@ struct FaceOf32 {
 
 // Green-Gauss sums of one cell over its faces in gather order; returns the
 // cell's own primitive state.  SL: every entry from the slots (3D); otherwise
-// from the gather list.  Each face's sums sit in a branch of their own: in one
+// through the gather entries.  Each face's sums sit in a branch of their own: in one
 // block the compiler interleaves all six faces' arithmetic (124 VGPRs instead
 // of 96, 4 waves per SIMD instead of 5).
 template <int D, int GRAD, bool VISC, bool SL, bool PK, bool NT>
@@ -463,24 +463,16 @@ __device__ __forceinline__ Prim32<D> grad32_sums(const KArgs32 &a, const int c, 
     // slower: O-grid gradients 0.97 -> 1.54 ms per step with three, 1.89 with
     // two.
     int e0 = 0, ne = U, key[U], oth[U];
-    if constexpr (D == 2) {
-        load_keys<D, NT>(a.g_key, a.nc, 0, c, key);
-        load_keys<D, NT>(a.g_oth, a.nc, 0, c, oth);
-    } else {
-        load_keys<D, NT>(a.g_key, a.nc, 0, c, key);
-    }
+    load_keys<D, NT>(a.g_key, a.nc, 0, c, key);
+    load_keys<D, NT>(a.g_oth, a.nc, 0, c, oth);
     if (a.more_faces) {
         e0 = a.g_off[c];
         ne = a.g_off[c + 1] - e0;
     }
 #pragma unroll
     for (int j = 0; j < U; j++) {
-        if constexpr (D == 2) {
-            f[j].load_face(a, key[j]);
-            f[j].other = oth[j];
-        } else {
-            f[j].load_list(a, key[j]);
-        }
+        f[j].load_face(a, key[j]);
+        f[j].other = oth[j];
         load_q32<D>(a, f[j].other, qo[j]);
     }
 #pragma unroll

@@ -614,7 +614,7 @@ void Solver::size_stage() {
     } else {
         // face fluxes, S, d, w, both cells; gather entries
         b += nf * ((3 * D + 3) * w + 2 * sizeof(int32_t)) + keys;
-        if (grads && !(fp32 && D == 3)) b += keys;  // the cells they lead to
+        if (grads && !(fp32 && D == 3)) b += keys;  // the cells they lead to (3D FP32: the slots below)
     }
     if (grads) b += nc * (size_t)(fp32 ? k32->gstride : k64.gstride) * w;
     if (grads && fp32 && D == 3) b += nc * GatherUnroll<3>::value * (sizeof(int32_t) + (D + 1) * w);  // slots

@@ -104,7 +104,7 @@ int create_fp32p(Solver *s) {
     }
     rc |= up(s, (int32_t **)&a.g_off, L.g_off.data(), nc + 1);
     rc |= up(s, (int32_t **)&a.g_ent, L.g_ent.data(), L.g_ent.size());
-    if (!rc) rc |= s->build_gather_keys(a, D == 2);
+    if (!rc) rc |= s->build_gather_keys(a, true);
     rc |= up(s, (int32_t **)&a.ghost_cell, L.ghost_cell.data(), L.ng);
     rc |= up(s, (int32_t **)&a.ghost_role, L.ghost_role.data(), L.ng);
     rc |= up(s, (double **)&a.vol_d, L.volume.data(), nc);
@@ -199,23 +199,31 @@ static void launch_gradvis32_v(Solver *s, bool fin) {
     s->stream_nt ? launch_gradvis32_nt<D, V, SL, PK, true>(s, fin) : launch_gradvis32_nt<D, V, SL, PK, false>(s, fin);
 }
 
-// 3D gradients read the face slots (same bits as the gather list; 4.2 M-cell
-// O-grid 0.98 -> 0.86 ms per step).  2D gradients keep the list: there the
+// 3D gradients of a mesh with a face table read its packed slots.  Without one
+// they read the faces' own data, from slots where the stage outgrows the
+// Infinity Cache (consecutive, 120 B per cell) and through the gather entries
+// where it does not (97 B, gathered); the bits are the same.  Slots against
+// entries per step: O-grid of 74 k cells 81.9 / 79.4 us, 193 k 131.8 / 130.1,
+// 1 M 615 / 640, 4.2 M 2399 / 2548.  2D gradients use the entries: there the
 // slot streams cost more than the cached face records they replace (1 M-cell
-// annulus 0.114 -> 0.134 ms per step with slots).  fin: the launch also
-// reduces the previous step's CFL maxima in one extra block (the caller
-// knows the launch happens: full, viscous or M2AUSM).
+// annulus 0.114 -> 0.134 ms per step with slots).  fin: the launch also reduces
+// the previous step's CFL maxima in one extra block (the caller knows the
+// launch happens: full, viscous or M2AUSM).
 template <int D>
 void launch_gradvis32(Solver *s, bool full, bool fin) {
     if (!full && !s->visc && s->prm.solver != 2) return;
     const bool V = full || s->visc;
     if constexpr (D == 3) {
-        if (s->ensure_slots32()) {
-            if (s->k32->pk)
+        if ((s->stream_nt || s->table32.n > 0 || s->k32->pk) && s->ensure_slots32()) {
+            if (s->k32->pk) {
                 V ? launch_gradvis32_v<D, true, true, true>(s, fin) : launch_gradvis32_v<D, false, true, true>(s, fin);
-            else
-                V ? launch_gradvis32_v<D, true, true, false>(s, fin) : launch_gradvis32_v<D, false, true, false>(s, fin);
-            return;
+                return;
+            }
+            if (s->stream_nt) {
+                V ? launch_gradvis32_nt<D, true, true, false, true>(s, fin)
+                  : launch_gradvis32_nt<D, false, true, false, true>(s, fin);
+                return;
+            }
         }
     }
     V ? launch_gradvis32_v<D, true, false, false>(s, fin) : launch_gradvis32_v<D, false, false, false>(s, fin);
