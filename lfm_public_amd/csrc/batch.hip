@@ -19,17 +19,21 @@ struct Batch {
     hipStream_t stream = nullptr;
     std::vector<Solver *> members;
     KArgs32 *d_args = nullptr;
-    int32_t *d_maps = nullptr;
+    int2 *d_maps = nullptr;
     size_t maps_cap = 0, args_cap = 0;
     BatchMap map_cells{}, map_faces{};
     int nb_cells = 0, nb_faces = 0;
     int D = 2, solver = 0, minmod = 0, nstages = 0;
     bool visc = true;
-    // inviscid M1 / M2 members with their second buffers and face slots:
-    // the stages after the first `separate` ones are one launch each
+    // inviscid M1 / M2 members with their second buffers and face slots: one
+    // launch per stage, from one buffer into the other (side 1: the state is in
+    // the second).  A graph ends in the first: one that holds an odd number of
+    // stages takes its first as separate launches, which update in place (256 k
+    // cells in four members: 15 us where a one-launch stage takes 8).
     bool fused = false;
-    int separate = 0;
+    int side = 0;
     double A[5]{}, B[5]{};
+    int separate = 0;      // first stages of each step that stay separate launches
     bool drop_dq = false;  // the step being enqueued is followed by another one of its graph
     int dq_mode(int rk) const { return (rk == 0 ? kDqZero : 0) | (drop_dq && rk == nstages - 1 ? kDqDrop : 0); }
     // one step, and kSteps of them for runs of many.  A graph launch costs
@@ -37,6 +41,7 @@ struct Batch {
     // capturing it costs 0.6 (6 launches per step) to 1.3 ms (16), what it
     // saves in kManyAfter steps, and is done once that many were run.
     static constexpr int kSteps = Solver::kGraphSteps;
+    static_assert(kSteps % 2 == 0);
     static constexpr long kManyAfter = 128;
     hipGraph_t graph = nullptr, graph_many = nullptr;
     hipGraphExec_t exec = nullptr, exec_many = nullptr;
@@ -77,9 +82,8 @@ static void enqueue_step_nt(Batch *b) {
     const dim3 blk(256);
     for (int rk = 0; rk < b->nstages; rk++) {
         if (b->fused && rk >= b->separate) {
-            // an even number of one-launch stages: each step ends in a.q
-            const int flip = (rk - b->separate) & 1;
-            b->solver == 0 ? enqueue_fused<D, 0, NT>(b, rk, flip) : enqueue_fused<D, 1, NT>(b, rk, flip);
+            b->solver == 0 ? enqueue_fused<D, 0, NT>(b, rk, b->side) : enqueue_fused<D, 1, NT>(b, rk, b->side);
+            b->side ^= 1;
             continue;
         }
         // ghosts are refreshed by the update kernel (members join with fresh ghosts);
@@ -124,6 +128,8 @@ static void enqueue_step(Batch *b) {
 static hipError_t capture(Batch *b, int n, hipGraph_t *graph, hipGraphExec_t *exec) {
     hipError_t e = hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) {
+        b->side = 0;
+        b->separate = n * b->nstages % 2;  // n is 1 or even
         for (int i = 0; i < n; i++) {
             b->drop_dq = i + 1 < n;
             if (b->D == 2)
@@ -163,7 +169,7 @@ static int batch_set_locked(Batch *b, lfm_solver *const *hs, int n) {
     if (n == 0) return LFM_OK;
     bool fused = true;
     std::vector<KArgs32> args;
-    std::vector<int32_t> req_c, req_f, first_c, first_f;
+    std::vector<int2> slot_c, slot_f;
     for (int i = 0; i < n; i++) {
         if (!hs[i] || !hs[i]->impl) return fail(LFM_EINVAL, "null solver in batch");
         Solver *s = hs[i]->impl.get();
@@ -197,22 +203,20 @@ static int batch_set_locked(Batch *b, lfm_solver *const *hs, int n) {
         args.push_back(*s->k32);
         args.back().q_alt = s->q_alt32;
         fused = fused && s->fused_ok && s->q_alt32 && !s->post_forces;
-        auto add = [&](std::vector<int32_t> &req, std::vector<int32_t> &first, long count) {
-            first.push_back((int32_t)req.size());
-            const long nb = (count + 255) / 256;
-            for (long k = 0; k < nb; k++) req.push_back(i);
+        auto add = [&](std::vector<int2> &slot, long count) {
+            const int nb = (int)((count + 255) / 256);
+            for (int k = 0; k < nb; k++) slot.push_back(make_int2(i, k));
         };
-        add(req_c, first_c, s->L.nc);
-        add(req_f, first_f, s->L.nf);
+        add(slot_c, s->L.nc);
+        add(slot_f, s->L.nf);
     }
-    b->nb_cells = (int)req_c.size();
-    b->nb_faces = (int)req_f.size();
+    b->nb_cells = (int)slot_c.size();
+    b->nb_faces = (int)slot_f.size();
     b->fused = fused && b->solver < 2 && !b->visc;
-    b->separate = b->nstages % 2;  // leaves an even number of one-launch stages
-    const size_t nmap = req_c.size() + req_f.size() + 2 * (size_t)n;
+    const size_t nmap = slot_c.size() + slot_f.size();
     if (nmap > b->maps_cap) {
         if (b->d_maps) HIP_TRY(hipFree(b->d_maps));
-        HIP_TRY(hipMalloc((void **)&b->d_maps, nmap * sizeof(int32_t)));
+        HIP_TRY(hipMalloc((void **)&b->d_maps, nmap * sizeof(int2)));
         b->maps_cap = nmap;
     }
     if ((size_t)n > b->args_cap) {
@@ -220,18 +224,10 @@ static int batch_set_locked(Batch *b, lfm_solver *const *hs, int n) {
         HIP_TRY(hipMalloc((void **)&b->d_args, n * sizeof(KArgs32)));
         b->args_cap = n;
     }
-    std::vector<int32_t> maps;
-    maps.reserve(nmap);
-    auto put = [&](const std::vector<int32_t> &v) {
-        const size_t off = maps.size();
-        maps.insert(maps.end(), v.begin(), v.end());
-        return b->d_maps + off;
-    };
-    b->map_cells = {put(req_c), nullptr};
-    b->map_cells.first = put(first_c);
-    b->map_faces = {put(req_f), nullptr};
-    b->map_faces.first = put(first_f);
-    HIP_TRY(hipMemcpy(b->d_maps, maps.data(), maps.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    b->map_cells.slot = b->d_maps;
+    b->map_faces.slot = b->d_maps + slot_c.size();
+    HIP_TRY(hipMemcpy(b->d_maps, slot_c.data(), slot_c.size() * sizeof(int2), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(b->d_maps + slot_c.size(), slot_f.data(), slot_f.size() * sizeof(int2), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(b->d_args, args.data(), n * sizeof(KArgs32), hipMemcpyHostToDevice));
     const hipError_t e = capture(b, 1, &b->graph, &b->exec);
     if (e != hipSuccess) {

@@ -1443,19 +1443,18 @@ __global__ void __launch_bounds__(256) vis_tensor_field32(KArgs32 a, float *tmc_
 
 // ---------------------------------------------------------------------------
 // batched kernels: one launch covers several resident solvers of one scheme
-// class.  Block b belongs to solver bmap[b] (sorted) and is its local block
-// b - bfirst[solver]; each solver computes exactly what its single launch
-// computes.
+// class; each solver computes exactly what its single launch computes.  A
+// block's solver and its number within that solver lie together: one load
+// before the solver's arguments can be asked for.
 // ---------------------------------------------------------------------------
 struct BatchMap {
-    const int32_t *req;    // [nblocks] solver of each block
-    const int32_t *first;  // [nsolvers] first block of each solver
+    const int2 *slot;  // [nblocks] solver (sorted) and local block
 };
 
 __device__ __forceinline__ void batch_slot(const BatchMap &m, int &r, int &lblk) {
-    const int b = LFM_BLK();
-    r = m.req[b];
-    lblk = b - m.first[r];
+    const int2 v = m.slot[LFM_BLK()];
+    r = v.x;
+    lblk = v.y;
 }
 
 template <int D, int GRAD, bool VISC, bool RG, bool NT>
