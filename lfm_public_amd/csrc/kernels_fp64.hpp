@@ -1,12 +1,16 @@
 // kernels_fp64.hpp -- gfx950 kernels of the plain FP64 time step.
 //
-// One RK stage is four launches over SoA arrays:
-//   bc_fill      one thread per boundary ghost   (set_boundary_conditions)
+// One RK stage is three launches,
 //   grad_vis     one thread per cell, gathering its faces in the reference's
 //                processing order (calc_gradients[_M2AUSM] + calc_VIS)
 //   face_flux    one thread per face, each face once (one_rk_step_* body)
 //   cell_update  one thread per cell, gathering face fluxes in the
-//                reference's accumulation order, then sponge and RK update
+//                reference's accumulation order, then sponge, RK update and
+//                the cell's boundary ghosts (set_boundary_conditions)
+// or, for inviscid M1 / M2,
+//   stage_fused64  one thread per cell, forming its faces' fluxes as it
+//                  gathers them, into a second state buffer
+// bc_fill fills the boundary ghosts after the state was set from outside.
 // The gathers replace the reference's owner/neighbour scatter: every cell
 // sums the same terms in the same order as the reference's in-place loop,
 // so no atomics are needed and the result does not depend on scheduling.
@@ -469,14 +473,16 @@ __device__ __forceinline__ void vis_tensors(const KArgs &a, const double (&dudx)
 }
 
 // Bound: latency (at a few 100 k cells a launch has 2-3 waves per SIMD to hide
-// its dependent loads), so registers decide.  Faces in groups whose loads are
-// issued together: all four in 2D (176 k-cell annulus, four 171, two 176 us per
-// step), two in 3D at 3 waves per SIMD (193 k-cell O-grid: three spill and take
-// 415, two 397, one 397; 1 M cells: two 1531, one 1586).
-template <int D>
-constexpr int kGradGroup64 = D == 2 ? 4 : 2;
+// its dependent loads), so registers decide; in 3D past the cache, memory.
+// Faces in groups whose loads are issued together: all four in 2D (176 k-cell
+// annulus, four 171, two 176 us per step), two in 3D at 3 waves per SIMD (193
+// k-cell O-grid: three spill and take 415, two 397, one 397) and, where the
+// stage outgrows the cache, all six at 2 (1 M cells 1400 -> 1351, 4.2 M 5983 ->
+// 5873).
+template <int D, bool NT>
+constexpr int kGradGroup64 = D == 2 ? 4 : NT ? 6 : 2;
 template <int D, int GRAD, bool VISC, bool RG, bool NT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) grad_vis(KArgs a) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGradGroup64<D, NT> == 6 ? 2 : 3))) grad_vis(KArgs a) {
     const int c = LFM_TID(blockIdx.x);
     using R = GradRec64<D, RG>;
     // every thread reaches the record write-out below (LDS staging)
@@ -558,7 +564,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) g
         }
     };
     // groups of G faces in gather order, their loads issued together
-    constexpr int U = GatherUnroll<D>::value, G = kGradGroup64<D>;
+    constexpr int U = GatherUnroll<D>::value, G = kGradGroup64<D, NT>;
     static_assert(U % G == 0);
     int key[G], oth[G], e0 = 0, ne = U;
     load_keys<D, NT>(a.g_key, a.nc, 0, c, key);
@@ -579,8 +585,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) g
             load_q<D>(a, oth[u], qj[u]);
         }
         const int jn = j0 + G;
-        load_keys<D, NT>(a.g_key, a.nc, jn < U ? jn : 0, c, nkey);
-        load_keys<D, NT>(a.g_oth, a.nc, jn < U ? jn : 0, c, noth);
+#pragma unroll
+        for (int u = 0; u < G; u++) nkey[u] = noth[u] = kNoFace;
+        if constexpr (G < U) {
+            load_keys<D, NT>(a.g_key, a.nc, jn < U ? jn : 0, c, nkey);
+            load_keys<D, NT>(a.g_oth, a.nc, jn < U ? jn : 0, c, noth);
+        }
         if (a.more_faces && jn >= U) {  // entries beyond the first U
 #pragma unroll
             for (int u = 0; u < G; u++) {
@@ -632,29 +642,52 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) g
     }
     }
     if (VISC) {
-        // the wave's records are contiguous from its first cell: four 16-byte
-        // words of each at a time are staged in LDS and written as 64-byte
-        // runs (without minmod the rho / p / U gradient slots are written
-        // zero, as they stay).  Staging whole records (57 KB per block for 3D
-        // M2AUSM) held the kernel at 2 waves per SIMD.
-        constexpr int W = R::kStride / 2, C = 4;
-        __shared__ double2 stage[256 / 64][64 * C];
+        // the wave's records are contiguous from its first cell.  In 2D where the
+        // stage fits the cache, four 16-byte words of each at a time are staged
+        // in LDS and written as 64-byte runs, which L2 joins (176 k-cell
+        // annulus 171 against 174 us per step); otherwise the records of 16
+        // cells at a time, written as consecutive words (64-byte runs wrote
+        // 540 MB where the records of a 4.2 M-cell O-grid are 403).  The face
+        // launch reads the records next: plain stores (1 M-cell annulus 802
+        // against 828 us per step non-temporal, 2.1 M 1627 against 1607).
+        // Staging whole blocks (57 KB for 3D M2AUSM) held the kernel at 2 waves
+        // per SIMD; without minmod the rho / p / U slots are written zero.
+        constexpr bool kRuns = D == 2 && !NT;
+        constexpr int W = R::kStride / 2, C = 4, M = 16;
+        __shared__ double2 stage[256 / 64][kRuns ? 64 * C : M * W];
         double2 *st = stage[threadIdx.x >> 6];
         const int lane = threadIdx.x & 63, c0 = c - lane;
         d2v *dst = reinterpret_cast<d2v *>(a.dudx + (size_t)c0 * R::kStride);
+        if constexpr (kRuns) {
 #pragma unroll
-        for (int w0 = 0; w0 < W; w0 += C) {
-            const int n = W - w0 < C ? W - w0 : C;
+            for (int w0 = 0; w0 < W; w0 += C) {
+                const int n = W - w0 < C ? W - w0 : C;
 #pragma unroll
-            for (int k = 0; k < n; k++) st[lane * n + k] = make_double2(rec[2 * (w0 + k)], rec[2 * (w0 + k) + 1]);
-            wave_sync_lds();
+                for (int k = 0; k < n; k++) st[lane * n + k] = make_double2(rec[2 * (w0 + k)], rec[2 * (w0 + k) + 1]);
+                wave_sync_lds();
 #pragma unroll
-            for (int i = 0; i < n; i++) {
-                const int j = i * 64 + lane, r = j / n;
-                const double2 v = st[j];
-                if (c0 + r < a.nc) st_once<NT>(dst + r * W + w0 + j % n, d2v{v.x, v.y});
+                for (int i = 0; i < n; i++) {
+                    const int j = i * 64 + lane, r = j / n;
+                    const double2 v = st[j];
+                    if (c0 + r < a.nc) st_once<false>(dst + r * W + w0 + j % n, d2v{v.x, v.y});
+                }
+                wave_sync_lds();
             }
-            wave_sync_lds();
+        } else {
+#pragma unroll
+            for (int g = 0; g < 64 / M; g++) {
+                if (lane / M == g)
+#pragma unroll
+                    for (int k = 0; k < W; k++) st[(lane % M) * W + k] = make_double2(rec[2 * k], rec[2 * k + 1]);
+                wave_sync_lds();
+                const int n = min(a.nc - c0 - g * M, M) * W;
+#pragma unroll
+                for (int j = lane; j < M * W; j += 64) {
+                    const double2 v = st[j];
+                    if (j < n) st_once<false>(dst + g * M * W + j, d2v{v.x, v.y});
+                }
+                wave_sync_lds();
+            }
         }
     }
 }

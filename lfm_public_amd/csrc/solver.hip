@@ -539,11 +539,12 @@ static void *upload_records(const std::vector<uint16_t> &rec) {
 }
 
 // the per-cell face slots (each cell's first GatherUnroll gather entries:
-// other cell, area vector, weight), read by the one-launch stages and the
+// other cell, area vector, weight), read by the one-launch stages and the 3D
 // FP32 gradient kernel; allocated on first use (under the set-up mutex, as a
 // capture on another thread requires) and filled from the gather list on
-// the handle's stream.  When memory cannot be had the kernels read the
-// gather list and the face arrays, which gives the same bits.
+// the handle's stream.  When memory cannot be had the gradients read the
+// gather entries and the face arrays and the step runs the separate launches,
+// which gives the same bits.
 bool Solver::ensure_slots32() {
     if (!fp32 || slots_failed) return false;
     if (k32->pk || k32->sl_nb) return true;
