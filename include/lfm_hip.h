@@ -179,6 +179,9 @@ int lfm_synchronize(lfm_solver *s);
 /* Time n steps (as lfm_run launches them, without post-processing) with
  * HIP events on the handle's stream (ms). */
 int lfm_time_steps(lfm_solver *s, int nsteps, double *ms_out);
+/* How many of the handle's steps were replays of a graph of several steps
+ * (long runs build one; results do not depend on it). */
+int lfm_replayed_steps(lfm_solver *s, int64_t *n);
 
 /* Time n steps launched kernel by kernel with HIP events around every
  * kernel group on the handle's stream: ms_per_group[6] = bc fill,
@@ -298,14 +301,14 @@ int lfm_post_forces_read(lfm_solver *s, int32_t max_rows, double *rows, int32_t 
  * reference, which runs one solve per process): the FP32-perturbation
  * solvers of one scheme class (dimension, solver, minmod, rkOrder; constant
  * dt, no residual output) are stepped by single kernel launches covering all
- * of them, one RK step captured as a hipGraph and replayed.  Each solver
+ * of them, one RK step as a hipGraph that is replayed.  Each solver
  * computes exactly what lfm_run would compute for it alone.  While a solver
  * is in a batch, only the batch may step it.
  * --------------------------------------------------------------------- */
 typedef struct lfm_batch lfm_batch;
 int lfm_batch_create(lfm_batch **out);
 int lfm_batch_destroy(lfm_batch *b);
-/* Replace the member set (may be empty) and capture the step graph.
+/* Replace the member set (may be empty) and build the step graph.
  * Inviscid M1 / M2 members get the one-launch stages' second state buffer
  * and face slots here if they lack them (their lfm_info.device_bytes grows);
  * where that memory cannot be had the batch runs separate launches. */
@@ -313,6 +316,8 @@ int lfm_batch_set(lfm_batch *b, lfm_solver *const *solvers, int n);
 /* Queue n steps of every member on the batch's stream. */
 int lfm_batch_run(lfm_batch *b, int nsteps);
 int lfm_batch_synchronize(lfm_batch *b);
+/* How many of the batch's steps were replays of a graph of several steps. */
+int lfm_batch_replayed_steps(lfm_batch *b, int64_t *n);
 
 #ifdef __cplusplus
 }

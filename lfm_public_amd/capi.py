@@ -34,7 +34,8 @@ EXPORTS = ("lfm_patch_role", "lfm_solver_create", "lfm_solver_destroy", "lfm_las
            "lfm_part_group_destroy", "lfm_case_open", "lfm_case_close", "lfm_case_mesh", "lfm_case_params",
            "lfm_case_fields", "lfm_case_time", "lfm_case_dict_scalar", "lfm_case_write_time",
            "lfm_case_post", "lfm_case_write_scalar", "lfm_post_configure", "lfm_post_average",
-           "lfm_post_average_fields", "lfm_post_walls", "lfm_post_forces", "lfm_post_forces_read")
+           "lfm_post_average_fields", "lfm_post_walls", "lfm_post_forces", "lfm_post_forces_read",
+           "lfm_replayed_steps", "lfm_batch_replayed_steps")
 HALO_SOLVARS, HALO_VISCOUS, HALO_PACKED = 1, 2, 3
 
 
@@ -115,6 +116,8 @@ def load() -> C.CDLL:
     L.lfm_compute_cfl.argtypes = [vp, dbl, C.POINTER(dbl)]
     L.lfm_run.argtypes = [vp, C.c_int]
     L.lfm_time_steps.argtypes = [vp, C.c_int, C.POINTER(dbl)]
+    L.lfm_replayed_steps.argtypes = [vp, C.POINTER(C.c_int64)]
+    L.lfm_batch_replayed_steps.argtypes = [vp, C.POINTER(C.c_int64)]
     L.lfm_profile_steps.argtypes = [vp, C.c_int, vp, C.POINTER(dbl)]
     L.lfm_get_field.argtypes = [vp, C.c_int, vp]
     L.lfm_set_field.argtypes = [vp, C.c_int, vp]
@@ -290,6 +293,12 @@ class GpuSolver:
         ms = C.c_double()
         _check(load().lfm_time_steps(self.h, nsteps, C.byref(ms)))
         return ms.value
+
+    def replayed_steps(self) -> int:
+        """Steps taken by replays of a graph of several steps."""
+        n = C.c_int64()
+        _check(load().lfm_replayed_steps(self.h, C.byref(n)))
+        return n.value
 
     PROFILE_GROUPS = ("bc_fill", "grad_vis", "face_flux", "cell_update", "cfl_dt", "cell_update_cfl")
 
@@ -468,6 +477,12 @@ class Batch:
 
     def run(self, nsteps: int):
         _check(load().lfm_batch_run(self.h, nsteps))
+
+    def replayed_steps(self) -> int:
+        """Steps taken by replays of a graph of several steps."""
+        n = C.c_int64()
+        _check(load().lfm_batch_replayed_steps(self.h, C.byref(n)))
+        return n.value
 
     def synchronize(self):
         _check(load().lfm_batch_synchronize(self.h))

@@ -1,5 +1,5 @@
 // batch.hip -- shared launches over several resident FP32-perturbation
-// solvers of one scheme class, one RK step captured in a hipGraph.
+// solvers of one scheme class, one RK step as a hipGraph.
 //
 // The reference has no serving mode; this is the device half of the
 // continuous-batching service: the host side admits and retires solvers and
@@ -38,15 +38,18 @@ struct Batch {
     int dq_mode(int rk) const { return (rk == 0 ? kDqZero : 0) | (drop_dq && rk == nstages - 1 ? kDqDrop : 0); }
     // one step, and kSteps of them for runs of many.  A graph launch costs
     // some 9 us beside its kernels, so the longer graph saves 8 us per step;
-    // capturing it costs 0.6 (6 launches per step) to 1.3 ms (16), what it
-    // saves in kManyAfter steps, and is done once that many were run.
+    // building it costs 0.6 (6 launches per step) to 1.3 ms (16), what it
+    // saves in kManyAfter steps, and is done once that many were run (twice as
+    // many after each time that it could not be had).
     static constexpr int kSteps = Solver::kGraphSteps;
     static_assert(kSteps % 2 == 0);
     static constexpr long kManyAfter = 128;
     hipGraph_t graph = nullptr, graph_many = nullptr;
     hipGraphExec_t exec = nullptr, exec_many = nullptr;
-    long singles = 0;  // single-step launches since the members were set
-    bool many_failed = false;
+    long singles = 0;  // single-step launches since the members were set or a failure
+    long many_after = kManyAfter;
+    int64_t replayed_many = 0;  // steps taken by graphs of kSteps
+    GraphBuild *building = nullptr;
 
     void drop_graphs() {
         if (exec) (void)hipGraphExecDestroy(exec);
@@ -56,7 +59,7 @@ struct Batch {
         exec = exec_many = nullptr;
         graph = graph_many = nullptr;
         singles = 0;
-        many_failed = false;
+        many_after = kManyAfter;
     }
     ~Batch() {
         drop_graphs();
@@ -70,10 +73,10 @@ template <int D, int SOLVER, bool NT>
 static void enqueue_fused(Batch *b, int rk, int flip) {
     const dim3 blk(256);
     if (rk == b->nstages - 1)
-        hipLaunchKernelGGL((stage_fused32_b<D, SOLVER, 1, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
+        launch(b, (stage_fused32_b<D, SOLVER, 1, NT>), dim3(b->nb_cells), blk, b->d_args,
                            b->map_cells, (float)b->A[rk], (float)b->B[rk], b->dq_mode(rk), flip);
     else
-        hipLaunchKernelGGL((stage_fused32_b<D, SOLVER, -1, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
+        launch(b, (stage_fused32_b<D, SOLVER, -1, NT>), dim3(b->nb_cells), blk, b->d_args,
                            b->map_cells, (float)b->A[rk], (float)b->B[rk], b->dq_mode(rk), flip);
 }
 
@@ -90,29 +93,29 @@ static void enqueue_step_nt(Batch *b) {
         // without viscosity solvers 0/1 consume no gradient or tensor
         if (V || b->solver == 2) {
             if (b->solver == 2 && b->minmod)
-                hipLaunchKernelGGL((grad_vis32_b<D, 2, V, true, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
+                launch(b, (grad_vis32_b<D, 2, V, true, NT>), dim3(b->nb_cells), blk, b->d_args,
                                    b->map_cells);
             else if (b->solver == 2)
-                hipLaunchKernelGGL((grad_vis32_b<D, 0, V, true, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
+                launch(b, (grad_vis32_b<D, 0, V, true, NT>), dim3(b->nb_cells), blk, b->d_args,
                                    b->map_cells);
             else
-                hipLaunchKernelGGL((grad_vis32_b<D, 0, V, false, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
+                launch(b, (grad_vis32_b<D, 0, V, false, NT>), dim3(b->nb_cells), blk, b->d_args,
                                    b->map_cells);
         }
         switch (b->solver) {
-        case 0: hipLaunchKernelGGL((face_flux32_b<D, 0, V, NT>), dim3(b->nb_faces), blk, 0, b->stream, b->d_args, b->map_faces); break;
-        case 1: hipLaunchKernelGGL((face_flux32_b<D, 1, V, NT>), dim3(b->nb_faces), blk, 0, b->stream, b->d_args, b->map_faces); break;
-        default: hipLaunchKernelGGL((face_flux32_b<D, 2, V, NT>), dim3(b->nb_faces), blk, 0, b->stream, b->d_args, b->map_faces); break;
+        case 0: launch(b, (face_flux32_b<D, 0, V, NT>), dim3(b->nb_faces), blk, b->d_args, b->map_faces); break;
+        case 1: launch(b, (face_flux32_b<D, 1, V, NT>), dim3(b->nb_faces), blk, b->d_args, b->map_faces); break;
+        default: launch(b, (face_flux32_b<D, 2, V, NT>), dim3(b->nb_faces), blk, b->d_args, b->map_faces); break;
         }
         // the last stage's update also forms the step's compute_cfl partials
         if (rk == b->nstages - 1)
-            hipLaunchKernelGGL((cell_update32_b<D, 1, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
+            launch(b, (cell_update32_b<D, 1, NT>), dim3(b->nb_cells), blk, b->d_args,
                                b->map_cells, (float)b->A[rk], (float)b->B[rk], b->dq_mode(rk));
         else
-            hipLaunchKernelGGL((cell_update32_b<D, -1, NT>), dim3(b->nb_cells), blk, 0, b->stream, b->d_args,
+            launch(b, (cell_update32_b<D, -1, NT>), dim3(b->nb_cells), blk, b->d_args,
                                b->map_cells, (float)b->A[rk], (float)b->B[rk], b->dq_mode(rk));
     }
-    hipLaunchKernelGGL(cfl_final32_b, dim3((unsigned)b->members.size()), blk, 0, b->stream, b->d_args);
+    launch(b, cfl_final32_b, dim3((unsigned)b->members.size()), blk, b->d_args);
 }
 
 // one launch walks every member: NT by what they touch together
@@ -123,45 +126,28 @@ static void enqueue_step(Batch *b) {
     outgrows_cache(bytes) ? enqueue_step_nt<D, V, true>(b) : enqueue_step_nt<D, V, false>(b);
 }
 
-// n RK steps of the batch as a graph; on failure no capture or sticky error is
-// left behind (the caller holds the set-up mutex)
-static hipError_t capture(Batch *b, int n, hipGraph_t *graph, hipGraphExec_t *exec) {
-    hipError_t e = hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal);
-    if (e == hipSuccess) {
-        b->side = 0;
-        b->separate = n * b->nstages % 2;  // n is 1 or even
-        for (int i = 0; i < n; i++) {
-            b->drop_dq = i + 1 < n;
-            if (b->D == 2)
-                b->visc ? enqueue_step<2, true>(b) : enqueue_step<2, false>(b);
-            else
-                b->visc ? enqueue_step<3, true>(b) : enqueue_step<3, false>(b);
-        }
-        e = hipStreamEndCapture(b->stream, graph);
+// n RK steps of the batch as a graph
+static hipError_t build_steps(Batch *b, int n, hipGraph_t *graph, hipGraphExec_t *exec) {
+    GraphBuild build;
+    b->building = &build;
+    b->side = 0;
+    b->separate = n * b->nstages % 2;  // n is 1 or even
+    for (int i = 0; i < n; i++) {
+        b->drop_dq = i + 1 < n;
+        if (b->D == 2)
+            b->visc ? enqueue_step<2, true>(b) : enqueue_step<2, false>(b);
+        else
+            b->visc ? enqueue_step<3, true>(b) : enqueue_step<3, false>(b);
     }
-    if (e == hipSuccess) e = hipGraphInstantiate(exec, *graph, nullptr, nullptr, 0);
-    if (e != hipSuccess) {
-        if (*graph) (void)hipGraphDestroy(*graph);
-        *graph = nullptr;
-        *exec = nullptr;
-        (void)hipGetLastError();
-    }
-    return e;
+    b->building = nullptr;
+    return build.finish(graph, exec);
 }
-
-static int batch_set_locked(Batch *b, lfm_solver *const *hs, int n);
 
 static int batch_set(Batch *b, lfm_solver *const *hs, int n) {
-    // the one-launch stages' buffers of eligible members, allocated (under
-    // the set-up mutex, which ensure_alt32 takes itself) before the batch
-    // takes it; a member without them keeps the batch on separate launches
+    // the one-launch stages' buffers of eligible members; a member without them
+    // keeps the batch on separate launches
     for (int i = 0; i < n; i++)
         if (hs && hs[i] && hs[i]->impl && hs[i]->impl->fp32) (void)hs[i]->impl->ensure_alt32();
-    std::lock_guard<std::mutex> lock(device_setup_mutex());
-    return batch_set_locked(b, hs, n);
-}
-
-static int batch_set_locked(Batch *b, lfm_solver *const *hs, int n) {
     if (b->exec) HIP_TRY(hipStreamSynchronize(b->stream));
     b->drop_graphs();
     b->members.clear();
@@ -229,20 +215,21 @@ static int batch_set_locked(Batch *b, lfm_solver *const *hs, int n) {
     HIP_TRY(hipMemcpy(b->d_maps, slot_c.data(), slot_c.size() * sizeof(int2), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(b->d_maps + slot_c.size(), slot_f.data(), slot_f.size() * sizeof(int2), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(b->d_args, args.data(), n * sizeof(KArgs32), hipMemcpyHostToDevice));
-    const hipError_t e = capture(b, 1, &b->graph, &b->exec);
+    const hipError_t e = build_steps(b, 1, &b->graph, &b->exec);
     if (e != hipSuccess) {
         b->members.clear();
-        return fail(LFM_EDEVICE, std::string("step graph capture: ") + hipGetErrorString(e));
+        return fail(LFM_EDEVICE, std::string("step graph: ") + hipGetErrorString(e));
     }
     return LFM_OK;
 }
 
 // the graph of kSteps steps, once the single ones have cost as much
-static bool capture_many(Batch *b) {
-    if (b->many_failed || b->singles < Batch::kManyAfter) return false;
-    std::lock_guard<std::mutex> lock(device_setup_mutex());
-    b->many_failed = capture(b, Batch::kSteps, &b->graph_many, &b->exec_many) != hipSuccess;
-    return !b->many_failed;
+static bool build_many(Batch *b) {
+    if (b->singles < b->many_after) return false;
+    if (build_steps(b, Batch::kSteps, &b->graph_many, &b->exec_many) == hipSuccess) return true;
+    b->singles = 0;
+    b->many_after *= 2;
+    return false;
 }
 
 }  // namespace lfm
@@ -281,13 +268,20 @@ int lfm_batch_run(lfm_batch *b, int nsteps) {
     if (b->impl.members.empty() || !b->impl.exec) return nsteps == 0 ? LFM_OK : lfm::fail(LFM_ESTATE, "empty batch");
     lfm::Batch &x = b->impl;
     for (int i = 0; i < nsteps;) {
-        const bool many = nsteps - i >= x.kSteps && (x.exec_many || lfm::capture_many(&x));
+        const bool many = nsteps - i >= x.kSteps && (x.exec_many || lfm::build_many(&x));
         const hipError_t e = hipGraphLaunch(many ? x.exec_many : x.exec, x.stream);
         if (e != hipSuccess) return lfm::fail(LFM_EDEVICE, std::string("hipGraphLaunch: ") + hipGetErrorString(e));
         i += many ? x.kSteps : 1;
         x.singles += many ? 0 : 1;
+        x.replayed_many += many ? x.kSteps : 0;
     }
     for (lfm::Solver *s : b->impl.members) s->steps_done += nsteps;
+    return LFM_OK;
+}
+
+int lfm_batch_replayed_steps(lfm_batch *b, int64_t *n) {
+    if (!b || !n) return lfm::fail(LFM_EINVAL, "null argument");
+    *n = b->impl.replayed_many;
     return LFM_OK;
 }
 

@@ -179,7 +179,6 @@ int lfm_halo_import(lfm_solver *h, int32_t rank, int32_t n_faces, const int32_t 
         return fail(LFM_ENOMEM, std::string("applying the set-up message: ") + e.what());
     }
     if (!err.empty()) return fail(LFM_EINVAL, err);
-    std::lock_guard<std::mutex> lock(lfm::device_setup_mutex());
     int rc = s->halo_upload_geometry();
     if (rc) return rc;
     const lfm::HaloNbr &hn = s->L.halo[ni];
@@ -258,7 +257,6 @@ int lfm_part_group_create(lfm_solver *const *hs, int n, lfm_part_group **out) {
             g->peer[q].push_back(j);
         }
     }
-    std::lock_guard<std::mutex> lock(lfm::device_setup_mutex());
     HIP_TRY(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking));
     HIP_TRY(hipEventCreateWithFlags(&g->done, hipEventDisableTiming));
     const size_t el = p0->fp32 ? 4 : 8;

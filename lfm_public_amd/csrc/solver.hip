@@ -27,11 +27,6 @@ int fail(int code, const std::string &msg) {
     return code;
 }
 
-std::mutex &device_setup_mutex() {
-    static std::mutex m;
-    return m;
-}
-
 // records of the FP64 geometry table: both orientations of them are at most
 // 192 KiB, which stay in an XCD's 4 MiB L2 beside the gathered states
 static constexpr int kMaxTable64 = 2048;
@@ -242,18 +237,18 @@ static int create_fp64(Solver *s) {
 // ---------------------------------------------------------------------------
 template <int D>
 static void launch_bc64(Solver *s) {
-    if (s->L.ng) hipLaunchKernelGGL(bc_fill<D>, dim3(nblocks(s->L.ng)), dim3(kBlock), 0, s->stream, s->k64);
+    if (s->L.ng) launch(s, bc_fill<D>, dim3(nblocks(s->L.ng)), dim3(kBlock), s->k64);
 }
 
 template <int D, bool V, bool NT>
 static void launch_gradvis64_nt(Solver *s) {
     const int nb = nblocks(s->L.nc);
     if (s->prm.solver == 2 && s->prm.minmod)
-        hipLaunchKernelGGL((grad_vis<D, 2, V, true, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64);
+        launch(s, (grad_vis<D, 2, V, true, NT>), dim3(nb), dim3(kBlock), s->k64);
     else if (s->prm.solver == 2)
-        hipLaunchKernelGGL((grad_vis<D, 0, V, true, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64);
+        launch(s, (grad_vis<D, 0, V, true, NT>), dim3(nb), dim3(kBlock), s->k64);
     else
-        hipLaunchKernelGGL((grad_vis<D, 0, V, false, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64);
+        launch(s, (grad_vis<D, 0, V, false, NT>), dim3(nb), dim3(kBlock), s->k64);
 }
 
 template <int D, bool V>
@@ -275,9 +270,9 @@ template <int D, bool V, bool ST, bool NT>
 static void launch_flux64_nt(Solver *s) {
     const int nb = nblocks(s->L.nf);
     switch (s->prm.solver) {
-    case 0: hipLaunchKernelGGL((face_flux<D, 0, V, ST, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64); break;
-    case 1: hipLaunchKernelGGL((face_flux<D, 1, V, ST, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64); break;
-    default: hipLaunchKernelGGL((face_flux<D, 2, V, ST, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64); break;
+    case 0: launch(s, (face_flux<D, 0, V, ST, NT>), dim3(nb), dim3(kBlock), s->k64); break;
+    case 1: launch(s, (face_flux<D, 1, V, ST, NT>), dim3(nb), dim3(kBlock), s->k64); break;
+    default: launch(s, (face_flux<D, 2, V, ST, NT>), dim3(nb), dim3(kBlock), s->k64); break;
     }
 }
 
@@ -299,18 +294,18 @@ static void launch_update64_nt(Solver *s, double A, double B, int dq_mode, bool 
                                const Solver::CflJob *cfl) {
     const int nb = nblocks(s->L.nc);
     if (res) {
-        hipLaunchKernelGGL((cell_update<D, true, -1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
+        launch(s, (cell_update<D, true, -1, NT>), dim3(nb), dim3(kBlock), s->k64, A, B,
                            dq_mode, 0.0);
-        hipLaunchKernelGGL(reduce_sum, dim3(1), dim3(kBlock), 0, s->stream, s->k64.partial, nb, D + 2, s->d_res,
+        launch(s, reduce_sum, dim3(1), dim3(kBlock), s->k64.partial, nb, D + 2, s->d_res,
                            (int)accumulate_res);
     } else if (cfl && cfl->mode == 0) {
-        hipLaunchKernelGGL((cell_update<D, false, 0, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
+        launch(s, (cell_update<D, false, 0, NT>), dim3(nb), dim3(kBlock), s->k64, A, B,
                            dq_mode, cfl->param);
     } else if (cfl) {
-        hipLaunchKernelGGL((cell_update<D, false, 1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
+        launch(s, (cell_update<D, false, 1, NT>), dim3(nb), dim3(kBlock), s->k64, A, B,
                            dq_mode, cfl->param);
     } else {
-        hipLaunchKernelGGL((cell_update<D, false, -1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, A, B,
+        launch(s, (cell_update<D, false, -1, NT>), dim3(nb), dim3(kBlock), s->k64, A, B,
                            dq_mode, 0.0);
     }
 }
@@ -326,21 +321,21 @@ template <int D>
 static void launch_cfl_dt64(Solver *s, int mode, double param, double *out, double *dt_dst) {
     const int nb = nblocks(s->L.nc);
     if (mode == 0) {
-        hipLaunchKernelGGL((cfl_dt_cells<D, 0>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, param);
-        hipLaunchKernelGGL(cfl_dt_final<0>, dim3(1), dim3(kFinalBlock), 0, s->stream, s->k64.partial, nb, out, dt_dst);
+        launch(s, (cfl_dt_cells<D, 0>), dim3(nb), dim3(kBlock), s->k64, param);
+        launch(s, cfl_dt_final<0>, dim3(1), dim3(kFinalBlock), s->k64.partial, nb, out, dt_dst);
     } else {
-        hipLaunchKernelGGL((cfl_dt_cells<D, 1>), dim3(nb), dim3(kBlock), 0, s->stream, s->k64, param);
-        hipLaunchKernelGGL(cfl_dt_final<1>, dim3(1), dim3(kFinalBlock), 0, s->stream, s->k64.partial, nb, out, dt_dst);
+        launch(s, (cfl_dt_cells<D, 1>), dim3(nb), dim3(kBlock), s->k64, param);
+        launch(s, cfl_dt_final<1>, dim3(1), dim3(kFinalBlock), s->k64.partial, nb, out, dt_dst);
     }
 }
 
 int integrals64(Solver *s, double *out_dev) {
     const int nb = nblocks(s->L.nc);
     if (s->L.D == 2)
-        hipLaunchKernelGGL(integrals64<2>, dim3(nb), dim3(kBlock), 0, s->stream, s->k64);
+        launch(s, integrals64<2>, dim3(nb), dim3(kBlock), s->k64);
     else
-        hipLaunchKernelGGL(integrals64<3>, dim3(nb), dim3(kBlock), 0, s->stream, s->k64);
-    hipLaunchKernelGGL(reduce_sum, dim3(1), dim3(kBlock), 0, s->stream, s->k64.partial, nb, s->L.D + 2, out_dev, 0);
+        launch(s, integrals64<3>, dim3(nb), dim3(kBlock), s->k64);
+    launch(s, reduce_sum, dim3(1), dim3(kBlock), s->k64.partial, nb, s->L.D + 2, out_dev, 0);
     return 0;
 }
 
@@ -349,13 +344,13 @@ static void launch_fused64_nt(Solver *s, double A, double B, int dq_mode, const 
                              const Solver::CflJob *cfl, bool fin) {
     const int nb = nblocks(s->L.nc);
     if (!cfl)
-        hipLaunchKernelGGL((stage_fused64<D, SOLVER, -1, PK, SYM, NT>), dim3(nb + (fin ? 1 : 0)), dim3(kBlock), 0, s->stream, a,
+        launch(s, (stage_fused64<D, SOLVER, -1, PK, SYM, NT>), dim3(nb + (fin ? 1 : 0)), dim3(kBlock), a,
                            qout, A, B, dq_mode, 0.0, fin ? nb : 0, s->d_cfl);
     else if (cfl->mode == 0)
-        hipLaunchKernelGGL((stage_fused64<D, SOLVER, 0, PK, SYM, NT>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
+        launch(s, (stage_fused64<D, SOLVER, 0, PK, SYM, NT>), dim3(nb), dim3(kBlock), a, qout, A, B,
                            dq_mode, cfl->param, 0, s->d_cfl);
     else
-        hipLaunchKernelGGL((stage_fused64<D, SOLVER, 1, PK, SYM, NT>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
+        launch(s, (stage_fused64<D, SOLVER, 1, PK, SYM, NT>), dim3(nb), dim3(kBlock), a, qout, A, B,
                            dq_mode, cfl->param, 0, s->d_cfl);
 }
 
@@ -435,10 +430,10 @@ void Solver::update(double A, double B, int dq_mode, bool res, bool accumulate_r
 void Solver::cfl_final(const CflJob &job) {
     const int nb = nblocks(L.nc);
     if (job.mode == 0)
-        hipLaunchKernelGGL(cfl_dt_final<0>, dim3(1), dim3(kFinalBlock), 0, stream, k64.partial, nb, job.out,
+        launch(this, cfl_dt_final<0>, dim3(1), dim3(kFinalBlock), k64.partial, nb, job.out,
                            job.dt_dst);
     else
-        hipLaunchKernelGGL(cfl_dt_final<1>, dim3(1), dim3(kFinalBlock), 0, stream, k64.partial, nb, job.out,
+        launch(this, cfl_dt_final<1>, dim3(1), dim3(kFinalBlock), k64.partial, nb, job.out,
                            job.dt_dst);
 }
 
@@ -540,16 +535,14 @@ static void *upload_records(const std::vector<uint16_t> &rec) {
 
 // the per-cell face slots (each cell's first GatherUnroll gather entries:
 // other cell, area vector, weight), read by the one-launch stages and the 3D
-// FP32 gradient kernel; allocated on first use (under the set-up mutex, as a
-// capture on another thread requires) and filled from the gather list on
-// the handle's stream.  When memory cannot be had the gradients read the
+// FP32 gradient kernel; allocated on first use and filled from the gather list
+// on the handle's stream.  When memory cannot be had the gradients read the
 // gather entries and the face arrays and the step runs the separate launches,
 // which gives the same bits.
 bool Solver::ensure_slots32() {
     if (!fp32 || slots_failed) return false;
     if (k32->pk || k32->sl_nb) return true;
     const int D = L.D, U = D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value, nt = table32.n;
-    std::lock_guard<std::mutex> lock(device_setup_mutex());
     void *p[3] = {nullptr, nullptr, nullptr}, *rec = nullptr;
     slots_failed = true;
     if (nt) {
@@ -644,7 +637,6 @@ bool Solver::ensure_slots64() {
     if (k64.s_perm) return true;
     const int D = L.D, U = D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value;
     const size_t words = slot_array_len(L.nc, U, 1) * sizeof(int32_t), perm = (size_t)L.nc * sizeof(int32_t);
-    std::lock_guard<std::mutex> lock(device_setup_mutex());
     void *p[4] = {nullptr, nullptr, nullptr, nullptr}, *rec = nullptr;
     const int nt = table64.n;
     std::vector<double> tab;
@@ -715,10 +707,7 @@ bool Solver::ensure_alt64() {
     void *p = nullptr;
     const size_t bytes = (size_t)(L.D + 2) * ((size_t)L.nc + L.ng) * sizeof(double);
     fused_ok = ensure_slots64();
-    if (fused_ok) {
-        std::lock_guard<std::mutex> lock(device_setup_mutex());
-        fused_ok = alloc_all(&p, &bytes, 1);
-    }
+    if (fused_ok) fused_ok = alloc_all(&p, &bytes, 1);
     q_alt64 = (double *)p;
     return fused_ok;
 }
@@ -731,7 +720,6 @@ bool Solver::ensure_alt32() {
         return false;
     }
     const size_t nq = (size_t)(L.D + 2) * ((size_t)L.nc + L.ng);
-    std::lock_guard<std::mutex> lock(device_setup_mutex());
     void *p = nullptr;
     if (hipMalloc(&p, nq * sizeof(float)) != hipSuccess) {
         (void)hipGetLastError();
@@ -836,19 +824,20 @@ void Solver::step() {
 }
 
 // ---------------------------------------------------------------------------
-// Steps as a captured graph.  A launch costs 2.7 us of host time and 3.6 us
+// Steps as a graph.  A launch costs 2.7 us of host time and 3.6 us
 // from one small kernel to the next; inside a graph of 40 kernels or more the
 // next one starts after 1.8 (4 blocks) to 2.4 us (256 blocks).  A graph of one
 // step's five launches gains nothing (3.7 us per kernel), so it holds
-// kGraphSteps steps.  Capturing costs what it saves in some 500 launches: it is
-// done by a run that continues past kGraphAfter of them.
+// kGraphSteps steps.  Building it costs what it saves in some 500 launches: it is
+// done by a run that continues past kGraphAfter of them, and, where it could not
+// be had, tried again after twice as many.
 // ---------------------------------------------------------------------------
 constexpr long kGraphAfter = 512;
 
 struct Solver::StepGraph {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    // all that the captured launches depend on
+    // all that its launches depend on
     KArgs k64;
     KArgs32 k32;
     const void *alt = nullptr;
@@ -881,7 +870,7 @@ void Solver::free_step_graph() {
 
 // whether the next kGraphSteps steps are one graph launch
 bool Solver::graph_ready() {
-    if (post || prof || graph_failed || ghosts_stale || nstages == 0) return false;
+    if (post || prof || ghosts_stale || nstages == 0) return false;
     // a step leaves its CFL reduction to the next one wherever it can: the
     // steps before the first such step are launched one by one
     if (!prm.adjust_dt && carry_target() != 0 && !cfl_pending) return false;
@@ -892,33 +881,29 @@ bool Solver::graph_ready() {
     // an odd number of one-launch stages swaps the buffers each step: the
     // graph's turn comes with the next one
     if (step_graph && ++graph_misses < 2) return false;
-    return eager_launches >= kGraphAfter && graph_capture();
+    return eager_launches >= std::max(kGraphAfter, graph_after) && graph_build();
 }
 
-bool Solver::graph_capture() {
+bool Solver::graph_build() {
     free_step_graph();
-    auto *g = new StepGraph;
-    std::lock_guard<std::mutex> lock(device_setup_mutex());
+    auto g = std::make_unique<StepGraph>();
     g->note(*this);
-    hipError_t e = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
-    if (e == hipSuccess) {
-        const int64_t done = steps_done;
-        defer_cfl = drop_dq = true;
-        for (int i = 0; i < kGraphSteps; i++) step();
-        steps_done = done;
-        e = hipStreamEndCapture(stream, &g->graph);
-        if (e == hipSuccess) e = hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0);
-    }
+    GraphBuild build;
+    building = &build;
+    const int64_t done = steps_done;
+    defer_cfl = drop_dq = true;
+    for (int i = 0; i < kGraphSteps; i++) step();
+    steps_done = done;
+    building = nullptr;
     eager_launches = 0;
     graph_misses = 0;
-    if (e != hipSuccess || !g->matches(*this)) {
+    if (build.finish(&g->graph, &g->exec) != hipSuccess || !g->matches(*this)) {
         // nothing was launched: the steps follow as launches of their own
-        (void)hipGetLastError();
-        delete g;
-        graph_failed = true;
+        graph_after = 2 * std::max(kGraphAfter, graph_after);
         return false;
     }
-    step_graph = g;
+    graph_after = 0;
+    step_graph = g.release();
     return true;
 }
 
@@ -928,6 +913,7 @@ int Solver::run_steps(int n, bool with_post) {
         if (n - i > kGraphSteps && graph_ready()) {
             HIP_TRY(hipGraphLaunch(step_graph->exec, stream));
             steps_done += kGraphSteps;
+            replayed_steps += kGraphSteps;
             if (prm.have_res) res_valid = true;
             i += kGraphSteps;
             continue;
@@ -989,7 +975,6 @@ int lfm_solver_create_part(const lfm_polymesh *mesh, const lfm_partition *part, 
     s->fp32 = prm->precision == LFM_PREC_FP32P;
     // the Smagorinsky stress does not scale with mu
     s->visc = prm->mu != 0.0 || !prm->laminar;
-    std::lock_guard<std::mutex> lock(lfm::device_setup_mutex());
     HIP_TRY(hipGetDevice(&s->device));
     HIP_TRY(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
     HIP_TRY(hipEventCreate(&s->ev0));
@@ -1152,6 +1137,12 @@ int lfm_run(lfm_solver *h, int nsteps) {
     const int rc = s->run_steps(nsteps, true);
     if (rc) return rc;
     HIP_TRY(hipGetLastError());
+    return LFM_OK;
+}
+
+int lfm_replayed_steps(lfm_solver *h, int64_t *n) {
+    if (!h || !n) return fail(LFM_EINVAL, "null argument");
+    *n = h->impl->replayed_steps;
     return LFM_OK;
 }
 

@@ -178,7 +178,7 @@ int create_fp32p(Solver *s) {
 
 template <int D>
 void launch_bc32(Solver *s) {
-    if (s->L.ng) hipLaunchKernelGGL(bc_fill32<D>, dim3(nblocks(s->L.ng)), dim3(kBlock), 0, s->stream, *s->k32);
+    if (s->L.ng) launch(s, bc_fill32<D>, dim3(nblocks(s->L.ng)), dim3(kBlock), *s->k32);
 }
 
 template <int D, bool V, bool SL, bool PK, bool NT>
@@ -187,11 +187,11 @@ static void launch_gradvis32_nt(Solver *s, bool fin) {
     const dim3 grid(nb + (fin ? 1 : 0));
     const int fb = fin ? nb : 0;
     if (s->prm.solver == 2 && s->prm.minmod)
-        hipLaunchKernelGGL((grad_vis32<D, 2, V, true, SL, PK, NT>), grid, dim3(kBlock), 0, s->stream, *s->k32, fb);
+        launch(s, (grad_vis32<D, 2, V, true, SL, PK, NT>), grid, dim3(kBlock), *s->k32, fb);
     else if (s->prm.solver == 2)
-        hipLaunchKernelGGL((grad_vis32<D, 0, V, true, SL, PK, NT>), grid, dim3(kBlock), 0, s->stream, *s->k32, fb);
+        launch(s, (grad_vis32<D, 0, V, true, SL, PK, NT>), grid, dim3(kBlock), *s->k32, fb);
     else
-        hipLaunchKernelGGL((grad_vis32<D, 0, V, false, SL, PK, NT>), grid, dim3(kBlock), 0, s->stream, *s->k32, fb);
+        launch(s, (grad_vis32<D, 0, V, false, SL, PK, NT>), grid, dim3(kBlock), *s->k32, fb);
 }
 
 template <int D, bool V, bool SL, bool PK>
@@ -233,9 +233,9 @@ template <int D, bool V, bool ST, bool NT>
 static void launch_flux32_nt(Solver *s) {
     const int nb = nblocks(s->L.nf);
     switch (s->prm.solver) {
-    case 0: hipLaunchKernelGGL((face_flux32<D, 0, V, ST, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32); break;
-    case 1: hipLaunchKernelGGL((face_flux32<D, 1, V, ST, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32); break;
-    default: hipLaunchKernelGGL((face_flux32<D, 2, V, ST, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32); break;
+    case 0: launch(s, (face_flux32<D, 0, V, ST, NT>), dim3(nb), dim3(kBlock), *s->k32); break;
+    case 1: launch(s, (face_flux32<D, 1, V, ST, NT>), dim3(nb), dim3(kBlock), *s->k32); break;
+    default: launch(s, (face_flux32<D, 2, V, ST, NT>), dim3(nb), dim3(kBlock), *s->k32); break;
     }
 }
 
@@ -257,18 +257,18 @@ static void launch_update32_nt(Solver *s, double A, double B, int dq_mode, bool 
                                const Solver::CflJob *cfl) {
     const int nb = nblocks(s->L.nc);
     if (res) {
-        hipLaunchKernelGGL((cell_update32<D, true, -1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
+        launch(s, (cell_update32<D, true, -1, NT>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
                            (float)B, dq_mode, 0.0);
-        hipLaunchKernelGGL(reduce_sum, dim3(1), dim3(kBlock), 0, s->stream, s->k32->partial, nb, D + 2, s->d_res,
+        launch(s, reduce_sum, dim3(1), dim3(kBlock), s->k32->partial, nb, D + 2, s->d_res,
                            (int)accumulate_res);
     } else if (cfl && cfl->mode == 0) {
-        hipLaunchKernelGGL((cell_update32<D, false, 0, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
+        launch(s, (cell_update32<D, false, 0, NT>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
                            (float)B, dq_mode, cfl->param);
     } else if (cfl) {
-        hipLaunchKernelGGL((cell_update32<D, false, 1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
+        launch(s, (cell_update32<D, false, 1, NT>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
                            (float)B, dq_mode, cfl->param);
     } else {
-        hipLaunchKernelGGL((cell_update32<D, false, -1, NT>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, (float)A,
+        launch(s, (cell_update32<D, false, -1, NT>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
                            (float)B, dq_mode, 0.0);
     }
 }
@@ -287,15 +287,15 @@ static void launch_fused32_nt(Solver *s, float A, float B, int dq_mode, const KA
                              const Solver::CflJob *cfl, bool fin) {
     const int nb = nblocks(s->L.nc);
     if (!cfl) {
-        hipLaunchKernelGGL((stage_fused32<D, SOLVER, -1, PK, HALF, NT>), dim3(nb + (fin ? 1 : 0)), dim3(kBlock), 0, s->stream, a,
+        launch(s, (stage_fused32<D, SOLVER, -1, PK, HALF, NT>), dim3(nb + (fin ? 1 : 0)), dim3(kBlock), a,
                            qout, A, B, dq_mode, 0.0, fin ? nb : 0);
         return;
     }
     if (cfl->mode == 0)
-        hipLaunchKernelGGL((stage_fused32<D, SOLVER, 0, PK, HALF, NT>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
+        launch(s, (stage_fused32<D, SOLVER, 0, PK, HALF, NT>), dim3(nb), dim3(kBlock), a, qout, A, B,
                            dq_mode, cfl->param, 0);
     else
-        hipLaunchKernelGGL((stage_fused32<D, SOLVER, 1, PK, HALF, NT>), dim3(nb), dim3(kBlock), 0, s->stream, a, qout, A, B,
+        launch(s, (stage_fused32<D, SOLVER, 1, PK, HALF, NT>), dim3(nb), dim3(kBlock), a, qout, A, B,
                            dq_mode, cfl->param, 0);
 }
 
@@ -334,19 +334,19 @@ template <int D>
 void launch_cfl_dt32(Solver *s, int mode, double param, double *out, double *dt_dst) {
     const int nb = nblocks(s->L.nc);
     if (mode == 0) {
-        hipLaunchKernelGGL((cfl_dt_cells32<D, 0>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, param);
-        hipLaunchKernelGGL(cfl_dt_final<0>, dim3(1), dim3(kFinalBlock), 0, s->stream, s->k32->partial, nb, out, dt_dst);
+        launch(s, (cfl_dt_cells32<D, 0>), dim3(nb), dim3(kBlock), *s->k32, param);
+        launch(s, cfl_dt_final<0>, dim3(1), dim3(kFinalBlock), s->k32->partial, nb, out, dt_dst);
     } else {
-        hipLaunchKernelGGL((cfl_dt_cells32<D, 1>), dim3(nb), dim3(kBlock), 0, s->stream, *s->k32, param);
-        hipLaunchKernelGGL(cfl_dt_final<1>, dim3(1), dim3(kFinalBlock), 0, s->stream, s->k32->partial, nb, out, dt_dst);
+        launch(s, (cfl_dt_cells32<D, 1>), dim3(nb), dim3(kBlock), *s->k32, param);
+        launch(s, cfl_dt_final<1>, dim3(1), dim3(kFinalBlock), s->k32->partial, nb, out, dt_dst);
     }
 }
 
 template <int D>
 void launch_integrals32(Solver *s, double *out) {
     const int nb = nblocks(s->L.nc);
-    hipLaunchKernelGGL(integrals32<D>, dim3(nb), dim3(kBlock), 0, s->stream, *s->k32);
-    hipLaunchKernelGGL(reduce_sum, dim3(1), dim3(kBlock), 0, s->stream, s->k32->partial, nb, D + 2, out, 0);
+    launch(s, integrals32<D>, dim3(nb), dim3(kBlock), *s->k32);
+    launch(s, reduce_sum, dim3(1), dim3(kBlock), s->k32->partial, nb, D + 2, out, 0);
 }
 
 template <int D>

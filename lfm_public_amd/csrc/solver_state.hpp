@@ -5,10 +5,10 @@
 
 #include <cstdint>
 #include <memory>
-#include <mutex>
 #include <string>
 #include <vector>
 
+#include "graph_build.hpp"
 #include "kernels_fp64.hpp"
 #include "lfm_hip.h"
 #include "mesh_builder.hpp"
@@ -32,11 +32,6 @@ int fail(int code, const std::string &msg);
         if (e_ != hipSuccess)                                                                    \
             return fail(LFM_EDEVICE, std::string(#expr) + ": " + hipGetErrorString(e_));       \
     } while (0)
-
-// Serialises device set-up (allocation, synchronous uploads) of new solvers
-// with hipGraph capture on other threads: a synchronous copy issued while a
-// capture is open would invalidate it.
-std::mutex &device_setup_mutex();
 
 struct Solver {
     lfm_params prm{};
@@ -187,8 +182,7 @@ struct Solver {
     bool stream_nt = false;
     void size_stage();
     bool sym64 = false;  // every record's weights allow flux_m1_sym
-    // device memory for a set of arrays of one kind, all or none, under the
-    // set-up mutex (which the caller holds)
+    // device memory for a set of arrays of one kind, all or none
     bool alloc_all(void **p, const size_t *bytes, int n);
     // per-cell face slots of the FP32 kernels (k32->pk or k32->sl_*), on
     // first use
@@ -214,16 +208,18 @@ struct Solver {
     void flush_cfl();
     void end_step(bool own_dt);
     // n steps; with_post: the post-processing after each.  Long runs replay
-    // kGraphSteps steps at a time as a captured graph.
+    // kGraphSteps steps at a time as a graph.
     int run_steps(int n, bool with_post);
     static constexpr int kGraphSteps = 8;  // even: the state buffers' roles return
     struct StepGraph;
     StepGraph *step_graph = nullptr;
-    bool graph_failed = false;
-    int graph_misses = 0;        // steps in a row whose launches were not the graph's
-    long eager_launches = 0;     // since the last capture
+    GraphBuild *building = nullptr;  // set while launches become its nodes (launch)
+    int graph_misses = 0;            // steps in a row whose launches were not the graph's
+    long eager_launches = 0;         // since the last graph was built
+    long graph_after = 0;            // and how many of them the next one waits for (0: kGraphAfter)
+    int64_t replayed_steps = 0;
     bool graph_ready();
-    bool graph_capture();
+    bool graph_build();
     void free_step_graph();
     void zero_state_for_step();
 

@@ -8,7 +8,7 @@ Requests (independent 2D cases of uneven size) arrive over time.  The loop
   thread while the GPU keeps stepping the resident ones;
 * keeps every admitted state resident and steps all residents of one scheme
   class with shared launches (lfm_batch: one kernel launch per stage piece
-  covers all of them, one RK step captured as a hipGraph);
+  covers all of them, one RK step as a hipGraph);
 * re-forms the batches at step boundaries, advancing in chunks that end
   exactly when the next resident finishes, so no request over-runs its step
   count and finished ones free their memory at once;
