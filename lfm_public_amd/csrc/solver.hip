@@ -885,7 +885,11 @@ bool Solver::graph_ready() {
 }
 
 bool Solver::graph_build() {
-    free_step_graph();
+    if (step_graph) {
+        // its replays may still be queued: they read what it holds
+        if (hipStreamSynchronize(stream) != hipSuccess) return false;
+        free_step_graph();
+    }
     auto g = std::make_unique<StepGraph>();
     g->note(*this);
     GraphBuild build;
