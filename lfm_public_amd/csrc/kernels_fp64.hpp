@@ -1731,6 +1731,9 @@ static __global__ void __launch_bounds__(256) fill_zero(T *p, T *r, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = r[i] = 0;
 }
+static __global__ void __launch_bounds__(64) set_scalar(double *x, double v) {
+    if (threadIdx.x == 0) *x = v;
+}
 // n <= 64 device values to pinned host memory: 2 us less than a copy of theirs
 static __global__ void __launch_bounds__(64) export_scalars(const double *x, int n, double *host) {
     if ((int)threadIdx.x < n) host[threadIdx.x] = x[threadIdx.x];

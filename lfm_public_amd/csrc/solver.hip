@@ -1091,10 +1091,11 @@ int lfm_one_rk_step(lfm_solver *h, int rk, double dt, double *res) {
     if (!s->halo_ready()) return fail(LFM_ESTATE, "halo set-up not imported for every neighbour");
     const double B = s->B[rk];
     // without adjustTimeStep nothing on the device writes its deltaT, which
-    // is then the last one that was copied there
+    // is then the last one that was set there.  The value goes with the
+    // launch: a copy from host scratch may run after a later call's value is
+    // in it.
     if (s->prm.adjust_dt || !(dt == s->dt)) {
-        s->h_scalar[0] = dt;
-        HIP_TRY(hipMemcpyAsync(s->d_dt_ptr(), s->h_scalar, sizeof(double), hipMemcpyHostToDevice, s->stream));
+        hipLaunchKernelGGL(lfm::set_scalar, dim3(1), dim3(64), 0, s->stream, s->d_dt_ptr(), dt);
         s->dt = dt;
     }
     const bool want_res = res && rk == 0 && s->prm.have_res;
