@@ -68,6 +68,7 @@ struct KArgs32 {
     const int32_t *sl_nb;
     const float *sl_S, *sl_w;
     int more_faces;
+    int own_nb;  // some cell is its own neighbour: no slots, two entries for such a face
     // the second state buffer, in a batch's copy of a member's arguments
     // (the solver's own copy leaves it null)
     float *q_alt;
@@ -946,7 +947,8 @@ __device__ __forceinline__ void refresh_ghost32(const KArgs32 &a, const int g, f
 // ordered gather of one cell's stored face fluxes, sponge and RK update in
 // place, with the cell's boundary ghosts refreshed; res receives the
 // residual, q the updated state
-template <int D, bool RES, bool NT>
+// MORE: some cell may have gather entries beyond the first U
+template <int D, bool RES, bool NT, bool MORE>
 __device__ __forceinline__ void cell_update32_cell(const KArgs32 &a, float A, float B, int dq_mode, const bool drop,
                                                    const int c, float (&res)[D + 2], float (&q)[D + 2], float &vinv) {
     const float dt = (float)(*a.dt);
@@ -988,10 +990,10 @@ __device__ __forceinline__ void cell_update32_cell(const KArgs32 &a, float A, fl
     for (int k = 0; k < D + 2; k++) dq[k] *= A;
 #pragma unroll
     for (int u = 0; u < U; u++) add(u, key[u], key[u] != kNoFace, fr[u]);
-    int e1 = 0, ne = 0;  // entries beyond the first U (a cell has at most kMaxFaces)
-    if (U < kMaxFaces && a.more_faces) {
+    int e1 = 0, ne = 0;  // entries beyond the first U
+    if (MORE && a.more_faces) {
         e1 = a.g_off[c] + U;
-        ne = min(a.g_off[c + 1] - e1, kMaxFaces - U);
+        ne = a.g_off[c + 1] - e1;
         for (int j = 0; j < ne; j++) {
             const int ent = a.g_ent[e1 + j];
             float f1[D + 2];
@@ -1003,23 +1005,19 @@ __device__ __forceinline__ void cell_update32_cell(const KArgs32 &a, float A, fl
     // refresh this cell's boundary ghosts for the next stage
     for (unsigned m = gmask; m; m &= m - 1) {
         const int j = __builtin_ctz(m);
-        const int ent = U >= kMaxFaces || j < U ? a.g_key[key_at<D>(a.nc, j, c)] : a.g_ent[e1 + j - U];
+        const int ent = !MORE || j < U ? a.g_key[key_at<D>(a.nc, j, c)] : a.g_ent[e1 + j - U];
         refresh_ghost32<D, NT>(a, a.fN[ent & kFaceMask] - a.nc, a.q, q);
     }
 }
 
-template <int D, int MODE>
+template <int D, int MODE, bool MORE>
 __device__ __forceinline__ double cfl_cell32(const KArgs32 &a, const int c, const float (&qc)[D + 2], float vinv,
                                              double param);
-
-template <int D, int MODE, class FA>
-__device__ __forceinline__ double cfl_cell32(const KArgs32 &a, const FA &fa, const int c, const float (&qc)[D + 2],
-                                             float vinv, double param);
 
 // every thread of the block must call this (block-wide reductions when RES
 // or CFL).  CFL >= 0 (the last stage of a step): the step's compute_dt (0) /
 // compute_cfl (1) of the updated cells, per-block extrema into a.partial.
-template <int D, bool RES, int CFL, bool NT>
+template <int D, bool RES, int CFL, bool NT, bool MORE>
 __device__ __forceinline__ void cell_update32_body(const KArgs32 &a, float A, float B, int dq_mode, const int c,
                                                    const int lblk, double cfl_param) {
     static_assert(!(RES && CFL >= 0), "the residual and the CFL share a.partial");
@@ -1030,8 +1028,8 @@ __device__ __forceinline__ void cell_update32_body(const KArgs32 &a, float A, fl
     for (int k = 0; k < D + 2; k++) rsq[k] = 0.0;
     if (c < a.nc) {
         float res[D + 2], q[D + 2], vinv;
-        cell_update32_cell<D, RES, NT>(a, A, B, dq_mode, CFL >= 0 && (dq_mode & kDqDrop), c, res, q, vinv);
-        if constexpr (CFL >= 0) cv = cfl_cell32<D, CFL>(a, c, q, vinv, cfl_param);
+        cell_update32_cell<D, RES, NT, MORE>(a, A, B, dq_mode, CFL >= 0 && (dq_mode & kDqDrop), c, res, q, vinv);
+        if constexpr (CFL >= 0) cv = cfl_cell32<D, CFL, MORE>(a, c, q, vinv, cfl_param);
         if (RES) {
 #pragma unroll
             for (int k = 0; k < D + 2; k++) {
@@ -1101,23 +1099,28 @@ struct CflSum32 {
         return v;
     }
 };
-template <int D, int MODE>
+template <int D, int MODE, bool MORE>
 __device__ __forceinline__ double cfl_cell32(const KArgs32 &a, const int c, const float (&qc)[D + 2], float vinv,
                                              double param) {
     CflSum32<D, MODE> t(a, qc);
     constexpr int U = GatherUnroll<D>::value;
     int key[U];
     float S[U][D];
+    // a face counts once: a cell's own face not again as its N
+    auto counted = [&](const int ent) {
+        return ent != kNoFace && !(MORE && a.own_nb && ent < 0 && a.fP[face_of(ent)] == c);
+    };
     load_keys<D, false>(a.g_key, a.nc, 0, c, key);
 #pragma unroll
     for (int j = 0; j < U; j++) load_S32<D>(a.S, face_of(key[j]), S[j]);
 #pragma unroll
-    for (int j = 0; j < U; j++) t.add(S[j], key[j] != kNoFace);
-    if (U < kMaxFaces && a.more_faces) {
-        const int e0 = a.g_off[c], ne = min(a.g_off[c + 1] - e0, kMaxFaces);
+    for (int j = 0; j < U; j++) t.add(S[j], counted(key[j]));
+    if (MORE && a.more_faces) {
+        const int e0 = a.g_off[c], ne = a.g_off[c + 1] - e0;
         for (int j = U; j < ne; j++) {
-            load_S32<D>(a.S, face_of(a.g_ent[e0 + j]), S[0]);
-            t.add(S[0], true);
+            const int ent = a.g_ent[e0 + j];
+            load_S32<D>(a.S, face_of(ent), S[0]);
+            t.add(S[0], counted(ent));
         }
     }
     return t.value(a, qc[0], vinv, param);
@@ -1131,7 +1134,7 @@ __device__ __forceinline__ void cfl_dt_cells32_body(const KArgs32 &a, double par
     if (c < a.nc) {
         float q[D + 2];
         load_q32<D>(a, c, q);
-        v = cfl_cell32<D, MODE>(a, c, q, a.vinv[c], param);
+        v = cfl_cell32<D, MODE, true>(a, c, q, a.vinv[c], param);
     }
     block_extremum<MODE>(v, a.partial + lblk);
 }
@@ -1210,9 +1213,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 3
 face_flux32(KArgs32 a) {
     face_flux32_body<D, SOLVER, VISC, STORED, NT>(a, LFM_TID(blockIdx.x));
 }
-template <int D, bool RES, int CFL, bool NT>
+// MORE in 3D only where some cell is its own neighbour: elsewhere no 3D cell
+// has more than the U entries (O-grid of 1 M cells: 149 us of updates per step
+// without the rest of the list in the kernel, 154 with it)
+template <int D, bool RES, int CFL, bool NT, bool MORE>
 __global__ void __launch_bounds__(256) cell_update32(KArgs32 a, float A, float B, int dq_mode, double cfl_param) {
-    cell_update32_body<D, RES, CFL, NT>(a, A, B, dq_mode, LFM_TID(blockIdx.x), LFM_BLK(), cfl_param);
+    cell_update32_body<D, RES, CFL, NT, MORE>(a, A, B, dq_mode, LFM_TID(blockIdx.x), LFM_BLK(), cfl_param);
 }
 // ---------------------------------------------------------------------------
 // One RK stage in one launch for inviscid M1 / M2: each cell forms its faces'
@@ -1477,7 +1483,7 @@ __global__ void __launch_bounds__(256) cell_update32_b(const KArgs32 *args, Batc
     int r, lb;
     batch_slot(m, r, lb);
     const KArgs32 &a = args[r];
-    cell_update32_body<D, false, CFL, NT>(a, A, B, dq_mode, lb * 256 + threadIdx.x, lb, CFL >= 0 ? *a.dt : 0.0);
+    cell_update32_body<D, false, CFL, NT, true>(a, A, B, dq_mode, lb * 256 + threadIdx.x, lb, CFL >= 0 ? *a.dt : 0.0);
 }
 // one-launch stage over a batch (inviscid M1 / M2), each member from one
 // of its state buffers into the other: flip 0 from a.q into a.q_alt, flip 1

@@ -108,6 +108,14 @@ inline int max_entries(const SolverLayout &L) {
     return m;
 }
 
+// whether some cell is its own neighbour (a cyclic pair one cell apart): it has
+// two gather entries for such a face, as its P and as its N
+inline bool own_neighbour(const SolverLayout &L) {
+    for (int f = 0; f < L.nf; f++)
+        if (L.fP[f] == L.fN[f]) return true;
+    return false;
+}
+
 // bits that hold an index below n
 inline int index_bits(long n) {
     int b = 1;

@@ -218,8 +218,7 @@ static int create_fp64(Solver *s) {
     // one-launch stages; a cell that is its own neighbour (a cyclic pair one
     // cell apart) has more gather entries than slots and keeps the launches
     // that walk the list
-    s->fused_ok = !s->visc && s->prm.solver < 2 && L.halo.empty();
-    for (size_t f = 0; f < nf && s->fused_ok; f++) s->fused_ok = L.fP[f] != L.fN[f];
+    s->fused_ok = !s->visc && s->prm.solver < 2 && L.halo.empty() && !own_neighbour(L);
     a.more_faces = max_entries(L) > (D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value);
     if (s->build_gather_keys(a, true)) return LFM_EDEVICE;
     if (s->fused_ok) {

@@ -124,11 +124,13 @@ int create_fp32p(Solver *s) {
         // one-launch stages (a second state buffer, allocated on the first
         // step that uses it; its unset-patch ghosts are copied from q by the
         // first fused stage)
-        s->fused_ok = !s->visc && s->prm.solver < 2 && L.halo.empty();
+        a.own_nb = own_neighbour(L);
+        s->fused_ok = !s->visc && s->prm.solver < 2 && L.halo.empty() && !a.own_nb;
         a.more_faces = max_entries(L) > (D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value);
         // slots are read by the one-launch stage and by 3D gradients (a halo
-        // face has its weight only after the import: no table there)
-        if (s->fused_ok || (D == 3 && L.halo.empty())) {
+        // face has its weight only after the import: no table there; a cell that
+        // is its own neighbour has more entries than slots)
+        if (s->fused_ok || (D == 3 && L.halo.empty() && !a.own_nb)) {
             a.pk_shift = index_bits((long)ntot);
             const long fit = ((1L << (32 - a.pk_shift)) - 1) / 2;
             s->table32 = face_table<float>(L, (int)std::min<long>(fit, kMaxTable32));
@@ -214,7 +216,7 @@ void launch_gradvis32(Solver *s, bool full, bool fin) {
     if (!full && !s->visc && s->prm.solver != 2) return;
     const bool V = full || s->visc;
     if constexpr (D == 3) {
-        if ((s->stream_nt || s->table32.n > 0 || s->k32->pk) && s->ensure_slots32()) {
+        if (!s->k32->own_nb && (s->stream_nt || s->table32.n > 0 || s->k32->pk) && s->ensure_slots32()) {
             if (s->k32->pk) {
                 V ? launch_gradvis32_v<D, true, true, true>(s, fin) : launch_gradvis32_v<D, false, true, true>(s, fin);
                 return;
@@ -252,23 +254,23 @@ void launch_flux32(Solver *s) {
         launch_flux32_v<D, false, false>(s);
 }
 
-template <int D, bool NT>
+template <int D, bool NT, bool MORE>
 static void launch_update32_nt(Solver *s, double A, double B, int dq_mode, bool res, bool accumulate_res,
                                const Solver::CflJob *cfl) {
     const int nb = nblocks(s->L.nc);
     if (res) {
-        launch(s, (cell_update32<D, true, -1, NT>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
+        launch(s, (cell_update32<D, true, -1, NT, MORE>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
                            (float)B, dq_mode, 0.0);
         launch(s, reduce_sum, dim3(1), dim3(kBlock), s->k32->partial, nb, D + 2, s->d_res,
                            (int)accumulate_res);
     } else if (cfl && cfl->mode == 0) {
-        launch(s, (cell_update32<D, false, 0, NT>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
+        launch(s, (cell_update32<D, false, 0, NT, MORE>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
                            (float)B, dq_mode, cfl->param);
     } else if (cfl) {
-        launch(s, (cell_update32<D, false, 1, NT>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
+        launch(s, (cell_update32<D, false, 1, NT, MORE>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
                            (float)B, dq_mode, cfl->param);
     } else {
-        launch(s, (cell_update32<D, false, -1, NT>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
+        launch(s, (cell_update32<D, false, -1, NT, MORE>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
                            (float)B, dq_mode, 0.0);
     }
 }
@@ -276,8 +278,10 @@ static void launch_update32_nt(Solver *s, double A, double B, int dq_mode, bool 
 template <int D>
 void launch_update32(Solver *s, double A, double B, int dq_mode, bool res, bool accumulate_res,
                      const Solver::CflJob *cfl) {
-    s->stream_nt ? launch_update32_nt<D, true>(s, A, B, dq_mode, res, accumulate_res, cfl)
-                 : launch_update32_nt<D, false>(s, A, B, dq_mode, res, accumulate_res, cfl);
+    if constexpr (D == 3)
+        if (s->k32->own_nb) return launch_update32_nt<3, false, true>(s, A, B, dq_mode, res, accumulate_res, cfl);
+    s->stream_nt ? launch_update32_nt<D, true, D == 2>(s, A, B, dq_mode, res, accumulate_res, cfl)
+                 : launch_update32_nt<D, false, D == 2>(s, A, B, dq_mode, res, accumulate_res, cfl);
 }
 
 // fin: one block more reduces the CFL maxima of the previous step's last
