@@ -58,8 +58,9 @@ struct KArgs32 {
     // (the first GatherUnroll gather entries of each cell): either packed
     // words (pk_at; the other cell in the low pk_shift bits, above them the
     // face's record in the geometry table pk_tab) or, where the mesh has too
-    // many distinct records, the other cell, the area vector out of the cell
-    // and the cell's own weight (sl_*, as slot_at places them).  A slot past
+    // many distinct records, the other cell (~other where the cell is the face's
+    // N), the area vector out of the cell and P's weight (sl_*, as slot_at
+    // places them).  A slot past
     // the cell's last entry holds the cell itself with zero area, so its flux
     // is zero.  more_faces: some cell has entries beyond the slots.
     const uint32_t *pk;
@@ -80,13 +81,22 @@ struct KArgs32 {
 
 #define LERP32(w, a, b) ((w) * (a) + (1.0f - (w)) * (b))
 
-// A face value from its two cells, wc c + wo o, with both products rounded
-// before the sum: exchanging the cells gives the same bits, so a face seen
-// from either side has one value (also where the products are subnormal).
-__device__ __forceinline__ float face_value32(float wc, float c, float wo, float o) {
+// The same from the cell's side: wc of its own value, wo of the other's
+__device__ __forceinline__ float cell_lerp32(float wc, float c, float wo, float o) {
+    return __builtin_fmaf(wc, c, wo * o);
+}
+// LERP32 at w = 1/2, both products rounded before the sum (they are exact, short
+// of the subnormal range): exchanging the cells gives the same bits
+__device__ __forceinline__ float half_lerp32(float c, float o) {
 #pragma clang fp contract(off)
-    const float x = wc * c, y = wo * o;
+    const float x = 0.5f * c, y = 0.5f * o;
     return x + y;
+}
+// LERP32 of a face's P and N where the one-launch stage must find the bits of
+// the face kernel: from half_lerp32 where w is 1/2
+__device__ __forceinline__ float face_lerp32(float w, float P, float N) {
+    const float v = __builtin_fmaf(w, P, (1.0f - w) * N), h = half_lerp32(P, N);
+    return w == 0.5f ? h : v;
 }
 // M2's midpoint
 __device__ __forceinline__ float midpoint32(float c, float o) { return 0.5f * (c + o); }
@@ -351,33 +361,39 @@ __device__ __forceinline__ size_t pk_at(int nc, int j, int c) {
 inline size_t pk_len(int D, int nc, int U) { return D == 2 ? (size_t)U * nc : slot_array_len(nc, U, 1); }
 
 // one face as one of its cells sees it: the other cell, the area vector out
-// of the cell and the cell's weight (the other's is 1 - wc, exactly:
-// canonical_w)
+// of the cell, P's weight and whether the cell is the face's P
 template <int D, bool PK, bool NT>
 struct FaceOf32 {
     int other;
-    float S[D], wc;
-    // key: the packed word, or the slot's other cell
+    float S[D], w;
+    bool isP;
+    // the weights of the cell's value and of the other's
+    __device__ __forceinline__ float wc() const { return isP ? w : 1.0f - w; }
+    __device__ __forceinline__ float wo() const { return isP ? 1.0f - w : w; }
+    // key: the packed word (an odd record is N's), or the slot's other cell (~other
+    // where the cell is the face's N)
     __device__ __forceinline__ static int load_key(const KArgs32 &a, const int j, const int c) {
         if constexpr (PK) return (int)ld_once<NT>(a.pk + pk_at<D>(a.nc, j, c));
         return ld_once<NT>(a.sl_nb + slot_at<D, 1>(a.nc, j, 0, c));
     }
     __device__ __forceinline__ static int other_of(const KArgs32 &a, const int key) {
         if constexpr (PK) return (int)((uint32_t)key & ((1u << a.pk_shift) - 1u));
-        return key;
+        return key >= 0 ? key : ~key;
     }
     __device__ __forceinline__ void load(const KArgs32 &a, const int j, const int c, const int key) {
         other = other_of(a, key);
         if constexpr (PK) {
+            isP = !((uint32_t)key >> a.pk_shift & 1u);
             const float4 v = reinterpret_cast<const float4 *>(a.pk_tab)[(uint32_t)key >> a.pk_shift];
             const float r[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
             for (int k = 0; k < D; k++) S[k] = r[k];
-            wc = r[D];
+            w = r[D];
         } else {
 #pragma unroll
             for (int k = 0; k < D; k++) S[k] = ld_once<NT>(a.sl_S + slot_at<D, D>(a.nc, j, k, c));
-            wc = ld_once<NT>(a.sl_w + slot_at<D, 1>(a.nc, j, 0, c));
+            w = ld_once<NT>(a.sl_w + slot_at<D, 1>(a.nc, j, 0, c));
+            isP = key >= 0;
         }
     }
     // an entry of the gather list
@@ -387,13 +403,12 @@ struct FaceOf32 {
     }
     // its face's data alone
     __device__ __forceinline__ void load_face(const KArgs32 &a, const int ent) {
-        const bool isP = ent >= 0;
+        isP = ent >= 0;
         const int f = face_of(ent);
-        const float w = a.w[f];
+        w = a.w[f];
         load_S32<D>(a.S, f, S);
 #pragma unroll
         for (int k = 0; k < D; k++) S[k] = isP ? S[k] : -S[k];
-        wc = isP ? w : 1.0f - w;
     }
 };
 
@@ -420,14 +435,14 @@ __device__ __forceinline__ Prim32<D> grad32_sums(const KArgs32 &a, const int c, 
     // one face's contribution
     auto add = [&](const F &f, const float (&qo)[D + 2]) {
         const Prim32<D> so = prim32<D>(a, qo);
-        const float wo = 1.0f - f.wc;
+        const float wc = f.wc(), wo = f.wo();
         float sv[D];
 #pragma unroll
         for (int k = 0; k < D; k++) sv[k] = f.S[k] * vinv;
         float fU[D];
 #pragma unroll
-        for (int k = 0; k < D; k++) fU[k] = face_value32(f.wc, own.up[k], wo, so.up[k]);
-        const float fT = VISC ? face_value32(f.wc, own.Rp, wo, so.Rp) * a.R_inv : 0.f;
+        for (int k = 0; k < D; k++) fU[k] = cell_lerp32(wc, own.up[k], wo, so.up[k]);
+        const float fT = VISC ? cell_lerp32(wc, own.Rp, wo, so.Rp) * a.R_inv : 0.f;
 #pragma unroll
         for (int i = 0; i < D; i++) {
 #pragma unroll
@@ -435,8 +450,8 @@ __device__ __forceinline__ Prim32<D> grad32_sums(const KArgs32 &a, const int c, 
             if (VISC) dTdx[i] += fT * sv[i];
         }
         if (GRAD == 2) {
-            const float rf = face_value32(f.wc, own.rp, wo, so.rp);
-            const float pf = face_value32(f.wc, own.pp, wo, so.pp);
+            const float rf = cell_lerp32(wc, own.rp, wo, so.rp);
+            const float pf = cell_lerp32(wc, own.pp, wo, so.pp);
 #pragma unroll
             for (int i = 0; i < D; i++) {
                 pg[i] += pf * sv[i];
@@ -610,38 +625,38 @@ struct GradGlobal32 {
 // ---------------------------------------------------------------------------
 // The convective flux of one face (M1 cfd_v0.cpp:2590-2637, M2 1968-2023)
 // seen from one of its cells: c the cell, o the other, S out of the cell.
-// Every face value is the same from both sides and every other term changes
-// sign with S, so the flux from N is P's negated, bit for bit, and the
-// one-launch stage forms a face from either side without selecting.
+// Every face value is formed from P's and N's, whichever of them c is (isP; M2's
+// midpoint and M1 at w = 1/2 are the same with the two exchanged and need no
+// selecting), and every other term changes sign with S, so the flux from N is
+// P's negated, bit for bit.  HALF: every weight is 1/2.
 template <int D>
 struct Conv32 {
-    float rp, rho, mp[D], phip, phi, pp, Gdev;
+    float rp, rho, mp[D], phi_inf, phip, phi, pp, Gdev;
 };
 template <int D, int SOLVER, bool HALF>
 __device__ __forceinline__ Conv32<D> conv32(const KArgs32 &a, const float (&qc)[D + 2], const Prim32<D> &sc,
                                             const float (&qo)[D + 2], const Prim32<D> &so, const float (&S)[D],
-                                            const float wc, const float wo) {
+                                            const float w, const bool isP) {
     Conv32<D> f;
     auto face = [&](const float c, const float o) {
         if constexpr (SOLVER != 0) return midpoint32(c, o);
-        // every weight 1/2: the cell's own products are formed once per cell
-        if constexpr (HALF) return face_value32(0.5f, c, 0.5f, o);
-        return face_value32(wc, c, wo, o);
+        if constexpr (HALF) return half_lerp32(c, o);  // the cell's own products are formed once per cell
+        return face_lerp32(w, isP ? c : o, isP ? o : c);
     };
     f.rp = face(qc[0], qo[0]);
     f.rho = a.rho_inf + f.rp;
     const float ri = rcp32(f.rho);
-    float phi_inf = 0.f, du2 = 0.f;
-    f.phip = 0.f;
+    float du2 = 0.f;
+    f.phip = f.phi_inf = 0.f;
 #pragma unroll
     for (int k = 0; k < D; k++) {
-        phi_inf += a.uinf[k] * S[k];
+        f.phi_inf += a.uinf[k] * S[k];
         f.mp[k] = face(qc[k + 1], qo[k + 1]);
         const float up = (f.mp[k] - a.uinf[k] * f.rp) * ri;
         f.phip += up * S[k];
         if (SOLVER == 0) du2 += up * (2.f * a.uinf[k] + up);
     }
-    f.phi = phi_inf + f.phip;
+    f.phi = f.phi_inf + f.phip;
     const float Rp = face(sc.Rp, so.Rp);
     f.pp = f.rp * a.Rpsi_inf + f.rho * Rp;
     // M1: G = rhoE + p = rho (g/(g-1) Rpsi + |u|^2/2) of the face state; M2:
@@ -693,10 +708,10 @@ __device__ __forceinline__ void face_flux32_states(const KArgs32 &a, const int f
 #pragma unroll
     for (int k = 0; k < D; k++) Sm2 += S[k] * S[k];
     const float Sm = sqrt32(Sm2);
-    const Conv32<D> cv = conv32<D, SOLVER, false>(a, qP, sp, qN, sn, S, w, 1.0f - w);
+    const Conv32<D> cv = conv32<D, SOLVER, false>(a, qP, sp, qN, sn, S, w, true);
     float pp = cv.pp;
     if (SOLVER == 2) {
-        const float phi_inf = cv.phi - cv.phip;
+        const float phi_inf = cv.phi_inf;
         const float cP = sqrt32(a.gamma * sp.R), cN = sqrt32(a.gamma * sn.R);
         const float cavg = 0.5f * (cP + cN);
         float cdiv = 0.f, ndiv = 0.f, ccurl = 0.f, ncurl = 0.f, unP = 0.f, unN = 0.f;
@@ -1267,7 +1282,7 @@ __device__ __forceinline__ void stage32_body(const KArgs32 &a, float *qout, floa
         const float s = dt * vinv;
         auto add = [&](const F &f, const float (&qo)[D + 2]) {
             const Prim32<D> so = prim32<D>(a, qo);
-            const Conv32<D> cf = conv32<D, SOLVER, HALF>(a, qc, sc, qo, so, f.S, f.wc, 1.0f - f.wc);
+            const Conv32<D> cf = conv32<D, SOLVER, HALF>(a, qc, sc, qo, so, f.S, f.w, f.isP);
             float r[D + 2];
             conv_rhs32<D>(a, cf, cf.pp, f.S, r);
 #pragma unroll
@@ -1377,7 +1392,8 @@ __global__ void __launch_bounds__(256) build_slots32(KArgs32 a, const uint16_t *
     for (int j = 0; j < U; j++) {
         FaceOf32<D, false, false> f;
         f.other = c;
-        f.wc = 0.5f;
+        f.w = 0.5f;
+        f.isP = true;
         for (int k = 0; k < D; k++) f.S[k] = 0.f;
         int rec = none;
         if (j < ne) {
@@ -1389,10 +1405,10 @@ __global__ void __launch_bounds__(256) build_slots32(KArgs32 a, const uint16_t *
             pk[pk_at<D>(a.nc, j, c)] = (uint32_t)f.other | (uint32_t)rec << a.pk_shift;
             continue;
         }
-        nb[slot_at<D, 1>(a.nc, j, 0, c)] = f.other;
+        nb[slot_at<D, 1>(a.nc, j, 0, c)] = f.isP ? f.other : ~f.other;
 #pragma unroll
         for (int k = 0; k < D; k++) S[slot_at<D, D>(a.nc, j, k, c)] = f.S[k];
-        w[slot_at<D, 1>(a.nc, j, 0, c)] = f.wc;
+        w[slot_at<D, 1>(a.nc, j, 0, c)] = f.w;
     }
 }
 
@@ -1499,10 +1515,12 @@ __global__ void __launch_bounds__(256) stage_fused32_b(const KArgs32 *args, Batc
     const int c = lb * 256 + threadIdx.x;
     const double dt = CFL >= 0 ? *a.dt : 0.0;
     // members may hold either slot form
-    if (a.pk)
-        stage32_body<D, SOLVER, CFL, true, false, NT>(a, qout, A, B, dq_mode, c, lb, dt);
+    if (a.pk && (SOLVER == 1 || a.pk_half))
+        stage32_body<D, SOLVER, CFL, true, true, NT>(a, qout, A, B, dq_mode, c, lb, dt);
+    else if (a.pk)
+        stage32_body<D, SOLVER, CFL, true, SOLVER == 1, NT>(a, qout, A, B, dq_mode, c, lb, dt);
     else
-        stage32_body<D, SOLVER, CFL, false, false, NT>(a, qout, A, B, dq_mode, c, lb, dt);
+        stage32_body<D, SOLVER, CFL, false, SOLVER == 1, NT>(a, qout, A, B, dq_mode, c, lb, dt);
 }
 // one block per solver: max of its partials into its CFL scalar
 static __global__ void __launch_bounds__(256) cfl_final32_b(const KArgs32 *args) {

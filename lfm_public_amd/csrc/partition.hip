@@ -95,7 +95,7 @@ int Solver::halo_upload_geometry() {
     if (fp32) {
         std::vector<float> d(L.d.size()), w(L.w.size());
         for (size_t i = 0; i < d.size(); i++) d[i] = (float)L.d[i];
-        for (size_t i = 0; i < w.size(); i++) w[i] = canonical_w((float)L.w[i]);
+        for (size_t i = 0; i < w.size(); i++) w[i] = (float)L.w[i];
         HIP_TRY(hipMemcpy((void *)k32->d, d.data(), D * nf * sizeof(float), hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy((void *)k32->w, w.data(), nf * sizeof(float), hipMemcpyHostToDevice));
     } else {

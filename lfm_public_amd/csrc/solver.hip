@@ -545,16 +545,16 @@ bool Solver::ensure_slots32() {
     void *p[3] = {nullptr, nullptr, nullptr}, *rec = nullptr;
     slots_failed = true;
     if (nt) {
-        // each record as P sees it, then as N does, and a placeholder's
+        // each record with S as P sees it, then as N does, and a placeholder's
         std::vector<float> tab((size_t)(2 * nt + 1) * 4, 0.f);
         bool half = true;
         for (int i = 0; i < 2 * nt; i++) {
-            const float w = canonical_w(table32.w[i / 2]);
+            const float w = table32.w[i / 2];
             for (int k = 0; k < D; k++) {
                 const float x = table32.S[(size_t)(i / 2) * D + k];
                 tab[(size_t)i * 4 + k] = i % 2 ? -x : x;
             }
-            tab[(size_t)i * 4 + D] = i % 2 ? 1.0f - w : w;
+            tab[(size_t)i * 4 + D] = w;
             half = half && w == 0.5f;
         }
         tab[(size_t)2 * nt * 4 + D] = 0.5f;

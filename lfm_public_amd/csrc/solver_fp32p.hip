@@ -88,7 +88,6 @@ int create_fp32p(Solver *s) {
         for (size_t f = 0; f < nf; f++)
             for (int k = 0; k < D; k++) S[f * D + k] = (float)L.S[(size_t)k * nf + f];
         auto d = to_f32(L.d), w = to_f32(L.w);
-        for (float &x : w) x = canonical_w(x);
         rc |= up(s, (float **)&a.S, S.data(), S.size());
         rc |= up(s, (float **)&a.d, d.data(), d.size());
         rc |= up(s, (float **)&a.w, w.data(), w.size());

@@ -174,7 +174,7 @@ struct Solver {
     // the FP64 one-launch stage's slots (k64.pk or k64.sl_*, k64.s_perm), on
     // first use; the distinct face records found when the handle was created
     FaceTable<double> table64;
-    FaceTable<float> table32;  // of the FP32 slots (canonical_w weights)
+    FaceTable<float> table32;  // of the FP32 slots
     bool ensure_slots64();
     // bytes one stage touches; whether it outgrows the Infinity Cache, so that
     // its kernels stream what they touch once past the caches
@@ -248,12 +248,6 @@ struct Solver {
 // 384 (139), 881 / 837 (356); FP64 O-grid 382 / 441 (157), 756 / 789 (314), 1440
 // / 1363 (558); FP64 box 386 / 460 (225), 645 / 654 (336), 915 / 903 (478).
 inline bool outgrows_cache(size_t bytes) { return bytes > (size_t)330 * 1000 * 1000; }
-
-// The FP32 path's weights are rounded to those whose complement is exact, so
-// that w and 1 - w, formed from either cell's side, are the same two numbers
-// (a change of at most 2^-25 to weights below one half, what rounding 1 - w
-// takes from them anyway).
-inline float canonical_w(float w) { return 1.0f - (1.0f - w); }
 
 int create_fp32p(Solver *s);
 void free_k32(KArgs32 *k);
