@@ -87,7 +87,7 @@ def cpu_sample_case(workload, case):
 def launch_plan(prm, nstages):
     """Launches per time step by profiling group, as Solver::step issues them:
     {group: (launches, kernel name up to the parameters that depend on the
-    mesh)}.  Inviscid M1/M2 runs every stage (but a residual stage 0) as one
+    mesh: slot form, non-temporal marks)}.  Inviscid M1/M2 runs every stage (but a residual stage 0) as one
     stage_fused32 / stage_fused64 launch; other paths run
     grad_vis (when it has work), face_flux and cell_update per stage.  The
     last stage's launch also forms the CFL/dt block extrema, except on the
@@ -109,18 +109,16 @@ def launch_plan(prm, nstages):
             plan["face_flux"] = (first, f"face_flux{sfx}<{D}, {S}, false, false")
         return plan
     rg = S == 2 and prm.get("minmod")
-    plan = {"face_flux": (nstages, f"face_flux{sfx}<{D}, {S}, {str(visc).lower()}, false>")}
+    plan = {"face_flux": (nstages, f"face_flux{sfx}<{D}, {S}, {str(visc).lower()}, false")}
     if fp32 or D == 2:
-        plan["cell_update"] = (nstages - 1, f"cell_update{sfx}<{D}, false, -1>")
-        plan["cell_update_cfl"] = (1, f"cell_update{sfx}<{D}, false, {mode}>")
+        plan["cell_update"] = (nstages - 1, f"cell_update{sfx}<{D}, false, -1")
+        plan["cell_update_cfl"] = (1, f"cell_update{sfx}<{D}, false, {mode}")
     else:
-        plan["cell_update"] = (nstages, f"cell_update<{D}, false, -1>")
+        plan["cell_update"] = (nstages, f"cell_update<{D}, false, -1")
         plan["cfl_dt"] = (1, f"cfl_dt_cells<{D}, {mode}>")
     if visc or S == 2:
-        # FP32 3D gradients read the face slots (the kernel's last parameter)
-        slots = f", {str(D == 3).lower()}" if fp32 else ">"
         plan["grad_vis"] = (nstages, f"grad_vis{sfx}<{D}, {2 if rg else 0}, {str(visc).lower()}, "
-                                     f"{str(S == 2).lower()}{slots}")
+                                     f"{str(S == 2).lower()}")
     return plan
 
 
