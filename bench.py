@@ -330,6 +330,13 @@ def roofline(case, nf, path_prm, nstages, prof, nprof, ms_step, w, traffic_key):
     out["traffic"] = traffic
     if traffic:
         out["traffic_source"] = src
+        # what the dominant kernel moves over HBM, over its mean launch time
+        moved = traffic / (per_launch[dom] * 1e-3) / 1e9
+        out["traffic_achieved"] = round(moved, 1)
+        out["traffic_frac"] = round(moved / HBM_PEAK_GBS, 4)
+        if one_stage and traffic < B:
+            out["frac_basis"] = ("frac and step_frac count every face's geometry, which packed slots do not move; "
+                                 "traffic_frac is the measured share of the HBM peak")
         out["traffic_over_algorithmic"] = round(traffic / B, 3) if one_stage else None
     return out
 
