@@ -123,6 +123,45 @@ inline int index_bits(long n) {
     return b;
 }
 
+// What one RK stage touches, in bytes, each array once.
+struct StageShape {
+    int D = 3;
+    size_t word = 4, nc = 0, nf = 0;  // bytes per value; cells, faces
+    bool one_launch = false;          // stage_fused32 / 64, otherwise gradients, fluxes and update
+    bool packed = false;              // slots of one word over a face table
+    size_t grad_values = 0;           // values of a cell's gradient record (0: no gradients)
+};
+inline size_t stage_footprint(const StageShape &s) {
+    const size_t D = s.D, w = s.word, U = D == 2 ? 4 : 6, key = sizeof(int32_t);
+    size_t cell = (2 * (D + 2) + 2) * w, face = 0;  // state, RK register, 1/V, sponge
+    if (s.one_launch) {
+        // second state; slots: one word each, or a face's own data
+        cell += (D + 2) * w + U * (s.packed ? key : key + (D + 1) * w);
+    } else {
+        // face fluxes, S, d, w, both cells; the update's gather entries
+        face += (3 * D + 3) * w + 2 * key;
+        cell += U * key;
+        // gradients: the record, and one word more per entry (the cell it leads
+        // to, or a packed slot).  Unpacked slots are not counted: gradients read
+        // them only past the line that this footprint is held against.
+        if (s.grad_values) cell += s.grad_values * w + U * key;
+    }
+    return s.nc * cell + s.nf * face;
+}
+// Streams are marked non-temporal from 330 MB touched per stage: below, part of
+// what one launch writes is still in the 256 MB Infinity Cache when the next
+// reads it, and marking loses that; above, marking keeps the gathered
+// neighbours in L2.  us per step plain / marked (MB per stage): FP32 3D box
+// 117 / 150 (81), 229 / 307 (193), 383 / 424 (275), 573 / 566 (377), 978 / 946
+// (651); viscous 251 / 306 (161), 526 / 542 (313), 659 / 670 (394), 923 / 890
+// (541); FP32 O-grid 182 / 218 (92), 327 / 377 (186), 365 / 399 (204), 535 / 548
+// (286), 609 / 615 (327), 709 / 695 (368), 1015 / 957 (516), M2AUSM 447 / 484
+// (220), 645 / 655 (308); FP32 annulus 317 / 389 (177); FP64 annulus 181 / 188
+// (60), 343 / 384 (139), 881 / 837 (356); FP64 O-grid 382 / 441 (157), 756 / 789
+// (314), 1440 / 1363 (558); FP64 box 386 / 460 (225), 645 / 654 (336), 915 / 903
+// (478).
+inline bool outgrows_cache(size_t bytes) { return bytes > (size_t)330 * 1000 * 1000; }
+
 // Gas constants derived as set_init_conditions does (cfd_v0.cpp:880-902).
 struct Gas {
     double R, R_inv, gamma, gm1, cp, mu, pr_inv;

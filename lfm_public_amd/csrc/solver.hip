@@ -595,24 +595,16 @@ bool Solver::ensure_slots32() {
 // What one RK stage touches, and whether its kernels mark what they touch once
 // as non-temporal.
 void Solver::size_stage() {
-    const size_t D = L.D, w = fp32 ? sizeof(float) : sizeof(double), nc = L.nc, nf = L.nf;
-    const bool grads = visc || prm.solver == 2;
-    const size_t keys = keys_len(L.D, L.nc) * sizeof(int32_t);  // gather entries
-    size_t b = nc * ((2 * (D + 2) + 2) * w);  // state, RK register, 1/V, sponge
-    if (fused_ok) {
-        // second state; slots: one word each, or a face's own data
-        const bool packed = fp32 ? table32.n > 0 : table64.n > 0;
-        const size_t U = D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value;
-        b += nc * ((D + 2) * w + U * (packed ? sizeof(int32_t) : sizeof(int32_t) + (D + 1) * w));
-    } else {
-        // face fluxes, S, d, w, both cells; gather entries
-        b += nf * ((3 * D + 3) * w + 2 * sizeof(int32_t)) + keys;
-        if (grads && !(fp32 && D == 3)) b += keys;  // the cells they lead to (3D FP32: the slots below)
-    }
-    if (grads) b += nc * (size_t)(fp32 ? k32->gstride : k64.gstride) * w;
-    if (grads && fp32 && D == 3) b += nc * GatherUnroll<3>::value * (sizeof(int32_t) + (D + 1) * w);  // slots
-    stage_bytes = b;
-    stream_nt = outgrows_cache(b);
+    StageShape sh;
+    sh.D = L.D;
+    sh.word = fp32 ? sizeof(float) : sizeof(double);
+    sh.nc = L.nc;
+    sh.nf = L.nf;
+    sh.one_launch = fused_ok;
+    sh.packed = fp32 ? table32.n > 0 : table64.n > 0;
+    if (visc || prm.solver == 2) sh.grad_values = fp32 ? k32->gstride : k64.gstride;
+    stage_bytes = stage_footprint(sh);
+    stream_nt = outgrows_cache(stage_bytes);
 }
 
 bool Solver::alloc_all(void **p, const size_t *bytes, int n) {

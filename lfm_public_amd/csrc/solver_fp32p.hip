@@ -204,8 +204,8 @@ static void launch_gradvis32_v(Solver *s, bool fin) {
 // they read the faces' own data, from slots where the stage outgrows the
 // Infinity Cache (consecutive, 120 B per cell) and through the gather entries
 // where it does not (97 B, gathered); the bits are the same.  Slots against
-// entries per step: O-grid of 74 k cells 81.9 / 79.4 us, 193 k 131.8 / 130.1,
-// 1 M 615 / 640, 4.2 M 2399 / 2548.  2D gradients use the entries: there the
+// entries, us per step: O-grid of 74 k cells 81.9 / 79.4, 193 k 131.8 / 130.1,
+// 0.92 M 548 / 535, 1.05 M (327 MB) 615 / 609, 1.18 M 695 / 709, 4.2 M 2399 / 2548.  2D gradients use the entries: there the
 // slot streams cost more than the cached face records they replace (1 M-cell
 // annulus 0.114 -> 0.134 ms per step with slots).  fin: the launch also reduces
 // the previous step's CFL maxima in one extra block (the caller knows the

@@ -238,17 +238,6 @@ struct Solver {
     int check_finite_noalloc(int64_t *n_bad);
 };
 
-// Streams are marked non-temporal from 330 MB touched per stage: below, part of
-// what one launch writes is still in the 256 MB Infinity Cache when the next
-// reads it, and marking loses that; above, marking keeps the gathered
-// neighbours in L2.  us per step plain / marked (MB per stage): FP32 3D box
-// 117 / 150 (81), 229 / 307 (193), 383 / 424 (275), 573 / 566 (377), 978 / 946
-// (651); FP32 O-grid 182 / 218 (121), 327 / 377 (243), 640 / 628 (432), 1015 /
-// 957 (675); FP32 annulus 317 / 389 (177); FP64 annulus 181 / 188 (60), 343 /
-// 384 (139), 881 / 837 (356); FP64 O-grid 382 / 441 (157), 756 / 789 (314), 1440
-// / 1363 (558); FP64 box 386 / 460 (225), 645 / 654 (336), 915 / 903 (478).
-inline bool outgrows_cache(size_t bytes) { return bytes > (size_t)330 * 1000 * 1000; }
-
 int create_fp32p(Solver *s);
 void free_k32(KArgs32 *k);
 int get_field32(Solver *s, int which, double *out);
