@@ -184,6 +184,7 @@ static int batch_set(Batch *b, lfm_solver *const *hs, int n) {
             s->bc();
             s->ghosts_stale = false;
         }
+        if (int rc = s->ensure_keys(s->visc || s->prm.solver == 2)) return rc;
         HIP_TRY(hipStreamSynchronize(s->stream));
         b->members.push_back(s);
         args.push_back(*s->k32);

@@ -240,6 +240,8 @@ int lfm_part_group_create(lfm_solver *const *hs, int n, lfm_part_group **out) {
         if (p->fp32 != p0->fp32 || p->L.D != p0->L.D || p->prm.solver != p0->prm.solver ||
             p->prm.minmod != p0->prm.minmod || p->nstages != p0->nstages || p->prm.adjust_dt != p0->prm.adjust_dt)
             return fail(LFM_EINVAL, "partitions must share precision, dimension, scheme, rkOrder and adjustTimeStep");
+    for (Solver *p : parts)
+        if (int rc = p->ensure_keys(p->visc || p->prm.solver == 2)) return rc;
     auto g = std::make_unique<lfm_part_group>();
     g->parts = parts;
     g->adjust = p0->prm.adjust_dt != 0;

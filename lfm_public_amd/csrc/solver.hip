@@ -95,25 +95,45 @@ static int dev_zeros(Solver *s, T **dst, size_t n) {
     return s->dev_fill(*dst, nullptr, n * sizeof(T));
 }
 
-// the fixed-width gather entries of an argument block whose lists are on the
-// device (on the null stream, as the uploads of the set-up)
+// The fixed-width gather entries of an argument block whose lists are on the
+// device.  At set-up among its arrays (on the null stream, as the uploads);
+// later on the handle's stream, which is waited for (a batch or a group reads
+// them on its own).
 template <class Args>
-int Solver::build_gather_keys(Args &a, bool others) {
+int Solver::build_gather_keys(Args &a, bool others, bool setup) {
     const size_t n = keys_len(L.D, L.nc) * sizeof(int32_t);
-    void *key = nullptr, *oth = nullptr;
-    if (int rc = dev_alloc(&key, n)) return rc;
-    if (others)
-        if (int rc = dev_alloc(&oth, n)) return rc;
-    if (int rc = slab_flush()) return rc;
+    void *key = (void *)a.g_key, *oth = (void *)a.g_oth;
+    for (void **p : {&key, &oth}) {
+        if (*p || (p == &oth && !others)) continue;
+        if (setup) {
+            if (int rc = dev_alloc(p, n)) return rc;
+        } else if (!alloc_all(p, &n, 1)) {
+            return fail(LFM_EDEVICE, "no device memory for the gather entries");
+        }
+    }
+    if (setup)
+        if (int rc = slab_flush()) return rc;
     auto build = L.D == 2 ? build_keys<2> : build_keys<3>;
-    hipLaunchKernelGGL(build, dim3(nblocks(L.nc)), dim3(kBlock), 0, nullptr, L.nc, a.g_off, a.g_ent, a.fP, a.fN,
-                       (int32_t *)key, (int32_t *)oth);
+    hipLaunchKernelGGL(build, dim3(nblocks(L.nc)), dim3(kBlock), 0, setup ? nullptr : stream, L.nc, a.g_off, a.g_ent,
+                       a.fP, a.fN, (int32_t *)key, (int32_t *)oth);
     HIP_TRY(hipGetLastError());
+    if (!setup) HIP_TRY(hipStreamSynchronize(stream));
     a.g_key = (const int32_t *)key;
     a.g_oth = (const int32_t *)oth;
     return 0;
 }
-template int Solver::build_gather_keys<KArgs32>(KArgs32 &, bool);
+template int Solver::build_gather_keys<KArgs32>(KArgs32 &, bool, bool);
+
+int Solver::ensure_keys(bool others) {
+    const int32_t *key = fp32 ? k32->g_key : k64.g_key, *oth = fp32 ? k32->g_oth : k64.g_oth;
+    if (key && (oth || !others)) return LFM_OK;
+    return fp32 ? build_gather_keys(*k32, others, false) : build_gather_keys(k64, others, false);
+}
+
+int Solver::ensure_step_keys() {
+    if (nstages > 0 && fused_ok && ensure_alt() && fused_from() == 0) return LFM_OK;
+    return ensure_keys(visc || prm.solver == 2);
+}
 
 Solver::~Solver() {
     free_step_graph();
@@ -220,7 +240,7 @@ static int create_fp64(Solver *s) {
     // that walk the list
     s->fused_ok = !s->visc && s->prm.solver < 2 && L.halo.empty() && !own_neighbour(L);
     a.more_faces = max_entries(L) > (D == 2 ? GatherUnroll<2>::value : GatherUnroll<3>::value);
-    if (s->build_gather_keys(a, true)) return LFM_EDEVICE;
+    if (s->keys_at_setup() && s->build_gather_keys(a, s->visc || s->prm.solver == 2, true)) return LFM_EDEVICE;
     if (s->fused_ok) {
         // records in both orientations and a placeholder's fit above the
         // cell index; kMaxTable64 keeps the table in an XCD's L2
@@ -903,6 +923,8 @@ bool Solver::graph_build() {
 }
 
 int Solver::run_steps(int n, bool with_post) {
+    if (n > 0)
+        if (int rc = ensure_step_keys()) return rc;
     for (int i = 0; i < n;) {
         // the run's last step is never in the graph: it reduces its own CFL
         if (n - i > kGraphSteps && graph_ready()) {
@@ -1070,6 +1092,7 @@ int lfm_calc_gradients(lfm_solver *h) {
 int lfm_calc_vis(lfm_solver *h) {
     if (!h) return fail(LFM_EINVAL, "null handle");
     if (!h->impl->halo_ready()) return fail(LFM_ESTATE, "halo set-up not imported for every neighbour");
+    if (int rc = h->impl->ensure_keys(true)) return rc;
     h->impl->gradvis(true);
     HIP_TRY(hipGetLastError());
     return LFM_OK;
@@ -1080,6 +1103,7 @@ int lfm_one_rk_step(lfm_solver *h, int rk, double dt, double *res) {
     Solver *s = h->impl.get();
     if (rk < 0 || rk > 4) return fail(LFM_EINVAL, "rk stage out of range");
     if (!s->halo_ready()) return fail(LFM_ESTATE, "halo set-up not imported for every neighbour");
+    if (int rc = s->ensure_keys(false)) return rc;
     const double B = s->B[rk];
     // without adjustTimeStep nothing on the device writes its deltaT, which
     // is then the last one that was set there.  The value goes with the
@@ -1107,6 +1131,8 @@ int lfm_one_rk_step(lfm_solver *h, int rk, double dt, double *res) {
 int lfm_compute_dt(lfm_solver *h, double max_co, double *dt_out) {
     if (!h || !dt_out) return fail(LFM_EINVAL, "null argument");
     Solver *s = h->impl.get();
+    if (s->fp32)  // FP64 sums over the slot lists
+        if (int rc = s->ensure_keys(false)) return rc;
     s->cfl_dt(0, max_co, s->d_dtmin, s->h_scalar + 9);  // pinned: the kernel writes it there as well
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s->stream));
@@ -1117,6 +1143,8 @@ int lfm_compute_dt(lfm_solver *h, double max_co, double *dt_out) {
 int lfm_compute_cfl(lfm_solver *h, double dt, double *cfl_out) {
     if (!h || !cfl_out) return fail(LFM_EINVAL, "null argument");
     Solver *s = h->impl.get();
+    if (s->fp32)  // FP64 sums over the slot lists
+        if (int rc = s->ensure_keys(false)) return rc;
     s->cfl_dt(1, dt, s->d_cfl, s->h_scalar + 8);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s->stream));
@@ -1171,6 +1199,7 @@ int lfm_profile_steps(lfm_solver *h, int nsteps, double *ms_per_group, double *m
     if (!s->L.halo.empty())
         return fail(LFM_ESTATE, "a partition with processor patches steps through lfm_part_group_run or the "
                                 "per-stage calls with halo exchange");
+    if (int rc = s->ensure_step_keys()) return rc;
     const size_t need = (size_t)nsteps * (s->nstages * 8 + 2);
     for (hipEvent_t e : s->prof_ev) (void)hipEventDestroy(e);
     s->prof_ev.assign(need, nullptr);

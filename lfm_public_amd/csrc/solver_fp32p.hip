@@ -103,7 +103,6 @@ int create_fp32p(Solver *s) {
     }
     rc |= up(s, (int32_t **)&a.g_off, L.g_off.data(), nc + 1);
     rc |= up(s, (int32_t **)&a.g_ent, L.g_ent.data(), L.g_ent.size());
-    if (!rc) rc |= s->build_gather_keys(a, true);
     rc |= up(s, (int32_t **)&a.ghost_cell, L.ghost_cell.data(), L.ng);
     rc |= up(s, (int32_t **)&a.ghost_role, L.ghost_role.data(), L.ng);
     rc |= up(s, (double **)&a.vol_d, L.volume.data(), nc);
@@ -135,6 +134,7 @@ int create_fp32p(Solver *s) {
             s->table32 = face_table<float>(L, (int)std::min<long>(fit, kMaxTable32));
         }
     }
+    if (!rc && s->keys_at_setup()) rc |= s->build_gather_keys(a, s->visc || s->prm.solver == 2, true);
     rc |= up(s, &a.dq, (float *)nullptr, (size_t)(D + 2) * nc);
     rc |= up(s, &a.res_cell, (float *)nullptr, (size_t)(D + 2) * nc);
     // gradient records (GradRec32): dudx, dTdx and (M2AUSM) rho / p gradients

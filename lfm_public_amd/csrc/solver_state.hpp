@@ -61,8 +61,15 @@ struct Solver {
     int dev_alloc(void **p, size_t bytes);
     int dev_fill(void *p, const void *src, size_t bytes);  // src null: zeros
     int slab_flush();  // what was filled so far, before a kernel reads it
+    // The gather entries (g_key, and g_oth where gradients are formed).  A solver
+    // whose steps are one-launch stages reads neither: it gets them with the
+    // first call that does (per-stage calls, FP32 compute_dt / compute_cfl,
+    // separate launches of a batch or a group): 48 B per 3D cell, 32 per 2D cell.
     template <class Args>
-    int build_gather_keys(Args &a, bool others);
+    int build_gather_keys(Args &a, bool others, bool setup);
+    bool keys_at_setup() const { return !fused_ok || prm.have_res; }
+    int ensure_keys(bool others);
+    int ensure_step_keys();
     char *slab = nullptr;
     size_t slab_used = 0, slab_copied = 0;
     std::unique_ptr<char[]> slab_host;
