@@ -478,10 +478,14 @@ __device__ __forceinline__ void vis_tensors(const KArgs &a, const double (&dudx)
 // annulus, four 171, two 176 us per step), two in 3D at 3 waves per SIMD (193
 // k-cell O-grid: three spill and take 415, two 397, one 397) and, where the
 // stage outgrows the cache, all six at 2 (1 M cells 1400 -> 1351, 4.2 M 5983 ->
-// 5873).
+// 5873).  There the M1 / M2 gradients are one straight line of six faces: as the
+// body of the rolled loop, which is run once, the same faces take 8 % longer
+// (4.2 M cells, us of gradients per step: loop 1749, straight 1618; the loop with
+// the gather list 1850, straight with it 1684; 3 waves 2140).  With the M2AUSM
+// records the two are equal (1 M cells 574 / 574).
 template <int D, bool NT>
 constexpr int kGradGroup64 = D == 2 ? 4 : NT ? 6 : 2;
-template <int D, int GRAD, bool VISC, bool RG, bool NT>
+template <int D, int GRAD, bool VISC, bool RG, bool NT, bool RNT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGradGroup64<D, NT> == 6 ? 2 : 3))) grad_vis(KArgs a) {
     const int c = LFM_TID(blockIdx.x);
     using R = GradRec64<D, RG>;
@@ -565,11 +569,35 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGradG
     };
     // groups of G faces in gather order, their loads issued together
     constexpr int U = GatherUnroll<D>::value, G = kGradGroup64<D, NT>;
-    static_assert(U % G == 0);
+    constexpr bool kStraight = D == 3 && NT && !RG;
+    static_assert(U % G == 0 && (!kStraight || G == U));
     int key[G], oth[G], e0 = 0, ne = U;
     load_keys<D, NT>(a.g_key, a.nc, 0, c, key);
     load_keys<D, NT>(a.g_oth, a.nc, 0, c, oth);
-    if (a.more_faces) {
+    if constexpr (kStraight) {
+        double wj[G], Sj[G][D], qj[G][D + 2];
+#pragma unroll
+        for (int u = 0; u < G; u++) {
+            const int f = face_of(key[u]);
+            wj[u] = a.w[f];
+            load_S64<D>(a.S, f, Sj[u]);
+            load_q<D>(a, oth[u], qj[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < G; u++)
+            if (key[u] != kNoFace) add(key[u] >= 0, wj[u], Sj[u], qj[u]);
+        if (a.more_faces) {  // entries beyond the first U
+            const int e2 = a.g_off[c + 1];
+            for (int e = a.g_off[c] + U; e < e2; e++) {
+                const int ent = a.g_ent[e], f = face_of(ent);
+                double S1[D], q1[D + 2];
+                load_S64<D>(a.S, f, S1);
+                load_q<D>(a, ent >= 0 ? a.fN[f] : a.fP[f], q1);
+                add(ent >= 0, a.w[f], S1, q1);
+            }
+        }
+        ne = 0;
+    } else if (a.more_faces) {
         e0 = a.g_off[c];
         ne = max(U, a.g_off[c + 1] - e0);
     }
@@ -648,8 +676,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGradG
         // annulus 171 against 174 us per step); otherwise the records of 16
         // cells at a time, written as consecutive words (64-byte runs wrote
         // 540 MB where the records of a 4.2 M-cell O-grid are 403).  The face
-        // launch reads the records next: plain stores (1 M-cell annulus 802
-        // against 828 us per step non-temporal, 2.1 M 1627 against 1607).
+        // launch reads the records next: non-temporal stores only where they
+        // outgrow what the Infinity Cache keeps for it (RNT, from 190 MB; MB of
+        // records, us per step plain / non-temporal: M1 / M2 O-grid 101 MB 1312 /
+        // 1366, 201 2810 / 2790, 403 5691 / 5611; M2AUSM 117 970 / 1010, 176 1459 /
+        // 1485, 235 1993 / 1947; annulus 117 801 / 834, 235 1613 / 1602).
         // Staging whole blocks (57 KB for 3D M2AUSM) held the kernel at 2 waves
         // per SIMD; without minmod the rho / p / U slots are written zero.
         constexpr bool kRuns = D == 2 && !NT;
@@ -684,7 +715,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGradG
 #pragma unroll
                 for (int j = lane; j < M * W; j += 64) {
                     const double2 v = st[j];
-                    if (j < n) st_once<false>(dst + g * M * W + j, d2v{v.x, v.y});
+                    if (j < n) st_once<RNT>(dst + g * M * W + j, d2v{v.x, v.y});
                 }
                 wave_sync_lds();
             }
@@ -1236,7 +1267,10 @@ __global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, 
         load_dq64<D, NT>(a, dq_mode, c, dq);
 #pragma unroll
         for (int k = 0; k < D + 2; k++) res[k] = 0.0;
-        load_q<D>(a, c, q);
+        // in 3D the state is asked for after the fluxes, which it would only queue
+        // before (O-grid, us of updates per step with it first / last: 4.2 M cells
+        // 1530 / 1477, 1 M 381 / 368, 193 k 84 / 81)
+        if constexpr (D == 2) load_q<D>(a, c, q);
         constexpr int U = GatherUnroll<D>::value;
         int key[U];
         load_keys<D, NT>(a.g_key, a.nc, 0, c, key);
@@ -1278,6 +1312,7 @@ __global__ void __launch_bounds__(256) cell_update(KArgs a, double A, double B, 
                 add(U + j, ent, f1);
             }
         }
+        if constexpr (D == 3) load_q<D>(a, c, q);
         if (a.sigma) sponge64<D, NT>(a, c, dt, q, dq);
 #pragma unroll
         for (int k = 0; k < D + 2; k++) q[k] += B * dq[k];

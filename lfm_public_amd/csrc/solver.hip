@@ -259,20 +259,22 @@ static void launch_bc64(Solver *s) {
     if (s->L.ng) launch(s, bc_fill<D>, dim3(nblocks(s->L.ng)), dim3(kBlock), s->k64);
 }
 
-template <int D, bool V, bool NT>
+template <int D, bool V, bool NT, bool RNT>
 static void launch_gradvis64_nt(Solver *s) {
     const int nb = nblocks(s->L.nc);
     if (s->prm.solver == 2 && s->prm.minmod)
-        launch(s, (grad_vis<D, 2, V, true, NT>), dim3(nb), dim3(kBlock), s->k64);
+        launch(s, (grad_vis<D, 2, V, true, NT, RNT>), dim3(nb), dim3(kBlock), s->k64);
     else if (s->prm.solver == 2)
-        launch(s, (grad_vis<D, 0, V, true, NT>), dim3(nb), dim3(kBlock), s->k64);
+        launch(s, (grad_vis<D, 0, V, true, NT, RNT>), dim3(nb), dim3(kBlock), s->k64);
     else
-        launch(s, (grad_vis<D, 0, V, false, NT>), dim3(nb), dim3(kBlock), s->k64);
+        launch(s, (grad_vis<D, 0, V, false, NT, RNT>), dim3(nb), dim3(kBlock), s->k64);
 }
 
 template <int D, bool V>
 static void launch_gradvis64_v(Solver *s) {
-    s->stream_nt ? launch_gradvis64_nt<D, V, true>(s) : launch_gradvis64_nt<D, V, false>(s);
+    if constexpr (V)  // without viscosity the records are not written whole
+        if (s->records_nt) return launch_gradvis64_nt<D, V, true, true>(s);
+    s->stream_nt ? launch_gradvis64_nt<D, V, true, false>(s) : launch_gradvis64_nt<D, V, false, false>(s);
 }
 
 // full: every tensor calc_VIS forms (the per-stage entry point); otherwise
@@ -625,6 +627,7 @@ void Solver::size_stage() {
     if (visc || prm.solver == 2) sh.grad_values = fp32 ? k32->gstride : k64.gstride;
     stage_bytes = stage_footprint(sh);
     stream_nt = outgrows_cache(stage_bytes);
+    records_nt = stream_nt && sh.nc * sh.grad_values * sh.word > (size_t)190 * 1000 * 1000;
 }
 
 bool Solver::alloc_all(void **p, const size_t *bytes, int n) {

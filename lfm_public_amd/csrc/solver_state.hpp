@@ -187,6 +187,7 @@ struct Solver {
     // its kernels stream what they touch once past the caches
     size_t stage_bytes = 0;
     bool stream_nt = false;
+    bool records_nt = false;  // the FP64 gradient records alone do not stay in it
     void size_stage();
     bool sym64 = false;  // every record's weights allow flux_m1_sym
     // device memory for a set of arrays of one kind, all or none
