@@ -73,11 +73,11 @@ template <int D, int SOLVER, bool NT>
 static void enqueue_fused(Batch *b, int rk, int flip) {
     const dim3 blk(256);
     if (rk == b->nstages - 1)
-        launch(b, (stage_fused32_b<D, SOLVER, 1, NT>), dim3(b->nb_cells), blk, b->d_args,
-                           b->map_cells, (float)b->A[rk], (float)b->B[rk], b->dq_mode(rk), flip);
+        launch(b, (stage_fused32_b<D, SOLVER, 1, NT>), dim3(b->nb_cells), blk, b->d_args, b->map_cells, (float)b->A[rk],
+               (float)b->B[rk], b->dq_mode(rk), flip);
     else
-        launch(b, (stage_fused32_b<D, SOLVER, -1, NT>), dim3(b->nb_cells), blk, b->d_args,
-                           b->map_cells, (float)b->A[rk], (float)b->B[rk], b->dq_mode(rk), flip);
+        launch(b, (stage_fused32_b<D, SOLVER, -1, NT>), dim3(b->nb_cells), blk, b->d_args, b->map_cells,
+               (float)b->A[rk], (float)b->B[rk], b->dq_mode(rk), flip);
 }
 
 template <int D, bool V, bool NT>
@@ -93,14 +93,11 @@ static void enqueue_step_nt(Batch *b) {
         // without viscosity solvers 0/1 consume no gradient or tensor
         if (V || b->solver == 2) {
             if (b->solver == 2 && b->minmod)
-                launch(b, (grad_vis32_b<D, 2, V, true, NT>), dim3(b->nb_cells), blk, b->d_args,
-                                   b->map_cells);
+                launch(b, (grad_vis32_b<D, 2, V, true, NT>), dim3(b->nb_cells), blk, b->d_args, b->map_cells);
             else if (b->solver == 2)
-                launch(b, (grad_vis32_b<D, 0, V, true, NT>), dim3(b->nb_cells), blk, b->d_args,
-                                   b->map_cells);
+                launch(b, (grad_vis32_b<D, 0, V, true, NT>), dim3(b->nb_cells), blk, b->d_args, b->map_cells);
             else
-                launch(b, (grad_vis32_b<D, 0, V, false, NT>), dim3(b->nb_cells), blk, b->d_args,
-                                   b->map_cells);
+                launch(b, (grad_vis32_b<D, 0, V, false, NT>), dim3(b->nb_cells), blk, b->d_args, b->map_cells);
         }
         switch (b->solver) {
         case 0: launch(b, (face_flux32_b<D, 0, V, NT>), dim3(b->nb_faces), blk, b->d_args, b->map_faces); break;
@@ -109,11 +106,11 @@ static void enqueue_step_nt(Batch *b) {
         }
         // the last stage's update also forms the step's compute_cfl partials
         if (rk == b->nstages - 1)
-            launch(b, (cell_update32_b<D, 1, NT>), dim3(b->nb_cells), blk, b->d_args,
-                               b->map_cells, (float)b->A[rk], (float)b->B[rk], b->dq_mode(rk));
+            launch(b, (cell_update32_b<D, 1, NT>), dim3(b->nb_cells), blk, b->d_args, b->map_cells, (float)b->A[rk],
+                   (float)b->B[rk], b->dq_mode(rk));
         else
-            launch(b, (cell_update32_b<D, -1, NT>), dim3(b->nb_cells), blk, b->d_args,
-                               b->map_cells, (float)b->A[rk], (float)b->B[rk], b->dq_mode(rk));
+            launch(b, (cell_update32_b<D, -1, NT>), dim3(b->nb_cells), blk, b->d_args, b->map_cells, (float)b->A[rk],
+                   (float)b->B[rk], b->dq_mode(rk));
     }
     launch(b, cfl_final32_b, dim3((unsigned)b->members.size()), blk, b->d_args);
 }

@@ -215,7 +215,6 @@ inline int grad_record_stride64(int D, bool rg) {
     return (n + 1) / 2 * 2;
 }
 
-// face flux record: components 0-3 as 32 bytes per face, component 4 after
 // Gather entries of fixed width.  A kernel that walks the gather list waits for
 // the list's offsets, then the entry, then (gradients) the face's cells before
 // it can ask for the other cell's state; from these arrays the face's data and
@@ -270,6 +269,7 @@ __global__ void __launch_bounds__(256) build_keys(int nc, const int32_t *g_off, 
     }
 }
 
+// face flux record: components 0-3 as 32 bytes per face, component 4 after
 template <int D>
 __device__ __forceinline__ void load_frhs(const KArgs &a, int f, double (&r)[D + 2]) {
     const double2 *p = reinterpret_cast<const double2 *>(a.frhs + 4 * (size_t)f);

@@ -315,19 +315,14 @@ static void launch_update64_nt(Solver *s, double A, double B, int dq_mode, bool 
                                const Solver::CflJob *cfl) {
     const int nb = nblocks(s->L.nc);
     if (res) {
-        launch(s, (cell_update<D, true, -1, NT>), dim3(nb), dim3(kBlock), s->k64, A, B,
-                           dq_mode, 0.0);
-        launch(s, reduce_sum, dim3(1), dim3(kBlock), s->k64.partial, nb, D + 2, s->d_res,
-                           (int)accumulate_res);
+        launch(s, (cell_update<D, true, -1, NT>), dim3(nb), dim3(kBlock), s->k64, A, B, dq_mode, 0.0);
+        launch(s, reduce_sum, dim3(1), dim3(kBlock), s->k64.partial, nb, D + 2, s->d_res, (int)accumulate_res);
     } else if (cfl && cfl->mode == 0) {
-        launch(s, (cell_update<D, false, 0, NT>), dim3(nb), dim3(kBlock), s->k64, A, B,
-                           dq_mode, cfl->param);
+        launch(s, (cell_update<D, false, 0, NT>), dim3(nb), dim3(kBlock), s->k64, A, B, dq_mode, cfl->param);
     } else if (cfl) {
-        launch(s, (cell_update<D, false, 1, NT>), dim3(nb), dim3(kBlock), s->k64, A, B,
-                           dq_mode, cfl->param);
+        launch(s, (cell_update<D, false, 1, NT>), dim3(nb), dim3(kBlock), s->k64, A, B, dq_mode, cfl->param);
     } else {
-        launch(s, (cell_update<D, false, -1, NT>), dim3(nb), dim3(kBlock), s->k64, A, B,
-                           dq_mode, 0.0);
+        launch(s, (cell_update<D, false, -1, NT>), dim3(nb), dim3(kBlock), s->k64, A, B, dq_mode, 0.0);
     }
 }
 
@@ -365,14 +360,14 @@ static void launch_fused64_nt(Solver *s, double A, double B, int dq_mode, const 
                              const Solver::CflJob *cfl, bool fin) {
     const int nb = nblocks(s->L.nc);
     if (!cfl)
-        launch(s, (stage_fused64<D, SOLVER, -1, PK, SYM, NT>), dim3(nb + (fin ? 1 : 0)), dim3(kBlock), a,
-                           qout, A, B, dq_mode, 0.0, fin ? nb : 0, s->d_cfl);
+        launch(s, (stage_fused64<D, SOLVER, -1, PK, SYM, NT>), dim3(nb + (fin ? 1 : 0)), dim3(kBlock), a, qout, A, B,
+               dq_mode, 0.0, fin ? nb : 0, s->d_cfl);
     else if (cfl->mode == 0)
-        launch(s, (stage_fused64<D, SOLVER, 0, PK, SYM, NT>), dim3(nb), dim3(kBlock), a, qout, A, B,
-                           dq_mode, cfl->param, 0, s->d_cfl);
+        launch(s, (stage_fused64<D, SOLVER, 0, PK, SYM, NT>), dim3(nb), dim3(kBlock), a, qout, A, B, dq_mode,
+               cfl->param, 0, s->d_cfl);
     else
-        launch(s, (stage_fused64<D, SOLVER, 1, PK, SYM, NT>), dim3(nb), dim3(kBlock), a, qout, A, B,
-                           dq_mode, cfl->param, 0, s->d_cfl);
+        launch(s, (stage_fused64<D, SOLVER, 1, PK, SYM, NT>), dim3(nb), dim3(kBlock), a, qout, A, B, dq_mode,
+               cfl->param, 0, s->d_cfl);
 }
 
 template <int D, int SOLVER, bool PK, bool SYM>
@@ -451,11 +446,9 @@ void Solver::update(double A, double B, int dq_mode, bool res, bool accumulate_r
 void Solver::cfl_final(const CflJob &job) {
     const int nb = nblocks(L.nc);
     if (job.mode == 0)
-        launch(this, cfl_dt_final<0>, dim3(1), dim3(kFinalBlock), k64.partial, nb, job.out,
-                           job.dt_dst);
+        launch(this, cfl_dt_final<0>, dim3(1), dim3(kFinalBlock), k64.partial, nb, job.out, job.dt_dst);
     else
-        launch(this, cfl_dt_final<1>, dim3(1), dim3(kFinalBlock), k64.partial, nb, job.out,
-                           job.dt_dst);
+        launch(this, cfl_dt_final<1>, dim3(1), dim3(kFinalBlock), k64.partial, nb, job.out, job.dt_dst);
 }
 
 void Solver::cfl_dt(int mode, double param, double *out, double *dt_dst) {

@@ -258,19 +258,18 @@ static void launch_update32_nt(Solver *s, double A, double B, int dq_mode, bool 
                                const Solver::CflJob *cfl) {
     const int nb = nblocks(s->L.nc);
     if (res) {
-        launch(s, (cell_update32<D, true, -1, NT, MORE>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
-                           (float)B, dq_mode, 0.0);
-        launch(s, reduce_sum, dim3(1), dim3(kBlock), s->k32->partial, nb, D + 2, s->d_res,
-                           (int)accumulate_res);
+        launch(s, (cell_update32<D, true, -1, NT, MORE>), dim3(nb), dim3(kBlock), *s->k32, (float)A, (float)B, dq_mode,
+               0.0);
+        launch(s, reduce_sum, dim3(1), dim3(kBlock), s->k32->partial, nb, D + 2, s->d_res, (int)accumulate_res);
     } else if (cfl && cfl->mode == 0) {
-        launch(s, (cell_update32<D, false, 0, NT, MORE>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
-                           (float)B, dq_mode, cfl->param);
+        launch(s, (cell_update32<D, false, 0, NT, MORE>), dim3(nb), dim3(kBlock), *s->k32, (float)A, (float)B, dq_mode,
+               cfl->param);
     } else if (cfl) {
-        launch(s, (cell_update32<D, false, 1, NT, MORE>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
-                           (float)B, dq_mode, cfl->param);
+        launch(s, (cell_update32<D, false, 1, NT, MORE>), dim3(nb), dim3(kBlock), *s->k32, (float)A, (float)B, dq_mode,
+               cfl->param);
     } else {
-        launch(s, (cell_update32<D, false, -1, NT, MORE>), dim3(nb), dim3(kBlock), *s->k32, (float)A,
-                           (float)B, dq_mode, 0.0);
+        launch(s, (cell_update32<D, false, -1, NT, MORE>), dim3(nb), dim3(kBlock), *s->k32, (float)A, (float)B, dq_mode,
+               0.0);
     }
 }
 
@@ -290,16 +289,16 @@ static void launch_fused32_nt(Solver *s, float A, float B, int dq_mode, const KA
                              const Solver::CflJob *cfl, bool fin) {
     const int nb = nblocks(s->L.nc);
     if (!cfl) {
-        launch(s, (stage_fused32<D, SOLVER, -1, PK, HALF, NT>), dim3(nb + (fin ? 1 : 0)), dim3(kBlock), a,
-                           qout, A, B, dq_mode, 0.0, fin ? nb : 0);
+        launch(s, (stage_fused32<D, SOLVER, -1, PK, HALF, NT>), dim3(nb + (fin ? 1 : 0)), dim3(kBlock), a, qout, A, B,
+               dq_mode, 0.0, fin ? nb : 0);
         return;
     }
     if (cfl->mode == 0)
-        launch(s, (stage_fused32<D, SOLVER, 0, PK, HALF, NT>), dim3(nb), dim3(kBlock), a, qout, A, B,
-                           dq_mode, cfl->param, 0);
+        launch(s, (stage_fused32<D, SOLVER, 0, PK, HALF, NT>), dim3(nb), dim3(kBlock), a, qout, A, B, dq_mode,
+               cfl->param, 0);
     else
-        launch(s, (stage_fused32<D, SOLVER, 1, PK, HALF, NT>), dim3(nb), dim3(kBlock), a, qout, A, B,
-                           dq_mode, cfl->param, 0);
+        launch(s, (stage_fused32<D, SOLVER, 1, PK, HALF, NT>), dim3(nb), dim3(kBlock), a, qout, A, B, dq_mode,
+               cfl->param, 0);
 }
 
 template <int D, int SOLVER, bool PK, bool HALF>

@@ -19,7 +19,23 @@ def _ogrid(nz, **kw):
     return cases.cylinder_3d(nr=96, nth=96, nz=nz, pert=0.05, **kw)
 
 
-# cells: what a stage touches is past 330 MB from 0.4 M (FP64 3D M2AUSM) to 0.9 M
+def _past_the_line(s, grad_values, word):
+    """The stage's bytes, each array once (tests/test_stage_footprint.py)."""
+    i = s.info()
+    D = i.dim
+    cell = (2 * (D + 2) + 2) * word + 2 * 4 * (4 if D == 2 else 6) + grad_values * word
+    return i.n_cells * cell + i.n_faces * ((3 * D + 3) * word + 8) > 330e6
+
+
+# values of a gradient record: dudx, dTdx, with M2AUSM rho and p (FP64 also U)
+RECORD = {(64, 2): 14, (64, 3): 28, (32, 2): 10, (32, 3): 18}
+
+
+def _record(c, prec):
+    D = c.params["dim"]
+    return RECORD[prec, D] if c.params["solver"] == 2 else D * D + D
+
+
 FP64 = {
     "ogrid_M2AUSM": lambda: _ogrid(56, solver=2, minmod=1),
     "ogrid_M2AUSM_nominmod": lambda: _ogrid(56, solver=2, minmod=0),
@@ -32,7 +48,7 @@ FP32 = {
     "ogrid_M1": lambda: _ogrid(129, solver=0, minmod=0),
     # packed slots
     "box_M2_visc": lambda: cases.acoustic_box(n=106, solver=1, mu=1e-3, amp=1e-2),
-    "poly_M2AUSM": lambda: sc.poly(nx=1100, ny=900, solver=2, mu=0.02, minmod=1),
+    "poly_M2AUSM": lambda: sc.poly(nx=1200, ny=900, solver=2, mu=0.02, minmod=1),
 }
 
 
@@ -41,6 +57,7 @@ def test_fp64_past_the_cache_matches_oracle(name, oracle_lib):
     c = FP64[name]()
     print(f"[marked] FP64 {name} {c.n_cells} cells", flush=True)
     g, o = _pair(c, oracle_lib)
+    assert _past_the_line(g, _record(c, 64), 8)
     g.run(1)
     o.run(1)
     assert np.all(np.isfinite(o.q()))
@@ -55,6 +72,7 @@ def test_fp32_past_the_cache_matches_fp64(name):
     c = FP32[name]()
     print(f"[marked] FP32 {name} {c.n_cells} cells", flush=True)
     g, f = (capi.GpuSolver.from_case(c, precision=p) for p in (capi.PREC_FP64, capi.PREC_FP32P))
+    assert _past_the_line(f, _record(c, 32), 4)
     for s in (g, f):
         s.run(1)
     for k, v in _errors(c, f.q(), g.q()).items():
