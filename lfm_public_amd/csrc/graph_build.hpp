@@ -12,8 +12,8 @@ namespace lfm {
 // A chain of kernel nodes.  The launches of a step become nodes here instead of
 // being captured from the stream: a synchronous copy on any other thread of the
 // process (another handle's set_field, or the program's own code) invalidates
-// an open capture, also one of thread-local mode, and every later call on the
-// capturing stream then fails.
+// an open capture, also one of thread-local mode, and the launches that follow on
+// that stream fail.
 struct GraphBuild {
     hipGraph_t graph = nullptr;
     hipGraphNode_t last = nullptr;
